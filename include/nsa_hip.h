@@ -252,6 +252,14 @@ int nsa_rmsnorm_fwd(int64_t rows, int32_t dim, const void* x, int64_t x_row_stri
 int nsa_rmsnorm_bwd(int64_t rows, int32_t dim, const void* x, int64_t x_row_stride, const void* weight, const float* rstd,
                     const void* dy, void* dx, void* dweight, int32_t dweight_fp32, float* partials, void* stream);
 
+/* Projection of a few rows: y[r] = norm(x[r]) weight^T + bias for rows <= 32, the shape of a decode step (one token per
+ * sequence: NSA.py:356-364, 545).  x: bf16 [rows, k], row stride x_row_stride; weight: bf16 [n, k] contiguous; bias
+ * (optional): bf16 [n]; y: bf16 [rows, n].  norm_weight (optional, bf16 [k]): x is RMS-normed first, as nsa_rmsnorm_fwd does
+ * (rounded to bf16 before the product).  k a multiple of 32, rows * (k + 8) <= 65536 (NSA_E_UNSUPPORTED otherwise), rows
+ * 16-byte aligned. */
+int nsa_skinny_linear(int32_t rows, int32_t k, int32_t n, const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
+                      const void* weight, const void* bias, void* y, int64_t y_row_stride, void* stream);
+
 /* Column sums of a bf16 matrix in fp32: the bias gradient of a projection (the sum of d_out over tokens that
  * autograd takes for the nn.Linear layers of NSA.py:244-262, 853) and the gradient of the intra-window positions
  * (the sum of the window gradients over batch and windows, NSA.py:599-600).  Row (o, i) of group g starts at

@@ -94,6 +94,8 @@ def lib():
         L.nsa_topk.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         L.nsa_topk_prefix.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         fp = C.POINTER(C.c_float)
+        L.nsa_skinny_linear.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, C.c_float, vp, vp, vp, C.c_int64, vp]
+        L.nsa_skinny_linear.restype = C.c_int
         L.nsa_rmsnorm_partials.argtypes = [C.c_int64]
         L.nsa_rmsnorm_fwd.argtypes = [C.c_int64, C.c_int32, vp, C.c_int64, vp, C.c_float, vp, vp, vp]
         L.nsa_rmsnorm_bwd.argtypes = [C.c_int64, C.c_int32, vp, C.c_int64, vp, vp, vp, vp, vp, C.c_int32, vp, vp]

@@ -4,10 +4,11 @@
 `SparseAttention.forward_inference` (NSA.py:338-547) derives every shape of a step on the host and
 issues about a dozen launches; at small batch the host-side work is several times the kernels' run
 time.  A `DecodeSession` owns fixed-capacity caches, keeps the token position and the number of
-compressed keys in device memory (the kernels read them when they run, `nsa_decode_step_dyn`) and
-records norm, projections, the attention step and the output projection into a HIP graph that is
-replayed for every token.  Every `compress_block_sliding_stride` tokens a compression window is
-complete (NSA.py:422-441); those steps replay a second graph that also gathers the window (rows
+compressed keys in device memory (the kernels read them when they run, `nsa_decode_step_dyn`), so a
+step's calls have the same arguments for every token: they are prepared once, five launches through
+three library calls (`direct`), or, for modules or batches those kernels do not serve, recorded into
+a HIP graph that is replayed.  Every `compress_block_sliding_stride` tokens a compression window is
+complete (NSA.py:422-441); those steps also replay a graph that gathers the window (rows
 indexed from the device-side position), compresses it and appends the compressed key / value.
 
     out, cache = attn(prompt, return_cache=True)           # prefill, as in the reference
@@ -26,7 +27,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from .ops import _kernel_dim, _pad_dim
+from .ops import _kernel_dim, _pad_dim, rms_norm_supported, skinny_linear, skinny_linear_supported
 
 _BF16 = torch.bfloat16
 
@@ -115,7 +116,19 @@ class DecodeSession:
         else:                                                       # a caller-supplied strategy network runs as it is
             self.w_cat, self.gate_bias = w_qkv.contiguous(), None
         self.x_buf = torch.zeros((b, 1, m.to_qkv.in_features), dtype=_BF16, device=dev)
+        # The projections as this library's kernels for a few rows, with the module's norm (an nn.RMSNorm of the model dimension)
+        # inside the first: both unhooked layers of the default kind
+        norm, out = m.norm, m.combine_heads
+        self.own_norm = (m._plain(norm, torch.nn.RMSNorm) and tuple(norm.normalized_shape) == (m.to_qkv.in_features,)
+                         and rms_norm_supported(self.x_buf, norm.weight))
+        self.own_in = skinny_linear_supported(self.x_buf, self.w_cat) and self.fused_gate and m.to_qkv.bias is None
+        merged = torch.empty((b, 1, m.heads * d), dtype=_BF16, device=dev)
+        self.own_out = m._plain(out, torch.nn.Linear) and out.weight.dtype == _BF16 and skinny_linear_supported(merged, out.weight)
         self._desc, self._ws = self._make_desc(dev)
+        # Direct steps pay where their launches take the host less time than the GPU: with this library's kernels always (five
+        # launches, ~35 us), with the GEMM library's (~20 us of host time each) when the weights are what takes time
+        self.direct = self.own_norm and self.fused_gate and m._plain(out, torch.nn.Linear) and m.to_qkv.bias is None and (
+            (self.own_in and self.own_out) or self.w_cat.numel() * 2 >= 32 << 20)
         self.graphs = None
         if capture:
             # the libraries initialise themselves on first use (outside the capture); the warm-up steps write row `pos` of
@@ -127,15 +140,22 @@ class DecodeSession:
                     self.layer_step(self.x_buf, advance=0)
                     self.compress_window(count=False)
             torch.cuda.current_stream(dev).wait_stream(side)
+            # [0]: ordinary step, [1]: step that completes a window.  A direct step reads the caller's token and writes a new
+            # result itself (recorded, it would need a copy of the token into a fixed buffer and one of the result out of
+            # another, each a launch like the other five): of its second graph only the window is recorded
             self.graphs, self.outs = [], []
-            for event in (False, True):                             # [0]: ordinary step, [1]: step that completes a window
+            for event in (False, True):
                 g = torch.cuda.CUDAGraph()
+                out = None
                 with torch.no_grad(), torch.cuda.graph(g):
-                    out = self.layer_step(self.x_buf, advance=1)
+                    if not (self.direct and event):
+                        out = self.layer_step(self.x_buf, advance=1)
                     if event:
                         self.compress_window()
                 self.graphs.append(g)
                 self.outs.append(out)
+            if self.direct:
+                self._prepare_direct(merged)
 
     # ---------------------------------------------------------------------------------------
 
@@ -167,26 +187,68 @@ class DecodeSession:
         """The layer's decode step on `x_in` 'b 1 dim' as a sequence of launches with no host-side dependence on the
         position (recordable into a graph); advance != 0 increments the device-side position afterwards."""
         m = self.module
-        x = m.norm(x_in)
-        qkvg = torch.nn.functional.linear(x, self.w_cat)             # 'b 1 ((hq + 2 hk) d + 3 hq)', contiguous
         hq, hk, d = self.hq, self.hk, self.d
-        merged = torch.empty((self.b, 1, hq * d), dtype=_BF16, device=x.device)
-        p = qkvg.data_ptr()
-        if self.fused_gate:
-            gate_ptr, gate_row = p + 2 * (hq + 2 * hk) * d, qkvg.shape[-1]
+        if self.own_in and self.own_norm:
+            qkvg = skinny_linear(x_in, self.w_cat, None, m.norm.weight, self._eps())
         else:
-            gl = m.to_strategy_combine[0](x).to(_BF16).contiguous()
-            gate_ptr, gate_row = gl.data_ptr(), 0
-        _lib.check(_lib.lib().nsa_decode_step_dyn(
-            C.byref(self._desc), self.state.data_ptr(), p, p + 2 * hq * d, p + 2 * (hq + hk) * d, self.freqs.data_ptr(),
-            self.K.data_ptr(), self.V.data_ptr(), self.CK.data_ptr(), self.CV.data_ptr(), self.mem_k.data_ptr(), self.mem_v.data_ptr(),
-            self.ring_k.data_ptr(), self.ring_v.data_ptr(), self.ring_k.stride(2), self.ring_v.stride(2), self.ring,
-            gate_ptr, gate_row, self.gate_bias.data_ptr() if self.gate_bias is not None else None,
-            self._ws.data_ptr(), self._ws.numel(), merged.data_ptr(), int(advance),
-            torch.cuda.current_stream(x.device).cuda_stream), "nsa_decode_step_dyn")
-        if self.w_out is not None:
-            return torch.nn.functional.linear(merged, self.w_out, m.combine_heads.bias)
-        return m.combine_heads(merged)
+            x = m.norm(x_in)
+            qkvg = torch.nn.functional.linear(x, self.w_cat)         # 'b 1 ((hq + 2 hk) d + 3 hq)', contiguous
+        merged = torch.empty((self.b, 1, hq * d), dtype=_BF16, device=qkvg.device)
+        gl = qkvg if self.fused_gate else m.to_strategy_combine[0](x).to(_BF16).contiguous()
+        _lib.check(_lib.lib().nsa_decode_step_dyn(*self._step_args(qkvg, gl, merged, advance),
+                                                  torch.cuda.current_stream(qkvg.device).cuda_stream), "nsa_decode_step_dyn")
+        w_out = self.w_out if self.w_out is not None else m.combine_heads.weight
+        if self.own_out:
+            return skinny_linear(merged, w_out, m.combine_heads.bias)
+        return m.combine_heads(merged) if self.w_out is None else torch.nn.functional.linear(merged, w_out, m.combine_heads.bias)
+
+    def _eps(self) -> float:
+        eps = self.module.norm.eps
+        return torch.finfo(torch.float32).eps if eps is None else eps      # as the library's kernel takes it for a bf16 input
+
+    def _step_args(self, qkvg, gl, merged, advance):
+        """Arguments of nsa_decode_step_dyn up to the stream; `gl`: the gate logits' tensor (qkvg itself: its last columns)."""
+        hq, hk, d = self.hq, self.hk, self.d
+        p = qkvg.data_ptr()
+        gate_ptr, gate_row = (p + 2 * (hq + 2 * hk) * d, qkvg.shape[-1]) if gl is qkvg else (gl.data_ptr(), 0)
+        return (C.byref(self._desc), self.state.data_ptr(), p, p + 2 * hq * d, p + 2 * (hq + hk) * d, self.freqs.data_ptr(),
+                self.K.data_ptr(), self.V.data_ptr(), self.CK.data_ptr(), self.CV.data_ptr(), self.mem_k.data_ptr(), self.mem_v.data_ptr(),
+                self.ring_k.data_ptr(), self.ring_v.data_ptr(), self.ring_k.stride(2), self.ring_v.stride(2), self.ring,
+                gate_ptr, gate_row, self.gate_bias.data_ptr() if self.gate_bias is not None else None,
+                self._ws.data_ptr(), self._ws.numel(), merged.data_ptr(), int(advance))
+
+    def _prepare_direct(self, merged):
+        """The arguments of a direct step that do not change from token to token, converted once."""
+        qkvg = torch.empty((self.b, 1, self.w_cat.shape[0]), dtype=_BF16, device=merged.device)
+        rstd = torch.empty((self.b,), dtype=torch.float32, device=merged.device)
+        self._direct_bufs = (qkvg, merged, rstd)
+        fn = _lib.lib().nsa_decode_step_dyn
+        self._direct_args = tuple(a if not isinstance(a, (int, type(None))) else t(a) for a, t in zip(self._step_args(qkvg, qkvg, merged, 1), fn.argtypes))
+
+    def _step_direct(self, x: torch.Tensor) -> torch.Tensor:
+        m, L = self.module, _lib.lib()
+        qkvg, merged, rstd = self._direct_bufs
+        if x.dtype != _BF16 or x.shape != self.x_buf.shape or not x.is_contiguous() or x.data_ptr() % 16 or x.device != merged.device:
+            x = x.to(device=merged.device, dtype=_BF16).reshape(self.x_buf.shape).clone(memory_format=torch.contiguous_format)
+        st = torch.cuda.current_stream(merged.device).cuda_stream
+        b, dim = self.b, x.shape[-1]
+        w_out = self.w_out if self.w_out is not None else m.combine_heads.weight
+        bias = m.combine_heads.bias
+        if self.own_in:
+            rc = L.nsa_skinny_linear(b, dim, qkvg.shape[-1], x.data_ptr(), dim, m.norm.weight.data_ptr(), self._eps(), self.w_cat.data_ptr(), None,
+                                     qkvg.data_ptr(), qkvg.shape[-1], st)
+        else:
+            rc = L.nsa_rmsnorm_fwd(b, dim, x.data_ptr(), dim, m.norm.weight.data_ptr(), self._eps(), self.x_buf.data_ptr(), rstd.data_ptr(), st)
+            torch.mm(self.x_buf.view(b, dim), self.w_cat.t(), out=qkvg.view(b, -1))
+        rc = rc or L.nsa_decode_step_dyn(*self._direct_args, st)
+        if self.own_out:
+            y = torch.empty_like(x)
+            rc = rc or L.nsa_skinny_linear(b, merged.shape[-1], dim, merged.data_ptr(), merged.shape[-1], None, 0.0, w_out.data_ptr(),
+                                           None if bias is None else bias.data_ptr(), y.data_ptr(), dim, st)
+        else:
+            y = torch.nn.functional.linear(merged, w_out, bias)
+        _lib.check(rc, "decode step")
+        return y
 
     def compress_window(self, count: bool = True):
         """Compress the window that ends at the device-side position (already advanced past the newest token) and append it
@@ -212,12 +274,18 @@ class DecodeSession:
 
     @torch.no_grad()
     def step(self, x: torch.Tensor) -> torch.Tensor:
-        """x 'b 1 dim': the token at position `self.pos`.  Returns the layer output 'b 1 dim' (a new tensor)."""
+        """x 'b 1 dim' on the session's device: the token at position `self.pos`.  Returns the layer output 'b 1 dim' (a new tensor)."""
         if self.graphs is None:
             raise RuntimeError("DecodeSession was built with capture=False (its launches belong to an enclosing graph)")
         if self.pos >= self.max_len:
             raise RuntimeError(f"DecodeSession: capacity of {self.max_len} tokens reached")
         event = self.completes_window()
+        if self.direct:
+            out = self._step_direct(x)
+            if event:
+                self.graphs[1].replay()
+            self.advance_host(event)
+            return out
         self.x_buf.copy_(x)
         self.graphs[event].replay()
         self.advance_host(event)

@@ -1486,6 +1486,25 @@ def rms_norm(x: Tensor, weight: Tensor, eps: float | None = None) -> Tensor:
 
 # ------------------------------------------------------------------ projections
 
+def skinny_linear_supported(x: Tensor, weight: Tensor) -> bool:
+    """A projection of a few rows (a decode step) that `skinny_linear` serves."""
+    rows, k = x.numel() // x.shape[-1], x.shape[-1]
+    return bool(x.is_cuda and x.dtype == _BF16 and weight.dtype == _BF16 and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+                and weight.shape[1] == k and 1 <= rows <= 32 and k % 32 == 0 and rows * (k + 8) <= 65536)
+
+
+@torch.no_grad()
+def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_weight: Tensor | None = None, eps: float = 0.0) -> Tensor:
+    """linear(rms_norm(x), weight, bias) for at most 32 rows in one kernel (see nsa_skinny_linear); without norm_weight plain
+    linear.  Inference only."""
+    k, n = x.shape[-1], weight.shape[0]
+    x2 = _rms_rows(x)
+    y = torch.empty((x2.shape[0], n), dtype=_BF16, device=x.device)
+    _lib.check(_lib.lib().nsa_skinny_linear(x2.shape[0], k, n, _ptr(x2), x2.stride(0), _ptr(norm_weight), eps, _ptr(weight), _ptr(bias), _ptr(y), n,
+                                            _stream()), "nsa_skinny_linear")
+    return y.view(*x.shape[:-1], n)
+
+
 def _wgrad_splits(rows: int, n_in: int, n_out: int, replayed: bool = False) -> int:
     """How many slices of the token axis the weight gradient 'o i' = dy^T x is cut into.  The library's GEMM gives one work-group
     per output tile the whole token axis: with a few dozen tiles of a small weight and tens of thousands of tokens most of the

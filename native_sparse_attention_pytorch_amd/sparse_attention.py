@@ -224,8 +224,22 @@ class SparseAttention(nn.Module):
         G, bf16 = self.num_grouped_queries, torch.bfloat16
         freqs = self.rotary_emb.freqs
 
-        x = self.norm(inp)
-        q, k, v = self.to_qkv(x).split(self.qkv_split, dim=-1)
+        # a bf16 layer's projections of a few rows: one kernel each, the norm inside (as decode_session.DecodeSession runs them)
+        norm, gate, gates = self.norm, self.to_strategy_combine[0], None
+        if (inp.dtype == bf16 and self._plain(norm, nn.RMSNorm) and self._plain(self.to_qkv, nn.Linear) and not torch.is_autocast_enabled()
+                and tuple(norm.normalized_shape) == tuple(inp.shape[-1:]) and ops.rms_norm_supported(inp, norm.weight)
+                and ops.skinny_linear_supported(inp, self.to_qkv.weight)):
+            eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
+            x = None
+            qkv = ops.skinny_linear(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight, eps)
+            if self._plain(gate, nn.Linear) and ops.skinny_linear_supported(inp, gate.weight):
+                gates = ops.skinny_linear(inp, gate.weight, gate.bias, norm.weight, eps)
+            else:
+                x = norm(inp)
+        else:
+            x = norm(inp)
+            qkv = self.to_qkv(x)
+        q, k, v = qkv.split(self.qkv_split, dim=-1)
         q, k, v = self._split_heads(q), self._split_heads(k), self._split_heads(v)
         if (self.fp32_kernels and q.dtype == torch.float32 and self.dim_head <= 128 and self.dim_head % 4 == 0
                 and all(t.dtype == torch.float32 for t in (cache_k, cache_v, cache_ck, cache_cv, run_k, run_v))):
@@ -258,7 +272,7 @@ class SparseAttention(nn.Module):
             ck16 = pad(cache_ck if cache_ck.dtype == bf16 else cache_ck.to(bf16))
             cv16 = pad(cache_cv if cache_cv.dtype == bf16 else cache_cv.to(bf16))
         merged, _, _ = ops.decode_step(q16, k16, v16, freqs, t, keys, vals, ck16, cv16, pad(self.compress_mem_kv[0]), pad(self.compress_mem_kv[1]),
-                                       rk_row if fused_run else None, rv_row if fused_run else None, self.to_strategy_combine[0](x),
+                                       rk_row if fused_run else None, rv_row if fused_run else None, gate(x) if gates is None else gates,
                                        per_block=B // st, block=B, num_sel=self.num_selected_blocks,
                                        share=self.query_heads_share_selected_kv, window=self.sliding_window_size, scale=self.scale)
 
@@ -275,7 +289,11 @@ class SparseAttention(nn.Module):
 
         if D != d:
             merged = merged.reshape(b, 1, self.heads, D)[..., :d].reshape(b, 1, self.heads * d)
-        out = self.combine_heads(merged.to(x.dtype))
+        merged = merged.to(qkv.dtype)
+        if self._plain(self.combine_heads, nn.Linear) and not torch.is_autocast_enabled() and ops.skinny_linear_supported(merged, self.combine_heads.weight):
+            out = ops.skinny_linear(merged, self.combine_heads.weight, self.combine_heads.bias)
+        else:
+            out = self.combine_heads(merged)
         if not return_cache:
             return out
         return out, ((keys, vals), ((ck, cv), (run_k, run_v)))
