@@ -252,13 +252,15 @@ int nsa_rmsnorm_fwd(int64_t rows, int32_t dim, const void* x, int64_t x_row_stri
 int nsa_rmsnorm_bwd(int64_t rows, int32_t dim, const void* x, int64_t x_row_stride, const void* weight, const float* rstd,
                     const void* dy, void* dx, void* dweight, int32_t dweight_fp32, float* partials, void* stream);
 
-/* Projection of a few rows: y[r] = norm(x[r]) weight^T + bias for rows <= 32, the shape of a decode step (one token per
- * sequence: NSA.py:356-364, 545).  x: bf16 [rows, k], row stride x_row_stride; weight: bf16 [n, k] contiguous; bias
- * (optional): bf16 [n]; y: bf16 [rows, n].  norm_weight (optional, bf16 [k]): x is RMS-normed first, as nsa_rmsnorm_fwd does
- * (rounded to bf16 before the product).  k a multiple of 32, rows * (k + 8) <= 65536 (NSA_E_UNSUPPORTED otherwise), rows
- * 16-byte aligned. */
+/* Projection of a few rows: y[r] = act(norm(x[r]) weight^T + bias) + residual[r] for rows <= 32, the shape of a decode step (one
+ * token per sequence: NSA.py:356-364, 545; transformer.py:130-138).  x: bf16 [rows, k], row stride x_row_stride; weight: bf16
+ * [n, k] contiguous; bias (optional): bf16 [n]; residual (optional): bf16 [rows, n]; y: bf16 [rows, n].  norm_weight (optional,
+ * bf16 [k]): x is RMS-normed first, as nsa_rmsnorm_fwd does.  Every step is rounded to bf16 as a layer of its own would.
+ * k a multiple of 32, rows * (k + 8) <= 65536 (NSA_E_UNSUPPORTED otherwise), rows of x and weight 16-byte aligned. */
+enum { NSA_ACT_NONE = 0, NSA_ACT_GELU = 1, NSA_ACT_RELU = 2 };
 int nsa_skinny_linear(int32_t rows, int32_t k, int32_t n, const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
-                      const void* weight, const void* bias, void* y, int64_t y_row_stride, void* stream);
+                      const void* weight, const void* bias, int32_t act, const void* residual, int64_t residual_row_stride, void* y,
+                      int64_t y_row_stride, void* stream);
 
 /* Column sums of a bf16 matrix in fp32: the bias gradient of a projection (the sum of d_out over tokens that
  * autograd takes for the nn.Linear layers of NSA.py:244-262, 853) and the gradient of the intra-window positions
@@ -376,6 +378,17 @@ int nsa_decode_step(const nsa_decode_step_desc* desc, const void* q, const void*
                     void* k_cache, void* v_cache, const void* ck_cache, const void* cv_cache, const void* mem_k,
                     const void* mem_v, void* k_run_row, void* v_run_row, const void* gate_logits, void* ws, size_t ws_bytes,
                     void* out, void* stream);
+
+/* The decode step of a whole bf16 layer (NSA.py:338-547 without the compression of a completed window) as one host call:
+ * RMS norm, qkv projection and gate logits, nsa_decode_step, output projection and residual - five launches.  x, residual
+ * (optional), out: bf16 [batch, dim] contiguous; w_qkv: [(heads + 2 kv_heads) d, dim], w_gate: [3 heads, dim], b_gate
+ * (optional): [3 heads], w_out: [dim, heads d], b_out (optional): [dim], all bf16 contiguous; the limits of nsa_skinny_linear
+ * hold for both projections.  freqs: fp32, or bf16 when freqs_bf16.  desc's q / k / v strides are not read.  The selection is left in ws as by nsa_decode_step. */
+int nsa_decode_layer_workspace_bytes(const nsa_decode_step_desc* desc, size_t* bytes);
+int nsa_decode_layer(const nsa_decode_step_desc* desc, int32_t dim, const void* x, const void* norm_weight, float eps, const void* w_qkv,
+                     const void* w_gate, const void* b_gate, const void* freqs, int32_t freqs_bf16, void* k_cache, void* v_cache, const void* ck_cache,
+                     const void* cv_cache, const void* mem_k, const void* mem_v, void* k_run_row, void* v_run_row, const void* w_out,
+                     const void* b_out, const void* residual, void* ws, size_t ws_bytes, void* out, void* stream);
 
 /* nsa_decode_step with the lengths read from device memory when the kernels run, so that the whole step can be
  * recorded once into a HIP graph and replayed for every token (the host-side cost of a step is otherwise several

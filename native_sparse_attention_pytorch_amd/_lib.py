@@ -94,7 +94,7 @@ def lib():
         L.nsa_topk.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         L.nsa_topk_prefix.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         fp = C.POINTER(C.c_float)
-        L.nsa_skinny_linear.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, C.c_float, vp, vp, vp, C.c_int64, vp]
+        L.nsa_skinny_linear.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, C.c_float, vp, vp, C.c_int32, vp, C.c_int64, vp, C.c_int64, vp]
         L.nsa_skinny_linear.restype = C.c_int
         L.nsa_rmsnorm_partials.argtypes = [C.c_int64]
         L.nsa_rmsnorm_fwd.argtypes = [C.c_int64, C.c_int32, vp, C.c_int64, vp, C.c_float, vp, vp, vp]
@@ -126,6 +126,9 @@ def lib():
         L.nsa_decode_step_workspace_bytes.argtypes = [ds, C.POINTER(sz), C.POINTER(sz), C.POINTER(sz), C.POINTER(C.c_int32)]
         L.nsa_decode_step.argtypes = [ds] + [vp] * 14 + [sz, vp, vp]
         L.nsa_decode_step_workspace_bytes.restype = L.nsa_decode_step.restype = C.c_int
+        L.nsa_decode_layer_workspace_bytes.argtypes = [vp, C.POINTER(sz)]
+        L.nsa_decode_layer.argtypes = [vp, C.c_int32, vp, vp, C.c_float] + [vp] * 4 + [C.c_int32] + [vp] * 11 + [vp, sz, vp, vp]
+        L.nsa_decode_layer_workspace_bytes.restype = L.nsa_decode_layer.restype = C.c_int
         L.nsa_decode_step_dyn.argtypes = [ds] + [vp] * 13 + [C.c_int64, C.c_int64, C.c_int32, vp, C.c_int64, vp, vp, sz, vp, C.c_int32, vp]
         L.nsa_decode_step_dyn.restype = C.c_int
         L.nsa_windows_fwd.argtypes = [vp, i3, vp] + [C.c_int32] * 6 + [vp, vp]

@@ -127,7 +127,8 @@ struct PoolOut {                     // kPooled: fp32 [batch, units, stride]; on
 struct NewToken {                    // kNewToken
   const __bf16 *k, *v;               // projections, un-rotated, element strides {batch, head}
   long k0, k1, v0, v1;
-  const float* freqs;
+  const void* freqs;                 // fp32, or bf16 when freqs_bf16
+  int freqs_bf16;
   __bf16* rq;                        // rotated queries [batch, heads, D] for the selected-block branch
   __bf16 *kc, *vc;                   // the caches (strides as in the plan)
   __bf16 *krun, *vrun;               // open compression window (optional): row address, or a ring when ring > 0
@@ -352,7 +353,10 @@ __device__ __forceinline__ void decode_attend_body(const AttendArgs& A, const in
   if constexpr (ROLE == kNewToken) {
     const int pos = P.dyn != nullptr ? P.dyn[0] : P.start + P.count - 1;
     fresh = pos >= 0 && (P.dyn == nullptr || pos < P.cap_len);
-    if (threadIdx.x < D / 2) sincosf((float)pos * A.nt.freqs[threadIdx.x], &step_s[1][threadIdx.x], &step_s[0][threadIdx.x]);
+    if (threadIdx.x < D / 2) {
+      const float f = A.nt.freqs_bf16 ? (float)reinterpret_cast<const __bf16*>(A.nt.freqs)[threadIdx.x] : reinterpret_cast<const float*>(A.nt.freqs)[threadIdx.x];
+      sincosf((float)pos * f, &step_s[1][threadIdx.x], &step_s[0][threadIdx.x]);
+    }
     __syncthreads();
     auto rotate = [&](bf16x8 x, int pair0) {
       bf16x8 o;
@@ -985,8 +989,8 @@ int decode_topk_launch(const float* logits, int32_t batch, int32_t kv_heads, int
 
 // The launches of a step.  state == nullptr: the lengths are the descriptor's; otherwise they are read from it when the
 // kernels run and the descriptor's are capacities.  krun / vrun: the row for the new token (ring == 0) or a ring of rows.
-static int run_step(const nsa_decode_step_desc* d, int32_t* state, const void* q, const void* k, const void* v, const float* freqs, void* k_cache,
-                    void* v_cache, const void* ck_cache, const void* cv_cache, const void* mem_k, const void* mem_v, void* krun, void* vrun,
+int run_decode_step(const nsa_decode_step_desc* d, int32_t* state, const void* q, const void* k, const void* v, const void* freqs, int freqs_bf16,
+                    void* k_cache, void* v_cache, const void* ck_cache, const void* cv_cache, const void* mem_k, const void* mem_v, void* krun, void* vrun,
                     int64_t krun_row, int64_t vrun_row, int32_t ring, const void* gate_logits, int64_t gate_row, const void* gate_bias, void* ws,
                     size_t ws_bytes, void* out, bool advance, void* stream) {
   StepLayout L;
@@ -1025,7 +1029,7 @@ static int run_step(const nsa_decode_step_desc* d, int32_t* state, const void* q
   AttendArgs S = attend_args(Ps, q, k_cache, v_cache, nullptr, nullptr, nullptr, nullptr, w + L.off_wss, nullptr);
   for (int i = 0; i < 2; ++i) S.P.sq[i] = d->q_stride[i];                  // the projection's queries, rotated on the way in
   if ((S.P.sq[0] | S.P.sq[1]) & 7) return NSA_E_ARG;
-  S.nt = NewToken{(const __bf16*)k, (const __bf16*)v, (long)d->k_stride[0], (long)d->k_stride[1], (long)d->v_stride[0], (long)d->v_stride[1], freqs,
+  S.nt = NewToken{(const __bf16*)k, (const __bf16*)v, (long)d->k_stride[0], (long)d->k_stride[1], (long)d->v_stride[0], (long)d->v_stride[1], freqs, freqs_bf16,
                   (__bf16*)rq, (__bf16*)k_cache, (__bf16*)v_cache, (__bf16*)krun, (__bf16*)vrun, (long)d->krun_stride[0], (long)d->krun_stride[1],
                   (long)d->vrun_stride[0], (long)d->vrun_stride[1], (long)krun_row, (long)vrun_row, ring};
   if (has_c) {
@@ -1056,7 +1060,7 @@ extern "C" int nsa_decode_step(const nsa_decode_step_desc* d, const void* q, con
                                void* k_cache, void* v_cache, const void* ck_cache, const void* cv_cache, const void* mem_k,
                                const void* mem_v, void* k_run_row, void* v_run_row, const void* gate_logits, void* ws, size_t ws_bytes,
                                void* out, void* stream) {
-  return nsa::run_step(d, nullptr, q, k, v, freqs, k_cache, v_cache, ck_cache, cv_cache, mem_k, mem_v, k_run_row, v_run_row, 0, 0, 0, gate_logits, 0,
+  return nsa::run_decode_step(d, nullptr, q, k, v, freqs, 0, k_cache, v_cache, ck_cache, cv_cache, mem_k, mem_v, k_run_row, v_run_row, 0, 0, 0, gate_logits, 0,
                        nullptr, ws, ws_bytes, out, false, stream);
 }
 
@@ -1066,6 +1070,6 @@ extern "C" int nsa_decode_step_dyn(const nsa_decode_step_desc* cap, int32_t* sta
                                    int64_t vrun_row_stride, int32_t run_ring, const void* gate_logits, int64_t gate_row_stride,
                                    const void* gate_bias, void* ws, size_t ws_bytes, void* out, int32_t advance, void* stream) {
   if (!state || ((k_run || v_run) && run_ring <= 0)) return NSA_E_ARG;
-  return nsa::run_step(cap, state, q, k, v, freqs, k_cache, v_cache, ck_cache, cv_cache, mem_k, mem_v, k_run, v_run, krun_row_stride, vrun_row_stride,
+  return nsa::run_decode_step(cap, state, q, k, v, freqs, 0, k_cache, v_cache, ck_cache, cv_cache, mem_k, mem_v, k_run, v_run, krun_row_stride, vrun_row_stride,
                        run_ring, gate_logits, gate_row_stride, gate_bias, ws, ws_bytes, out, advance != 0, stream);
 }

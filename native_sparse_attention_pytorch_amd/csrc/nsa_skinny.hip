@@ -4,7 +4,8 @@
 // Bound by reading W once: 2 K N bytes.  A work-group of eight waves owns 16 output features and shares the K axis, so 4096
 // features are 2048 waves that each request up to 16 KB of W before waiting for the first; the batch is the other side of a
 // 16x16x32 MFMA.  While W is on its way the work-group brings x into LDS and norms it there - the norm costs no launch and
-// no pass of its own.  The waves' partial sums meet in LDS.
+// no pass of its own.  The waves' partial sums meet in LDS; bias, activation and residual are added there, each rounded to
+// bf16 as the layers they replace would (a decode step of a small model is bound by the number of its launches).
 // Measured (weights from HBM, launch included): 4096 -> 6240 with norm, batch 1 14.5 us, batch 8 18.1 us, of which the 51 MB
 // of W take 9.8 us at the rate of a large copy (norm kernel + library GEMM: 20.6 / 20.8 us); 4096 -> 4096, batch 1 10.2 us (15.6 us);
 // 1024 -> 1584 with norm, batch 16 6.4 us (9.3 us).
@@ -17,19 +18,39 @@ constexpr int kSkinnyWaves = 8, kSkinnyThreads = 64 * kSkinnyWaves;
 constexpr int kSkinnyAhead = 16;                 // K steps (of 32) whose W operands a wave holds
 constexpr size_t kSkinnyLds = 128 << 10;         // of x
 
+struct SkinnyArgs {
+  int rows, K;
+  const __bf16* x;
+  long xs;
+  const __bf16* nw;                // norm weight or null
+  float eps;
+  int tiles0;                      // work-groups of output 0; the rest are output 1's
+  int n[2];
+  const __bf16 *w[2], *bias[2];
+  __bf16* y[2];
+  long ys[2];
+  int act;                         // NSA_ACT_*
+  const __bf16* res;               // added to output 0, or null
+  long rs;
+};
+
 // NB: groups of 16 rows
 template <int NB>
-__global__ __launch_bounds__(kSkinnyThreads, 4) void skinny_linear_kernel(int rows, int K, int N, const __bf16* __restrict__ x, long xs,
-                                                                          const __bf16* __restrict__ nw, float eps,
-                                                                          const __bf16* __restrict__ w, const __bf16* __restrict__ bias,
-                                                                          __bf16* __restrict__ y, long ys) {
+__global__ __launch_bounds__(kSkinnyThreads, 4) void skinny_linear_kernel(const SkinnyArgs A) {
   extern __shared__ __align__(16) char lds[];
   __shared__ float ss_s[kSkinnyWaves];
   float (*part_s)[NB][16][17] = reinterpret_cast<float (*)[NB][16][17]>(lds);                                 // [wave]
   __bf16* x_s = reinterpret_cast<__bf16*>(lds + sizeof(float) * kSkinnyWaves * NB * 16 * 17);
+  const int o = (int)blockIdx.x < A.tiles0 ? 0 : 1;
+  const int rows = A.rows, K = A.K, N = A.n[o];
+  const __bf16* __restrict__ x = A.x;
+  const __bf16* __restrict__ nw = A.nw;
+  const __bf16* __restrict__ w = A.w[o];
+  const long xs = A.xs;
+  const float eps = A.eps;
   const int RS = K + 8;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, kq = lane >> 4;
-  const int n0 = blockIdx.x * 16;
+  const int n0 = ((int)blockIdx.x - (o ? A.tiles0 : 0)) * 16;
   const int steps = K >> 5, per = (steps + kSkinnyWaves - 1) / kSkinnyWaves;
   const int s0 = wave * per, s1 = min(steps, s0 + per);
   const __bf16* wp = w + (long)min(n0 + r, N - 1) * K + 8 * kq;
@@ -59,7 +80,7 @@ __global__ __launch_bounds__(kSkinnyThreads, 4) void skinny_linear_kernel(int ro
     }
     if (nw != nullptr) {
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
       if (share > 1) {                                                       // (a single round)
         if (lane == 0) ss_s[wave] = ss;
         __syncthreads();
@@ -110,30 +131,109 @@ __global__ __launch_bounds__(kSkinnyThreads, 4) void skinny_linear_kernel(int ro
     float t = 0.f;
 #pragma unroll
     for (int v = 0; v < kSkinnyWaves; ++v) t += part_s[v][g][br][f];
-    if (bias != nullptr) t += (float)bias[n0 + f];
-    y[(long)(16 * g + br) * ys + n0 + f] = (__bf16)t;
+    if (A.bias[o] != nullptr) t += (float)A.bias[o][n0 + f];
+    const int row = 16 * g + br;
+    if (A.act == NSA_ACT_GELU) {
+      const float u = (float)(__bf16)t;
+      t = 0.5f * u * (1.0f + erff(u * 0.70710678118654752f));
+    } else if (A.act == NSA_ACT_RELU) {
+      t = fmaxf(t, 0.f);
+    }
+    if (o == 0 && A.res != nullptr) t = (float)(__bf16)t + (float)A.res[row * A.rs + n0 + f];
+    A.y[o][row * A.ys[o] + n0 + f] = (__bf16)t;
   }
+}
+
+static int launch_skinny(const SkinnyArgs& A, void* stream) {
+  if (A.rows <= 0 || A.K <= 0 || A.n[0] <= 0 || A.n[1] < 0 || !A.x || !A.w[0] || !A.y[0] || (A.n[1] > 0 && (!A.w[1] || !A.y[1]))) return NSA_E_ARG;
+  const size_t xb = (size_t)A.rows * (A.K + 8) * 2;
+  if (A.rows > 32 || (A.K & 31) || xb > kSkinnyLds) return NSA_E_UNSUPPORTED;
+  if ((A.xs & 7) || ((reinterpret_cast<uintptr_t>(A.x) | reinterpret_cast<uintptr_t>(A.w[0]) | reinterpret_cast<uintptr_t>(A.w[1]) |
+                      reinterpret_cast<uintptr_t>(A.nw)) & 15))
+    return NSA_E_ARG;
+  const int nb = A.rows <= 16 ? 1 : 2;
+  const size_t shm = sizeof(float) * kSkinnyWaves * nb * 16 * 17 + xb;
+  const dim3 grid((unsigned)(A.tiles0 + (A.n[1] + 15) / 16)), block(kSkinnyThreads);
+  hipStream_t st = (hipStream_t)stream;
+  if (nb == 1) hipLaunchKernelGGL((skinny_linear_kernel<1>), grid, block, shm, st, A);
+  else hipLaunchKernelGGL((skinny_linear_kernel<2>), grid, block, shm, st, A);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : (int)e;
 }
 
 }  // namespace nsa
 
 extern "C" int nsa_skinny_linear(int32_t rows, int32_t k, int32_t n, const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
-                                 const void* weight, const void* bias, void* y, int64_t y_row_stride, void* stream) {
+                                 const void* weight, const void* bias, int32_t act, const void* residual, int64_t residual_row_stride, void* y,
+                                 int64_t y_row_stride, void* stream) {
   using namespace nsa;
-  if (rows <= 0 || k <= 0 || n <= 0 || !x || !weight || !y) return NSA_E_ARG;
-  const size_t xb = (size_t)rows * (k + 8) * 2;
-  if (rows > 32 || (k & 31) || xb > kSkinnyLds) return NSA_E_UNSUPPORTED;
-  if ((x_row_stride & 7) || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(norm_weight)) & 15))
-    return NSA_E_ARG;
-  const int nb = rows <= 16 ? 1 : 2;
-  const size_t shm = sizeof(float) * kSkinnyWaves * nb * 16 * 17 + xb;
-  const dim3 grid((unsigned)((n + 15) / 16)), block(kSkinnyThreads);
-  hipStream_t st = (hipStream_t)stream;
-#define NSA_SKINNY(NB)                                                                                                                           \
-  hipLaunchKernelGGL((skinny_linear_kernel<NB>), grid, block, shm, st, rows, k, n, (const __bf16*)x, (long)x_row_stride, (const __bf16*)norm_weight, \
-                     eps, (const __bf16*)weight, (const __bf16*)bias, (__bf16*)y, (long)y_row_stride)
-  if (nb == 1) NSA_SKINNY(1); else NSA_SKINNY(2);
-#undef NSA_SKINNY
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? 0 : (int)e;
+  if (act < NSA_ACT_NONE || act > NSA_ACT_RELU) return NSA_E_ARG;
+  SkinnyArgs A{};
+  A.rows = rows; A.K = k; A.x = (const __bf16*)x; A.xs = x_row_stride; A.nw = (const __bf16*)norm_weight; A.eps = eps;
+  A.tiles0 = (n + 15) / 16; A.n[0] = n; A.w[0] = (const __bf16*)weight; A.bias[0] = (const __bf16*)bias; A.y[0] = (__bf16*)y; A.ys[0] = y_row_stride;
+  A.act = act; A.res = (const __bf16*)residual; A.rs = residual_row_stride;
+  return launch_skinny(A, stream);
+}
+
+// ---------------------------------------------------------------------------- a layer's decode step
+// Norm + qkv projection + gate logits (one launch), the attention step (nsa_decode_step: three), output projection + residual:
+// one host call, because at small sizes the host's work between the launches is most of the step.
+
+namespace nsa {
+// nsa_decode.hip
+int run_decode_step(const nsa_decode_step_desc* d, int32_t* state, const void* q, const void* k, const void* v, const void* freqs, int freqs_bf16,
+                    void* k_cache, void* v_cache, const void* ck_cache, const void* cv_cache, const void* mem_k, const void* mem_v, void* krun,
+                    void* vrun, int64_t krun_row, int64_t vrun_row, int32_t ring, const void* gate_logits, int64_t gate_row, const void* gate_bias,
+                    void* ws, size_t ws_bytes, void* out, bool advance, void* stream);
+
+struct LayerLayout { size_t step, off_qkv, off_gate, off_merged, total; };
+
+static int make_layer_layout(const nsa_decode_step_desc* d, LayerLayout& L) {
+  if (int e = nsa_decode_step_workspace_bytes(d, &L.step, nullptr, nullptr, nullptr)) return e;
+  auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  L.off_qkv = up(L.step);
+  L.off_gate = up(L.off_qkv + (size_t)d->batch * (d->heads + 2 * d->kv_heads) * d->dim_head * 2);
+  L.off_merged = up(L.off_gate + (size_t)d->batch * 3 * d->heads * 2);
+  L.total = up(L.off_merged + (size_t)d->batch * d->heads * d->dim_head * 2);
+  return 0;
+}
+}  // namespace nsa
+
+extern "C" int nsa_decode_layer_workspace_bytes(const nsa_decode_step_desc* desc, size_t* bytes) {
+  nsa::LayerLayout L;
+  if (!desc || !bytes) return NSA_E_ARG;
+  if (int e = nsa::make_layer_layout(desc, L)) return e;
+  *bytes = L.total;
+  return 0;
+}
+
+extern "C" int nsa_decode_layer(const nsa_decode_step_desc* desc, int32_t dim, const void* x, const void* norm_weight, float eps, const void* w_qkv,
+                                const void* w_gate, const void* b_gate, const void* freqs, int32_t freqs_bf16, void* k_cache, void* v_cache, const void* ck_cache,
+                                const void* cv_cache, const void* mem_k, const void* mem_v, void* k_run_row, void* v_run_row, const void* w_out,
+                                const void* b_out, const void* residual, void* ws, size_t ws_bytes, void* out, void* stream) {
+  using namespace nsa;
+  if (!desc || !norm_weight || !w_gate || !ws || !out) return NSA_E_ARG;
+  LayerLayout L;
+  if (int e = make_layer_layout(desc, L)) return e;
+  if (ws_bytes < L.total) return NSA_E_WORKSPACE;
+  char* w = (char*)ws;
+  const int hd = desc->heads * desc->dim_head, kd = desc->kv_heads * desc->dim_head, width = hd + 2 * kd;
+  SkinnyArgs P{};
+  P.rows = desc->batch; P.K = dim; P.x = (const __bf16*)x; P.xs = dim; P.nw = (const __bf16*)norm_weight; P.eps = eps;
+  P.tiles0 = (width + 15) / 16;
+  P.n[0] = width; P.w[0] = (const __bf16*)w_qkv; P.y[0] = (__bf16*)(w + L.off_qkv); P.ys[0] = width;
+  P.n[1] = 3 * desc->heads; P.w[1] = (const __bf16*)w_gate; P.bias[1] = (const __bf16*)b_gate; P.y[1] = (__bf16*)(w + L.off_gate); P.ys[1] = 3 * desc->heads;
+  if (int e = launch_skinny(P, stream)) return e;
+  nsa_decode_step_desc d = *desc;
+  d.q_stride[0] = d.k_stride[0] = d.v_stride[0] = width;
+  d.q_stride[1] = d.k_stride[1] = d.v_stride[1] = desc->dim_head;
+  const __bf16* q = (const __bf16*)(w + L.off_qkv);
+  if (int e = run_decode_step(&d, nullptr, q, q + hd, q + hd + kd, freqs, freqs_bf16, k_cache, v_cache, ck_cache, cv_cache, mem_k, mem_v, k_run_row,
+                              v_run_row, 0, 0, 0, w + L.off_gate, 0, nullptr, ws, L.step, w + L.off_merged, false, stream))
+    return e;
+  SkinnyArgs O{};
+  O.rows = desc->batch; O.K = hd; O.x = (const __bf16*)(w + L.off_merged); O.xs = hd;
+  O.tiles0 = (dim + 15) / 16; O.n[0] = dim; O.w[0] = (const __bf16*)w_out; O.bias[0] = (const __bf16*)b_out; O.y[0] = (__bf16*)out; O.ys[0] = dim;
+  O.res = (const __bf16*)residual; O.rs = dim;
+  return launch_skinny(O, stream);
 }

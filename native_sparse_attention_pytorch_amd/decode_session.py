@@ -236,7 +236,7 @@ class DecodeSession:
         bias = m.combine_heads.bias
         if self.own_in:
             rc = L.nsa_skinny_linear(b, dim, qkvg.shape[-1], x.data_ptr(), dim, m.norm.weight.data_ptr(), self._eps(), self.w_cat.data_ptr(), None,
-                                     qkvg.data_ptr(), qkvg.shape[-1], st)
+                                     0, None, 0, qkvg.data_ptr(), qkvg.shape[-1], st)
         else:
             rc = L.nsa_rmsnorm_fwd(b, dim, x.data_ptr(), dim, m.norm.weight.data_ptr(), self._eps(), self.x_buf.data_ptr(), rstd.data_ptr(), st)
             torch.mm(self.x_buf.view(b, dim), self.w_cat.t(), out=qkvg.view(b, -1))
@@ -244,7 +244,7 @@ class DecodeSession:
         if self.own_out:
             y = torch.empty_like(x)
             rc = rc or L.nsa_skinny_linear(b, merged.shape[-1], dim, merged.data_ptr(), merged.shape[-1], None, 0.0, w_out.data_ptr(),
-                                           None if bias is None else bias.data_ptr(), y.data_ptr(), dim, st)
+                                           None if bias is None else bias.data_ptr(), 0, None, 0, y.data_ptr(), dim, st)
         else:
             y = torch.nn.functional.linear(merged, w_out, bias)
         _lib.check(rc, "decode step")
@@ -258,8 +258,8 @@ class DecodeSession:
         wk = self.ring_k.index_select(2, rows)[..., :self.d0]
         wv = self.ring_v.index_select(2, rows)[..., :self.d0]
         at = self.state[1:2].long().clamp(max=self.CK.shape[2] - 1)    # the spare last row at most, whatever the counter holds
-        self.CK.index_copy_(2, at, _pad_dim(m.k_compress((wk + m.k_intrablock_positions)[:, :, None]).to(_BF16), self.d))
-        self.CV.index_copy_(2, at, _pad_dim(m.v_compress((wv + m.v_intrablock_positions)[:, :, None]).to(_BF16), self.d))
+        self.CK.index_copy_(2, at, _pad_dim(m._compress_rows(m.k_compress, wk + m.k_intrablock_positions).to(_BF16), self.d))
+        self.CV.index_copy_(2, at, _pad_dim(m._compress_rows(m.v_compress, wv + m.v_intrablock_positions).to(_BF16), self.d))
         if count:
             self.state[1:2].add_(1)
 
@@ -338,8 +338,8 @@ class TransformerDecodeSession:
             if event:
                 sess.compress_window(count)
             x = a + x
-            x = ff(x) + x
-        return model.to_logits(model.norm(x))
+            x = model._decode_feed_forward(ff, x)
+        return model._decode_logits(x)
 
     @property
     def pos(self) -> int:

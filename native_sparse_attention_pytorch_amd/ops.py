@@ -9,7 +9,8 @@ missing library raise.
 from __future__ import annotations
 
 import ctypes as C
-from typing import Optional
+import struct
+from typing import NamedTuple, Optional
 
 import torch
 from torch import Tensor
@@ -20,7 +21,9 @@ _BF16 = torch.bfloat16
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the current stream of the current device without building a Stream object around it (2 us a call: a decode step of a small
+    # model is bound by its host work)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: Tensor | None) -> int:
@@ -1233,15 +1236,87 @@ def decode_importance_topk(logits: Tensor, kv_heads: int, per_block: int, share:
     return vals, idx, fm.view(torch.bool)
 
 
+class DecodeLayer(NamedTuple):
+    """The parts of a layer that `decode_step(layer=...)` runs around the attention: everything bf16, weights contiguous."""
+    x: Tensor                      # 'b 1 dim'
+    heads: int
+    norm_weight: Tensor
+    eps: float
+    w_qkv: Tensor
+    w_gate: Tensor
+    b_gate: Optional[Tensor]
+    w_out: Tensor
+    b_out: Optional[Tensor]
+    residual: Optional[Tensor]     # 'b 1 dim', added to the output
+
+
+class _StepResult:
+    """(output, idx, fmask) of a step; the selection's views of the workspace are made when somebody asks for them."""
+    __slots__ = ("out", "ws", "desc", "units")
+
+    def __init__(self, out, ws, desc, units):
+        self.out, self.ws, self.desc, self.units = out, ws, desc, units
+
+    def _selection(self):
+        n, io, fo, k = C.c_size_t(), C.c_size_t(), C.c_size_t(), C.c_int32()
+        _lib.check(_lib.lib().nsa_decode_step_workspace_bytes(C.cast(self.desc, C.POINTER(_lib.DecodeStepDesc)), C.byref(n), C.byref(io), C.byref(fo),
+                                                              C.byref(k)), "nsa_decode_step_workspace_bytes")
+        b, kk = self.out.shape[0], k.value
+        shape, cnt = (b, self.units, 1, kk), b * self.units * kk
+        return self.ws[io.value:io.value + 4 * cnt].view(torch.int32).view(shape), self.ws[fo.value:fo.value + cnt].view(torch.bool).view(shape)
+
+    def __getitem__(self, i):
+        return self.out if i == 0 else self._selection()[i - 1]
+
+    def __iter__(self):
+        return iter((self.out, *self._selection()))
+
+
+_STEP_DESC = struct.Struct("@12if22q")      # nsa_decode_step_desc
+assert _STEP_DESC.size == C.sizeof(_lib.DecodeStepDesc)
+
+
+def _decode_layer(layer: DecodeLayer, freqs, pos, keys, vals, ck, cv, mem, run_k, run_v, per_block, block, num_sel, share, window, scale):
+    x = layer.x
+    b, _, dim = x.shape
+    _, hk, _, d = keys.shape
+    nc = 0 if ck is None else ck.shape[2]
+    m = mem.shape[2] if nc else 0
+    rk, rv = run_k.stride(), run_v.stride()
+    last = run_k.shape[2] - 1
+    zero = (0, 0, 0)
+    desc = _STEP_DESC.pack(b, layer.heads, hk, d, pos, nc, m, per_block, block, num_sel, bool(share), window, d ** -0.5 if scale is None else scale,
+                           0, 0, 0, 0, 0, 0, *keys.stride()[:3], *vals.stride()[:3], *(ck.stride()[:3] if nc else zero),
+                           *(cv.stride()[:3] if nc else zero), rk[0], rk[1], rv[0], rv[1])
+    L = _lib.lib()
+    nbytes = C.c_size_t()
+    _lib.check(L.nsa_decode_layer_workspace_bytes(desc, C.byref(nbytes)), "nsa_decode_layer_workspace_bytes")
+    dev = x.device
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
+    out = torch.empty((b, 1, dim), dtype=_BF16, device=dev)
+    mem_p = mem.data_ptr() if m else None
+    _lib.check(L.nsa_decode_layer(desc, dim, x.data_ptr(), layer.norm_weight.data_ptr(), layer.eps, layer.w_qkv.data_ptr(), layer.w_gate.data_ptr(),
+                                  _ptr(layer.b_gate), freqs.data_ptr(), freqs.dtype == _BF16, keys.data_ptr(), vals.data_ptr(),
+                                  ck.data_ptr() if nc else None, cv.data_ptr() if nc else None, mem_p, mem_p + 2 * hk * m * d if m else None,
+                                  run_k.data_ptr() + 2 * last * rk[2], run_v.data_ptr() + 2 * last * rv[2], layer.w_out.data_ptr(), _ptr(layer.b_out),
+                                  _ptr(layer.residual), ws.data_ptr(), nbytes.value, out.data_ptr(), _stream()), "nsa_decode_layer")
+    return _StepResult(out, ws, desc, hk if share else layer.heads)
+
+
 @torch.no_grad()
 def decode_step(q: Tensor, k: Tensor, v: Tensor, freqs: Tensor, pos: int, keys: Tensor, vals: Tensor, ck: Tensor | None, cv: Tensor | None,
                 mem_k: Tensor | None, mem_v: Tensor | None, k_run_row: Tensor | None, v_run_row: Tensor | None, gate_logits: Tensor,
-                *, per_block: int, block: int, num_sel: int, share: bool, window: int, scale: float | None = None):
+                *, per_block: int, block: int, num_sel: int, share: bool, window: int, scale: float | None = None, layer=None):
     """The attention part of one decode step in a single library call (see nsa_decode_step in
     include/nsa_hip.h).  q 'b hq 1 d', k, v 'b hk 1 d': the new token's projections; keys, vals: the
     caches with row `pos` free ('b hk >=pos+1 d' views from the start of their buffers); ck, cv: the
     compressed caches (None or empty before the first compressed key); mem_k, mem_v 'hk m d'.
-    Returns (merged 'b 1 (h d)', idx int32, fmask bool) with idx / fmask 'b hk|hq 1 k'."""
+    Returns (merged 'b 1 (h d)', idx int32, fmask bool) with idx / fmask 'b hk|hq 1 k'.
+    With `layer` (a DecodeLayer) the projections around it are part of the call: q, k, v and gate_logits are None, k_run_row /
+    v_run_row the whole window tensors whose last row is the new token's, mem_k the parameter '2 hk m d' holding both, and
+    the first result is the layer's output 'b 1 dim'."""
+    if layer is not None:
+        return _decode_layer(layer, freqs, pos, keys, vals, ck, cv, mem_k, k_run_row, v_run_row, per_block, block, num_sel, share, window, scale)
     q, k, v = _prep(q), _prep(k), _prep(v)
     b, hq, _, d = q.shape
     hk = k.shape[1]
@@ -1493,16 +1568,25 @@ def skinny_linear_supported(x: Tensor, weight: Tensor) -> bool:
                 and weight.shape[1] == k and 1 <= rows <= 32 and k % 32 == 0 and rows * (k + 8) <= 65536)
 
 
-@torch.no_grad()
-def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_weight: Tensor | None = None, eps: float = 0.0) -> Tensor:
-    """linear(rms_norm(x), weight, bias) for at most 32 rows in one kernel (see nsa_skinny_linear); without norm_weight plain
-    linear.  Inference only."""
+_ACTS = {None: 0, "gelu": 1, "relu": 2}
+
+
+def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_weight: Tensor | None = None, eps: float = 0.0,
+                  act: str | None = None, residual: Tensor | None = None) -> Tensor:
+    """act(linear(rms_norm(x), weight, bias)) + residual for at most 32 rows in one kernel (see nsa_skinny_linear): a bf16
+    projection of a decode step with what stands around it, every part optional.  Inference only (no autograd)."""
     k, n = x.shape[-1], weight.shape[0]
     x2 = _rms_rows(x)
-    y = torch.empty((x2.shape[0], n), dtype=_BF16, device=x.device)
-    _lib.check(_lib.lib().nsa_skinny_linear(x2.shape[0], k, n, _ptr(x2), x2.stride(0), _ptr(norm_weight), eps, _ptr(weight), _ptr(bias), _ptr(y), n,
-                                            _stream()), "nsa_skinny_linear")
-    return y.view(*x.shape[:-1], n)
+    rows = x2.shape[0]
+    if residual is not None:
+        residual = residual.reshape(rows, n)
+        if residual.dtype != _BF16 or residual.stride(1) != 1:
+            raise RuntimeError("skinny_linear: the residual must be bf16 with unit stride")
+    y = torch.empty((*x.shape[:-1], n), dtype=_BF16, device=x.device)
+    _lib.check(_lib.lib().nsa_skinny_linear(rows, k, n, x2.data_ptr(), x2.stride(0), _ptr(norm_weight), eps, weight.data_ptr(), _ptr(bias), _ACTS[act],
+                                            _ptr(residual), 0 if residual is None else residual.stride(0), y.data_ptr(), n, _stream()),
+               "nsa_skinny_linear")
+    return y
 
 
 def _wgrad_splits(rows: int, n_in: int, n_out: int, replayed: bool = False) -> int:

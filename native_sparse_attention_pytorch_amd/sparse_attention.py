@@ -68,6 +68,16 @@ def _append_rows(t: torch.Tensor, extra: int = 1, dtype=torch.bfloat16, min_capa
     return base[:, :, :n + extra], base[:, :, n:n + extra]
 
 
+def _grown(t: torch.Tensor, min_capacity: int = 128) -> torch.Tensor:
+    """`_append_rows` of one row to a bf16 cache of its own width, without the view of the new row."""
+    base, n = t._base, t.shape[2]
+    if (base is not None and getattr(base, "_nsa_filled", -1) == n and base.dim() == 4 and base.shape[2] > n and base.shape[:2] == t.shape[:2]
+            and base.shape[3] == t.shape[3] and base.dtype == torch.bfloat16 and t.data_ptr() == base.data_ptr() and t.stride() == base.stride()):
+        base._nsa_filled = n + 1
+        return base.narrow(2, 0, n + 1)
+    return _append_rows(t, min_capacity=min_capacity)[0]
+
+
 class _FlattenWindow(nn.Module):
     def forward(self, x):                                   # 'b h w n d -> b h w (n d)'
         return x.flatten(-2)
@@ -81,6 +91,16 @@ class _GateLayout(nn.Module):
     def forward(self, x):                                   # 'b n (h s) -> b h n s'
         b, n, _ = x.shape
         return x.reshape(b, n, self.heads, 3).permute(0, 2, 1, 3)
+
+
+def _global_hooks():
+    from torch.nn.modules import module as M
+    return tuple(h for h in (getattr(M, name, None) for name in (
+        "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks",
+        "_global_forward_hooks_always_called")) if h is not None)
+
+
+_GLOBAL_HOOKS = _global_hooks()          # torch's registries themselves: hooks registered later are seen
 
 
 class SparseAttention(nn.Module):
@@ -173,11 +193,8 @@ class SparseAttention(nn.Module):
     def _plain(layer, kind):
         """A library layer of exactly this kind on which nothing is hooked, neither on the instance nor globally: only then may
         its weights be used directly (any hook is skipped when the layer's own `__call__` is)."""
-        from torch.nn.modules import module as M
-        own = (layer._forward_hooks, layer._forward_pre_hooks, layer._backward_hooks, layer._backward_pre_hooks)
-        glob = tuple(getattr(M, name, None) for name in ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
-                                                         "_global_backward_pre_hooks", "_global_forward_hooks_always_called"))
-        return type(layer) is kind and not any(own) and not any(glob)
+        return (type(layer) is kind and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
+                and not any(_GLOBAL_HOOKS))
 
     def _front_is_one_node(self, inp):
         """Norm, qkv projection and gate logits as ops.normed_projections: a bf16 module with its default layers, under autograd."""
@@ -211,6 +228,69 @@ class SparseAttention(nn.Module):
         b, n, hd = t.shape
         return t.view(b, n, hd // self.dim_head, self.dim_head).permute(0, 2, 1, 3)
 
+    def _decode_whole(self, inp, cache, return_cache=True, residual=None):
+        """The decode step of a bf16 layer with its default parts over bf16 caches as one library call (nsa_decode_layer: five
+        launches; `residual` is added to the output); None when something about the layer, the caches or the sizes asks for the
+        general path.  Called without gradients."""
+        (cache_k, cache_v), ((cache_ck, cache_cv), (run_k, run_v)) = cache
+        norm, qkv, gate, out, bf16 = self.norm, self.to_qkv, self.to_strategy_combine[0], self.combine_heads, torch.bfloat16
+        plain, d = self._plain, self.dim_head
+        if not (d in (64, 128) and inp.dtype == bf16 and plain(norm, nn.RMSNorm) and plain(qkv, nn.Linear) and plain(gate, nn.Linear)
+                and plain(out, nn.Linear) and qkv.bias is None and norm.weight is not None and inp.dim() == 3 and inp.shape[1] == 1):
+            return None
+        b, dim, hd = inp.shape[0], inp.shape[2], self.heads * d
+        mem, freqs, device = self.compress_mem_kv, self.rotary_emb.freqs, inp.device
+        if (b > 32 or dim % 32 or b * (max(dim, hd) + 8) > 65536 or norm.normalized_shape != (dim,)
+                or torch.is_autocast_enabled() or torch.compiler.is_compiling()):
+            return None
+        for w in (norm.weight, qkv.weight, gate.weight, gate.bias, out.weight, out.bias, mem):
+            if w is not None and (w.dtype != bf16 or w.device != device or not w.is_contiguous() or w.data_ptr() % 16):
+                return None
+        if not inp.is_contiguous() or inp.data_ptr() % 16:
+            inp = inp.clone(memory_format=torch.contiguous_format)
+        if residual is not None and not residual.is_contiguous():
+            residual = residual.contiguous()
+        if gate.weight.shape != (3 * self.heads, dim) or freqs.dtype not in (bf16, torch.float32) or not freqs.is_contiguous():
+            return None
+        for c in (cache_k, cache_v, cache_ck, cache_cv, run_k, run_v):
+            if c.dtype != bf16 or c.shape[3] != d or c.device != device:
+                return None
+        st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
+        nc, npf = cache_ck.shape[2], B // st
+        if min(self.num_selected_blocks, nc // npf) > 64 or nc // npf > 2048 or (nc and not (ops._rows_ok(cache_ck) and ops._rows_ok(cache_cv))):
+            return None
+        run_k, run_v = _grown(run_k, cbs), _grown(run_v, cbs)
+        keys, vals = _grown(cache_k), _grown(cache_v)
+        eps = norm.eps
+        layer = ops.DecodeLayer(inp, self.heads, norm.weight, torch.finfo(torch.float32).eps if eps is None else eps, qkv.weight, gate.weight, gate.bias,
+                                out.weight, out.bias, residual)
+        y = ops.decode_step(None, None, None, freqs, cache_k.shape[2], keys, vals, cache_ck if nc else None, cache_cv if nc else None, mem, None,
+                            run_k, run_v, None, per_block=npf, block=B, num_sel=self.num_selected_blocks, share=self.query_heads_share_selected_kv,
+                            window=self.sliding_window_size, scale=self.scale, layer=layer)[0]
+        ck, cv = cache_ck, cache_cv
+        if run_k.shape[2] % cbs == 0:
+            next_ck = self._compress_rows(self.k_compress, run_k + self.k_intrablock_positions)
+            next_cv = self._compress_rows(self.v_compress, run_v + self.v_intrablock_positions)
+            run_k, run_v = run_k[..., st:, :], run_v[..., st:, :]
+            ck, ck_row = _append_rows(cache_ck)
+            cv, cv_row = _append_rows(cache_cv)
+            ck_row.copy_(next_ck)
+            cv_row.copy_(next_cv)
+        return (y, ((keys, vals), ((ck, cv), (run_k, run_v)))) if return_cache else y
+
+    @classmethod
+    def _compress_rows(cls, mlp, window):
+        """The compression network on one complete window per sequence, 'b h cbs d' -> 'b h 1 d'."""
+        b, h, n, d = window.shape
+        if cls._plain(mlp, nn.Sequential) and len(mlp) == 4 and type(mlp[0]) is _FlattenWindow and window.dtype == torch.bfloat16:
+            _, up, act, down = mlp
+            x = window.reshape(b * h, n * d)
+            if (cls._plain(up, nn.Linear) and cls._plain(act, nn.ReLU) and cls._plain(down, nn.Linear) and not torch.is_autocast_enabled()
+                    and ops.skinny_linear_supported(x, up.weight) and up.weight.shape[0] % 32 == 0
+                    and b * h * (up.weight.shape[0] + 8) <= 65536 and down.weight.is_contiguous()):
+                return ops.skinny_linear(ops.skinny_linear(x, up.weight, up.bias, act="relu"), down.weight, down.bias).view(b, h, 1, -1)
+        return mlp(window[:, :, None])
+
     @torch.no_grad()
     def forward_inference(self, inp, cache, return_cache=True):
         """One decode step (NSA.py:338-547): `inp` 'b 1 dim' is the token at position t = cached
@@ -224,7 +304,10 @@ class SparseAttention(nn.Module):
         G, bf16 = self.num_grouped_queries, torch.bfloat16
         freqs = self.rotary_emb.freqs
 
-        # a bf16 layer's projections of a few rows: one kernel each, the norm inside (as decode_session.DecodeSession runs them)
+        out = self._decode_whole(inp, cache, return_cache)
+        if out is not None:
+            return out
+        # projections of a few rows by the same kernels (bit-equal to the whole-layer call and to decode_session.DecodeSession)
         norm, gate, gates = self.norm, self.to_strategy_combine[0], None
         if (inp.dtype == bf16 and self._plain(norm, nn.RMSNorm) and self._plain(self.to_qkv, nn.Linear) and not torch.is_autocast_enabled()
                 and tuple(norm.normalized_shape) == tuple(inp.shape[-1:]) and ops.rms_norm_supported(inp, norm.weight)
@@ -279,8 +362,8 @@ class SparseAttention(nn.Module):
         # a compression window is complete: compress it, keep the overlap (NSA.py:422-441)
         ck, cv = cache_ck, cache_cv
         if run_k.shape[-2] % cbs == 0:
-            next_ck = self.k_compress((run_k[..., :d] + self.k_intrablock_positions)[:, :, None])
-            next_cv = self.v_compress((run_v[..., :d] + self.v_intrablock_positions)[:, :, None])
+            next_ck = self._compress_rows(self.k_compress, run_k[..., :d] + self.k_intrablock_positions)
+            next_cv = self._compress_rows(self.v_compress, run_v[..., :d] + self.v_intrablock_positions)
             run_k, run_v = run_k[..., st:, :], run_v[..., st:, :]
             ck, ck_row = _append_rows(cache_ck)
             cv, cv_row = _append_rows(cache_cv)

@@ -57,6 +57,51 @@ class Transformer(nn.Module):
             return ff(tokens)
         return ops.linear(act(ops.linear(norm(tokens), up.weight, up.bias)), down.weight, down.bias)
 
+    @staticmethod
+    def _decode_feed_forward(ff, tokens):
+        """ff(tokens) + tokens for one token per sequence: a bf16 block of the default layers as two kernels (norm, linear, GELU;
+        linear, residual), each step rounded as the layers would."""
+        from . import ops
+        plain = SparseAttention._plain
+        if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+                and plain(ff, nn.Sequential) and len(ff) == 4):
+            norm, up, act, down = ff
+            if (plain(norm, nn.RMSNorm) and plain(up, nn.Linear) and plain(act, nn.GELU) and plain(down, nn.Linear) and act.approximate == 'none'
+                    and norm.normalized_shape == tuple(tokens.shape[-1:]) and ops.rms_norm_supported(tokens, norm.weight)
+                    and ops.skinny_linear_supported(tokens, up.weight) and down.weight.dtype == torch.bfloat16 and down.weight.is_contiguous()
+                    and up.weight.shape[0] % 32 == 0 and tokens.numel() // tokens.shape[-1] * (up.weight.shape[0] + 8) <= 65536):
+                eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
+                hidden = ops.skinny_linear(tokens, up.weight, up.bias, norm.weight, eps, act="gelu")
+                return ops.skinny_linear(hidden, down.weight, down.bias, residual=tokens)
+        return ff(tokens) + tokens
+
+    def _decode_logits(self, tokens):
+        """to_logits(norm(tokens)) for one token per sequence."""
+        from . import ops
+        plain, norm, out = SparseAttention._plain, self.norm, self.to_logits
+        if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+                and plain(norm, nn.RMSNorm) and plain(out, nn.Linear) and norm.normalized_shape == tuple(tokens.shape[-1:])
+                and ops.rms_norm_supported(tokens, norm.weight) and ops.skinny_linear_supported(tokens, out.weight)):
+            return ops.skinny_linear(tokens, out.weight, out.bias, norm.weight, torch.finfo(torch.float32).eps if norm.eps is None else norm.eps)
+        return out(norm(tokens))
+
+    def _decode(self, ids, caches):
+        """One token per sequence through the caches: (logits 'b 1 vocab', advanced caches)."""
+        tokens = self.token_emb(ids[:, -1:])
+        new = []
+        whole = not torch.is_grad_enabled()
+        for (attn, ff), cache in zip(self.layers, caches):
+            # a layer nothing is hooked on takes the residual into its last kernel
+            step = attn._decode_whole(tokens, cache, residual=tokens) if whole and SparseAttention._plain(attn, SparseAttention) else None
+            if step is None:
+                attn_out, cache = attn(tokens, cache=cache, return_cache=True)
+                tokens = attn_out + tokens
+            else:
+                tokens, cache = step
+            new.append(cache)
+            tokens = self._decode_feed_forward(ff, tokens)
+        return self._decode_logits(tokens), new
+
     def forward(self, ids, return_loss=False, disable_flex=False, disable_triton_kernel=False, cache=None, return_cache=False):
         if return_loss:
             ids, labels = ids[:, :-1], ids[:, 1:]
@@ -64,7 +109,10 @@ class Transformer(nn.Module):
             from . import ops
             if not ops.capturing():
                 self._launched_grad_steps = True      # training.GraphedStep must be recorded before the first of these
-        # with caches only the newest token is embedded and every layer takes one decode step
+        if cache is not None and len(cache) == len(self.layers) and not return_loss:
+            # with caches only the newest token is embedded and every layer takes one decode step
+            logits, caches = self._decode(ids, cache)
+            return (logits, caches) if return_cache else logits
         tokens = self.token_emb(ids if cache is None else ids[:, -1:])
         layer_caches = iter(cache or [])
         caches = []

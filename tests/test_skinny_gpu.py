@@ -42,3 +42,50 @@ def test_skinny_limits():
     assert not ops.skinny_linear_supported(z(16, 4096), z(8, 4096))
     with pytest.raises(RuntimeError):
         ops.skinny_linear(z(33, 64), z(8, 64))
+
+
+@pytest.mark.parametrize("rows,k,n,act,res", [(1, 64, 40, "gelu", False), (7, 512, 33, "gelu", True), (20, 128, 16, "relu", True), (32, 64, 100, None, True)])
+def test_skinny_epilogue(rows, k, n, act, res):
+    """Activation and residual: as the layers they replace, each result rounded to bf16."""
+    from native_sparse_attention_pytorch_amd import ops
+    g = torch.Generator().manual_seed(rows + k + n)
+    r = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    x, w, b, add = r(rows, 1, k), r(n, k) * k ** -0.5, r(n), r(rows, 1, n)
+    got = ops.skinny_linear(x.to(DEV), w.to(DEV), b.to(DEV), act=act, residual=add.to(DEV) if res else None)
+    torch.cuda.synchronize()
+    y = x.double() @ w.double().t() + b.double()
+    fn = {"gelu": torch.nn.functional.gelu, "relu": torch.relu, None: lambda t: t}[act]
+    want = fn(y) + (add.double() if res else 0.)
+    # the linear's rounding through a function of slope <= 1.13, the activation's own, the sum's
+    tol = 2 ** -8 * (1.13 * y.abs() + fn(y).abs() + want.abs()) + 1e-6
+    err = (got.double().cpu() - want).abs()
+    assert got.shape == (rows, 1, n) and (err <= tol).all(), (err - tol).max().item()
+
+
+def test_decode_layer_fills_the_newest_rows_and_reports_the_selection():
+    """The whole-layer call: rows of the caches and of the open window, the selection's views, against the general path."""
+    from native_sparse_attention_pytorch_amd import SparseAttention, ops
+    torch.manual_seed(3)
+    m = SparseAttention(dim=96, dim_head=64, heads=4, kv_heads=2, sliding_window_size=20, compress_block_size=8, compress_block_sliding_stride=4,
+                        selection_block_size=8, num_selected_blocks=3, causal=True).to(DEV).bfloat16()
+    x = torch.randn(2, 41, 96, device=DEV, dtype=torch.bfloat16)
+    seen = []
+    orig = ops.decode_step
+    def spy(*a, **kw):
+        r = orig(*a, **kw)
+        seen.append((r[1].clone(), r[2].clone(), kw.get("layer") is not None))
+        return r
+    with torch.no_grad():
+        _, cache = m(x[:, :40], return_cache=True)
+        ops.decode_step = spy
+        try:
+            a, ca = m(x[:, 40:], cache=cache, return_cache=True)
+            m._decode_whole = lambda *args, **kw: None
+            b_, cb = m(x[:, 40:], cache=cache, return_cache=True)
+        finally:
+            ops.decode_step = orig
+    torch.cuda.synchronize()
+    assert seen[0][2] and not seen[1][2]
+    assert torch.equal(seen[0][0], seen[1][0]) and torch.equal(seen[0][1], seen[1][1])
+    flat = lambda c: [t for pair in (c[0], c[1][0], c[1][1]) for t in pair]
+    assert torch.equal(a, b_) and all(torch.equal(s, t) for s, t in zip(flat(ca), flat(cb)))
