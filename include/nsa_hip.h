@@ -166,6 +166,11 @@ int nsa_compress_topk_fwd(const nsa_dense_desc* d, const void* q, const void* k,
  * comes out as value NaN with fmask 0.  Limits: nb <= 2048, k <= min(nb, 64) (NSA_E_UNSUPPORTED otherwise). */
 int nsa_topk(const float* scores, int64_t rows, int32_t nb, int32_t k, int32_t apply_softmax,
              int32_t* idx, float* vals, uint8_t* fmask, void* stream);
+/* nsa_topk (with the softmax) on unscaled, unmasked logits: entry = score * scale; row r belongs to query r % seq; causal_block > 0:
+ * only the columns below floor(query / causal_block) can be selected (the rest is not read), own_block > 0: the column
+ * floor(query / own_block) cannot (NSA.py:676-691).  rows must be a multiple of seq. */
+int nsa_importance_topk(const float* scores, int64_t rows, int32_t nb, int32_t k, float scale, int32_t seq, int32_t causal_block,
+                        int32_t own_block, int32_t* idx, float* vals, uint8_t* fmask, void* stream);
 /* The same for the logits of a causal compressed forward (nsa_dense_fwd with pool = 2): row r belongs to query
  * r % seq, and only its columns below floor(query / block) - the selection blocks that lie completely before the
  * query, NSA.py:676-689 - are defined; the rest counts as -inf and is never read (about half the matrix).  Same
@@ -182,6 +187,10 @@ int nsa_topk_prefix(const float* scores, int64_t rows, int32_t nb, int32_t k, in
 int nsa_gate_fwd(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, const void* logits,
                  const void* c, const int64_t* c_stride, const void* f, const int64_t* f_stride,
                  const void* s, const int64_t* s_stride, void* out, void* stream);
+/* nsa_gate_fwd in fp32 for any dim_head <= 128 that is a multiple of 4. */
+int nsa_gate_fwd_f32(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, const float* logits, const float* c,
+                     const int64_t* c_stride, const float* f, const int64_t* f_stride, const float* s, const int64_t* s_stride, float* out,
+                     void* stream);
 int nsa_gate_bwd(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, const void* logits,
                  const void* c, const int64_t* c_stride, const void* f, const int64_t* f_stride,
                  const void* s, const int64_t* s_stride, const void* d_out,
@@ -262,6 +271,12 @@ int nsa_skinny_linear(int32_t rows, int32_t k, int32_t n, const void* x, int64_t
                       const void* weight, const void* bias, int32_t act, const void* residual, int64_t residual_row_stride, void* y,
                       int64_t y_row_stride, void* stream);
 
+/* y = act(x weight^T + bias) in fp32 for few rows (see nsa_skinny.hip): x [rows, k] with row stride x_row_stride, weight [n, k]
+ * contiguous, bias (optional) [n], y [rows, n] contiguous; act NSA_ACT_NONE or NSA_ACT_RELU.  k a multiple of 8
+ * (NSA_E_UNSUPPORTED otherwise), rows 16-byte aligned. */
+int nsa_linear_f32(int32_t rows, int32_t k, int32_t n, const float* x, int64_t x_row_stride, const float* weight, const float* bias, int32_t act,
+                   float* y, void* stream);
+
 /* Column sums of a bf16 matrix in fp32: the bias gradient of a projection (the sum of d_out over tokens that
  * autograd takes for the nn.Linear layers of NSA.py:244-262, 853) and the gradient of the intra-window positions
  * (the sum of the window gradients over batch and windows, NSA.py:599-600).  Row (o, i) of group g starts at
@@ -290,6 +305,11 @@ int nsa_colsum(const void* x, int32_t groups, int64_t group_stride, int64_t oute
  * any group size, any block size; no backward. */
 int nsa_dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, float* out, float* lse,
                       int32_t q_offset, void* stream);
+/* nsa_dense_fwd_f32 of mode 1 with the memory rows in arrays of their own: mem_k, mem_v fp32 [kv_heads, num_mem, d] contiguous,
+ * k / v hold the num_keys compressed rows alone. */
+int nsa_compress_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, const float* mem_k, const float* mem_v,
+                         float* out, float* lse, int32_t q_offset, void* stream);
+/* (non-causal, no offset, num_keys = seq: a query whose slots are all dead attends their blocks uniformly, NSA.py:809-815; its lse is -inf) */
 int nsa_select_fwd_f32(const nsa_select_desc* d, const float* q, const float* k, const float* v, const void* idx,
                        const uint8_t* fmask, float* out, float* lse, int32_t num_keys, int32_t q_offset, void* stream);
 

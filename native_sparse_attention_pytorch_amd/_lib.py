@@ -93,6 +93,9 @@ def lib():
         L.nsa_compress_topk_supported.restype = L.nsa_compress_topk_fwd.restype = C.c_int
         L.nsa_topk.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         L.nsa_topk_prefix.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
+        L.nsa_importance_topk.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_float, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
+        L.nsa_linear_f32.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, vp, C.c_int32, vp, vp]
+        L.nsa_importance_topk.restype = L.nsa_linear_f32.restype = C.c_int
         fp = C.POINTER(C.c_float)
         L.nsa_skinny_linear.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, C.c_float, vp, vp, C.c_int32, vp, C.c_int64, vp, C.c_int64, vp]
         L.nsa_skinny_linear.restype = C.c_int
@@ -108,6 +111,8 @@ def lib():
         i3 = C.POINTER(C.c_int64)
         L.nsa_gate_fwd.argtypes = [C.c_int32] * 4 + [vp, vp, i3, vp, i3, vp, i3, vp, vp]
         L.nsa_gate_bwd.argtypes = [C.c_int32] * 4 + [vp, vp, i3, vp, i3, vp, i3, vp, vp, vp, vp, vp, vp]
+        L.nsa_gate_fwd_f32.argtypes = L.nsa_gate_fwd.argtypes
+        L.nsa_gate_fwd_f32.restype = C.c_int
         L.nsa_rope.argtypes = [vp, i3, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp, C.c_int32, C.c_int32, vp, i3, vp]
         L.nsa_rope.restype = C.c_int
         L.nsa_decode_workspace_bytes.argtypes = [C.POINTER(DecodeDesc), C.POINTER(sz)]
@@ -138,6 +143,8 @@ def lib():
         L.nsa_qkv_prep_bwd.argtypes = [C.POINTER(QkvDesc)] + [vp] * 9
         L.nsa_qkv_prep_fwd.restype = L.nsa_qkv_prep_bwd.restype = C.c_int
         L.nsa_dense_fwd_f32.argtypes = [C.POINTER(DenseDesc)] + [vp] * 5 + [C.c_int32, vp]
+        L.nsa_compress_fwd_f32.argtypes = [C.POINTER(DenseDesc)] + [vp] * 7 + [C.c_int32, vp]
+        L.nsa_compress_fwd_f32.restype = C.c_int
         L.nsa_select_fwd_f32.argtypes = [C.POINTER(SelectDesc)] + [vp] * 7 + [C.c_int32, C.c_int32, vp]
         L.nsa_dense_fwd_f32.restype = L.nsa_select_fwd_f32.restype = C.c_int
         for name in ("nsa_dense_workspace_bytes", "nsa_dense_fwd", "nsa_dense_bwd", "nsa_topk", "nsa_topk_prefix", "nsa_gate_fwd", "nsa_gate_bwd"):

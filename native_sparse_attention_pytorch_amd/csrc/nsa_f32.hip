@@ -26,8 +26,9 @@ struct F32Args {
   long sq[3], sk[3], sv[3];
   // dense
   int mode, causal, wb, wf, st, mem;
+  const float *memk, *memv;       // the memory rows [hk, mem, d] when they are not the first rows of k / v, else null
   // selection
-  int S, B, W, idx64;
+  int S, B, W, idx64, uniform;
 };
 
 __device__ __forceinline__ floatx16 mfma32x2(float a, float b, floatx16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
@@ -77,21 +78,25 @@ __device__ __forceinline__ float sum_mod4(float v) {
 
 struct RowsStage { floatx4 x[16]; };
 
-// this lane's 16 bytes of rows 4 r + lane / 16, r = 0 .. 15, of the tile whose rows `rows_s` lists.  `zeros` (wave-uniform): some
-// of them are padding keys (row -1), or this piece's chunks reach past the head dimension; those read as zeros.
-__device__ __forceinline__ void rows_load(RowsStage& st, const float* __restrict__ base, long stride, const int* __restrict__ rows_s, int r0, int col,
-                                          bool inside, bool zeros) {
+// this lane's 16 bytes of rows 4 r + lane / 16, r = 0 .. 15, of the tile whose rows `rows_s` lists.  `special` (wave-uniform): some
+// of them are padding keys (row -1: zeros) or memory rows of an array of their own (row -2 - m: row m of `mem`), or this piece's
+// chunks reach past the head dimension (zeros).
+__device__ __forceinline__ void rows_load(RowsStage& st, const float* __restrict__ base, long stride, const float* __restrict__ mem, int d,
+                                          const int* __restrict__ rows_s, int r0, int col, bool inside, bool special) {
   const float* bc = base + (inside ? col : 0);
-  if (!zeros) {
+  if (!special) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) st.x[r] = *reinterpret_cast<const floatx4*>(bc + (long)rows_s[4 * r + r0] * stride);
   } else {
+    const float* mc = mem + (inside ? col : 0);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int row = rows_s[4 * r + r0];
-      const floatx4 x = *reinterpret_cast<const floatx4*>(bc + (long)max(row, 0) * stride);
+      const bool real = inside && row != -1;
+      const float* p = row <= -2 ? mc + (long)(-2 - row) * d : bc + (long)max(row, 0) * stride;
+      const floatx4 x = *reinterpret_cast<const floatx4*>(p);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) st.x[r][e] = inside && row >= 0 ? x[e] : 0.f;
+      for (int e = 0; e < 4; ++e) st.x[r][e] = real ? x[e] : 0.f;
     }
   }
 }
@@ -104,28 +109,33 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// `total` keys; key(v) -> row of k / v (v < total), -1 for a padding key past the sequence end (logit 0, value 0).  Tiles first, first + step, ...
+// `total` keys; key(v) -> row of k / v (v < total), -1 for a padding key past the sequence end (logit 0, value 0), -2 - m for
+// row m of mk / mv.  Tiles first, first + step, ...
 template <int DT, class Key>
 __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ piece, int* __restrict__ rows_s, const float (&q)[DT][64], const float* __restrict__ kb,
-                                          const float* __restrict__ vb, int total, int first, int step, Key key, RowsState<DT>& S, int lane) {
+                                          const float* __restrict__ vb, const float* __restrict__ mk, const float* __restrict__ mv, int total,
+                                          int first, int step, Key key, RowsState<DT>& S, int lane) {
   const int tiles = (total + 63) >> 6;
   if (first >= tiles) return;
   const int chunk = lane & 15, r0 = lane >> 4;
-  bool pads = false;
+  bool special = false;
   // rows of tile t's keys; places behind the last key repeat it (their scores are masked)
   auto locate = [&](int t) {
     const int row = key(min(t * 64 + lane, total - 1));
-    pads = __any(row < 0);
+    special = __any(row < 0);
     __builtin_amdgcn_wave_barrier();
     rows_s[lane] = row;
     __builtin_amdgcn_wave_barrier();
   };
   RowsStage st;
-  auto load = [&](const float* base, long stride, int ft) {
-    rows_load(st, base, stride, rows_s, r0, 64 * ft + 4 * chunk, 64 * ft + 4 * chunk < A.d, pads || 64 * (ft + 1) > A.d);
+  auto load_k = [&](int ft) {
+    rows_load(st, kb, A.sk[2], mk, A.d, rows_s, r0, 64 * ft + 4 * chunk, 64 * ft + 4 * chunk < A.d, special || 64 * (ft + 1) > A.d);
+  };
+  auto load_v = [&](int ft) {
+    rows_load(st, vb, A.sv[2], mv, A.d, rows_s, r0, 64 * ft + 4 * chunk, 64 * ft + 4 * chunk < A.d, special || 64 * (ft + 1) > A.d);
   };
   locate(first);
-  load(kb, A.sk[2], 0);
+  load_k(0);
   for (int t = first; t < tiles; t += step) {
     floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -134,8 +144,8 @@ __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ 
 #pragma unroll
       for (int r = 0; r < 16; ++r) *reinterpret_cast<floatx4*>(piece + (4 * r + r0) * 64 + 4 * (chunk ^ ((4 * r + r0) & 15))) = st.x[r];
       __builtin_amdgcn_wave_barrier();
-      if (ft + 1 < DT) load(kb, A.sk[2], ft + 1);
-      else load(vb, A.sv[2], 0);
+      if (ft + 1 < DT) load_k(ft + 1);
+      else load_v(0);
 #pragma unroll
       for (int c = 0; c < 16; ++c) {
         const floatx4 kx = *reinterpret_cast<const floatx4*>(piece + lane * 64 + 4 * (c ^ (lane & 15)));
@@ -169,10 +179,10 @@ __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ 
 #pragma unroll
       for (int r = 0; r < 16; ++r) *reinterpret_cast<floatx4*>(piece + (4 * r + r0) * 64 + 4 * chunk) = st.x[r];
       __builtin_amdgcn_wave_barrier();
-      if (ft + 1 < DT) load(vb, A.sv[2], ft + 1);
+      if (ft + 1 < DT) load_v(ft + 1);
       else if (t + step < tiles) {
         locate(t + step);
-        load(kb, A.sk[2], 0);
+        load_k(0);
       }
       floatx4 o0 = S.acc[ft] * al, o1 = {0.f, 0.f, 0.f, 0.f};
       static_for<0, 16>([&](auto blk) {
@@ -206,6 +216,22 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
   int* blocks = blocks_s[wave];
   const int first = WPQ == 1 ? 0 : wave, step = WPQ;
   const int pos = i + A.qoff;
+  const float* mk = A.memk != nullptr ? A.memk + (long)hk * A.mem * A.d : kb;
+  const float* mv = A.memv != nullptr ? A.memv + (long)hk * A.mem * A.d : vb;
+  // A query of a non-causal selection whose slots are all dead attends their blocks uniformly, zero padding included: the
+  // reference fills all its logits with the same value (NSA.py:809-815).  Zero queries over all slots give the same.
+  bool dead = false;
+  if constexpr (SELECT) {
+    if (A.uniform) {
+      dead = true;
+      for (int s = lane; s < A.S; s += 64) {
+        const size_t at = ((size_t)bh * A.n + i) * A.S + s;
+        const long j = A.idx64 ? (long)reinterpret_cast<const long long*>(idx)[at] : (long)reinterpret_cast<const int*>(idx)[at];
+        if (fmask[at] && j >= 0 && j < A.W) dead = false;
+      }
+      dead = !__any(!dead);
+    }
+  }
   for (int g0 = 0; g0 < A.g; g0 += 4) {
     float qr[DT][64];
     {
@@ -218,6 +244,12 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
       for (int ft = 0; ft < DT; ++ft)
 #pragma unroll
         for (int e = 0; e < 64; ++e) qr[ft][e] = qp[min(64 * ft + e, last)];
+      if (SELECT && dead) {
+#pragma unroll
+        for (int ft = 0; ft < DT; ++ft)
+#pragma unroll
+          for (int e = 0; e < 64; ++e) qr[ft][e] = 0.f;
+      }
     }
     RowsState<DT> S;
     S.m = -INFINITY;
@@ -232,9 +264,10 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
         int blk = -1;
         if (s0 + lane < A.S) {
           const size_t at = ((size_t)bh * A.n + i) * A.S + s0 + lane;
-          if (fmask[at]) {
+          if (dead || fmask[at]) {
             const long j = A.idx64 ? (long)reinterpret_cast<const long long*>(idx)[at] : (long)reinterpret_cast<const int*>(idx)[at];
-            if (j >= 0 && j < A.W) blk = (int)j;
+            if (dead) blk = (int)min(max(j, 0l), (long)A.W - 1);
+            else if (j >= 0 && j < A.W) blk = (int)j;
           }
         }
         const unsigned long long live = __ballot(blk >= 0);
@@ -243,7 +276,7 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
         if (blk >= 0) blocks[__popcll(live & ((1ull << lane) - 1))] = blk;
         __builtin_amdgcn_wave_barrier();
         const bool last = s0 + 64 >= A.S;
-        rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, cnt * A.B + (last ? own_keys : 0), first, step, [&](int v) {
+        rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, kb, vb, cnt * A.B + (last ? own_keys : 0), first, step, [&](int v) {
           const int slot = v / A.B, off = v - slot * A.B;
           const int row = (slot < cnt ? blocks[slot] : own) * A.B + off;
           return row < A.nk ? row : -1;
@@ -253,7 +286,11 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
     } else {
       int lo, hi;
       f32_interval(A, pos, lo, hi);
-      rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, hi - lo + 1, first, step, [&](int v) { return lo + v; }, S, lane);
+      const int own_mem = A.memk != nullptr ? A.mem : 0;
+      rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, mk, mv, hi - lo + 1, first, step, [&](int v) {
+        const int u = lo + v;
+        return u < own_mem ? -2 - u : u - own_mem;
+      }, S, lane);
     }
     float l = sum_mod4(S.l);
     float* ob = out + (((long)b * A.hk * A.g + (long)hk * A.g + g0) * A.n + i) * A.d;
@@ -268,7 +305,7 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
           if (64 * ft + lane < A.d) ob[(long)h * A.n * A.d + 64 * ft + lane] = S.acc[ft][h] * inv;
       }
       if (lse != nullptr && lane < 4 && g0 + lane < A.g)
-        lse[((long)b * A.hk * A.g + (long)hk * A.g + g0 + lane) * A.n + i] = l > 0.f ? S.m + logf(l) : -INFINITY;
+        lse[((long)b * A.hk * A.g + (long)hk * A.g + g0 + lane) * A.n + i] = l > 0.f && !dead ? S.m + logf(l) : -INFINITY;
     } else {
       // merge of the four waves' partial results: wave w finishes head g0 + w
       __syncthreads();                                     // the pieces are free
@@ -299,7 +336,7 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
         for (int ft = 0; ft < DT; ++ft)
           if (64 * ft + lane < A.d) ob[(long)wave * A.n * A.d + 64 * ft + lane] = o[ft] * inv;
         if (lse != nullptr && lane == 0)
-          lse[((long)b * A.hk * A.g + (long)hk * A.g + g0 + wave) * A.n + i] = ll > 0.f ? mm + logf(ll) : -INFINITY;
+          lse[((long)b * A.hk * A.g + (long)hk * A.g + g0 + wave) * A.n + i] = ll > 0.f && !dead ? mm + logf(ll) : -INFINITY;
       }
       __syncthreads();                                     // before the next heads' pieces overwrite the partials
     }
@@ -360,6 +397,7 @@ __global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const
   for (int ft = 0; ft < D / 32; ++ft) o[ft] = zero_acc();
   float m = -INFINITY, l = 0.f;
 
+  const int own_mem = A.memk != nullptr ? A.mem : 0;
   floatx4 kx[LD], vx[LD];
   auto fetch = [&](int t0) {
 #pragma unroll
@@ -370,8 +408,9 @@ __global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const
       kx[u] = z;
       vx[u] = z;
       if (kr <= g_hi && 4 * c < A.d) {
-        kx[u] = *reinterpret_cast<const floatx4*>(kb + (long)kr * A.sk[2] + 4 * c);
-        vx[u] = *reinterpret_cast<const floatx4*>(vb + (long)kr * A.sv[2] + 4 * c);
+        const bool own = kr < own_mem;
+        kx[u] = *reinterpret_cast<const floatx4*>((own ? A.memk + ((long)hk * A.mem + kr) * A.d : kb + (long)(kr - own_mem) * A.sk[2]) + 4 * c);
+        vx[u] = *reinterpret_cast<const floatx4*>((own ? A.memv + ((long)hk * A.mem + kr) * A.d : vb + (long)(kr - own_mem) * A.sv[2]) + 4 * c);
       }
     }
   };
@@ -484,8 +523,8 @@ static void f32_launch_rows(const F32Args& A, const float* q, const float* k, co
 
 using namespace nsa;
 
-extern "C" int nsa_dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, float* out, float* lse,
-                                 int32_t q_offset, void* stream) {
+static int dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, const float* mem_k, const float* mem_v, float* out,
+                         float* lse, int32_t q_offset, void* stream) {
   if (!d || !q || !k || !v || !out) return NSA_E_ARG;
   F32Args A{};
   const int rc = f32_common(d->batch, d->kv_heads, d->group, d->seq, q_offset, d->dim_head, d->scale, d->q_stride, d->k_stride, d->v_stride, A);
@@ -493,6 +532,7 @@ extern "C" int nsa_dense_fwd_f32(const nsa_dense_desc* d, const float* q, const 
   if (d->num_keys < 0 || d->num_mem < 0 || d->num_mem > 64) return NSA_E_ARG;
   A.nk = d->num_keys; A.mem = d->num_mem; A.mode = d->mode; A.causal = d->causal ? 1 : 0;
   A.wb = A.wf = 0; A.st = 1;
+  A.memk = mem_k; A.memv = mem_v;
   if (d->mode == 0) {
     if (d->window < 0 || d->num_mem != 0) return NSA_E_ARG;
     A.wb = d->window; A.wf = A.causal ? 0 : d->window;
@@ -516,6 +556,18 @@ extern "C" int nsa_dense_fwd_f32(const nsa_dense_desc* d, const float* q, const 
   return e == hipSuccess ? 0 : (int)e;
 }
 
+extern "C" int nsa_dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, float* out, float* lse,
+                                 int32_t q_offset, void* stream) {
+  return dense_fwd_f32(d, q, k, v, nullptr, nullptr, out, lse, q_offset, stream);
+}
+
+extern "C" int nsa_compress_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, const float* mem_k, const float* mem_v,
+                                    float* out, float* lse, int32_t q_offset, void* stream) {
+  if (!d || d->mode != 1 || d->num_mem <= 0 || !mem_k || !mem_v || ((reinterpret_cast<uintptr_t>(mem_k) | reinterpret_cast<uintptr_t>(mem_v)) & 15))
+    return NSA_E_ARG;
+  return dense_fwd_f32(d, q, k, v, mem_k, mem_v, out, lse, q_offset, stream);
+}
+
 extern "C" int nsa_select_fwd_f32(const nsa_select_desc* d, const float* q, const float* k, const float* v, const void* idx,
                                   const uint8_t* fmask, float* out, float* lse, int32_t num_keys, int32_t q_offset, void* stream) {
   if (!d || !q || !k || !v || !out) return NSA_E_ARG;
@@ -526,6 +578,7 @@ extern "C" int nsa_select_fwd_f32(const nsa_select_desc* d, const float* q, cons
   if (num_keys <= 0 || (d->causal && d->seq + q_offset > num_keys)) return NSA_E_ARG;      // a query's own position must have a key row
   A.nk = num_keys; A.S = d->num_sel; A.B = d->block; A.W = (num_keys + d->block - 1) / d->block; A.causal = d->causal ? 1 : 0;
   A.idx64 = d->idx_is_int64 ? 1 : 0;
+  A.uniform = !A.causal && A.S > 0 && q_offset == 0 && num_keys == d->seq;
   f32_launch_rows<true>(A, q, k, v, idx, fmask, out, lse, (hipStream_t)stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;

@@ -175,6 +175,59 @@ extern "C" int nsa_skinny_linear(int32_t rows, int32_t k, int32_t n, const void*
   return launch_skinny(A, stream);
 }
 
+// ---------------------------------------------------------------------------- few rows in fp32
+// y = act(x W^T + bias) for matrices too small for the GEMM library's tiles (an fp32 layer on a few dozen tokens: 240 x 256 x
+// 256 takes it 65 us, one 256 x 256 tile and seven eighths of it idle).  A work-group owns a 32 x 32 tile of y and its eight waves
+// share K: v_mfma_f32_32x32x2, both operands 16 bytes per lane straight from memory (lane = row, half h: features
+// 8 t + 4 h + j in step j of group t), partial tiles added in LDS in a fixed order.
+
+namespace nsa {
+
+__global__ __launch_bounds__(512) void linear_f32_kernel(int rows, int K, int N, const float* __restrict__ x, long xs, const float* __restrict__ w,
+                                                         const float* __restrict__ bias, int act, float* __restrict__ y) {
+  __shared__ float part_s[8][32][33];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
+  const int n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
+  const int groups = K >> 3, per = (groups + 7) / 8, g0 = wave * per, g1 = min(groups, g0 + per);
+  const float* wp = w + (long)min(n0 + r, N - 1) * K + 4 * h;
+  const float* xp = x + (long)min(m0 + r, rows - 1) * xs + 4 * h;
+  floatx16 acc = zero_acc();
+#pragma unroll 4
+  for (int g = g0; g < g1; ++g) {
+    const floatx4 a = *reinterpret_cast<const floatx4*>(wp + 8 * g), b = *reinterpret_cast<const floatx4*>(xp + 8 * g);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], acc, 0, 0, 0);
+  }
+  // D: feature 8 (i / 4) + 4 h + i % 4, row r
+#pragma unroll
+  for (int i = 0; i < 16; ++i) part_s[wave][r][8 * (i / 4) + 4 * h + (i % 4)] = acc[i];
+  __syncthreads();
+  for (int e = threadIdx.x; e < 1024; e += 512) {
+    const int f = e & 31, row = e >> 5;
+    if (m0 + row >= rows || n0 + f >= N) continue;
+    float t = 0.f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) t += part_s[v][row][f];
+    if (bias != nullptr) t += bias[n0 + f];
+    if (act == NSA_ACT_RELU) t = fmaxf(t, 0.f);
+    y[(long)(m0 + row) * N + n0 + f] = t;
+  }
+}
+
+}  // namespace nsa
+
+extern "C" int nsa_linear_f32(int32_t rows, int32_t k, int32_t n, const float* x, int64_t x_row_stride, const float* weight, const float* bias,
+                              int32_t act, float* y, void* stream) {
+  using namespace nsa;
+  if (rows <= 0 || k <= 0 || n <= 0 || !x || !weight || !y || (act != NSA_ACT_NONE && act != NSA_ACT_RELU)) return NSA_E_ARG;
+  if ((k & 7) || (rows + 31) / 32 > 65535) return NSA_E_UNSUPPORTED;
+  if ((x_row_stride & 3) || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weight)) & 15)) return NSA_E_ARG;
+  hipLaunchKernelGGL(linear_f32_kernel, dim3((unsigned)((n + 31) / 32), (unsigned)((rows + 31) / 32)), dim3(512), 0, (hipStream_t)stream, rows, k, n, x,
+                     (long)x_row_stride, weight, bias, act, y);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : (int)e;
+}
+
 // ---------------------------------------------------------------------------- a layer's decode step
 // Norm + qkv projection + gate logits (one launch), the attention step (nsa_decode_step: three), output projection + residual:
 // one host call, because at small sizes the host's work between the launches is most of the step.

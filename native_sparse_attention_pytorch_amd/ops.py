@@ -1607,6 +1607,27 @@ def _wgrad_splits(rows: int, n_in: int, n_out: int, replayed: bool = False) -> i
     return s if s >= 4 else 1
 
 
+def linear_f32_supported(x: Tensor, weight: Tensor) -> bool:
+    """An fp32 projection small enough that the GEMM library's tiles leave most of the chip idle.  Measured, this kernel / the
+    library in us: 240 x 256 -> 256 4.8 / 64.7, 240 x 512 -> 24 6.2 / 19.9, 62 x 512 -> 1536 6.7 / 6.8, 256 x 512 -> 1536 11.6 / 8.5
+    (the library's call takes the host 14 us longer), 384 x 256 -> 256 4.8 / 6.1, 256 x 1024 -> 1024 12.3 / 9.1."""
+    rows, k = x.numel() // max(x.shape[-1], 1), x.shape[-1]
+    return bool(x.is_cuda and x.dtype == torch.float32 and weight.dtype == torch.float32 and weight.is_contiguous() and 0 < rows <= 256 and k <= 512 and k % 8 == 0
+                and weight.data_ptr() % 16 == 0)
+
+
+def linear_f32(x: Tensor, weight: Tensor, bias: Tensor | None = None, act: str | None = None) -> Tensor:
+    """act(linear(x, weight, bias)) in fp32 by nsa_linear_f32 (few rows, no gradient)."""
+    k, n = x.shape[-1], weight.shape[0]
+    x2 = x.reshape(-1, k)
+    if x2.stride(1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
+        x2 = x2.clone(memory_format=torch.contiguous_format)
+    y = torch.empty((*x.shape[:-1], n), dtype=torch.float32, device=x.device)
+    _lib.check(_lib.lib().nsa_linear_f32(x2.shape[0], k, n, _ptr(x2), x2.stride(0), _ptr(weight), _ptr(bias), _ACTS[act], _ptr(y), _stream()),
+               "nsa_linear_f32")
+    return y
+
+
 class _Linear(torch.autograd.Function):
     """F.linear whose weight gradient is a batched GEMM over slices of the token axis, summed in fp32 (see _wgrad_splits):
     the same products as the one GEMM autograd would launch (NSA.py:583 to_qkv, 853 to_strategy_combine, 858 combine_heads)."""
@@ -1636,6 +1657,8 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     """torch.nn.functional.linear with the split weight-gradient GEMM (see _Linear)."""
     if (not (torch.is_grad_enabled() and weight.requires_grad) or torch.compiler.is_compiling() or x.dtype != weight.dtype
             or torch.is_autocast_enabled()):               # under autocast the library casts the operands itself
+        if not torch.is_grad_enabled() and linear_f32_supported(x, weight) and not torch.compiler.is_compiling() and not torch.is_autocast_enabled():
+            return linear_f32(x, weight, bias)
         return torch.nn.functional.linear(x, weight, bias)
     return _Linear.apply(x, weight, bias)
 
@@ -1792,9 +1815,84 @@ def native_sparse_attend_f32(fq: Tensor, fk: Tensor, fv: Tensor, block_size: int
     _lib.check(_lib.lib().nsa_select_fwd_f32(C.byref(dsc), _ptr(q), _ptr(k), _ptr(v), _ptr(idx) if idx.numel() else None,
                                              _ptr(fm) if fm.numel() else None, _ptr(out), _ptr(lse), k.shape[2], int(q_offset), _stream()),
                "nsa_select_fwd_f32")
-    if not include_block_causal and idx.shape[-1] > 0 and q_offset == 0 and k.shape[2] == n:
-        out = _dead_rows_uniform(out, fv, selected_block_indices, fmask, int(block_size), q_heads, d)
     return (out, lse) if return_lse else out
+
+
+@torch.no_grad()
+def compress_attend_f32(q: Tensor, ck: Tensor, cv: Tensor, mem: Tensor, stride: int, causal: bool, q_offset: int = 0) -> Tensor:
+    """`dense_attend_f32` of the compressed branch with the memory rows 'kv hk m d' where the parameter has them, instead of in
+    front of the compressed keys / values."""
+    q, ck, cv = _f32(q), _f32(ck), _f32(cv)
+    b, hq, n, d = q.shape
+    _check_f32_dim(d)
+    mem = mem.contiguous()
+    hk, m = mem.shape[1], mem.shape[2]
+    out = torch.empty((b, hq, n, d), dtype=torch.float32, device=q.device)
+    dsc = _dense_desc(q, ck, cv, out, out, 1, bool(causal), 0, int(stride), 0, False, 1, True, float(d ** -0.5))
+    dsc.num_mem, dsc.num_keys = m, ck.shape[2]
+    p = mem.data_ptr()
+    # (no compressed key yet: the kernel is handed the memory rows' address for an array it does not read)
+    _lib.check(_lib.lib().nsa_compress_fwd_f32(C.byref(dsc), _ptr(q), _ptr(ck) or p, _ptr(cv) or p, p, p + 4 * hk * m * d, _ptr(out), None, int(q_offset),
+                                               _stream()), "nsa_compress_fwd_f32")
+    return out
+
+
+@torch.no_grad()
+def importance_topk_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool, causal: bool, num_selected: int, mask_own: bool = True):
+    """`importance_topk(importance_logits_f32(...))` without gradients: the products from the same fp32 GEMM, scale and masks
+    inside the top-k kernel.  Returns (values, idx, fmask)."""
+    raw = _importance_products_f32(q, ck, stride, sel_block, share)
+    n, nb = raw.shape[-2:]
+    own = mask_own and stride != sel_block
+    if nb > _TOPK_MAX_ROW or num_selected > _TOPK_MAX_K:
+        return importance_topk(_importance_mask_f32(raw * (q.shape[-1] ** -0.5), stride, sel_block, causal, mask_own).contiguous(), num_selected)
+    raw = raw.contiguous()
+    shp = (*raw.shape[:-1], int(num_selected))
+    idx = torch.empty(shp, dtype=torch.int32, device=raw.device)
+    vals = torch.empty(shp, dtype=torch.float32, device=raw.device)
+    fm = torch.empty(shp, dtype=torch.bool, device=raw.device)
+    _lib.check(_lib.lib().nsa_importance_topk(_ptr(raw), raw.numel() // nb, nb, int(num_selected), q.shape[-1] ** -0.5, n, int(sel_block) if causal else 0,
+                                              int(sel_block) if own else 0, _ptr(idx), _ptr(vals), _ptr(fm), _stream()), "nsa_importance_topk")
+    return vals, idx, fm
+
+
+@torch.no_grad()
+def gate_combine_f32(logits: Tensor, compressed: Tensor, selected: Tensor, sliding: Tensor) -> Tensor:
+    """`gate_combine` in fp32: pre-sigmoid logits 'b n (h s)', branches 'b h n d' -> 'b n (h d)'."""
+    c, f, s = _f32(compressed), _f32(selected), _f32(sliding)
+    logits = logits.contiguous()
+    b, h, n, d = c.shape
+    out = torch.empty((b, n, h * d), dtype=torch.float32, device=c.device)
+    _lib.check(_lib.lib().nsa_gate_fwd_f32(b, h, n, d, _ptr(logits), _ptr(c), _s3(c), _ptr(f), _s3(f), _ptr(s), _s3(s), _ptr(out), _stream()),
+               "nsa_gate_fwd_f32")
+    return out
+
+
+def _importance_products_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool) -> Tensor:
+    """Mean over a fine block's compressed keys and (if shared) the group's heads of q . ck, unscaled: one fp32 GEMM against
+    the block means."""
+    b, hq, n, d = q.shape
+    hk = ck.shape[1]
+    g = hq // hk
+    npf = sel_block // stride
+    nb = ck.shape[2] // npf
+    cbar = ck[:, :, :nb * npf].float().reshape(b, hk, nb, npf, d).mean(dim=3)
+    qq = q.float().reshape(b, hk, g, n, d).mean(dim=2) if share else q.float()
+    if not share:
+        cbar = cbar.repeat_interleave(g, dim=1)
+    return torch.matmul(qq, cbar.transpose(-1, -2))
+
+
+def _importance_mask_f32(imp: Tensor, stride: int, sel_block: int, causal: bool, mask_own: bool) -> Tensor:
+    n, nb = imp.shape[-2:]
+    i = torch.arange(n, device=imp.device)[:, None]
+    j = torch.arange(nb, device=imp.device)[None, :]
+    dead = torch.zeros((n, nb), dtype=torch.bool, device=imp.device)
+    if causal:
+        dead |= (j + 1) * sel_block > i
+    if stride != sel_block and mask_own:      # decode steps (mask_own False): every cached block lies before the query
+        dead |= (i // sel_block) == j
+    return imp.masked_fill(dead, float("-inf"))
 
 
 def importance_logits_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool, causal: bool, mask_own: bool = True):
@@ -1803,26 +1901,10 @@ def importance_logits_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, sh
     compressed keys `ck` 'b hk nc d' (memory slots excluded); -inf where the reference's fill values remove the block from
     the softmax (a block not entirely before the query; the query's own block when stride != sel_block).  None when no
     full fine block exists.  Plain torch, differentiable in q and ck."""
-    b, hq, n, d = q.shape
-    hk = ck.shape[1]
-    g = hq // hk
-    npf = sel_block // stride
-    nb = ck.shape[2] // npf
-    if nb == 0:
+    if ck.shape[2] // (sel_block // stride) == 0:
         return None
-    cbar = ck[:, :, :nb * npf].float().reshape(b, hk, nb, npf, d).mean(dim=3)
-    qq = q.float().reshape(b, hk, g, n, d).mean(dim=2) if share else q.float()
-    if not share:
-        cbar = cbar.repeat_interleave(g, dim=1)
-    imp = torch.matmul(qq, cbar.transpose(-1, -2)) * (d ** -0.5)
-    i = torch.arange(n, device=q.device)[:, None]
-    j = torch.arange(nb, device=q.device)[None, :]
-    dead = torch.zeros((n, nb), dtype=torch.bool, device=q.device)
-    if causal:
-        dead |= (j + 1) * sel_block > i
-    if stride != sel_block and mask_own:      # decode steps (mask_own False): every cached block lies before the query
-        dead |= (i // sel_block) == j
-    return imp.masked_fill(dead, float("-inf"))
+    imp = _importance_products_f32(q, ck, stride, sel_block, share) * (q.shape[-1] ** -0.5)
+    return _importance_mask_f32(imp, stride, sel_block, causal, mask_own)
 
 
 @torch.no_grad()

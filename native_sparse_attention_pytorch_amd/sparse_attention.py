@@ -220,6 +220,11 @@ class SparseAttention(nn.Module):
         # the default network (flatten, linear, relu, linear) layer by layer, so that its projections go through ops.linear
         if not cls._plain(mlp, nn.Sequential):
             return mlp(windows)
+        if (len(mlp) == 4 and windows.dtype == torch.float32 and type(mlp[0]) is _FlattenWindow and cls._plain(mlp[1], nn.Linear)
+                and cls._plain(mlp[2], nn.ReLU) and not torch.is_grad_enabled() and not torch.is_autocast_enabled()):
+            x = windows.flatten(-2)
+            if ops.linear_f32_supported(x, mlp[1].weight):
+                return cls._linear(mlp[3], ops.linear_f32(x, mlp[1].weight, mlp[1].bias, act="relu"))
         for layer in mlp:
             windows = cls._linear(layer, windows)
         return windows
@@ -388,7 +393,7 @@ class SparseAttention(nn.Module):
         (cache_k, cache_v), ((cache_ck, cache_cv), (run_k, run_v)) = cache
         b, t = x.shape[0], cache_k.shape[-2]
         st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
-        M, d, f32 = self.num_mem_compress_kv, self.dim_head, torch.float32
+        f32 = torch.float32
         rq, rk = self.rotary_emb.rotate(q, offset=t), self.rotary_emb.rotate(k, offset=t)
         run_k, rk_row = _append_rows(run_k, dtype=f32, min_capacity=cbs)
         run_v, rv_row = _append_rows(run_v, dtype=f32, min_capacity=cbs)
@@ -401,20 +406,12 @@ class SparseAttention(nn.Module):
 
         # compressed branch over every cached compressed key (NSA.py:396-420); none cached: the branch is zero
         nc = cache_ck.shape[-2]
-        if nc > 0:
-            ak = torch.cat((self.compress_mem_kv[0][None].expand(b, -1, -1, -1), cache_ck), dim=-2)
-            av = torch.cat((self.compress_mem_kv[1][None].expand(b, -1, -1, -1), cache_cv), dim=-2)
-            c_out, _ = ops.dense_attend_f32(q, ak, av, 1, False, 0, st, M)
-        else:
-            c_out = torch.zeros_like(q)
+        c_out = ops.compress_attend_f32(q, cache_ck, cache_cv, self.compress_mem_kv, st, False) if nc > 0 else torch.zeros_like(q)
 
         # selected blocks + own block up to the token (NSA.py:446-515)
-        imp = None
-        if self.num_selected_blocks > 0 and nc > 0:
-            imp = ops.importance_logits_f32(q, cache_ck, st, B, self.query_heads_share_selected_kv, False, mask_own=False)
-        num_sel = min(self.num_selected_blocks, imp.shape[-1]) if imp is not None else 0
+        num_sel = min(self.num_selected_blocks, nc // (B // st))
         if num_sel > 0:
-            _, idx, fmask = ops.importance_topk(imp.contiguous(), num_sel)
+            _, idx, fmask = ops.importance_topk_f32(q, cache_ck, st, B, self.query_heads_share_selected_kv, False, num_sel, mask_own=False)
         else:
             idx = torch.zeros((b, self.kv_heads, 1, 0), dtype=torch.int32, device=x.device)
             fmask = idx.bool()
@@ -433,9 +430,7 @@ class SparseAttention(nn.Module):
             ck_row.copy_(next_ck)
             cv_row.copy_(next_cv)
 
-        gates = self.to_strategy_combine(x)                                   # 'b h 1 3' after the sigmoid
-        merged = gates[..., 0:1] * c_out + gates[..., 1:2] * f_out + gates[..., 2:3] * s_out
-        out = self.combine_heads(merged.permute(0, 2, 1, 3).reshape(b, 1, self.heads * d))
+        out = self._linear(self.combine_heads, self._gate_fp32(x, c_out, f_out, s_out))
         if not return_cache:
             return out
         return out, ((keys, vals), ((ck, cv), (run_k, run_v)))
@@ -463,7 +458,9 @@ class SparseAttention(nn.Module):
                     return t.new_zeros((b, t.shape[1], 0, cbs, d)) + pos[None, :, None]
                 return F.pad(t[..., :L, :], (0, 0, cbs - st, 0)).unfold(2, cbs, st).permute(0, 1, 2, 4, 3) + pos[None, :, None]
             kw, vw = win_of(k, self.k_intrablock_positions), win_of(v, self.v_intrablock_positions)
-        ck0, cv0 = self.k_compress(kw), self.v_compress(vw)
+        ck0, cv0 = self._compress(self.k_compress, kw), self._compress(self.v_compress, vw)
+        if not torch.is_grad_enabled():
+            return self._forward_fp32_values(x, q, k, v, rq, rk, ck0, cv0, return_cache)
         ck = torch.cat((self.compress_mem_kv[0][None].expand(b, -1, -1, -1), ck0), dim=-2)
         cv = torch.cat((self.compress_mem_kv[1][None].expand(b, -1, -1, -1), cv0), dim=-2)
         nc = ck0.shape[-2]
@@ -503,6 +500,46 @@ class SparseAttention(nn.Module):
         if co > 0:
             run_k, run_v = F.pad(run_k, (0, 0, co, 0)), F.pad(run_v, (0, 0, co, 0))
         return out, ((rk, v), ((ck0, cv0), (run_k[..., L:, :], run_v[..., L:, :])))
+
+    def _forward_fp32_values(self, x, q, k, v, rq, rk, ck0, cv0, return_cache):
+        """The attention of `_forward_fp32` without gradients: a kernel per branch, the memory rows read from the parameter, scale
+        and masks of the importance scores inside the top-k kernel, gate and head merge one kernel."""
+        b, n, _ = x.shape
+        st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
+        causal, nc = self.causal, ck0.shape[-2]
+        c_out = ops.compress_attend_f32(q, ck0, cv0, self.compress_mem_kv, st, causal)
+        num_sel = min(self.num_selected_blocks, nc // (B // st))
+        block_causal = causal
+        if num_sel > 0:
+            _, idx, fmask = ops.importance_topk_f32(q, ck0, st, B, self.query_heads_share_selected_kv, causal, num_sel)
+        elif causal:
+            idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=x.device)
+            fmask = idx.bool()
+        else:
+            idx = (torch.arange(n, device=x.device, dtype=torch.int32) // B)[None, None, :, None].expand(b, self.kv_heads, n, 1).contiguous()
+            fmask = torch.ones_like(idx, dtype=torch.bool)
+        f_out = ops.native_sparse_attend_f32(rq, rk, v, B, idx, fmask, include_block_causal=block_causal)
+        s_out, _ = ops.dense_attend_f32(rq, rk, v, 0, causal, self.sliding_window_size)
+        out = self._linear(self.combine_heads, self._gate_fp32(x, c_out, f_out, s_out))
+        if not return_cache:
+            return out
+        L, co = (n // st) * st, cbs - st
+        run_k, run_v = k, v
+        if co > 0:
+            run_k, run_v = F.pad(run_k, (0, 0, co, 0)), F.pad(run_v, (0, 0, co, 0))
+        return out, ((rk, v), ((ck0, cv0), (run_k[..., L:, :], run_v[..., L:, :])))
+
+    def _gate_fp32(self, x, c_out, f_out, s_out):
+        """Strategy gate and head merge in fp32 without gradients: 'b n (h d)'."""
+        gate = self.to_strategy_combine
+        if (self._plain(gate, nn.Sequential) and len(gate) == 3 and self._plain(gate[1], nn.Sigmoid) and type(gate[2]) is _GateLayout):
+            logits = self._linear(gate[0], x)
+            if logits.dtype == torch.float32:
+                return ops.gate_combine_f32(logits, c_out, f_out, s_out)
+        gates = gate(x)                                                        # 'b h n 3' after the sigmoid
+        b, h, n, d = c_out.shape
+        merged = gates[..., 0:1] * c_out + gates[..., 1:2] * f_out + gates[..., 2:3] * s_out
+        return merged.permute(0, 2, 1, 3).reshape(b, n, h * d)
 
     def forward(self, inp, cache=None, disable_triton_kernel=False, sliding_window_flex_mask=None,
                 fine_selection_flex_mask=None, return_cache=False):

@@ -74,3 +74,74 @@ def test_selection(b, hq, hk, n, d, B, S, causal, qoff):
     torch.cuda.synchronize()
     assert_close(got, want, 1e-5, 1e-5, "out")
     assert_close(lse, want_lse, 1e-5, 1e-5, "lse")
+
+
+@pytest.mark.parametrize("rows,k,n,bias,act", [(1, 8, 1, True, None), (31, 264, 33, True, "relu"), (32, 512, 32, False, None), (33, 72, 100, True, None),
+                                               (256, 512, 40, True, "relu")])
+def test_linear_f32(rows, k, n, bias, act):
+    """Against float64: a sum of k products, each partial sum exact to 2^-24 of the sum of magnitudes per addition."""
+    from native_sparse_attention_pytorch_amd import ops
+    wide, w, b = _rand((rows, k + 4), 1), _rand((n, k), 2) * k ** -0.5, _rand((n,), 3)
+    x = wide[:, :k]
+    assert ops.linear_f32_supported(x.to(DEV), w.to(DEV))
+    got = ops.linear_f32(wide.to(DEV)[:, :k], w.to(DEV), b.to(DEV) if bias else None, act=act)
+    torch.cuda.synchronize()
+    want = x.double() @ w.double().t() + (b.double() if bias else 0.)
+    tol = k * 2 ** -24 * (x.double().abs() @ w.double().abs().t()) + 2 ** -23 * want.abs() + 1e-12
+    want = torch.relu(want) if act else want
+    assert ((got.double().cpu() - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("b,hq,hk,n,nc,st,B,share,causal,own,S", [
+    (2, 4, 2, 70, 35, 2, 8, True, True, True, 5),
+    (1, 6, 2, 31, 15, 2, 4, True, False, True, 2),          # not causal: only the own block is hidden
+    (1, 4, 4, 40, 40, 1, 1, False, False, True, 16),        # stride = block: nothing hidden
+    (1, 4, 2, 600, 600, 1, 1, True, True, True, 17),        # k > 16: a row per wave
+    (1, 2, 1, 1, 90, 4, 12, True, False, False, 7),         # a decode step
+])
+def test_importance_topk_f32(b, hq, hk, n, nc, st, B, share, causal, own, S):
+    """Scale and masks inside the top-k kernel: bit for bit what the kernel gives on the scaled, masked logits."""
+    from native_sparse_attention_pytorch_amd import ops
+    q, ck = _rand((b, hq, n, 64), 1).to(DEV), _rand((b, hk, nc, 64), 2).to(DEV)
+    vals, idx, fm = ops.importance_topk_f32(q, ck, st, B, share, causal, S, mask_own=own)
+    wv, wi, wf = ops.importance_topk(ops.importance_logits_f32(q, ck, st, B, share, causal, mask_own=own).contiguous(), S)
+    torch.cuda.synchronize()
+    assert torch.equal(vals, wv) and torch.equal(idx, wi) and torch.equal(fm, wf)
+
+
+@pytest.mark.parametrize("b,hk,g,n,nc,d,mem,causal,qoff", [(1, 2, 3, 40, 10, 64, 1, True, 0), (2, 4, 2, 600, 37, 36, 33, True, 0), (1, 1, 4, 7, 0, 128, 2, False, 0),
+                                                           (1, 8, 1, 1, 70, 64, 5, False, 300)])
+def test_compressed_f32_memory_rows_of_their_own(b, hk, g, n, nc, d, mem, causal, qoff):
+    """Memory rows read from the parameter instead of from in front of the keys: the same bits, in both kernels."""
+    from native_sparse_attention_pytorch_amd import ops
+    q, ck, cv, m = (_rand(s, i).to(DEV) for i, s in enumerate(((b, hk * g, n, d), (b, hk, nc, d), (b, hk, nc, d), (2, hk, mem, d))))
+    got = ops.compress_attend_f32(q, ck, cv, m, 4, causal, q_offset=qoff)
+    cat = lambda i, t: torch.cat((m[i][None].expand(b, -1, -1, -1), t), dim=2)
+    want, _ = ops.dense_attend_f32(q, cat(0, ck), cat(1, cv), 1, causal, 0, 4, mem, q_offset=qoff)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
+def test_selection_of_dead_blocks_only():
+    """Not causal, every slot of some queries dead: uniform over the dead slots' blocks, padding included (NSA.py:809-815)."""
+    from native_sparse_attention_pytorch_amd.ops import native_sparse_attend_f32
+    b, hq, hk, n, d, B, S = 1, 4, 2, 50, 64, 16, 3
+    q, k, v = _rand((b, hq, n, d), 1), _rand((b, hk, n, d), 2), _rand((b, hk, n, d), 3)
+    idx = torch.randint(0, 4, (b, hk, n, S), generator=torch.Generator().manual_seed(0))
+    msk = torch.ones(b, hk, n, S, dtype=torch.bool)
+    msk[:, :, ::3] = False
+    want = O.select_attend(q.double(), k.double(), v.double(), idx, msk, B, causal=False)
+    got = native_sparse_attend_f32(q.to(DEV), k.to(DEV), v.to(DEV), B, idx.to(DEV), msk.to(DEV), include_block_causal=False)
+    torch.cuda.synchronize()
+    assert_close(got, want, 1e-5, 1e-5, "out")
+
+
+@pytest.mark.parametrize("b,h,n,d", [(1, 1, 1, 4), (2, 3, 5, 128), (1, 5, 33, 60)])
+def test_gate_f32(b, h, n, d):
+    from native_sparse_attention_pytorch_amd import ops
+    lg, c, f, s = _rand((b, n, 3 * h), 1), *(_rand((b, h, n, d), i) for i in (2, 3, 4))
+    got = ops.gate_combine_f32(*(t.to(DEV) for t in (lg, c, f, s)))
+    torch.cuda.synchronize()
+    g = lg.double().sigmoid().view(b, n, h, 3).permute(0, 2, 1, 3)
+    want = (g[..., 0:1] * c.double() + g[..., 1:2] * f.double() + g[..., 2:3] * s.double()).permute(0, 2, 1, 3).reshape(b, n, h * d)
+    assert_close(got, want, 1e-6, 1e-6, "merged")
