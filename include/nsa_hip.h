@@ -191,6 +191,10 @@ int nsa_gate_fwd(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, co
 int nsa_gate_fwd_f32(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, const float* logits, const float* c,
                      const int64_t* c_stride, const float* f, const int64_t* f_stride, const float* s, const int64_t* s_stride, float* out,
                      void* stream);
+/* its gradients: branch gradients fp32 [batch, heads, seq, dim_head] contiguous, d_out as `out`, d_logits as `logits`. */
+int nsa_gate_bwd_f32(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, const float* logits, const float* c,
+                     const int64_t* c_stride, const float* f, const int64_t* f_stride, const float* s, const int64_t* s_stride,
+                     const float* d_out, float* d_logits, float* dc, float* df, float* ds, void* stream);
 int nsa_gate_bwd(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, const void* logits,
                  const void* c, const int64_t* c_stride, const void* f, const int64_t* f_stride,
                  const void* s, const int64_t* s_stride, const void* d_out,
@@ -238,8 +242,9 @@ int nsa_windows_bwd(const void* d_windows, int32_t batch, int32_t heads, int32_t
 typedef struct nsa_qkv_desc {
   int32_t batch, seq, heads, kv_heads, dim_head;
   int32_t block, stride;  /* compression window length and step (compress_block_size, compress_block_sliding_stride); block 0: no windows */
-  int32_t fp32;           /* 1: qkv, positions, windows and d_qkv are fp32; 0: bf16; 2 (forward only): as 1, and rq / rk are
-                             written as fp32 too, q16 / v16 are not written (inputs of the fp32 forward kernels below) */
+  int32_t fp32;           /* 1: qkv, positions, windows and d_qkv are fp32; 0: bf16; 2: as 1, and rq / rk are
+                             written as fp32 too, q16 / v16 are not written (inputs of the fp32 forward kernels below); the
+                             four gradients of nsa_qkv_prep_bwd that are bf16 otherwise are then fp32 */
   int32_t offset;         /* rotary position of token 0 */
   int64_t qkv_stride[2];
 } nsa_qkv_desc;

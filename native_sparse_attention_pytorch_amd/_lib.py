@@ -112,7 +112,8 @@ def lib():
         L.nsa_gate_fwd.argtypes = [C.c_int32] * 4 + [vp, vp, i3, vp, i3, vp, i3, vp, vp]
         L.nsa_gate_bwd.argtypes = [C.c_int32] * 4 + [vp, vp, i3, vp, i3, vp, i3, vp, vp, vp, vp, vp, vp]
         L.nsa_gate_fwd_f32.argtypes = L.nsa_gate_fwd.argtypes
-        L.nsa_gate_fwd_f32.restype = C.c_int
+        L.nsa_gate_bwd_f32.argtypes = L.nsa_gate_bwd.argtypes
+        L.nsa_gate_fwd_f32.restype = L.nsa_gate_bwd_f32.restype = C.c_int
         L.nsa_rope.argtypes = [vp, i3, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp, C.c_int32, C.c_int32, vp, i3, vp]
         L.nsa_rope.restype = C.c_int
         L.nsa_decode_workspace_bytes.argtypes = [C.POINTER(DecodeDesc), C.POINTER(sz)]

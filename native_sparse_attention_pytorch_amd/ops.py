@@ -764,11 +764,22 @@ class _ImportanceTopk(torch.autograd.Function):
         return dl, None
 
 
-def importance_topk(importance_logits: Tensor, num_selected: int, prefix=None):
+def importance_topk(importance_logits: Tensor, num_selected: int, prefix=None, raw=None):
     """softmax with the -1e3 pad column (NSA.py:693-695) + topk (NSA.py:713) + `> 1e-10` mask
     (NSA.py:721).  Returns (values fp32, indices int32, fmask bool), each [..., num_selected];
     `values` is differentiable with respect to the logits.  `prefix` = (n, sel_block) as returned by
-    `compress_attend(..., prefix_only=True)`: row i is read only below column i // sel_block (no gradient)."""
+    `compress_attend(..., prefix_only=True)`: row i is read only below column i // sel_block (no gradient).
+    `raw` = (scale, seq, causal block or 0, own block or 0): the logits are fp32 products that the kernel scales and masks
+    (`importance_topk_f32`; no gradient)."""
+    if raw is not None:
+        rows = importance_logits.detach().contiguous()
+        shp = (*rows.shape[:-1], int(num_selected))
+        idx = torch.empty(shp, dtype=torch.int32, device=rows.device)
+        vals = torch.empty(shp, dtype=torch.float32, device=rows.device)
+        fm = torch.empty(shp, dtype=torch.bool, device=rows.device)
+        _lib.check(_lib.lib().nsa_importance_topk(_ptr(rows), rows.numel() // rows.shape[-1], rows.shape[-1], int(num_selected), *raw,
+                                                  _ptr(idx), _ptr(vals), _ptr(fm), _stream()), "nsa_importance_topk")
+        return vals, idx, fm
     if prefix is not None:
         if torch.compiler.is_compiling():
             idx, vals, fm = topk_prefix_op(importance_logits.detach(), int(num_selected), True, int(prefix[0]), int(prefix[1]))
@@ -1846,26 +1857,41 @@ def importance_topk_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, shar
     own = mask_own and stride != sel_block
     if nb > _TOPK_MAX_ROW or num_selected > _TOPK_MAX_K:
         return importance_topk(_importance_mask_f32(raw * (q.shape[-1] ** -0.5), stride, sel_block, causal, mask_own).contiguous(), num_selected)
-    raw = raw.contiguous()
-    shp = (*raw.shape[:-1], int(num_selected))
-    idx = torch.empty(shp, dtype=torch.int32, device=raw.device)
-    vals = torch.empty(shp, dtype=torch.float32, device=raw.device)
-    fm = torch.empty(shp, dtype=torch.bool, device=raw.device)
-    _lib.check(_lib.lib().nsa_importance_topk(_ptr(raw), raw.numel() // nb, nb, int(num_selected), q.shape[-1] ** -0.5, n, int(sel_block) if causal else 0,
-                                              int(sel_block) if own else 0, _ptr(idx), _ptr(vals), _ptr(fm), _stream()), "nsa_importance_topk")
-    return vals, idx, fm
+    return importance_topk(raw, num_selected, raw=(q.shape[-1] ** -0.5, n, int(sel_block) if causal else 0, int(sel_block) if own else 0))
 
 
-@torch.no_grad()
+class _GateF32(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, logits, c, f, s):
+        c, f, s, logits = _f32(c), _f32(f), _f32(s), logits.contiguous()
+        b, h, n, d = c.shape
+        out = torch.empty((b, n, h * d), dtype=torch.float32, device=c.device)
+        _lib.check(_lib.lib().nsa_gate_fwd_f32(b, h, n, d, _ptr(logits), _ptr(c), _s3(c), _ptr(f), _s3(f), _ptr(s), _s3(s), _ptr(out), _stream()),
+                   "nsa_gate_fwd_f32")
+        ctx.save_for_backward(logits, c, f, s)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        logits, c, f, s = ctx.saved_tensors
+        b, h, n, d = c.shape
+        if torch.is_grad_enabled():                     # a graph of the gradient is wanted: the same sums by differentiable operators
+            g = logits.sigmoid().view(b, n, h, 3).permute(0, 2, 1, 3)
+            do = dout.reshape(b, n, h, d).permute(0, 2, 1, 3)
+            dg = torch.stack([(do * t).sum(-1) for t in (c, f, s)], dim=-1) * g * (1. - g)
+            return (dg.permute(0, 2, 1, 3).reshape(logits.shape), *(g[..., i:i + 1] * do for i in range(3)))
+        dout = dout.contiguous()
+        dout = dout.clone() if dout.data_ptr() % 16 else dout
+        dl = torch.empty_like(logits)
+        dc, df, ds = (torch.empty((b, h, n, d), dtype=torch.float32, device=c.device) for _ in range(3))
+        _lib.check(_lib.lib().nsa_gate_bwd_f32(b, h, n, d, _ptr(logits), _ptr(c), _s3(c), _ptr(f), _s3(f), _ptr(s), _s3(s), _ptr(dout),
+                                               _ptr(dl), _ptr(dc), _ptr(df), _ptr(ds), _stream()), "nsa_gate_bwd_f32")
+        return dl, dc, df, ds
+
+
 def gate_combine_f32(logits: Tensor, compressed: Tensor, selected: Tensor, sliding: Tensor) -> Tensor:
     """`gate_combine` in fp32: pre-sigmoid logits 'b n (h s)', branches 'b h n d' -> 'b n (h d)'."""
-    c, f, s = _f32(compressed), _f32(selected), _f32(sliding)
-    logits = logits.contiguous()
-    b, h, n, d = c.shape
-    out = torch.empty((b, n, h * d), dtype=torch.float32, device=c.device)
-    _lib.check(_lib.lib().nsa_gate_fwd_f32(b, h, n, d, _ptr(logits), _ptr(c), _s3(c), _ptr(f), _s3(f), _ptr(s), _s3(s), _ptr(out), _stream()),
-               "nsa_gate_fwd_f32")
-    return out
+    return _GateF32.apply(logits, compressed, selected, sliding)
 
 
 def _importance_products_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool) -> Tensor:
@@ -1907,29 +1933,85 @@ def importance_logits_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, sh
     return _importance_mask_f32(imp, stride, sel_block, causal, mask_own)
 
 
-@torch.no_grad()
+def rotate_pairs(t: Tensor, freqs: Tensor, offset: int = 0) -> Tensor:
+    """Feature pairs (2k, 2k+1) of 'b h n d' rotated by (i + offset) * freqs[k], in fp32 by differentiable operators."""
+    n = t.shape[-2]
+    pos = torch.arange(offset, offset + n, device=t.device, dtype=torch.float32)
+    ang = torch.outer(pos, freqs.float())
+    cos, sin = ang.cos().repeat_interleave(2, dim=-1), ang.sin().repeat_interleave(2, dim=-1)
+    tf = t.float()
+    rot = torch.stack((-tf[..., 1::2], tf[..., 0::2]), dim=-1).flatten(-2)
+    return (tf * cos + rot * sin).to(t.dtype)
+
+
+def windows_of(t: Tensor, pos: Tensor, block: int, stride: int) -> Tensor:
+    """Compression windows 'b h w block d' of 'b h n d' + intra-window positions (NSA.py:589-603) by differentiable operators."""
+    b, h, n, d = t.shape
+    L = (n // stride) * stride
+    if L == 0:                                                    # fewer tokens than one stride: no window yet
+        return t.new_zeros((b, h, 0, block, d)) + pos[None, :, None]
+    return torch.nn.functional.pad(t[..., :L, :], (0, 0, block - stride, 0)).unfold(2, block, stride).permute(0, 1, 2, 4, 3) + pos[None, :, None]
+
+
+class _QkvPrepF32(torch.autograd.Function):
+    """`_QkvPrep` with every tensor in fp32: one kernel over the projection in each direction, instead of about fifty launches of
+    rotation, window split, their gradients and the padded sums of the gradients of q, k and v."""
+
+    @staticmethod
+    def forward(ctx, qkv, freqs, kpos, vpos, heads, kv_heads, d, block, stride, offset):
+        b, n, width = qkv.shape
+        if qkv.stride(2) != 1 or qkv.stride(1) % 8 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
+            qkv = qkv.clone(memory_format=torch.contiguous_format)
+        w = n // stride if block > 0 else 0
+        rq = torch.empty((b, heads, n, d), dtype=torch.float32, device=qkv.device)
+        rk = torch.empty((b, kv_heads, n, d), dtype=torch.float32, device=qkv.device)
+        kw = torch.empty((b, kv_heads, w, block, d), dtype=torch.float32, device=qkv.device)
+        vw = torch.empty_like(kw)
+        freqs32 = freqs.detach().to(torch.float32).contiguous()
+        kp = kpos.detach().to(torch.float32).contiguous() if w > 0 else None
+        vp = vpos.detach().to(torch.float32).contiguous() if w > 0 else None
+        dsc = _qkv_desc(qkv, heads, kv_heads, d, block, stride, offset)
+        dsc.fp32 = 2
+        _lib.check(_lib.lib().nsa_qkv_prep_fwd(C.byref(dsc), _ptr(qkv), _ptr(freqs32), _ptr(kp), _ptr(vp), None, _ptr(rq), _ptr(rk), None,
+                                               _ptr(kw) if w > 0 else None, _ptr(vw) if w > 0 else None, _stream()), "nsa_qkv_prep_fwd")
+        q = qkv[..., :heads * d].view(b, n, heads, d).permute(0, 2, 1, 3)
+        v = qkv[..., (heads + kv_heads) * d:].view(b, n, kv_heads, d).permute(0, 2, 1, 3)
+        ctx.save_for_backward(freqs32)
+        ctx.meta = ((b, n, width), heads, kv_heads, d, block, stride, offset, tuple(kpos.shape), kpos.dtype, vpos.dtype)
+        ctx.set_materialize_grads(False)
+        return q, rq, rk, v, kw, vw
+
+    @staticmethod
+    def backward(ctx, dq, drq, drk, dv, dkw, dvw):
+        (freqs32,) = ctx.saved_tensors
+        shape, heads, kv_heads, d, block, stride, offset, pos_shape, kp_dtype, vp_dtype = ctx.meta
+        grads = (dq, drq, drk, dv, dkw, dvw)
+        pos = [t.sum(dim=(0, 2)).to(dt) if need and t is not None else None
+               for t, need, dt in zip((dkw, dvw), ctx.needs_input_grad[2:4], (kp_dtype, vp_dtype))]
+        if torch.is_grad_enabled():                     # a graph of the gradient is wanted: the operation is linear in qkv
+            z = freqs32.new_zeros(shape).requires_grad_()
+            zero = freqs32.new_zeros(pos_shape)
+            q, k, v = (u.unflatten(-1, (-1, d)).transpose(1, 2) for u in z.split((heads * d, kv_heads * d, kv_heads * d), dim=-1))
+            outs = (q, rotate_pairs(q, freqs32, offset), rotate_pairs(k, freqs32, offset), v, windows_of(k, zero, block, stride),
+                    windows_of(v, zero, block, stride))
+            used = [(o, g) for o, g in zip(outs, grads) if g is not None and o.requires_grad]      # (no window: not connected)
+            dqkv = torch.autograd.grad([o for o, _ in used], z, [g for _, g in used], create_graph=True)[0] if used else torch.zeros_like(z)
+            return dqkv, None, *pos, None, None, None, None, None, None
+        ready = lambda t: None if t is None or t.numel() == 0 else t.contiguous()
+        # (a gradient handed over as a slice at an odd place is copied: the kernel reads 16 bytes at a time)
+        aligned = [t if t is None or t.data_ptr() % 16 == 0 else t.clone() for t in map(ready, grads)]
+        dqkv = torch.empty(shape, dtype=torch.float32, device=freqs32.device)
+        dsc = _qkv_desc(dqkv, heads, kv_heads, d, block, stride, offset)
+        dsc.fp32 = 2
+        _lib.check(_lib.lib().nsa_qkv_prep_bwd(C.byref(dsc), *(_ptr(t) for t in aligned), _ptr(freqs32), _ptr(dqkv), _stream()), "nsa_qkv_prep_bwd")
+        return dqkv, None, *pos, None, None, None, None, None, None
+
+
 def qkv_prep_f32(qkv: Tensor, freqs: Tensor, k_positions: Tensor, v_positions: Tensor, heads: int, kv_heads: int, dim_head: int,
                  compress_block_size: int, compress_stride: int, offset: int = 0):
     """`qkv_prep` for the fp32 forward: (q, rotated q, rotated k, v, k windows, v windows), all fp32; q and v are views of
-    the projection.  dim_head 64 or 128."""
+    the projection.  dim_head 64 or 128.  Differentiable in the projection and the positions."""
     if qkv.dtype != torch.float32 or dim_head not in (64, 128) or not qkv.is_cuda:
         raise RuntimeError("qkv_prep_f32: needs an fp32 device projection with dim_head 64 or 128")
-    b, n, width = qkv.shape
-    heads, kv_heads, d, block, stride = int(heads), int(kv_heads), int(dim_head), int(compress_block_size), int(compress_stride)
-    if qkv.stride(2) != 1 or qkv.stride(1) % 8 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
-        qkv = qkv.contiguous()
-    w = n // stride if block > 0 else 0
-    rq = torch.empty((b, heads, n, d), dtype=torch.float32, device=qkv.device)
-    rk = torch.empty((b, kv_heads, n, d), dtype=torch.float32, device=qkv.device)
-    kw = torch.empty((b, kv_heads, w, block, d), dtype=torch.float32, device=qkv.device)
-    vw = torch.empty_like(kw)
-    freqs32 = freqs.detach().to(torch.float32).contiguous()
-    kp = k_positions.detach().to(torch.float32).contiguous() if w > 0 else None
-    vp = v_positions.detach().to(torch.float32).contiguous() if w > 0 else None
-    dsc = _qkv_desc(qkv, heads, kv_heads, d, block, stride, int(offset))
-    dsc.fp32 = 2
-    _lib.check(_lib.lib().nsa_qkv_prep_fwd(C.byref(dsc), _ptr(qkv), _ptr(freqs32), _ptr(kp), _ptr(vp), None, _ptr(rq), _ptr(rk), None,
-                                           _ptr(kw) if w > 0 else None, _ptr(vw) if w > 0 else None, _stream()), "nsa_qkv_prep_fwd")
-    q = qkv[..., :heads * d].view(b, n, heads, d).permute(0, 2, 1, 3)
-    v = qkv[..., (heads + kv_heads) * d:].view(b, n, kv_heads, d).permute(0, 2, 1, 3)
-    return q, rq, rk, v, kw, vw
+    return _QkvPrepF32.apply(qkv, freqs, k_positions, v_positions, int(heads), int(kv_heads), int(dim_head), int(compress_block_size),
+                             int(compress_stride), int(offset))

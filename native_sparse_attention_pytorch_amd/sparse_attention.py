@@ -36,13 +36,7 @@ class RotaryEmbedding(nn.Module):
         self.freqs = nn.Parameter(1.0 / (theta ** (torch.arange(0, dim, 2).float() / dim)), requires_grad=False)
 
     def rotate(self, t: torch.Tensor, offset: int = 0) -> torch.Tensor:
-        n = t.shape[-2]
-        pos = torch.arange(offset, offset + n, device=t.device, dtype=torch.float32)
-        ang = torch.outer(pos, self.freqs.float())
-        cos, sin = ang.cos().repeat_interleave(2, dim=-1), ang.sin().repeat_interleave(2, dim=-1)
-        tf = t.float()
-        rot = torch.stack((-tf[..., 1::2], tf[..., 0::2]), dim=-1).flatten(-2)
-        return (tf * cos + rot * sin).to(t.dtype)
+        return ops.rotate_pairs(t, self.freqs, offset)
 
     def rotate_queries_with_cached_keys(self, q, k):
         return self.rotate(q, offset=k.shape[-2] - q.shape[-2]), self.rotate(k)
@@ -208,6 +202,12 @@ class SparseAttention(nn.Module):
         if tuple(norm.normalized_shape) != tuple(inp.shape[-1:]) or torch.is_autocast_enabled():
             return False
         return ops.rms_norm_supported(inp, norm.weight) and (inp.requires_grad or any(p.requires_grad for p in self.parameters()))
+
+    def _plain_rotary(self, batch):
+        """Rotation and window split may be the kernel's under autograd: frequencies that are not trained, no hooks, its own types."""
+        rot = self.rotary_emb
+        return (self._plain(rot, RotaryEmbedding) and not rot.freqs.requires_grad and batch <= 65535
+                and all(p.dtype == torch.float32 for p in (self.k_intrablock_positions, self.v_intrablock_positions)))
 
     def _normed(self, x):
         norm = self.norm
@@ -437,9 +437,8 @@ class SparseAttention(nn.Module):
 
     def _forward_fp32(self, x, qkv, return_cache):
         """The parallel forward of an fp32 module: every attention branch through the fp32 kernels (ops.*_f32), the gate and
-        the merge in fp32 torch - the same steps as `forward` (NSA.py:579-862).  Under autograd the values are still those of
-        the fp32 kernels and each branch's gradient comes from the bf16 kernels (ops.fp32_value_bf16_grad); rotation and
-        window split are then plain differentiable torch."""
+        the merge in fp32 - the same steps as `forward` (NSA.py:579-862).  Under autograd the values are still those of
+        the fp32 kernels and each branch's gradient comes from the bf16 kernels (ops.fp32_value_bf16_grad)."""
         b, n, _ = x.shape
         st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
         M, d = self.num_mem_compress_kv, self.dim_head
@@ -448,16 +447,13 @@ class SparseAttention(nn.Module):
         q, k, v = self._split_heads(q), self._split_heads(k), self._split_heads(v)
         L = (n // st) * st
         recording = torch.is_grad_enabled() and (qkv.requires_grad or any(p.requires_grad for p in self.parameters()))
-        if d in (64, 128) and not recording:
-            _, rq, rk, _, kw, vw = ops.qkv_prep_f32(qkv, self.rotary_emb.freqs, self.k_intrablock_positions, self.v_intrablock_positions,
-                                                    self.heads, self.kv_heads, d, cbs, st)
+        qa, va = q, v                                    # as the attention branches read them (the caches hand out q, k, v themselves)
+        if d in (64, 128) and (not recording or self._plain_rotary(b)):
+            qa, rq, rk, va, kw, vw = ops.qkv_prep_f32(qkv, self.rotary_emb.freqs, self.k_intrablock_positions, self.v_intrablock_positions,
+                                                      self.heads, self.kv_heads, d, cbs, st)
         else:
             rq, rk = self.rotary_emb.rotate(q), self.rotary_emb.rotate(k)
-            def win_of(t, pos):
-                if L == 0:                                                    # fewer tokens than one stride: no window yet
-                    return t.new_zeros((b, t.shape[1], 0, cbs, d)) + pos[None, :, None]
-                return F.pad(t[..., :L, :], (0, 0, cbs - st, 0)).unfold(2, cbs, st).permute(0, 1, 2, 4, 3) + pos[None, :, None]
-            kw, vw = win_of(k, self.k_intrablock_positions), win_of(v, self.v_intrablock_positions)
+            kw, vw = ops.windows_of(k, self.k_intrablock_positions, cbs, st), ops.windows_of(v, self.v_intrablock_positions, cbs, st)
         ck0, cv0 = self._compress(self.k_compress, kw), self._compress(self.v_compress, vw)
         if not torch.is_grad_enabled():
             return self._forward_fp32_values(x, q, k, v, rq, rk, ck0, cv0, return_cache)
@@ -465,18 +461,15 @@ class SparseAttention(nn.Module):
         cv = torch.cat((self.compress_mem_kv[1][None].expand(b, -1, -1, -1), cv0), dim=-2)
         nc = ck0.shape[-2]
         c_out = ops.fp32_value_bf16_grad(lambda q_, k_, v_: ops.dense_attend_f32(q_, k_, v_, 1, causal, 0, st, M)[0],
-                                         lambda q_, k_, v_: ops.compress_attend(q_, k_, v_, M, st, causal)[0], q, ck, cv)
-        imp = None
-        if self.num_selected_blocks > 0 and nc > 0:
-            imp = ops.importance_logits_f32(q, ck0, st, B, share, causal)
-            if imp is not None and not self.use_diff_topk:
-                imp = imp.detach()
-        num_sel = min(self.num_selected_blocks, imp.shape[-1]) if imp is not None else 0
+                                         lambda q_, k_, v_: ops.compress_attend(q_, k_, v_, M, st, causal)[0], qa, ck, cv)
+        num_sel = min(self.num_selected_blocks, nc // (B // st))
         gates = None
         if num_sel > 0:
-            vals, idx, fmask = ops.importance_topk(imp.contiguous(), num_sel)
             if self.use_diff_topk:
+                vals, idx, fmask = ops.importance_topk(ops.importance_logits_f32(qa, ck0, st, B, share, causal).contiguous(), num_sel)
                 gates = vals + (1. - vals).detach()                              # straight-through gates (NSA.py:715)
+            else:
+                _, idx, fmask = ops.importance_topk_f32(qa, ck0, st, B, share, causal, num_sel)
             block_causal = causal
         elif causal:
             idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=x.device)
@@ -487,12 +480,10 @@ class SparseAttention(nn.Module):
         sel32 = lambda q_, k_, v_, *g_: ops.native_sparse_attend_f32(q_, k_, v_, B, idx, fmask, include_block_causal=block_causal)
         sel16 = lambda q_, k_, v_, *g_: ops.native_sparse_attend(q_, k_, v_, B, idx, fmask, sel_scale=g_[0] if g_ else None,
                                                                  include_block_causal=block_causal)
-        f_out = ops.fp32_value_bf16_grad(sel32, sel16, rq, rk, v, *(() if gates is None else (gates,)))
+        f_out = ops.fp32_value_bf16_grad(sel32, sel16, rq, rk, va, *(() if gates is None else (gates,)))
         s_out = ops.fp32_value_bf16_grad(lambda q_, k_, v_: ops.dense_attend_f32(q_, k_, v_, 0, causal, win)[0],
-                                         lambda q_, k_, v_: ops.sliding_attend(q_, k_, v_, win, causal=causal), rq, rk, v)
-        gates3 = self.to_strategy_combine(x)                                  # 'b h n 3' after the sigmoid
-        merged = gates3[..., 0:1] * c_out + gates3[..., 1:2] * f_out + gates3[..., 2:3] * s_out
-        out = self.combine_heads(merged.permute(0, 2, 1, 3).reshape(b, n, self.heads * d))
+                                         lambda q_, k_, v_: ops.sliding_attend(q_, k_, v_, win, causal=causal), rq, rk, va)
+        out = self.combine_heads(self._gate_fp32(x, c_out, f_out, s_out))
         if not return_cache:
             return out
         co = cbs - st
@@ -530,9 +521,9 @@ class SparseAttention(nn.Module):
         return out, ((rk, v), ((ck0, cv0), (run_k[..., L:, :], run_v[..., L:, :])))
 
     def _gate_fp32(self, x, c_out, f_out, s_out):
-        """Strategy gate and head merge in fp32 without gradients: 'b n (h d)'."""
+        """Strategy gate and head merge in fp32: 'b n (h d)'."""
         gate = self.to_strategy_combine
-        if (self._plain(gate, nn.Sequential) and len(gate) == 3 and self._plain(gate[1], nn.Sigmoid) and type(gate[2]) is _GateLayout):
+        if (self._plain(gate, nn.Sequential) and len(gate) == 3 and self._plain(gate[1], nn.Sigmoid) and self._plain(gate[2], _GateLayout)):
             logits = self._linear(gate[0], x)
             if logits.dtype == torch.float32:
                 return ops.gate_combine_f32(logits, c_out, f_out, s_out)

@@ -145,3 +145,72 @@ def test_gate_f32(b, h, n, d):
     g = lg.double().sigmoid().view(b, n, h, 3).permute(0, 2, 1, 3)
     want = (g[..., 0:1] * c.double() + g[..., 1:2] * f.double() + g[..., 2:3] * s.double()).permute(0, 2, 1, 3).reshape(b, n, h * d)
     assert_close(got, want, 1e-6, 1e-6, "merged")
+
+
+def _grads(outs, leaves, douts, **kw):
+    used = [(o, g) for o, g in zip(outs, douts) if g is not None]
+    return torch.autograd.grad([o for o, _ in used], leaves, [g for _, g in used], **kw)
+
+
+@pytest.mark.parametrize("b,h,n,d", [(1, 1, 1, 4), (2, 3, 5, 128), (1, 5, 33, 60)])
+def test_gate_f32_gradients(b, h, n, d):
+    """Against float64; also with a graph of the gradient, which takes other operators.  A sum of d products: d + 8 roundings of
+    the magnitudes (the sigmoid and its products among them)."""
+    from native_sparse_attention_pytorch_amd import ops
+    host = [_rand((b, n, 3 * h), 1), *(_rand((b, h, n, d), i) for i in (2, 3, 4))]
+    do = _rand((b, n, h * d), 5)
+
+    def merged(lg, c, f, s):
+        g = lg.sigmoid().view(b, n, h, 3).permute(0, 2, 1, 3)
+        return (g[..., 0:1] * c + g[..., 1:2] * f + g[..., 2:3] * s).permute(0, 2, 1, 3).reshape(b, n, h * d)
+
+    ref = [t.double().requires_grad_() for t in host]
+    want = torch.autograd.grad(merged(*ref), ref, do.double())
+    mags = [t.double().abs().requires_grad_() for t in host]
+    big = torch.autograd.grad(merged(*mags), mags, do.double().abs())
+    wide = torch.zeros(b, n, 3 * h * d).to(DEV)
+    wide[..., 1:1 + h * d] = do.to(DEV)                    # a gradient that is neither contiguous nor aligned
+    for graph in (False, True):
+        leaves = [t.to(DEV).requires_grad_() for t in host]
+        got = torch.autograd.grad(ops.gate_combine_f32(*leaves), leaves, wide[..., 1:1 + h * d], create_graph=graph)
+        torch.cuda.synchronize()
+        for w, g, m in zip(want, got, big):
+            assert ((g.double().cpu() - w).abs() <= (d + 8) * 2 ** -24 * (m.abs() + w.abs() + m.abs().max()) + 1e-30).all()
+
+
+@pytest.mark.parametrize("b,hq,hk,n,d,cbs,st,offset,missing", [
+    (1, 4, 2, 1, 64, 4, 2, 0, ()),                  # fewer tokens than a stride: no window
+    (2, 2, 1, 33, 64, 16, 8, 0, ()), (1, 3, 1, 70, 128, 6, 4, 5, ()), (1, 2, 2, 37, 128, 4, 4, 0, (0, 4)), (2, 8, 4, 130, 64, 5, 1, 0, (1, 2, 3)),
+])
+def test_qkv_prep_f32_gradients(b, hq, hk, n, d, cbs, st, offset, missing):
+    """Against float64 of the operators it stands for, outputs and gradients, gradients left out among them, and with a graph of
+    the gradient.  An angle is off by a rounding of its size (n + offset at most), a sum has at most 4 + cbs / st terms; the
+    gradients of the positions sum b * windows of them."""
+    from native_sparse_attention_pytorch_amd import ops
+    qkv, kp, vp = _rand((b, n, (hq + 2 * hk) * d), 1), _rand((hk, cbs, d), 2), _rand((hk, cbs, d), 3)
+    freqs = 1.0 / (10000 ** (torch.arange(0, d, 2).float() / d))
+    douts = [None if i in missing else _rand((b, h, n, d), 4 + i) for i, h in enumerate((hq, hq, hk, hk))]
+    douts += [None if i in missing else _rand((b, hk, n // st, cbs, d), 4 + i) for i in (4, 5)]
+
+    def parts(z, kp, vp):
+        q, k, v = (u.unflatten(-1, (-1, d)).transpose(1, 2) for u in z.split((hq * d, hk * d, hk * d), dim=-1))
+        ang = torch.outer(torch.arange(offset, offset + n).double(), freqs.double())
+        cos, sin = ang.cos().repeat_interleave(2, -1), ang.sin().repeat_interleave(2, -1)
+        rot = lambda t: t * cos + torch.stack((-t[..., 1::2], t[..., 0::2]), -1).flatten(-2) * sin
+        return q, rot(q), rot(k), v, ops.windows_of(k, kp, cbs, st), ops.windows_of(v, vp, cbs, st)
+
+    ref = [t.double().requires_grad_() for t in (qkv, kp, vp)]
+    outs = parts(*ref)
+    want = _grads(outs, ref, [None if g is None else g.double() for g in douts], allow_unused=True)
+    tol = 2 ** -24 * (2 * (n + offset) + 16) * 5 * (4 + -(-cbs // st))
+    for graph in (False, True):
+        leaves = [t.to(DEV).requires_grad_() for t in (qkv, kp, vp)]
+        mine = ops.qkv_prep_f32(leaves[0], freqs.to(DEV), leaves[1], leaves[2], hq, hk, d, cbs, st, offset)
+        got = _grads(mine, leaves, [None if g is None else g.to(DEV) for g in douts], allow_unused=True, create_graph=graph)
+        torch.cuda.synchronize()
+        for o, w in zip(mine, outs):
+            assert o.shape == w.shape and ((o.detach().double().cpu() - w.detach()).abs() <= tol).all()
+        for i, (g, w) in enumerate(zip(got, want)):
+            assert (g is None) == (w is None)
+            if g is not None:
+                assert ((g.double().cpu() - w).abs() <= (tol if i == 0 else tol * b * max(1, n // st))).all()
