@@ -158,6 +158,16 @@ int nsa_compress_topk_supported(const nsa_dense_desc* d, int32_t num_selected);
 int nsa_compress_topk_fwd(const nsa_dense_desc* d, const void* q, const void* k, const void* v, void* out, float* lse,
                           int32_t num_selected, int32_t* idx, uint8_t* fmask, void* stream);
 
+/* Gradient of nsa_topk's values (with the softmax) with respect to the logits: logits, d_logits fp32 [rows, nb]; idx (the k
+ * different entries of a row), d_vals fp32 [rows, k].  nb <= 2048. */
+int nsa_importance_topk_bwd(const float* logits, int64_t rows, int32_t nb, int32_t k, const int32_t* idx, const float* d_vals,
+                            float* d_logits, void* stream);
+/* out = bf16(base + c * small), small's rows repeated: base (fp32 or bf16) and out [batch, heads, rows, d] contiguous (out may be
+ * base), small fp32 [batch, heads / head_repeat, small_rows, d]; row r takes small's row (r - row_offset) / row_repeat, rows outside
+ * keep base.  d a multiple of 8, 16-byte aligned. */
+int nsa_add_repeated(const void* base, int32_t base_fp32, int32_t batch, int32_t heads, int32_t rows, int32_t d, const float* small,
+                     int32_t head_repeat, int32_t row_offset, int32_t row_repeat, int32_t small_rows, float c, void* out, void* stream);
+
 /* Block-importance softmax + per-query top-k.  Replaces NSA.py:693-695 (pad -1e3, softmax, drop
  * pad), :713 (topk) and :721 (fmask = value > 1e-10).  scores: fp32 [rows, nb]; with
  * apply_softmax != 0 they are importance logits (-inf = not selectable), otherwise ready

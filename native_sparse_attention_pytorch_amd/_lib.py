@@ -94,6 +94,10 @@ def lib():
         L.nsa_topk.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         L.nsa_topk_prefix.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         L.nsa_importance_topk.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, C.c_float, C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
+        L.nsa_importance_topk_bwd.argtypes = [vp, C.c_int64, C.c_int32, C.c_int32, vp, vp, vp, vp]
+        L.nsa_add_repeated.argtypes = [vp, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp, C.c_int32, C.c_int32, C.c_int32, C.c_int32,
+                                       C.c_float, vp, vp]
+        L.nsa_importance_topk_bwd.restype = L.nsa_add_repeated.restype = C.c_int
         L.nsa_linear_f32.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, vp, C.c_int32, vp, vp]
         L.nsa_importance_topk.restype = L.nsa_linear_f32.restype = C.c_int
         fp = C.POINTER(C.c_float)

@@ -368,6 +368,117 @@ static int topk_launch(const float* scores, int64_t rows, int32_t nb, int32_t k,
   return e == hipSuccess ? 0 : (int)e;
 }
 
+namespace nsa {
+// Gradient of the selected values with respect to the logits: dl_j = p_j (dfull_j - sum_k p_idx(k) dvals_k), p the padded softmax,
+// dfull the values' gradients at their places.  A wave per row; the row and dfull stay in LDS between the three sweeps, so memory
+// sees one read and one write of the row.  32768 rows of 64, k = 4 (17 MB): 15 us, bound by its three
+// dependent reductions; as operators 70 us in 12 launches.
+__global__ __launch_bounds__(256) void topk_bwd_kernel(const float* __restrict__ logits, long rows, int nb, int k, const int* __restrict__ idx,
+                                                       const float* __restrict__ dvals, float* __restrict__ dlogits) {
+  extern __shared__ float topk_bwd_s[];                  // per wave: row, dfull
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long row = (long)blockIdx.x * 4 + wave;
+  if (row >= rows) return;                               // (no work-group barrier follows)
+  float* x = topk_bwd_s + (size_t)wave * 2 * nb;
+  float* df = x + nb;
+  const float* src = logits + row * nb;
+  float mx = -1e3f;                                      // the pad column
+  for (int j = lane; j < nb; j += 64) {
+    const float t = src[j];
+    x[j] = t;
+    df[j] = 0.f;
+    mx = fmaxf(mx, t);
+  }
+#pragma unroll
+  for (int mk = 32; mk >= 1; mk >>= 1) mx = fmaxf(mx, __shfl_xor(mx, mk, 64));
+  float sum = 0.f;
+  for (int j = lane; j < nb; j += 64) {
+    const float t = expf(x[j] - mx);
+    x[j] = t;
+    sum += t;
+  }
+#pragma unroll
+  for (int mk = 32; mk >= 1; mk >>= 1) sum += __shfl_xor(sum, mk, 64);
+  const float inv = 1.0f / (sum + expf(-1e3f - mx));
+  __builtin_amdgcn_wave_barrier();                       // LDS operations of one wave execute in order
+  float dot = 0.f;
+  for (int s = lane; s < k; s += 64) {
+    const int j = idx[row * k + s];
+    if (j < 0 || j >= nb) continue;
+    const float g = dvals[row * k + s];
+    df[j] = g;                                           // the k places of a row differ
+    dot += x[j] * inv * g;
+  }
+#pragma unroll
+  for (int mk = 32; mk >= 1; mk >>= 1) dot += __shfl_xor(dot, mk, 64);
+  __builtin_amdgcn_wave_barrier();
+  for (int j = lane; j < nb; j += 64) dlogits[row * nb + j] = x[j] * inv * (df[j] - dot);
+}
+
+// out = base + c * small, small's rows repeated: row r of head h takes row (r - off) / rdiv of head h / hdiv where that is one of
+// its `srows` rows.  The importance gradient joining the attention's: one launch for scale, repeat,
+// cast, sum, cast (five, 25-30 us at 8 x 1024 tokens x 8 heads x 64): 6.5 us there, HBM-bound.
+struct AddRepArgs { long total; int heads, rows, d8, hdiv, off, rdiv, srows; float c; };
+
+template <typename TB>
+__global__ __launch_bounds__(256) void add_repeated_kernel(const AddRepArgs A, const TB* base, const float* __restrict__ small, __bf16* out) {
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= A.total) return;
+  const int piece = (int)(t % A.d8);
+  const long row = t / A.d8;
+  const int r = (int)(row % A.rows) - A.off, sr = r >= 0 ? r / A.rdiv : -1;
+  const long bh = row / A.rows, b = bh / A.heads;
+  const int h = (int)(bh - b * A.heads);
+  float x[8];
+  if constexpr (sizeof(TB) == 4) {
+    const floatx4 lo = *reinterpret_cast<const floatx4*>(base + t * 8), hi = *reinterpret_cast<const floatx4*>(base + t * 8 + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { x[e] = lo[e]; x[4 + e] = hi[e]; }
+  } else {
+    const bf16x8 v = load8(base + t * 8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = (float)v[e];
+  }
+  if (sr >= 0 && sr < A.srows) {
+    const float* sp = small + (((b * (A.heads / A.hdiv) + h / A.hdiv) * A.srows + sr) * A.d8 + piece) * 8;
+    const floatx4 lo = *reinterpret_cast<const floatx4*>(sp), hi = *reinterpret_cast<const floatx4*>(sp + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { x[e] += A.c * lo[e]; x[4 + e] += A.c * hi[e]; }
+  }
+  bf16x8 v;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = (__bf16)x[e];
+  *reinterpret_cast<bf16x8*>(out + t * 8) = v;
+}
+}  // namespace nsa
+
+extern "C" int nsa_importance_topk_bwd(const float* logits, int64_t rows, int32_t nb, int32_t k, const int32_t* idx, const float* d_vals,
+                                       float* d_logits, void* stream) {
+  if (!logits || !idx || !d_vals || !d_logits || rows <= 0 || nb <= 0 || k <= 0 || k > nb) return NSA_E_ARG;
+  if (nb > 64 * 32 || rows > (int64_t)4 * 0x7fffffff) return NSA_E_UNSUPPORTED;           // (2 x 4 rows of LDS: 64 KB at most)
+  hipLaunchKernelGGL(nsa::topk_bwd_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), (size_t)8 * nb * sizeof(float), (hipStream_t)stream, logits,
+                     (long)rows, nb, k, idx, d_vals, d_logits);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : (int)e;
+}
+
+extern "C" int nsa_add_repeated(const void* base, int32_t base_fp32, int32_t batch, int32_t heads, int32_t rows, int32_t d, const float* small,
+                                int32_t head_repeat, int32_t row_offset, int32_t row_repeat, int32_t small_rows, float c, void* out, void* stream) {
+  if (!base || !small || !out || batch <= 0 || heads <= 0 || rows <= 0 || d <= 0 || head_repeat <= 0 || heads % head_repeat || row_offset < 0 ||
+      row_repeat <= 0 || small_rows <= 0)
+    return NSA_E_ARG;
+  if (d % 8 || ((uintptr_t)base | (uintptr_t)small | (uintptr_t)out) % 16) return NSA_E_UNSUPPORTED;
+  const long total = (long)batch * heads * rows * (d / 8);
+  if ((total + 255) / 256 > 0x7fffffffl) return NSA_E_UNSUPPORTED;
+  const nsa::AddRepArgs A{total, heads, rows, d / 8, head_repeat, row_offset, row_repeat, small_rows, c};
+  const dim3 grid((unsigned)((total + 255) / 256)), block(256);
+  hipStream_t st = (hipStream_t)stream;
+  if (base_fp32) hipLaunchKernelGGL((nsa::add_repeated_kernel<float>), grid, block, 0, st, A, (const float*)base, small, (__bf16*)out);
+  else hipLaunchKernelGGL((nsa::add_repeated_kernel<__bf16>), grid, block, 0, st, A, (const __bf16*)base, small, (__bf16*)out);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : (int)e;
+}
+
 extern "C" int nsa_topk(const float* scores, int64_t rows, int32_t nb, int32_t k, int32_t apply_softmax,
                         int32_t* idx, float* vals, uint8_t* fmask, void* stream) {
   return topk_launch(scores, rows, nb, k, apply_softmax, nsa::TopkMask{1, 0, 0, 1.f}, idx, vals, fmask, stream);

@@ -448,30 +448,45 @@ def _dense_setup(ctx, inputs, output):
     ctx.set_materialize_grads(False)
 
 
-def _importance_backward(q, ck, dpooled, num_mem, stride, sel_block, share, scale):
+def _importance_products_backward(q, ck, dpooled, num_mem, stride, sel_block, share, scale):
     """Gradient of the importance logits (NSA.py:652-680: mean of the scaled logits over a fine
     block's npf compressed keys and, if shared, the group's heads) with respect to q and ck.  The
     logits are linear in both, so this is two small dense GEMMs per (batch, kv head); entries that
-    were -inf carry zero gradient by construction of the softmax that follows."""
+    were -inf carry zero gradient by construction of the softmax that follows.  Returns (dq 'b hk n d' (shared) or 'b hq n d', dck
+    'b hk nb d' of every key of a block, c): both still to be multiplied by c."""
     b, hq, n, d = q.shape
     hk = ck.shape[1]
     g = hq // hk
     nb = dpooled.shape[-1]
     npf = sel_block // stride
     dp = torch.nan_to_num(dpooled.float(), nan=0.0, posinf=0.0, neginf=0.0)
-    ckb = ck[:, :, num_mem:num_mem + nb * npf].float().reshape(b, hk, nb, npf, d).sum(dim=3)       # [b,hk,nb,d]
-    qf = q.float()
+    ckb = ck[:, :, num_mem:num_mem + nb * npf].unflatten(2, (nb, npf)).sum(dim=3, dtype=torch.float32)        # [b,hk,nb,d]
     if share:
-        c = scale / (g * npf)
-        dq = (c * torch.matmul(dp, ckb)).repeat_interleave(g, dim=1)                                # every head of the group
-        dckb = c * torch.matmul(dp.transpose(-1, -2), qf.reshape(b, hk, g, n, d).sum(dim=2))         # [b,hk,nb,d]
-    else:
-        c = scale / npf
-        dq = c * torch.matmul(dp, ckb.repeat_interleave(g, dim=1))
-        dckb = c * torch.matmul(dp.transpose(-1, -2), qf).reshape(b, hk, g, nb, d).sum(dim=2)
+        dq = torch.matmul(dp, ckb)
+        dckb = torch.matmul(dp.transpose(-1, -2), q.unflatten(1, (hk, g)).sum(dim=2, dtype=torch.float32))   # [b,hk,nb,d]
+        return dq, dckb, scale / (g * npf)
+    dq = torch.matmul(dp, ckb.repeat_interleave(g, dim=1))
+    dckb = torch.matmul(dp.transpose(-1, -2), q.float()).unflatten(1, (hk, g)).sum(dim=2)
+    return dq, dckb, scale / npf
+
+
+def _importance_backward(q, ck, dpooled, num_mem, stride, sel_block, share, scale):
+    """(dq, dck) of `_importance_products_backward`, shaped as q and ck, in fp32."""
+    npf, nb = sel_block // stride, dpooled.shape[-1]
+    dq, dckb, c = _importance_products_backward(q, ck, dpooled, num_mem, stride, sel_block, share, scale)
+    dq = c * dq
     dck = torch.zeros_like(ck, dtype=torch.float32)
-    dck[:, :, num_mem:num_mem + nb * npf] = dckb.repeat_interleave(npf, dim=2)
-    return dq, dck
+    dck[:, :, num_mem:num_mem + nb * npf] = (c * dckb).repeat_interleave(npf, dim=2)
+    return (dq.repeat_interleave(q.shape[1] // ck.shape[1], dim=1) if share else dq), dck
+
+
+def _add_repeated(base: Tensor, small: Tensor, out: Tensor, head_repeat: int, row_offset: int, row_repeat: int, c: float) -> Tensor:
+    """out (bf16, may be base) = base + c * small, small's heads and rows repeated (nsa_add_repeated)."""
+    b, h, n, d = base.shape
+    small = small.contiguous()
+    _lib.check(_lib.lib().nsa_add_repeated(_ptr(base), int(base.dtype == torch.float32), b, h, n, d, _ptr(small), head_repeat, row_offset, row_repeat,
+                                           small.shape[2], float(c), _ptr(out), _stream()), "nsa_add_repeated")
+    return out
 
 
 def _dense_backward(ctx, dout, dlse, dpooled):
@@ -484,7 +499,12 @@ def _dense_backward(ctx, dout, dlse, dpooled):
         # importance term has been added
         dq, dk, dv = _direct(dense_bwd)(q, k, v, out, dout, lse, mode, causal, window, stride, num_mem, scale,
                                         mode == 1 and dpooled is not None and dpooled.numel() > 0)
-    if dpooled is not None and dpooled.numel() > 0:
+    if dq is not None and dpooled is not None and dpooled.numel() > 0 and not torch.compiler.is_compiling() and not torch.is_grad_enabled():
+        # both sums in one kernel each: scale, repetition over the group's heads / the block's keys, sum in fp32, one rounding
+        dq2, dckb, c = _importance_products_backward(q, k, dpooled, num_mem, stride, sel_block, share, scale)
+        dq = _add_repeated(dq, dq2, dq, q.shape[1] // dq2.shape[1], 0, 1, c)
+        dk = _add_repeated(dk, dckb, torch.empty(dk.shape, dtype=_BF16, device=dk.device), 1, num_mem, sel_block // stride, c)
+    elif dpooled is not None and dpooled.numel() > 0:
         dq2, dk2 = _importance_backward(q, k, dpooled, num_mem, stride, sel_block, share, scale)
         dq = dq2.to(q.dtype) if dq is None else (dq.float() + dq2).to(q.dtype)
         dk = dk2 if dk is None else dk.float() + dk2
@@ -743,9 +763,26 @@ def _(scores, k, apply_softmax, seq, block):
     return (scores.new_empty(shp, dtype=torch.int32), scores.new_empty(shp), scores.new_empty(shp, dtype=torch.uint8))
 
 
+@torch.library.custom_op("nsa_amd::topk_bwd", mutates_args=())
+def topk_bwd(logits: Tensor, idx: Tensor, dvals: Tensor) -> Tensor:
+    logits, idx, dvals = logits.contiguous(), idx.contiguous(), dvals.to(torch.float32).contiguous()
+    out = torch.empty_like(logits)
+    nb, k = logits.shape[-1], idx.shape[-1]
+    if out.numel():
+        _lib.check(_lib.lib().nsa_importance_topk_bwd(_ptr(logits), logits.numel() // nb, nb, k, _ptr(idx), _ptr(dvals), _ptr(out), _stream()),
+                   "nsa_importance_topk_bwd")
+    return out
+
+
+@topk_bwd.register_fake
+def _(logits, idx, dvals):
+    return logits.new_empty(logits.shape)
+
+
 class _ImportanceTopk(torch.autograd.Function):
-    """HIP top-k in the forward; the backward of `values` through the padded softmax (plain
-    elementwise torch, O(rows * nb)) - only used for the differentiable top-k gates."""
+    """HIP top-k in the forward; the backward of `values` through the padded softmax is one kernel (twelve elementwise launches
+    as operators, which rows of more than 2048 entries and a graph of the gradient still take) - only used for the differentiable
+    top-k gates."""
 
     @staticmethod
     def forward(ctx, logits, k):
@@ -757,6 +794,8 @@ class _ImportanceTopk(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dvals, _didx, _dfm):
         logits, idx = ctx.saved_tensors
+        if logits.shape[-1] <= _TOPK_MAX_ROW and not torch.is_grad_enabled():
+            return _direct(topk_bwd)(logits, idx, dvals), None
         padded = torch.nn.functional.pad(logits, (1, 0), value=-1e3)
         p = padded.softmax(dim=-1)[..., 1:]                     # -inf entries -> exactly 0
         dfull = torch.zeros_like(p).scatter_add_(-1, idx.long(), dvals.to(p.dtype))

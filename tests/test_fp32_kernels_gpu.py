@@ -214,3 +214,39 @@ def test_qkv_prep_f32_gradients(b, hq, hk, n, d, cbs, st, offset, missing):
             assert (g is None) == (w is None)
             if g is not None:
                 assert ((g.double().cpu() - w).abs() <= (tol if i == 0 else tol * b * max(1, n // st))).all()
+
+
+@pytest.mark.parametrize("rows,nb,k", [(1, 1, 1), (5, 3, 3), (7, 64, 4), (33, 65, 17), (3, 2048, 64), (2, 2049, 3)])
+def test_importance_topk_gradient(rows, nb, k):
+    """Against float64 of softmax with the pad column; rows with nothing to select and masked entries among them.  A product of a
+    probability (exp to 2 ulp, a sum of nb) and a difference of two sums of k terms."""
+    from native_sparse_attention_pytorch_amd import ops
+    x, dv = _rand((rows, nb), 1), _rand((rows, k), 2)
+    x[torch.rand(rows, nb, generator=torch.Generator().manual_seed(3)) < 0.2] = -math.inf
+    x[rows // 2] = -math.inf
+    for graph in (False, True):
+        leaf = x.to(DEV).requires_grad_()
+        vals, idx, _ = ops.importance_topk(leaf, k)
+        got, = torch.autograd.grad(vals, leaf, dv.to(DEV), create_graph=graph)
+        torch.cuda.synchronize()
+        p = torch.nn.functional.pad(x.double(), (1, 0), value=-1e3).softmax(-1)[:, 1:]
+        full = torch.zeros(rows, nb, dtype=torch.float64).scatter_add_(-1, idx.cpu().long(), dv.double())
+        dot = (p * full).sum(-1, keepdim=True)
+        tol = 2 ** -24 * (nb + k + 16) * p * (full.abs() + (p * full.abs()).sum(-1, keepdim=True)) + 1e-30
+        assert ((got.double().cpu() - p * (full - dot)).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("b,h,n,d,hrep,off,rrep,srows,base32", [(1, 1, 1, 8, 1, 0, 1, 1, False), (2, 4, 9, 64, 2, 0, 1, 9, False), (2, 6, 23, 128, 1, 2, 4, 5, True),
+                                                                (1, 3, 37, 64, 3, 1, 3, 12, True)])
+def test_add_repeated(b, h, n, d, hrep, off, rrep, srows, base32):
+    """bf16(base + c * small), rounded once; in place where the base is bf16."""
+    from native_sparse_attention_pytorch_amd import ops
+    base = _rand((b, h, n, d), 1) if base32 else _rand((b, h, n, d), 1).bfloat16()
+    small = _rand((b, h // hrep, srows, d), 2)
+    want = base.double().clone()
+    rep = small.double().repeat_interleave(hrep, 1).repeat_interleave(rrep, 2)
+    want[:, :, off:off + srows * rrep] += 0.3 * rep
+    dev = base.to(DEV)
+    got = ops._add_repeated(dev, small.to(DEV), torch.empty_like(dev, dtype=torch.bfloat16) if base32 else dev, hrep, off, rrep, 0.3)
+    torch.cuda.synchronize()
+    assert ((got.double().cpu() - want).abs() <= want.abs() * (2 ** -8 + 2 ** -20) + 2 ** -20).all()
