@@ -81,12 +81,14 @@ struct RowsStage { floatx4 x[16]; };
 // this lane's 16 bytes of rows 4 r + lane / 16, r = 0 .. 15, of the tile whose rows `rows_s` lists.  `special` (wave-uniform): some
 // of them are padding keys (row -1: zeros) or memory rows of an array of their own (row -2 - m: row m of `mem`), or this piece's
 // chunks reach past the head dimension (zeros).
+template <bool FULL>
 __device__ __forceinline__ void rows_load(RowsStage& st, const float* __restrict__ base, long stride, const float* __restrict__ mem, int d,
-                                          const int* __restrict__ rows_s, int r0, int col, bool inside, bool special) {
+                                          const int* __restrict__ rows_s, int r0, int col, bool inside, bool special, int quarters) {
   const float* bc = base + (inside ? col : 0);
   if (!special) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) st.x[r] = *reinterpret_cast<const floatx4*>(bc + (long)rows_s[4 * r + r0] * stride);
+    for (int r = 0; r < 16; ++r)
+      if (FULL || r < 4 || r / 4 < quarters) st.x[r] = *reinterpret_cast<const floatx4*>(bc + (long)rows_s[4 * r + r0] * stride);
   } else {
     const float* mc = mem + (inside ? col : 0);
 #pragma unroll
@@ -127,25 +129,39 @@ __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ 
     rows_s[lane] = row;
     __builtin_amdgcn_wave_barrier();
   };
+  // A tile's rows move 16 at a time and the last tile leaves out those that no key needs (with small blocks it holds little but
+  // the own block: 1 to 16 of 64 keys at a block of 16).  Rows of LDS that were left out hold old values: as keys they give scores
+  // that are masked, as values they are not multiplied.  4 blocks of 16 keys and the own one, 2 heads, d = 64, 32768
+  // queries: 195 -> 168 us; 17 blocks of 64 keys: the same as before (478 us, 16424 queries).
+  // (The full tiles' code holds no branch for it: with one around every quarter 17 blocks of 64 keys took 4 % longer.)
+  auto quarters_of = [&](int t) { return DT > 1 || special ? 4 : __builtin_amdgcn_readfirstlane((min(total - 64 * t, 64) + 15) >> 4); };
+  int quarters = 4;
   RowsStage st;
-  auto load_k = [&](int ft) {
-    rows_load(st, kb, A.sk[2], mk, A.d, rows_s, r0, 64 * ft + 4 * chunk, 64 * ft + 4 * chunk < A.d, special || 64 * (ft + 1) > A.d);
+  auto load_k = [&](auto full, int ft) {
+    rows_load<decltype(full)::value>(st, kb, A.sk[2], mk, A.d, rows_s, r0, 64 * ft + 4 * chunk, 64 * ft + 4 * chunk < A.d, special || 64 * (ft + 1) > A.d, quarters);
   };
-  auto load_v = [&](int ft) {
-    rows_load(st, vb, A.sv[2], mv, A.d, rows_s, r0, 64 * ft + 4 * chunk, 64 * ft + 4 * chunk < A.d, special || 64 * (ft + 1) > A.d);
+  auto load_v = [&](auto full, int ft) {
+    rows_load<decltype(full)::value>(st, vb, A.sv[2], mv, A.d, rows_s, r0, 64 * ft + 4 * chunk, 64 * ft + 4 * chunk < A.d, special || 64 * (ft + 1) > A.d, quarters);
   };
+  using Full = std::integral_constant<bool, true>;
+  using Part = std::integral_constant<bool, false>;
   locate(first);
-  load_k(0);
-  for (int t = first; t < tiles; t += step) {
+  quarters = quarters_of(first);
+  if (DT > 1 || quarters == 4) load_k(Full{}, 0);
+  else load_k(Part{}, 0);
+  auto tile = [&](auto full, int t) {
+    constexpr bool FULL = decltype(full)::value;
+    const int here = quarters;                           // of tile t; `quarters` moves on with the loads
     floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ft = 0; ft < DT; ++ft) {
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int r = 0; r < 16; ++r) *reinterpret_cast<floatx4*>(piece + (4 * r + r0) * 64 + 4 * (chunk ^ ((4 * r + r0) & 15))) = st.x[r];
+      for (int r = 0; r < 16; ++r)
+        if (FULL || r < 4 || r / 4 < here) *reinterpret_cast<floatx4*>(piece + (4 * r + r0) * 64 + 4 * (chunk ^ ((4 * r + r0) & 15))) = st.x[r];
       __builtin_amdgcn_wave_barrier();
-      if (ft + 1 < DT) load_k(ft + 1);
-      else load_v(0);
+      if (ft + 1 < DT) load_k(full, ft + 1);
+      else load_v(full, 0);
 #pragma unroll
       for (int c = 0; c < 16; ++c) {
         const floatx4 kx = *reinterpret_cast<const floatx4*>(piece + lane * 64 + 4 * (c ^ (lane & 15)));
@@ -177,24 +193,35 @@ __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ 
     for (int ft = 0; ft < DT; ++ft) {
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int r = 0; r < 16; ++r) *reinterpret_cast<floatx4*>(piece + (4 * r + r0) * 64 + 4 * chunk) = st.x[r];
+      for (int r = 0; r < 16; ++r)
+        if (FULL || r < 4 || r / 4 < here) *reinterpret_cast<floatx4*>(piece + (4 * r + r0) * 64 + 4 * chunk) = st.x[r];
       __builtin_amdgcn_wave_barrier();
-      if (ft + 1 < DT) load_v(ft + 1);
+      if (ft + 1 < DT) load_v(full, ft + 1);
       else if (t + step < tiles) {
         locate(t + step);
-        load_k(0);
+        quarters = quarters_of(t + step);
+        if (DT > 1 || quarters == 4) load_k(Full{}, 0);
+        else load_k(Part{}, 0);
       }
       floatx4 o0 = S.acc[ft] * al, o1 = {0.f, 0.f, 0.f, 0.f};
-      static_for<0, 16>([&](auto blk) {
-        constexpr int b = decltype(blk)::value;
-        const float* vr = piece + 4 * b * 64 + lane;
-        o0 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[0], vr[0], o0, 4, b, 0);
-        o1 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[1], vr[64], o1, 4, b, 0);
-        o0 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[2], vr[128], o0, 4, b, 0);
-        o1 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[3], vr[192], o1, 4, b, 0);
+      static_for<0, 4>([&](auto quarter) {
+        constexpr int qd = decltype(quarter)::value;
+        if (FULL || qd == 0 || qd < here)
+          static_for<4 * qd, 4 * qd + 4>([&](auto blk) {
+            constexpr int b = decltype(blk)::value;
+            const float* vr = piece + 4 * b * 64 + lane;
+            o0 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[0], vr[0], o0, 4, b, 0);
+            o1 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[1], vr[64], o1, 4, b, 0);
+            o0 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[2], vr[128], o0, 4, b, 0);
+            o1 = __builtin_amdgcn_mfma_f32_4x4x1f32(p[3], vr[192], o1, 4, b, 0);
+          });
       });
       S.acc[ft] = o0 + o1;
     }
+  };
+  for (int t = first; t < tiles; t += step) {
+    if (DT > 1 || quarters == 4) tile(Full{}, t);
+    else tile(Part{}, t);
   }
 }
 
