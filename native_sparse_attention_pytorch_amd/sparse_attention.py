@@ -257,8 +257,15 @@ class SparseAttention(nn.Module):
             residual = residual.contiguous()
         if gate.weight.shape != (3 * self.heads, dim) or freqs.dtype not in (bf16, torch.float32) or not freqs.is_contiguous():
             return None
-        for c in (cache_k, cache_v, cache_ck, cache_cv, run_k, run_v):
-            if c.dtype != bf16 or c.shape[3] != d or c.device != device:
+        hk = self.kv_heads
+        if (qkv.weight.shape != (hd + 2 * hk * d, dim) or out.weight.shape != (dim, hd) or freqs.shape != (d // 2,)
+                or mem.dim() != 4 or mem.shape[1] != hk or mem.shape[3] != d):
+            return None
+        # the kernels take batch, heads and lengths from one tensor of each pair
+        for c, v in ((cache_k, cache_v), (cache_ck, cache_cv), (run_k, run_v)):
+            if c.shape != v.shape or c.dim() != 4 or c.shape[:2] != (b, hk) or c.shape[3] != d:
+                return None
+            if c.dtype != bf16 or v.dtype != bf16 or c.device != device or v.device != device:
                 return None
         st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
         nc, npf = cache_ck.shape[2], B // st

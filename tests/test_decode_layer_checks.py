@@ -1,0 +1,61 @@
+"""What `SparseAttention._decode_whole` may hand to the kernels: caches and weights whose shapes agree.  The library call takes batch,
+heads and lengths from one tensor of each pair, so everything else goes to the general path, which refuses it."""
+import pytest
+import torch
+from torch import nn
+
+from native_sparse_attention_pytorch_amd import SparseAttention, ops
+
+BF16 = torch.bfloat16
+
+
+def _layer_and_cache(b=4, n=40, hk=2, d=64):
+    m = SparseAttention(dim=128, dim_head=d, heads=4, kv_heads=hk, causal=True, sliding_window_size=16, compress_block_size=16,
+                        compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2).to(BF16)
+    z = lambda rows, batch=b, heads=hk, width=d: torch.zeros(batch, heads, rows, width, dtype=BF16)
+    return m, z, ((z(n), z(n)), ((z(n // 8), z(n // 8)), (z(8), z(8))))
+
+
+@pytest.fixture
+def reached(monkeypatch):
+    calls = []
+
+    def decode_step(*args, layer=None, **kwargs):
+        calls.append(layer)
+        return (torch.zeros_like(layer.x),)
+
+    monkeypatch.setattr(ops, "decode_step", decode_step)
+    return calls
+
+
+def _run(m, cache, b=4):
+    with torch.no_grad():
+        return m._decode_whole(torch.zeros(b, 1, 128, dtype=BF16), cache)
+
+
+def test_matching_shapes_take_the_call(reached):
+    m, _, cache = _layer_and_cache()
+    assert _run(m, cache) is not None and len(reached) == 1
+
+
+@pytest.mark.parametrize("pair", [0, 1, 2])
+@pytest.mark.parametrize("member", [0, 1])
+@pytest.mark.parametrize("change", ["batch", "heads", "rows"])
+def test_caches_that_disagree_do_not(reached, pair, member, change):
+    m, z, ((k, v), ((ck, cv), (rk, rv))) = _layer_and_cache()
+    pairs = [[k, v], [ck, cv], [rk, rv]]
+    rows = pairs[pair][member].shape[2]
+    pairs[pair][member] = dict(batch=z(rows, batch=2), heads=z(rows, heads=1), rows=z(rows - 1))[change]
+    assert _run(m, (tuple(pairs[0]), (tuple(pairs[1]), tuple(pairs[2])))) is None and not reached
+
+
+def test_all_caches_of_another_batch_do_not(reached):
+    m, _, cache = _layer_and_cache(b=2)
+    assert _run(m, cache) is None and not reached
+
+
+@pytest.mark.parametrize("name, features", [("to_qkv", (128, 256)), ("to_qkv", (64, 512)), ("combine_heads", (256, 64)), ("combine_heads", (128, 128))])
+def test_replaced_projections_of_another_size_do_not(reached, name, features):
+    m, _, cache = _layer_and_cache()
+    setattr(m, name, nn.Linear(*features, bias=False).to(BF16))
+    assert _run(m, cache) is None and not reached

@@ -104,3 +104,14 @@ def test_selection_order(nb, k, scores):
     q = torch.ones(1, hq, 1, d, dtype=BF16, device=DEV)
     got, want, probs = _step(1, hq, hk, d, 4 * nb, nb, 1, 4, k, True, 16, 1, ck=ck, q=q)
     _check(got, want, probs, exact=True)
+
+
+@pytest.mark.parametrize("wrong", ["batch", "heads"])
+def test_caches_of_another_shape_are_refused(wrong):
+    from native_sparse_attention_pytorch_amd import ops
+    z = lambda *s: torch.zeros(*s, dtype=BF16, device=DEV)
+    b, hk = (1, 2) if wrong == "batch" else (2, 1)
+    q, k, gl, freqs = z(2, 4, 1, 64), z(2, 2, 1, 64), z(2, 1, 12), torch.zeros(32, device=DEV)
+    with pytest.raises(RuntimeError, match="batch, heads"):
+        ops.decode_step(q, k, k, freqs, 8, z(b, hk, 9, 64), z(b, hk, 9, 64), None, None, None, None, None, None, gl, per_block=2, block=16, num_sel=2,
+                        share=True, window=16)
