@@ -1619,7 +1619,8 @@ def skinny_linear_supported(x: Tensor, weight: Tensor) -> bool:
     """A projection of a few rows (a decode step) that `skinny_linear` serves."""
     rows, k = x.numel() // x.shape[-1], x.shape[-1]
     return bool(x.is_cuda and x.dtype == _BF16 and weight.dtype == _BF16 and weight.is_contiguous() and weight.data_ptr() % 16 == 0
-                and weight.shape[1] == k and 1 <= rows <= 32 and k % 32 == 0 and rows * (k + 8) <= 65536)
+                and weight.dim() == 2 and weight.shape[1] == k and weight.device == x.device and 1 <= rows <= 32 and k % 32 == 0
+                and rows * (k + 8) <= 65536)
 
 
 _ACTS = {None: 0, "gelu": 1, "relu": 2}
@@ -1629,6 +1630,8 @@ def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_we
                   act: str | None = None, residual: Tensor | None = None) -> Tensor:
     """act(linear(rms_norm(x), weight, bias)) + residual for at most 32 rows in one kernel (see nsa_skinny_linear): a bf16
     projection of a decode step with what stands around it, every part optional.  Inference only (no autograd)."""
+    _check_linear("skinny_linear", x, weight, bias, norm_weight)
+    bias, norm_weight = (t if t is None else t.contiguous() for t in (bias, norm_weight))
     k, n = x.shape[-1], weight.shape[0]
     x2 = _rms_rows(x)
     rows = x2.shape[0]
@@ -1667,11 +1670,27 @@ def linear_f32_supported(x: Tensor, weight: Tensor) -> bool:
     (the library's call takes the host 14 us longer), 384 x 256 -> 256 4.8 / 6.1, 256 x 1024 -> 1024 12.3 / 9.1."""
     rows, k = x.numel() // max(x.shape[-1], 1), x.shape[-1]
     return bool(x.is_cuda and x.dtype == torch.float32 and weight.dtype == torch.float32 and weight.is_contiguous() and 0 < rows <= 256 and k <= 512 and k % 8 == 0
-                and weight.data_ptr() % 16 == 0)
+                and weight.dim() == 2 and weight.shape[1] == k and weight.device == x.device and weight.data_ptr() % 16 == 0)
+
+
+def _check_linear(name: str, x: Tensor, weight: Tensor, *others):
+    """What the projection kernels take for granted; the library's F.linear refuses the same (`others`: bias, norm weight)."""
+    if weight.dim() != 2 or weight.shape[1] != x.shape[-1]:
+        raise RuntimeError(f"{name}: weight {tuple(weight.shape)} does not take inputs {tuple(x.shape)}")
+    for t, size in zip(others, (weight.shape[0], weight.shape[1])):
+        if t is not None and (t.shape != (size,) or t.dtype != x.dtype or t.device != x.device):
+            raise RuntimeError(f"{name}: bias and norm weight are vectors of the projection's own width, type and device")
+
+
+def _transformed() -> bool:
+    """Inside vmap, jvp or another functorch transform, or a forward-mode level: operators carry what a kernel would lose."""
+    return torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
 
 
 def linear_f32(x: Tensor, weight: Tensor, bias: Tensor | None = None, act: str | None = None) -> Tensor:
     """act(linear(x, weight, bias)) in fp32 by nsa_linear_f32 (few rows, no gradient)."""
+    _check_linear("linear_f32", x, weight, bias)
+    bias = bias if bias is None else bias.contiguous()
     k, n = x.shape[-1], weight.shape[0]
     x2 = x.reshape(-1, k)
     if x2.stride(1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
@@ -1711,7 +1730,9 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     """torch.nn.functional.linear with the split weight-gradient GEMM (see _Linear)."""
     if (not (torch.is_grad_enabled() and weight.requires_grad) or torch.compiler.is_compiling() or x.dtype != weight.dtype
             or torch.is_autocast_enabled()):               # under autocast the library casts the operands itself
-        if not torch.is_grad_enabled() and linear_f32_supported(x, weight) and not torch.compiler.is_compiling() and not torch.is_autocast_enabled():
+        if (not torch.is_grad_enabled() and linear_f32_supported(x, weight) and not torch.compiler.is_compiling()
+                and not torch.is_autocast_enabled() and not _transformed()
+                and (bias is None or (bias.shape == weight.shape[:1] and bias.dtype == x.dtype and bias.device == x.device))):
             return linear_f32(x, weight, bias)
         return torch.nn.functional.linear(x, weight, bias)
     return _Linear.apply(x, weight, bias)
