@@ -1900,8 +1900,11 @@ def compress_attend_f32(q: Tensor, ck: Tensor, cv: Tensor, mem: Tensor, stride: 
     q, ck, cv = _f32(q), _f32(ck), _f32(cv)
     b, hq, n, d = q.shape
     _check_f32_dim(d)
-    mem = mem.contiguous()
-    hk, m = mem.shape[1], mem.shape[2]
+    mem = mem.to(torch.float32).contiguous()
+    mem = mem.clone() if mem.data_ptr() % 16 else mem             # (a parameter that is a slice of a larger buffer)
+    hk, m = ck.shape[1], mem.shape[2]
+    if mem.shape != (2, hk, m, d) or cv.shape != ck.shape or ck.shape[0] != b or ck.shape[3] != d or mem.device != q.device:
+        raise RuntimeError("compress_attend_f32: memory rows '2 hk m d' and compressed keys / values 'b hk nc d' of the queries' batch and features")
     out = torch.empty((b, hq, n, d), dtype=torch.float32, device=q.device)
     dsc = _dense_desc(q, ck, cv, out, out, 1, bool(causal), 0, int(stride), 0, False, 1, True, float(d ** -0.5))
     dsc.num_mem, dsc.num_keys = m, ck.shape[2]
@@ -1955,6 +1958,9 @@ class _GateF32(torch.autograd.Function):
 
 def gate_combine_f32(logits: Tensor, compressed: Tensor, selected: Tensor, sliding: Tensor) -> Tensor:
     """`gate_combine` in fp32: pre-sigmoid logits 'b n (h s)', branches 'b h n d' -> 'b n (h d)'."""
+    b, h, n, _ = compressed.shape
+    if logits.dtype != torch.float32 or logits.shape != (b, n, 3 * h) or selected.shape != compressed.shape or sliding.shape != compressed.shape:
+        raise RuntimeError("gate_combine_f32: fp32 logits 'b n (h 3)' and three branches 'b h n d'")
     return _GateF32.apply(logits, compressed, selected, sliding)
 
 

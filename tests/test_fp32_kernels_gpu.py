@@ -122,6 +122,20 @@ def test_compressed_f32_memory_rows_of_their_own(b, hk, g, n, nc, d, mem, causal
     assert torch.equal(got, want)
 
 
+def test_compressed_f32_memory_rows_elsewhere():
+    """A parameter that is a slice at an odd place, or of another type, gives the same rows; one of another shape is refused."""
+    from native_sparse_attention_pytorch_amd import ops
+    q, ck, cv, m = (_rand(s, i).to(DEV) for i, s in enumerate(((1, 4, 9, 64), (1, 2, 4, 64), (1, 2, 4, 64), (2, 2, 3, 64))))
+    want = ops.compress_attend_f32(q, ck, cv, m.bfloat16().float(), 4, True)
+    odd = torch.empty(m.numel() + 1, device=DEV)[1:].view(m.shape).copy_(m.bfloat16())
+    assert odd.data_ptr() % 16
+    for t in (odd, m.bfloat16()):
+        assert torch.equal(ops.compress_attend_f32(q, ck, cv, t, 4, True), want)
+    for t in (m[:, :1], m[..., :32], m[:1]):
+        with pytest.raises(RuntimeError):
+            ops.compress_attend_f32(q, ck, cv, t, 4, True)
+
+
 def test_selection_of_dead_blocks_only():
     """Not causal, every slot of some queries dead: uniform over the dead slots' blocks, padding included (NSA.py:809-815)."""
     from native_sparse_attention_pytorch_amd.ops import native_sparse_attend_f32
@@ -145,6 +159,15 @@ def test_gate_f32(b, h, n, d):
     g = lg.double().sigmoid().view(b, n, h, 3).permute(0, 2, 1, 3)
     want = (g[..., 0:1] * c.double() + g[..., 1:2] * f.double() + g[..., 2:3] * s.double()).permute(0, 2, 1, 3).reshape(b, n, h * d)
     assert_close(got, want, 1e-6, 1e-6, "merged")
+
+
+def test_gate_f32_refuses():
+    from native_sparse_attention_pytorch_amd import ops
+    z = lambda *s: torch.zeros(*s, device=DEV)
+    t = z(1, 4, 5, 64)
+    for lg, f in ((z(1, 5, 9), t), (z(1, 4, 12), t), (z(1, 5, 12).bfloat16(), t), (z(1, 5, 12), z(1, 4, 4, 64))):
+        with pytest.raises(RuntimeError):
+            ops.gate_combine_f32(lg, t, f, t)
 
 
 def _grads(outs, leaves, douts, **kw):
