@@ -72,6 +72,17 @@ def _grown(t: torch.Tensor, min_capacity: int = 128) -> torch.Tensor:
     return _append_rows(t, min_capacity=min_capacity)[0]
 
 
+def _open_window(t: torch.Tensor, complete: int, overlap: int) -> torch.Tensor:
+    """Rows of the compression window that is still open after `complete` tokens: the last `overlap` of those (zeros before the
+    first) and what follows, as a copy that does not hold on to the projection.  A 30011-token prompt's k and v, 61 MB each, were
+    padded whole for the 38 rows of it (120 us of a prefill's 6.8 ms, and the 123 MB stayed allocated with the cache)."""
+    if overlap <= 0:
+        return t[..., complete:, :]
+    if complete >= overlap:
+        return t[..., complete - overlap:, :].clone(memory_format=torch.contiguous_format)
+    return F.pad(t, (0, 0, overlap - complete, 0))
+
+
 class _FlattenWindow(nn.Module):
     def forward(self, x):                                   # 'b h w n d -> b h w (n d)'
         return x.flatten(-2)
@@ -493,11 +504,7 @@ class SparseAttention(nn.Module):
         out = self.combine_heads(self._gate_fp32(x, c_out, f_out, s_out))
         if not return_cache:
             return out
-        co = cbs - st
-        run_k, run_v = k, v
-        if co > 0:
-            run_k, run_v = F.pad(run_k, (0, 0, co, 0)), F.pad(run_v, (0, 0, co, 0))
-        return out, ((rk, v), ((ck0, cv0), (run_k[..., L:, :], run_v[..., L:, :])))
+        return out, ((rk, v), ((ck0, cv0), (_open_window(k, L, cbs - st), _open_window(v, L, cbs - st))))
 
     def _forward_fp32_values(self, x, q, k, v, rq, rk, ck0, cv0, return_cache):
         """The attention of `_forward_fp32` without gradients: a kernel per branch, the memory rows read from the parameter, scale
@@ -521,11 +528,8 @@ class SparseAttention(nn.Module):
         out = self._linear(self.combine_heads, self._gate_fp32(x, c_out, f_out, s_out))
         if not return_cache:
             return out
-        L, co = (n // st) * st, cbs - st
-        run_k, run_v = k, v
-        if co > 0:
-            run_k, run_v = F.pad(run_k, (0, 0, co, 0)), F.pad(run_v, (0, 0, co, 0))
-        return out, ((rk, v), ((ck0, cv0), (run_k[..., L:, :], run_v[..., L:, :])))
+        L = (n // st) * st
+        return out, ((rk, v), ((ck0, cv0), (_open_window(k, L, cbs - st), _open_window(v, L, cbs - st))))
 
     def _gate_fp32(self, x, c_out, f_out, s_out):
         """Strategy gate and head merge in fp32: 'b n (h d)'."""
@@ -639,8 +643,4 @@ class SparseAttention(nn.Module):
 
         if not return_cache:
             return out
-        co = cbs - st
-        run_k, run_v = k, v
-        if co > 0:
-            run_k, run_v = F.pad(run_k, (0, 0, co, 0)), F.pad(run_v, (0, 0, co, 0))
-        return out, ((rk16.to(k.dtype), v), ((ck0, cv0), (run_k[..., L:, :], run_v[..., L:, :])))
+        return out, ((rk16.to(k.dtype), v), ((ck0, cv0), (_open_window(k, L, cbs - st), _open_window(v, L, cbs - st))))

@@ -2,6 +2,7 @@
 buffer with spare rows; appending takes a spare row in place, and any tensor that is not the
 live prefix of such a buffer (a prefill cache, an older tuple at a branch point, a full buffer)
 is copied into a new buffer first, so tensors handed out earlier never change."""
+import pytest
 import torch
 
 from native_sparse_attention_pytorch_amd.sparse_attention import _append_rows
@@ -108,3 +109,16 @@ def test_append_rows_into_wider_buffers():
     again, row2 = _append_rows(full, feat=64)
     assert again.data_ptr() == full.data_ptr() and again.shape == (2, 3, 7, 64)       # in place: same buffer
     assert torch.equal(again[:, :, 5], torch.ones(2, 3, 64, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("n, st, cbs", [(1, 2, 4), (7, 8, 16), (8, 8, 16), (37, 8, 32), (40, 8, 32), (41, 8, 8), (64, 16, 16), (2053, 16, 32)])
+def test_open_window_is_the_padded_sequence_from_the_last_complete_stride(n, st, cbs):
+    from native_sparse_attention_pytorch_amd.sparse_attention import _open_window
+    proj = torch.randn(2, n, 3 * 8, generator=torch.Generator().manual_seed(n))
+    t = proj.view(2, n, 3, 8).permute(0, 2, 1, 3)
+    L = n // st * st
+    got = _open_window(t, L, cbs - st)
+    assert torch.equal(got, torch.nn.functional.pad(t, (0, 0, cbs - st, 0))[..., L:, :])
+    if cbs > st:                                            # a copy: the cache neither changes with the projection nor keeps it
+        proj.zero_()
+        assert got.untyped_storage().data_ptr() != proj.untyped_storage().data_ptr()
