@@ -251,7 +251,7 @@ class SparseAttention(nn.Module):
         (cache_k, cache_v), ((cache_ck, cache_cv), (run_k, run_v)) = cache
         norm, qkv, gate, out, bf16 = self.norm, self.to_qkv, self.to_strategy_combine[0], self.combine_heads, torch.bfloat16
         plain, d = self._plain, self.dim_head
-        if not (d in (64, 128) and inp.dtype == bf16 and plain(norm, nn.RMSNorm) and plain(qkv, nn.Linear) and plain(gate, nn.Linear)
+        if not (d in (64, 128) and inp.is_cuda and inp.dtype == bf16 and plain(norm, nn.RMSNorm) and plain(qkv, nn.Linear) and plain(gate, nn.Linear)
                 and plain(out, nn.Linear) and qkv.bias is None and norm.weight is not None and inp.dim() == 3 and inp.shape[1] == 1):
             return None
         b, dim, hd = inp.shape[0], inp.shape[2], self.heads * d
@@ -266,7 +266,8 @@ class SparseAttention(nn.Module):
             inp = inp.clone(memory_format=torch.contiguous_format)
         if residual is not None and not residual.is_contiguous():
             residual = residual.contiguous()
-        if gate.weight.shape != (3 * self.heads, dim) or freqs.dtype not in (bf16, torch.float32) or not freqs.is_contiguous():
+        if (gate.weight.shape != (3 * self.heads, dim) or freqs.dtype not in (bf16, torch.float32) or not freqs.is_contiguous()
+                or freqs.device != device):
             return None
         hk = self.kv_heads
         if (qkv.weight.shape != (hd + 2 * hk * d, dim) or out.weight.shape != (dim, hd) or freqs.shape != (d // 2,)

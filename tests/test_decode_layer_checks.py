@@ -5,6 +5,7 @@ import torch
 from torch import nn
 
 from native_sparse_attention_pytorch_amd import SparseAttention, ops
+from native_sparse_attention_pytorch_amd.transformer import Transformer
 
 BF16 = torch.bfloat16
 
@@ -28,9 +29,14 @@ def reached(monkeypatch):
     return calls
 
 
+class OnDevice(torch.Tensor):
+    """A CPU tensor that says it lies on the GPU: with the library call replaced nothing reads its address."""
+    is_cuda = True
+
+
 def _run(m, cache, b=4):
     with torch.no_grad():
-        return m._decode_whole(torch.zeros(b, 1, 128, dtype=BF16), cache)
+        return m._decode_whole(torch.zeros(b, 1, 128, dtype=BF16).as_subclass(OnDevice), cache)
 
 
 def test_matching_shapes_take_the_call(reached):
@@ -59,3 +65,24 @@ def test_replaced_projections_of_another_size_do_not(reached, name, features):
     m, _, cache = _layer_and_cache()
     setattr(m, name, nn.Linear(*features, bias=False).to(BF16))
     assert _run(m, cache) is None and not reached
+
+
+def test_host_tensors_never_reach_the_library(reached):
+    """The library takes addresses: a layer, its caches or its frequencies in host memory are refused, whatever the grad mode."""
+    m, _, cache = _layer_and_cache()
+    with torch.no_grad():
+        assert m._decode_whole(torch.zeros(4, 1, 128, dtype=BF16), cache) is None
+        with pytest.raises(RuntimeError, match="GPU only"):
+            m(torch.zeros(4, 1, 128, dtype=BF16), cache=cache)
+    m.rotary_emb.freqs = nn.Parameter(m.rotary_emb.freqs.to("meta"), requires_grad=False)
+    assert _run(m, cache) is None and not reached
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_model_in_host_memory_is_refused(reached, grad):
+    m = Transformer(num_tokens=16, dim=128, depth=2, heads=4, kv_heads=2, sparse_attn_kwargs=dict(
+        sliding_window_size=16, compress_block_size=16, compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2)).to(BF16)
+    _, _, cache = _layer_and_cache()
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="GPU only"):
+        m(torch.zeros(4, 1, dtype=torch.long), cache=[cache, cache])
+    assert not reached
