@@ -251,8 +251,8 @@ class SparseAttention(nn.Module):
         (cache_k, cache_v), ((cache_ck, cache_cv), (run_k, run_v)) = cache
         norm, qkv, gate, out, bf16 = self.norm, self.to_qkv, self.to_strategy_combine[0], self.combine_heads, torch.bfloat16
         plain, d = self._plain, self.dim_head
-        if not (d in (64, 128) and inp.is_cuda and inp.dtype == bf16 and plain(norm, nn.RMSNorm) and plain(qkv, nn.Linear) and plain(gate, nn.Linear)
-                and plain(out, nn.Linear) and qkv.bias is None and norm.weight is not None and inp.dim() == 3 and inp.shape[1] == 1):
+        if not (self.causal and d in (64, 128) and inp.is_cuda and inp.dtype == bf16 and plain(norm, nn.RMSNorm) and plain(qkv, nn.Linear)
+                and plain(gate, nn.Linear) and plain(out, nn.Linear) and qkv.bias is None and norm.weight is not None and inp.dim() == 3 and inp.shape[1] == 1):
             return None
         b, dim, hd = inp.shape[0], inp.shape[2], self.heads * d
         mem, freqs, device = self.compress_mem_kv, self.rotary_emb.freqs, inp.device

@@ -86,3 +86,14 @@ def test_a_model_in_host_memory_is_refused(reached, grad):
     with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="GPU only"):
         m(torch.zeros(4, 1, dtype=torch.long), cache=[cache, cache])
     assert not reached
+
+
+def test_a_model_that_is_not_causal_is_refused(reached, monkeypatch):
+    m = Transformer(num_tokens=16, dim=128, depth=1, heads=4, kv_heads=2, causal=False, sparse_attn_kwargs=dict(
+        sliding_window_size=16, compress_block_size=16, compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2)).to(BF16)
+    embedded = torch.zeros(4, 1, 128, dtype=BF16).as_subclass(OnDevice)
+    monkeypatch.setattr(m.token_emb, "forward", lambda ids: embedded)
+    _, _, cache = _layer_and_cache()
+    with torch.no_grad(), pytest.raises(AssertionError, match="autoregressive"):
+        m(torch.zeros(4, 1, dtype=torch.long), cache=[cache])
+    assert not reached
