@@ -271,7 +271,8 @@ class SparseAttention(nn.Module):
             return None
         hk = self.kv_heads
         if (qkv.weight.shape != (hd + 2 * hk * d, dim) or out.weight.shape != (dim, hd) or freqs.shape != (d // 2,)
-                or mem.dim() != 4 or mem.shape[1] != hk or mem.shape[3] != d):
+                or norm.weight.shape != (dim,) or mem.dim() != 4 or mem.shape[:2] != (2, hk) or mem.shape[3] != d
+                or (gate.bias is not None and gate.bias.shape != (3 * self.heads,)) or (out.bias is not None and out.bias.shape != (dim,))):
             return None
         # the kernels take batch, heads and lengths from one tensor of each pair
         for c, v in ((cache_k, cache_v), (cache_ck, cache_cv), (run_k, run_v)):

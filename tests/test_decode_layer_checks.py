@@ -97,3 +97,13 @@ def test_a_model_that_is_not_causal_is_refused(reached, monkeypatch):
     with torch.no_grad(), pytest.raises(AssertionError, match="autoregressive"):
         m(torch.zeros(4, 1, dtype=torch.long), cache=[cache])
     assert not reached
+
+
+@pytest.mark.parametrize("name, shape", [("to_strategy_combine.0.bias", (1,)), ("to_strategy_combine.0.bias", (6,)), ("combine_heads.bias", (1,)),
+                                         ("norm.weight", (1,)), ("compress_mem_kv", (1, 2, 1, 64))])
+def test_replaced_vectors_of_another_size_do_not(reached, name, shape):
+    """The kernels read a whole vector from each; the layers broadcast or refuse the others."""
+    m, _, cache = _layer_and_cache()
+    owner, _, leaf = name.rpartition(".")
+    setattr(m.get_submodule(owner), leaf, nn.Parameter(torch.zeros(shape, dtype=BF16)))
+    assert _run(m, cache) is None and not reached
