@@ -1615,12 +1615,17 @@ def rms_norm(x: Tensor, weight: Tensor, eps: float | None = None) -> Tensor:
 
 # ------------------------------------------------------------------ projections
 
-def skinny_linear_supported(x: Tensor, weight: Tensor) -> bool:
-    """A projection of a few rows (a decode step) that `skinny_linear` serves."""
-    rows, k = x.numel() // x.shape[-1], x.shape[-1]
-    return bool(x.is_cuda and x.dtype == _BF16 and weight.dtype == _BF16 and weight.is_contiguous() and weight.data_ptr() % 16 == 0
-                and weight.dim() == 2 and weight.shape[1] == k and weight.device == x.device and 1 <= rows <= 32 and k % 32 == 0
-                and rows * (k + 8) <= 65536)
+def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
+    """A weight the projection kernels read where it lies: rows of `width`, x's type and device, contiguous from a 16-byte boundary on."""
+    return bool(weight.dtype == x.dtype and weight.device == x.device and weight.dim() == 2 and weight.shape[1] == width
+                and weight.shape[0] > 0 and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+
+
+def skinny_linear_supported(x: Tensor, weight: Tensor, width: int | None = None) -> bool:
+    """A projection of a few rows (a decode step) that `skinny_linear` serves.  `width`: the input is not x itself but as many rows
+    of this many features, x's own projection."""
+    rows, k = x.numel() // x.shape[-1], x.shape[-1] if width is None else width
+    return x.is_cuda and x.dtype == _BF16 and 1 <= rows <= 32 and k % 32 == 0 and rows * (k + 8) <= 65536 and _weight_ready(x, k, weight)
 
 
 _ACTS = {None: 0, "gelu": 1, "relu": 2}
@@ -1630,7 +1635,8 @@ def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_we
                   act: str | None = None, residual: Tensor | None = None) -> Tensor:
     """act(linear(rms_norm(x), weight, bias)) + residual for at most 32 rows in one kernel (see nsa_skinny_linear): a bf16
     projection of a decode step with what stands around it, every part optional.  Inference only (no autograd)."""
-    _check_linear("skinny_linear", x, weight, bias, norm_weight)
+    _check_linear("skinny_linear", _BF16, x, weight, bias, norm_weight)
+    weight = _laid_out(weight)
     bias, norm_weight = (t if t is None else t.contiguous() for t in (bias, norm_weight))
     k, n = x.shape[-1], weight.shape[0]
     x2 = _rms_rows(x)
@@ -1639,7 +1645,7 @@ def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_we
         residual = residual.reshape(rows, n)
         if residual.dtype != _BF16 or residual.stride(1) != 1:
             raise RuntimeError("skinny_linear: the residual must be bf16 with unit stride")
-    y = torch.empty((*x.shape[:-1], n), dtype=_BF16, device=x.device)
+    y = x.new_empty((*x.shape[:-1], n))
     _lib.check(_lib.lib().nsa_skinny_linear(rows, k, n, x2.data_ptr(), x2.stride(0), _ptr(norm_weight), eps, weight.data_ptr(), _ptr(bias), _ACTS[act],
                                             _ptr(residual), 0 if residual is None else residual.stride(0), y.data_ptr(), n, _stream()),
                "nsa_skinny_linear")
@@ -1669,12 +1675,18 @@ def linear_f32_supported(x: Tensor, weight: Tensor) -> bool:
     library in us: 240 x 256 -> 256 4.8 / 64.7, 240 x 512 -> 24 6.2 / 19.9, 62 x 512 -> 1536 6.7 / 6.8, 256 x 512 -> 1536 11.6 / 8.5
     (the library's call takes the host 14 us longer), 384 x 256 -> 256 4.8 / 6.1, 256 x 1024 -> 1024 12.3 / 9.1."""
     rows, k = x.numel() // max(x.shape[-1], 1), x.shape[-1]
-    return bool(x.is_cuda and x.dtype == torch.float32 and weight.dtype == torch.float32 and weight.is_contiguous() and 0 < rows <= 256 and k <= 512 and k % 8 == 0
-                and weight.dim() == 2 and weight.shape[1] == k and weight.device == x.device and weight.data_ptr() % 16 == 0)
+    return x.is_cuda and x.dtype == torch.float32 and 0 < rows <= 256 and k <= 512 and k % 8 == 0 and _weight_ready(x, k, weight)
 
 
-def _check_linear(name: str, x: Tensor, weight: Tensor, *others):
+def _laid_out(t: Tensor) -> Tensor:
+    """t, or a copy of it as the projection kernels read it."""
+    return t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
+def _check_linear(name: str, dtype: torch.dtype, x: Tensor, weight: Tensor, *others):
     """What the projection kernels take for granted; the library's F.linear refuses the same (`others`: bias, norm weight)."""
+    if not x.is_cuda or x.dtype != dtype or weight.dtype != dtype or weight.device != x.device:
+        raise RuntimeError(f"{name}: input and weight must be device tensors of {dtype}")
     if weight.dim() != 2 or weight.shape[1] != x.shape[-1]:
         raise RuntimeError(f"{name}: weight {tuple(weight.shape)} does not take inputs {tuple(x.shape)}")
     for t, size in zip(others, (weight.shape[0], weight.shape[1])):
@@ -1689,13 +1701,14 @@ def _transformed() -> bool:
 
 def linear_f32(x: Tensor, weight: Tensor, bias: Tensor | None = None, act: str | None = None) -> Tensor:
     """act(linear(x, weight, bias)) in fp32 by nsa_linear_f32 (few rows, no gradient)."""
-    _check_linear("linear_f32", x, weight, bias)
+    _check_linear("linear_f32", torch.float32, x, weight, bias)
+    weight = _laid_out(weight)
     bias = bias if bias is None else bias.contiguous()
     k, n = x.shape[-1], weight.shape[0]
     x2 = x.reshape(-1, k)
     if x2.stride(1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
         x2 = x2.clone(memory_format=torch.contiguous_format)
-    y = torch.empty((*x.shape[:-1], n), dtype=torch.float32, device=x.device)
+    y = x.new_empty((*x.shape[:-1], n))
     _lib.check(_lib.lib().nsa_linear_f32(x2.shape[0], k, n, _ptr(x2), x2.stride(0), _ptr(weight), _ptr(bias), _ACTS[act], _ptr(y), _stream()),
                "nsa_linear_f32")
     return y

@@ -311,8 +311,7 @@ class SparseAttention(nn.Module):
             _, up, act, down = mlp
             x = window.reshape(b * h, n * d)
             if (cls._plain(up, nn.Linear) and cls._plain(act, nn.ReLU) and cls._plain(down, nn.Linear) and not torch.is_autocast_enabled()
-                    and ops.skinny_linear_supported(x, up.weight) and up.weight.shape[0] % 32 == 0
-                    and b * h * (up.weight.shape[0] + 8) <= 65536 and down.weight.is_contiguous()):
+                    and ops.skinny_linear_supported(x, up.weight) and ops.skinny_linear_supported(x, down.weight, up.weight.shape[0])):
                 return ops.skinny_linear(ops.skinny_linear(x, up.weight, up.bias, act="relu"), down.weight, down.bias).view(b, h, 1, -1)
         return mlp(window[:, :, None])
 

@@ -68,8 +68,7 @@ class Transformer(nn.Module):
             norm, up, act, down = ff
             if (plain(norm, nn.RMSNorm) and plain(up, nn.Linear) and plain(act, nn.GELU) and plain(down, nn.Linear) and act.approximate == 'none'
                     and norm.normalized_shape == tuple(tokens.shape[-1:]) and ops.rms_norm_supported(tokens, norm.weight)
-                    and ops.skinny_linear_supported(tokens, up.weight) and down.weight.dtype == torch.bfloat16 and down.weight.is_contiguous()
-                    and up.weight.shape[0] % 32 == 0 and tokens.numel() // tokens.shape[-1] * (up.weight.shape[0] + 8) <= 65536):
+                    and ops.skinny_linear_supported(tokens, up.weight) and ops.skinny_linear_supported(tokens, down.weight, up.weight.shape[0])):
                 eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
                 hidden = ops.skinny_linear(tokens, up.weight, up.bias, norm.weight, eps, act="gelu")
                 return ops.skinny_linear(hidden, down.weight, down.bias, residual=tokens)

@@ -1,0 +1,89 @@
+"""What the projection kernels for a few rows are handed (`ops.skinny_linear`, `ops.linear_f32` and the decode paths around them), with the
+library replaced by a recorder: they read a weight as contiguous rows of the input's type in device memory, so everything else is
+refused, copied or left to the layer, as F.linear would have it."""
+import pytest
+import torch
+from torch import nn
+
+from native_sparse_attention_pytorch_amd import SparseAttention, _lib, ops
+from native_sparse_attention_pytorch_amd.transformer import FeedForward, Transformer
+
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+class OnDevice(torch.Tensor):
+    """A CPU tensor that says it lies on the GPU: with the library replaced nothing reads its address."""
+    is_cuda = True
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """(name, arguments) of every library call."""
+    seen = []
+
+    class Recorder:
+        def __getattr__(self, name):
+            return lambda *args: seen.append((name, args)) or 0
+
+    monkeypatch.setattr(_lib, "lib", Recorder)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    return seen
+
+
+def _dev(*shape, dtype=BF16):
+    return torch.ones(shape, dtype=dtype).as_subclass(OnDevice)
+
+
+KERNELS = [(ops.skinny_linear, BF16), (ops.linear_f32, F32)]
+
+
+@pytest.mark.parametrize("fn, dtype", KERNELS)
+def test_weights_and_inputs_the_kernel_cannot_read_are_refused(calls, fn, dtype):
+    other = F32 if dtype == BF16 else BF16
+    x = _dev(4, 64, dtype=dtype)
+    for args in ((x, _dev(16, 64, dtype=other)), (x, torch.ones(16, 64, dtype=dtype, device="meta")), (torch.ones(4, 64, dtype=dtype), _dev(16, 64, dtype=dtype)),
+                 (_dev(4, 64, dtype=other), _dev(16, 64, dtype=other)), (x, _dev(64, dtype=dtype))):
+        with pytest.raises(RuntimeError):
+            fn(*args)
+    assert not calls
+
+
+@pytest.mark.parametrize("fn, dtype", KERNELS)
+def test_a_weight_that_is_not_contiguous_is_copied(calls, fn, dtype):
+    w = _dev(64, 16, dtype=dtype).t()
+    fn(_dev(4, 64, dtype=dtype), w)
+    (_, args), = calls
+    assert w.data_ptr() not in args
+
+
+def _odd(linear, how):
+    """`linear` with a weight the kernel must not be handed."""
+    w = linear.weight.detach()
+    if how == "fp32":
+        linear.weight = nn.Parameter(w.float())
+    elif how == "strided":
+        linear.weight = nn.Parameter(w.t().contiguous().t())
+    elif how == "offset":                                     # a slice of a flat buffer, off a 16-byte boundary
+        flat = torch.zeros(w.numel() + 1, dtype=w.dtype)
+        linear.weight = nn.Parameter(flat[1:].view(w.shape).copy_(w))
+    return linear
+
+
+@pytest.mark.parametrize("how", ["plain", "fp32", "strided", "offset"])
+def test_second_projections_the_kernel_cannot_read_stay_with_the_layer(calls, monkeypatch, how):
+    """The compression network's and the feed-forward block's second linear: its call is the layer's own (which refuses fp32)."""
+    m = SparseAttention(dim=128, dim_head=64, heads=4, kv_heads=2, causal=True, sliding_window_size=16, compress_block_size=16,
+                        compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2).to(BF16)
+    ff = FeedForward(64).to(BF16)
+    layers = []
+    for down, run in ((m.k_compress[3], lambda: m._compress_rows(m.k_compress, _dev(2, 2, 16, 64))), (ff[3], lambda: Transformer._decode_feed_forward(ff, _dev(2, 1, 64)))):
+        monkeypatch.setattr(_odd(down, how), "forward", lambda x, n=down.out_features: layers.append(n) or torch.zeros(*x.shape[:-1], n, dtype=BF16))
+        with torch.no_grad():
+            out = run()
+        assert out.shape[-1] == down.out_features
+        if how == "plain":
+            assert not layers and [name for name, _ in calls] == ["nsa_skinny_linear"] * 2
+            calls.clear()
+            continue
+        assert len(layers) == 1 and not calls
+        layers.clear()
