@@ -1621,11 +1621,19 @@ def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
                 and weight.shape[0] > 0 and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
 
 
-def skinny_linear_supported(x: Tensor, weight: Tensor, width: int | None = None) -> bool:
+def _vectors_ready(x: Tensor, weight: Tensor, bias: Tensor | None, norm_weight: Tensor | None) -> bool:
+    """A bias of one value per output (F.linear broadcasts others) and a norm weight the kernels read where it lies."""
+    return ((bias is None or (bias.shape == weight.shape[:1] and bias.dtype == x.dtype and bias.device == x.device))
+            and (norm_weight is None or (norm_weight.shape == weight.shape[1:] and norm_weight.dtype == x.dtype and norm_weight.device == x.device
+                                         and norm_weight.is_contiguous() and norm_weight.data_ptr() % 16 == 0)))
+
+
+def skinny_linear_supported(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_weight: Tensor | None = None, width: int | None = None) -> bool:
     """A projection of a few rows (a decode step) that `skinny_linear` serves.  `width`: the input is not x itself but as many rows
     of this many features, x's own projection."""
     rows, k = x.numel() // x.shape[-1], x.shape[-1] if width is None else width
-    return x.is_cuda and x.dtype == _BF16 and 1 <= rows <= 32 and k % 32 == 0 and rows * (k + 8) <= 65536 and _weight_ready(x, k, weight)
+    return (x.is_cuda and x.dtype == _BF16 and 1 <= rows <= 32 and k % 32 == 0 and rows * (k + 8) <= 65536 and _weight_ready(x, k, weight)
+            and _vectors_ready(x, weight, bias, norm_weight))
 
 
 _ACTS = {None: 0, "gelu": 1, "relu": 2}
@@ -1637,9 +1645,11 @@ def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_we
     projection of a decode step with what stands around it, every part optional.  Inference only (no autograd)."""
     _check_linear("skinny_linear", _BF16, x, weight, bias, norm_weight)
     weight = _laid_out(weight)
-    bias, norm_weight = (t if t is None else t.contiguous() for t in (bias, norm_weight))
+    bias, norm_weight = (t if t is None else _laid_out(t) for t in (bias, norm_weight))
     k, n = x.shape[-1], weight.shape[0]
-    x2 = _rms_rows(x)
+    x2 = x.reshape(-1, k)
+    if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
+        x2 = x2.clone(memory_format=torch.contiguous_format)
     rows = x2.shape[0]
     if residual is not None:
         residual = residual.reshape(rows, n)

@@ -311,7 +311,7 @@ class SparseAttention(nn.Module):
             _, up, act, down = mlp
             x = window.reshape(b * h, n * d)
             if (cls._plain(up, nn.Linear) and cls._plain(act, nn.ReLU) and cls._plain(down, nn.Linear) and not torch.is_autocast_enabled()
-                    and ops.skinny_linear_supported(x, up.weight) and ops.skinny_linear_supported(x, down.weight, up.weight.shape[0])):
+                    and ops.skinny_linear_supported(x, up.weight, up.bias) and ops.skinny_linear_supported(x, down.weight, down.bias, width=up.weight.shape[0])):
                 return ops.skinny_linear(ops.skinny_linear(x, up.weight, up.bias, act="relu"), down.weight, down.bias).view(b, h, 1, -1)
         return mlp(window[:, :, None])
 
@@ -335,11 +335,11 @@ class SparseAttention(nn.Module):
         norm, gate, gates = self.norm, self.to_strategy_combine[0], None
         if (inp.dtype == bf16 and self._plain(norm, nn.RMSNorm) and self._plain(self.to_qkv, nn.Linear) and not torch.is_autocast_enabled()
                 and tuple(norm.normalized_shape) == tuple(inp.shape[-1:]) and ops.rms_norm_supported(inp, norm.weight)
-                and ops.skinny_linear_supported(inp, self.to_qkv.weight)):
+                and ops.skinny_linear_supported(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight)):
             eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
             x = None
             qkv = ops.skinny_linear(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight, eps)
-            if self._plain(gate, nn.Linear) and ops.skinny_linear_supported(inp, gate.weight):
+            if self._plain(gate, nn.Linear) and ops.skinny_linear_supported(inp, gate.weight, gate.bias, norm.weight):
                 gates = ops.skinny_linear(inp, gate.weight, gate.bias, norm.weight, eps)
             else:
                 x = norm(inp)
@@ -397,10 +397,11 @@ class SparseAttention(nn.Module):
         if D != d:
             merged = merged.reshape(b, 1, self.heads, D)[..., :d].reshape(b, 1, self.heads * d)
         merged = merged.to(qkv.dtype)
-        if self._plain(self.combine_heads, nn.Linear) and not torch.is_autocast_enabled() and ops.skinny_linear_supported(merged, self.combine_heads.weight):
-            out = ops.skinny_linear(merged, self.combine_heads.weight, self.combine_heads.bias)
+        heads = self.combine_heads
+        if self._plain(heads, nn.Linear) and not torch.is_autocast_enabled() and ops.skinny_linear_supported(merged, heads.weight, heads.bias):
+            out = ops.skinny_linear(merged, heads.weight, heads.bias)
         else:
-            out = self.combine_heads(merged)
+            out = heads(merged)
         if not return_cache:
             return out
         return out, ((keys, vals), ((ck, cv), (run_k, run_v)))

@@ -68,7 +68,8 @@ class Transformer(nn.Module):
             norm, up, act, down = ff
             if (plain(norm, nn.RMSNorm) and plain(up, nn.Linear) and plain(act, nn.GELU) and plain(down, nn.Linear) and act.approximate == 'none'
                     and norm.normalized_shape == tuple(tokens.shape[-1:]) and ops.rms_norm_supported(tokens, norm.weight)
-                    and ops.skinny_linear_supported(tokens, up.weight) and ops.skinny_linear_supported(tokens, down.weight, up.weight.shape[0])):
+                    and ops.skinny_linear_supported(tokens, up.weight, up.bias, norm.weight)
+                    and ops.skinny_linear_supported(tokens, down.weight, down.bias, width=up.weight.shape[0])):
                 eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
                 hidden = ops.skinny_linear(tokens, up.weight, up.bias, norm.weight, eps, act="gelu")
                 return ops.skinny_linear(hidden, down.weight, down.bias, residual=tokens)
@@ -80,7 +81,7 @@ class Transformer(nn.Module):
         plain, norm, out = SparseAttention._plain, self.norm, self.to_logits
         if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
                 and plain(norm, nn.RMSNorm) and plain(out, nn.Linear) and norm.normalized_shape == tuple(tokens.shape[-1:])
-                and ops.rms_norm_supported(tokens, norm.weight) and ops.skinny_linear_supported(tokens, out.weight)):
+                and ops.rms_norm_supported(tokens, norm.weight) and ops.skinny_linear_supported(tokens, out.weight, out.bias, norm.weight)):
             return ops.skinny_linear(tokens, out.weight, out.bias, norm.weight, torch.finfo(torch.float32).eps if norm.eps is None else norm.eps)
         return out(norm(tokens))
 

@@ -87,3 +87,51 @@ def test_second_projections_the_kernel_cannot_read_stay_with_the_layer(calls, mo
             continue
         assert len(layers) == 1 and not calls
         layers.clear()
+
+
+def _off_boundary(t):
+    flat = torch.zeros(t.numel() + 1, dtype=t.dtype)
+    return flat[1:].view(t.shape).copy_(t)
+
+
+def _decode_layer(norm_weight=None, out_bias=None):
+    m = SparseAttention(dim=128, dim_head=64, heads=4, kv_heads=2, causal=True, sliding_window_size=16, compress_block_size=16,
+                        compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2).to(BF16)
+    if norm_weight is not None:
+        m.norm.weight = nn.Parameter(norm_weight(m.norm.weight.detach()))
+    if out_bias is not None:
+        m.combine_heads.bias = nn.Parameter(out_bias)
+    z = lambda rows: torch.zeros(2, 2, rows, 64, dtype=BF16)
+    return m, ((z(40), z(40)), ((z(5), z(5)), (z(8), z(8))))
+
+
+@pytest.mark.parametrize("vector", ["norm weight off a boundary", "bias of one element"])
+def test_vectors_the_kernel_cannot_read_stay_with_the_layers(calls, monkeypatch, vector):
+    """A decode step, a feed-forward block and the logits whose norm weight lies elsewhere or whose bias is broadcast."""
+    norm_weight = _off_boundary if vector.startswith("norm") else None
+    bias = None if norm_weight else torch.ones(1, dtype=BF16)
+    m, cache = _decode_layer(norm_weight, bias)
+    monkeypatch.setattr(ops, "decode_step", lambda q, *a, **kw: (_dev(2, 1, 256), None, None))
+    with torch.no_grad():
+        m.forward_inference(_dev(2, 1, 128), cache)
+    assert "nsa_decode_layer" not in [n for n, _ in calls] and len(calls) == (1 if norm_weight else 2)       # output projection; qkv and gate logits
+    calls.clear()
+
+    model = Transformer(num_tokens=16, dim=64, depth=0).to(BF16)
+    ff = FeedForward(64).to(BF16)
+    if norm_weight:
+        for norm in (ff[0], model.norm):
+            norm.weight = nn.Parameter(_off_boundary(norm.weight.detach()))
+    else:
+        ff[1].bias, model.to_logits.bias = nn.Parameter(bias), nn.Parameter(bias)
+    with torch.no_grad():
+        assert Transformer._decode_feed_forward(ff, _dev(2, 1, 64)).shape == (2, 1, 64)
+        assert model._decode_logits(_dev(2, 1, 64)).shape == (2, 1, 16)
+    assert not calls
+
+
+def test_inputs_off_a_boundary_are_copied(calls):
+    x = _off_boundary(torch.ones(4, 64, dtype=BF16)).as_subclass(OnDevice)
+    ops.skinny_linear(x, _dev(16, 64), norm_weight=_off_boundary(torch.ones(64, dtype=BF16)).as_subclass(OnDevice))
+    (_, args), = calls
+    assert x.data_ptr() not in args and args[3] % 16 == 0 and args[5] % 16 == 0
