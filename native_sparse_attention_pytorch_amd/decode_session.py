@@ -120,10 +120,11 @@ class DecodeSession:
         # inside the first: both unhooked layers of the default kind
         norm, out = m.norm, m.combine_heads
         self.own_norm = (m._plain(norm, torch.nn.RMSNorm) and tuple(norm.normalized_shape) == (m.to_qkv.in_features,)
-                         and rms_norm_supported(self.x_buf, norm.weight))
+                         and rms_norm_supported(self.x_buf, norm.weight) and norm.weight.is_contiguous() and norm.weight.data_ptr() % 16 == 0)
         self.own_in = skinny_linear_supported(self.x_buf, self.w_cat) and self.fused_gate and m.to_qkv.bias is None
         merged = torch.empty((b, 1, m.heads * d), dtype=_BF16, device=dev)
-        self.own_out = m._plain(out, torch.nn.Linear) and out.weight.dtype == _BF16 and skinny_linear_supported(merged, out.weight)
+        self.own_out = (m._plain(out, torch.nn.Linear) and skinny_linear_supported(merged, out.weight, out.bias)
+                        and (out.bias is None or out.bias.is_contiguous()))
         self._desc, self._ws = self._make_desc(dev)
         # Direct steps pay where their launches take the host less time than the GPU: with this library's kernels always (five
         # launches, ~35 us), with the GEMM library's (~20 us of host time each) when the weights are what takes time

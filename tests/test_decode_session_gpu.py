@@ -1,0 +1,54 @@
+"""A directly launched decode session takes what a replayed one takes, and is not disturbed by what happens around it."""
+import pytest
+import torch
+from torch import nn
+
+pytestmark = pytest.mark.gpu
+DEV, BF16 = "cuda", torch.bfloat16
+
+
+def _session(b=4, dim=128):
+    from native_sparse_attention_pytorch_amd import SparseAttention
+    from native_sparse_attention_pytorch_amd.decode_session import DecodeSession
+    torch.manual_seed(b)
+    m = SparseAttention(dim=dim, dim_head=64, heads=4, kv_heads=2, causal=True, sliding_window_size=16, compress_block_size=16,
+                        compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2).to(DEV, BF16)
+    with torch.no_grad():
+        _, cache = m(torch.randn(b, 37, dim, device=DEV, dtype=BF16), return_cache=True)
+        return m, cache, DecodeSession(m, cache, max_len=64)
+
+
+def _off_boundary(t):
+    flat = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)
+    return nn.Parameter(flat[1:].view(t.shape).copy_(t.detach()))
+
+
+def _strided_bias(m):
+    m.combine_heads.bias = nn.Parameter(torch.randn(256, device=DEV, dtype=BF16)[::2])
+
+
+def _bias_of_one(m):
+    m.combine_heads.bias = nn.Parameter(torch.randn(1, device=DEV, dtype=BF16))
+
+
+def _weight_off_boundary(m):
+    m.combine_heads.weight = _off_boundary(m.combine_heads.weight)
+
+
+def _norm_off_boundary(m):
+    m.norm.weight = _off_boundary(m.norm.weight)
+
+
+@pytest.mark.parametrize("change", [_strided_bias, _bias_of_one, _weight_off_boundary, _norm_off_boundary])
+def test_parameters_of_other_layouts(change):
+    m, cache, session = _session()                        # (the parallel forward's norm kernel refuses a weight off a boundary)
+    change(m)
+    session = type(session)(m, cache, max_len=64)
+    x = torch.randn(4, 1, 128, device=DEV, dtype=BF16)
+    with torch.no_grad():
+        want = m(x, cache=cache, return_cache=True)[0]
+    got = session.step(x)
+    torch.cuda.synchronize()
+    # the same partial sums merged in another order, then one bf16 projection of 256 products: two roundings of its magnitude
+    mag = want.float().abs().max().item()
+    assert (got.float() - want.float()).abs().max().item() <= 2 ** -6 * mag
