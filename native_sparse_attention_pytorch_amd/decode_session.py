@@ -230,7 +230,7 @@ class DecodeSession:
         m, L = self.module, _lib.lib()
         qkvg, merged, rstd = self._direct_bufs
         if x.dtype != _BF16 or x.shape != self.x_buf.shape or not x.is_contiguous() or x.data_ptr() % 16 or x.device != merged.device:
-            x = x.to(device=merged.device, dtype=_BF16).reshape(self.x_buf.shape).clone(memory_format=torch.contiguous_format)
+            x = torch.empty_like(self.x_buf).copy_(x)                # converted and broadcast, as a replayed step copies it
         st = torch.cuda.current_stream(merged.device).cuda_stream
         b, dim = self.b, x.shape[-1]
         w_out = self.w_out if self.w_out is not None else m.combine_heads.weight
@@ -275,7 +275,7 @@ class DecodeSession:
 
     @torch.no_grad()
     def step(self, x: torch.Tensor) -> torch.Tensor:
-        """x 'b 1 dim' on the session's device: the token at position `self.pos`.  Returns the layer output 'b 1 dim' (a new tensor)."""
+        """x 'b 1 dim', or what is broadcast to it: the token at position `self.pos`.  Returns the layer output 'b 1 dim' (a new tensor)."""
         if self.graphs is None:
             raise RuntimeError("DecodeSession was built with capture=False (its launches belong to an enclosing graph)")
         if self.pos >= self.max_len:

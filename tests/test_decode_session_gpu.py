@@ -52,3 +52,15 @@ def test_parameters_of_other_layouts(change):
     # the same partial sums merged in another order, then one bf16 projection of 256 products: two roundings of its magnitude
     mag = want.float().abs().max().item()
     assert (got.float() - want.float()).abs().max().item() <= 2 ** -6 * mag
+
+
+def test_tokens_are_taken_as_a_copy_into_the_buffer_takes_them():
+    """`x` is broadcast to 'b 1 dim' and converted; what cannot be broadcast is refused."""
+    m, cache, first = _session()
+    one = torch.randn(128, device=DEV, dtype=BF16)
+    want = first.step(one.expand(4, 1, 128).contiguous())
+    for x in (one, one[None], one.view(1, 1, 128), one.expand(4, 1, 128), one.float().view(1, 1, 128), one.cpu()):
+        assert torch.equal(type(first)(m, cache, max_len=64).step(x), want)
+    for shape in ((4, 128), (1, 4, 128), (4, 2, 128), (512,)):
+        with pytest.raises(RuntimeError):
+            type(first)(m, cache, max_len=64).step(torch.zeros(shape, device=DEV, dtype=BF16))
