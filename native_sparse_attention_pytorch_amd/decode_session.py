@@ -219,7 +219,12 @@ class DecodeSession:
                 self._ws.data_ptr(), self._ws.numel(), merged.data_ptr(), int(advance))
 
     def _prepare_direct(self, merged):
-        """The arguments of a direct step that do not change from token to token, converted once."""
+        """The arguments of a direct step that do not change from token to token, converted once.  The parameters are held by what
+        they are now, as a recorded graph holds their memory: a module moved or converted later must not change the addresses."""
+        m = self.module
+        bias = m.combine_heads.bias
+        self._direct_params = (m.norm.weight.detach(), self._eps(), m.combine_heads.weight.detach() if self.w_out is None else self.w_out,
+                               None if bias is None else bias.detach())
         qkvg = torch.empty((self.b, 1, self.w_cat.shape[0]), dtype=_BF16, device=merged.device)
         rstd = torch.empty((self.b,), dtype=torch.float32, device=merged.device)
         self._direct_bufs = (qkvg, merged, rstd)
@@ -227,19 +232,18 @@ class DecodeSession:
         self._direct_args = tuple(a if not isinstance(a, (int, type(None))) else t(a) for a, t in zip(self._step_args(qkvg, qkvg, merged, 1), fn.argtypes))
 
     def _step_direct(self, x: torch.Tensor) -> torch.Tensor:
-        m, L = self.module, _lib.lib()
+        L = _lib.lib()
         qkvg, merged, rstd = self._direct_bufs
+        norm_weight, eps, w_out, bias = self._direct_params
         if x.dtype != _BF16 or x.shape != self.x_buf.shape or not x.is_contiguous() or x.data_ptr() % 16 or x.device != merged.device:
             x = torch.empty_like(self.x_buf).copy_(x)                # converted and broadcast, as a replayed step copies it
         st = torch.cuda.current_stream(merged.device).cuda_stream
         b, dim = self.b, x.shape[-1]
-        w_out = self.w_out if self.w_out is not None else m.combine_heads.weight
-        bias = m.combine_heads.bias
         if self.own_in:
-            rc = L.nsa_skinny_linear(b, dim, qkvg.shape[-1], x.data_ptr(), dim, m.norm.weight.data_ptr(), self._eps(), self.w_cat.data_ptr(), None,
+            rc = L.nsa_skinny_linear(b, dim, qkvg.shape[-1], x.data_ptr(), dim, norm_weight.data_ptr(), eps, self.w_cat.data_ptr(), None,
                                      0, None, 0, qkvg.data_ptr(), qkvg.shape[-1], st)
         else:
-            rc = L.nsa_rmsnorm_fwd(b, dim, x.data_ptr(), dim, m.norm.weight.data_ptr(), self._eps(), self.x_buf.data_ptr(), rstd.data_ptr(), st)
+            rc = L.nsa_rmsnorm_fwd(b, dim, x.data_ptr(), dim, norm_weight.data_ptr(), eps, self.x_buf.data_ptr(), rstd.data_ptr(), st)
             torch.mm(self.x_buf.view(b, dim), self.w_cat.t(), out=qkvg.view(b, -1))
         rc = rc or L.nsa_decode_step_dyn(*self._direct_args, st)
         if self.own_out:

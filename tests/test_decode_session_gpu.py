@@ -64,3 +64,17 @@ def test_tokens_are_taken_as_a_copy_into_the_buffer_takes_them():
     for shape in ((4, 128), (1, 4, 128), (4, 2, 128), (512,)):
         with pytest.raises(RuntimeError):
             type(first)(m, cache, max_len=64).step(torch.zeros(shape, device=DEV, dtype=BF16))
+
+
+def test_a_module_moved_afterwards_leaves_the_session_with_its_weights():
+    """The session keeps the memory its steps read: moving the module's parameters away neither changes nor invalidates it."""
+    m, cache, first = _session()
+    x = torch.randn(4, 1, 128, device=DEV, dtype=BF16)
+    want = first.step(x)
+    second = type(first)(m, cache, max_len=64)
+    m.norm.cpu(), m.combine_heads.cpu()
+    assert torch.equal(second.step(x), want)
+    third = type(first)(m.to(DEV), cache, max_len=64)
+    with torch.no_grad():
+        m.combine_heads.weight.mul_(2)                                 # values changed in place are followed, as by a replayed step
+    torch.testing.assert_close(third.step(x), want * 2, rtol=0, atol=0)
