@@ -251,7 +251,10 @@ class DecodeSession:
             rc = rc or L.nsa_skinny_linear(b, merged.shape[-1], dim, merged.data_ptr(), merged.shape[-1], None, 0.0, w_out.data_ptr(),
                                            None if bias is None else bias.data_ptr(), 0, None, 0, y.data_ptr(), dim, st)
         else:
-            y = torch.nn.functional.linear(merged, w_out, bias)
+            # (into a result of its own: autocast around the step has no say in it)
+            y = torch.empty_like(x)
+            rows, flat = merged.view(b, -1), y.view(b, -1)
+            torch.mm(rows, w_out.t(), out=flat) if bias is None else torch.addmm(bias, rows, w_out.t(), out=flat)
         _lib.check(rc, "decode step")
         return y
 

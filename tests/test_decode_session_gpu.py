@@ -7,11 +7,11 @@ pytestmark = pytest.mark.gpu
 DEV, BF16 = "cuda", torch.bfloat16
 
 
-def _session(b=4, dim=128):
+def _session(b=4, dim=128, heads=4, kv_heads=2):
     from native_sparse_attention_pytorch_amd import SparseAttention
     from native_sparse_attention_pytorch_amd.decode_session import DecodeSession
     torch.manual_seed(b)
-    m = SparseAttention(dim=dim, dim_head=64, heads=4, kv_heads=2, causal=True, sliding_window_size=16, compress_block_size=16,
+    m = SparseAttention(dim=dim, dim_head=64, heads=heads, kv_heads=kv_heads, causal=True, sliding_window_size=16, compress_block_size=16,
                         compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2).to(DEV, BF16)
     with torch.no_grad():
         _, cache = m(torch.randn(b, 37, dim, device=DEV, dtype=BF16), return_cache=True)
@@ -78,3 +78,16 @@ def test_a_module_moved_afterwards_leaves_the_session_with_its_weights():
     with torch.no_grad():
         m.combine_heads.weight.mul_(2)                                 # values changed in place are followed, as by a replayed step
     torch.testing.assert_close(third.step(x), want * 2, rtol=0, atol=0)
+
+
+def test_autocast_around_a_step_changes_nothing():
+    """A direct step whose output projection is the library's: bf16, as a recorded step leaves it whatever the step is run under."""
+    m, cache, _ = _session(dim=4096, heads=48, kv_heads=8)              # (35 MB of qkv and gate weights: launched directly)
+    _bias_of_one(m)
+    from native_sparse_attention_pytorch_amd.decode_session import DecodeSession
+    sessions = [DecodeSession(m, cache, max_len=64) for _ in range(2)]
+    assert sessions[0].direct and not sessions[0].own_out
+    x = torch.randn(4, 1, 4096, device=DEV, dtype=BF16)
+    with torch.autocast("cuda", dtype=torch.float16):
+        got = sessions[0].step(x)
+    assert got.dtype == BF16 and torch.equal(got, sessions[1].step(x))
