@@ -91,3 +91,16 @@ def test_autocast_around_a_step_changes_nothing():
     with torch.autocast("cuda", dtype=torch.float16):
         got = sessions[0].step(x)
     assert got.dtype == BF16 and torch.equal(got, sessions[1].step(x))
+
+
+def test_a_step_cannot_be_recorded():
+    """The host's position would stand still while a replay moves the device's: refused, as replaying a graph inside a capture is."""
+    m, cache, session = _session()
+    x = torch.randn(4, 1, 128, device=DEV, dtype=BF16)
+    kept, graph = torch.ones(4, device=DEV), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kept.add_(1)
+        with pytest.raises(RuntimeError, match="recorded"):
+            session.step(x)
+    assert session.pos == 37
+    assert torch.equal(session.step(x), type(session)(m, cache, max_len=64).step(x))
