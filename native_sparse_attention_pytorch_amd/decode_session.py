@@ -287,6 +287,9 @@ class DecodeSession:
             raise RuntimeError("DecodeSession was built with capture=False (its launches belong to an enclosing graph)")
         if self.pos >= self.max_len:
             raise RuntimeError(f"DecodeSession: capacity of {self.max_len} tokens reached")
+        if torch.cuda.current_device() != self.K.device.index:
+            with torch.cuda.device(self.K.device):
+                return self.step(x)
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("DecodeSession.step cannot be recorded into a graph: its position advances on the host")
         event = self.completes_window()
