@@ -5,6 +5,7 @@ same constructor arguments and parameter names."""
 from __future__ import annotations
 
 import math
+from itertools import islice
 
 import torch
 import torch.nn.functional as F
@@ -109,10 +110,12 @@ class Transformer(nn.Module):
             from . import ops
             if not ops.capturing():
                 self._launched_grad_steps = True      # training.GraphedStep must be recorded before the first of these
-        if cache is not None and len(cache) == len(self.layers) and not return_loss:
-            # with caches only the newest token is embedded and every layer takes one decode step
-            logits, caches = self._decode(ids, cache)
-            return (logits, caches) if return_cache else logits
+        if cache is not None:
+            cache = list(islice(cache or (), len(self.layers)))         # any iterable of layer caches; a layer without one starts one
+            if len(cache) == len(self.layers) and not return_loss and all(c is not None for c in cache):
+                # with caches only the newest token is embedded and every layer takes one decode step
+                logits, caches = self._decode(ids, cache)
+                return (logits, caches) if return_cache else logits
         tokens = self.token_emb(ids if cache is None else ids[:, -1:])
         layer_caches = iter(cache or [])
         caches = []

@@ -1,5 +1,7 @@
 """What `SparseAttention._decode_whole` may hand to the kernels: caches and weights whose shapes agree.  The library call takes batch,
 heads and lengths from one tensor of each pair, so everything else goes to the general path, which refuses it."""
+import itertools
+
 import pytest
 import torch
 from torch import nn
@@ -107,3 +109,44 @@ def test_replaced_vectors_of_another_size_do_not(reached, name, shape):
     owner, _, leaf = name.rpartition(".")
     setattr(m.get_submodule(owner), leaf, nn.Parameter(torch.zeros(shape, dtype=BF16)))
     assert _run(m, cache) is None and not reached
+
+
+def _model_with_spied_layers(monkeypatch, depth=2):
+    m = Transformer(num_tokens=16, dim=128, depth=depth, heads=4, kv_heads=2, sparse_attn_kwargs=dict(
+        sliding_window_size=16, compress_block_size=16, compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2)).to(BF16)
+    handed = []
+    for i, (attn, _) in enumerate(m.layers):
+        def forward(tokens, cache=None, return_cache=False, i=i):
+            handed.append((i, cache))
+            return torch.zeros_like(tokens), ("advanced", i)
+        monkeypatch.setattr(attn, "forward", forward)
+        monkeypatch.setattr(attn, "_decode_whole", lambda *a, **kw: None)
+    return m, handed
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("kind", ["list", "tuple", "iterator", "endless", "longer"])
+def test_layer_caches_from_any_iterable(monkeypatch, kind, grad):
+    """One cache per layer, from whatever yields them; what is left over is not read."""
+    m, handed = _model_with_spied_layers(monkeypatch)
+    caches = {"list": ["a", "b"], "tuple": ("a", "b"), "iterator": iter("ab"), "endless": itertools.cycle("ab"), "longer": ["a", "b", "c"]}[kind]
+    with torch.set_grad_enabled(grad):
+        logits, new = m(torch.zeros(3, 5, dtype=torch.long), cache=caches, return_cache=True)
+    assert handed == [(0, "a"), (1, "b")] and new == [("advanced", 0), ("advanced", 1)] and logits.shape == (3, 1, 16)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("caches", [[None, "b"], ["a"], []])
+def test_a_layer_without_a_cache_starts_one(monkeypatch, caches, grad):
+    m, handed = _model_with_spied_layers(monkeypatch)
+    with torch.set_grad_enabled(grad):
+        m(torch.zeros(3, 5, dtype=torch.long), cache=caches, return_cache=True)
+    assert [c for _, c in handed] == (caches + [None, None])[:2]
+
+
+def test_a_missing_cache_does_not_reach_the_layer_call():
+    m, _, _ = _layer_and_cache()
+    model = Transformer(num_tokens=16, dim=128, depth=1, heads=4, kv_heads=2).to(BF16)
+    model.layers[0][0] = m
+    with torch.no_grad(), pytest.raises(RuntimeError, match="GPU only"):      # the layer's own forward, which has no CPU path
+        model(torch.zeros(4, 1, dtype=torch.long), cache=[None])
