@@ -1615,6 +1615,15 @@ def rms_norm(x: Tensor, weight: Tensor, eps: float | None = None) -> Tensor:
 
 # ------------------------------------------------------------------ projections
 
+def plain_call() -> bool:
+    """Nothing is at work that an operator carries and a kernel launched by address loses: autocast, a compiler or another tracer (which
+    would record the result as a constant), vmap, jvp, a forward-mode level, a dispatch mode.  Asked before any address is read:
+    a batched or traced tensor has none."""
+    return not (torch.compiler.is_compiling() or torch.is_autocast_enabled() or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0
+                or torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0 or torch._C._get_tracing_state() is not None)
+
+
 def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
     """A weight the projection kernels read where it lies: rows of `width`, x's type and device, contiguous from a 16-byte boundary on."""
     return bool(weight.dtype == x.dtype and weight.device == x.device and weight.dim() == 2 and weight.shape[1] == width
@@ -1680,12 +1689,12 @@ def _wgrad_splits(rows: int, n_in: int, n_out: int, replayed: bool = False) -> i
     return s if s >= 4 else 1
 
 
-def linear_f32_supported(x: Tensor, weight: Tensor) -> bool:
+def linear_f32_supported(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> bool:
     """An fp32 projection small enough that the GEMM library's tiles leave most of the chip idle.  Measured, this kernel / the
     library in us: 240 x 256 -> 256 4.8 / 64.7, 240 x 512 -> 24 6.2 / 19.9, 62 x 512 -> 1536 6.7 / 6.8, 256 x 512 -> 1536 11.6 / 8.5
     (the library's call takes the host 14 us longer), 384 x 256 -> 256 4.8 / 6.1, 256 x 1024 -> 1024 12.3 / 9.1."""
     rows, k = x.numel() // max(x.shape[-1], 1), x.shape[-1]
-    return x.is_cuda and x.dtype == torch.float32 and 0 < rows <= 256 and k <= 512 and k % 8 == 0 and _weight_ready(x, k, weight)
+    return x.is_cuda and x.dtype == torch.float32 and 0 < rows <= 256 and k <= 512 and k % 8 == 0 and _weight_ready(x, k, weight) and _vectors_ready(x, weight, bias, None)
 
 
 def _laid_out(t: Tensor) -> Tensor:
@@ -1702,11 +1711,6 @@ def _check_linear(name: str, dtype: torch.dtype, x: Tensor, weight: Tensor, *oth
     for t, size in zip(others, (weight.shape[0], weight.shape[1])):
         if t is not None and (t.shape != (size,) or t.dtype != x.dtype or t.device != x.device):
             raise RuntimeError(f"{name}: bias and norm weight are vectors of the projection's own width, type and device")
-
-
-def _transformed() -> bool:
-    """Inside vmap, jvp or another functorch transform, or a forward-mode level: operators carry what a kernel would lose."""
-    return torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
 
 
 def linear_f32(x: Tensor, weight: Tensor, bias: Tensor | None = None, act: str | None = None) -> Tensor:
@@ -1753,9 +1757,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     """torch.nn.functional.linear with the split weight-gradient GEMM (see _Linear)."""
     if (not (torch.is_grad_enabled() and weight.requires_grad) or torch.compiler.is_compiling() or x.dtype != weight.dtype
             or torch.is_autocast_enabled()):               # under autocast the library casts the operands itself
-        if (not torch.is_grad_enabled() and linear_f32_supported(x, weight) and not torch.compiler.is_compiling()
-                and not torch.is_autocast_enabled() and not _transformed()
-                and (bias is None or (bias.shape == weight.shape[:1] and bias.dtype == x.dtype and bias.device == x.device))):
+        if not torch.is_grad_enabled() and plain_call() and linear_f32_supported(x, weight, bias):
             return linear_f32(x, weight, bias)
         return torch.nn.functional.linear(x, weight, bias)
     return _Linear.apply(x, weight, bias)

@@ -232,9 +232,9 @@ class SparseAttention(nn.Module):
         if not cls._plain(mlp, nn.Sequential):
             return mlp(windows)
         if (len(mlp) == 4 and windows.dtype == torch.float32 and type(mlp[0]) is _FlattenWindow and cls._plain(mlp[1], nn.Linear)
-                and cls._plain(mlp[2], nn.ReLU) and not torch.is_grad_enabled() and not torch.is_autocast_enabled()):
+                and cls._plain(mlp[2], nn.ReLU) and not torch.is_grad_enabled() and ops.plain_call()):
             x = windows.flatten(-2)
-            if ops.linear_f32_supported(x, mlp[1].weight):
+            if ops.linear_f32_supported(x, mlp[1].weight, mlp[1].bias):
                 return cls._linear(mlp[3], ops.linear_f32(x, mlp[1].weight, mlp[1].bias, act="relu"))
         for layer in mlp:
             windows = cls._linear(layer, windows)
@@ -257,7 +257,7 @@ class SparseAttention(nn.Module):
         b, dim, hd = inp.shape[0], inp.shape[2], self.heads * d
         mem, freqs, device = self.compress_mem_kv, self.rotary_emb.freqs, inp.device
         if (b > 32 or dim % 32 or b * (max(dim, hd) + 8) > 65536 or norm.normalized_shape != (dim,)
-                or torch.is_autocast_enabled() or torch.compiler.is_compiling()):
+                or not ops.plain_call()):
             return None
         for w in (norm.weight, qkv.weight, gate.weight, gate.bias, out.weight, out.bias, mem):
             if w is not None and (w.dtype != bf16 or w.device != device or not w.is_contiguous() or w.data_ptr() % 16):
@@ -310,7 +310,7 @@ class SparseAttention(nn.Module):
         if cls._plain(mlp, nn.Sequential) and len(mlp) == 4 and type(mlp[0]) is _FlattenWindow and window.dtype == torch.bfloat16:
             _, up, act, down = mlp
             x = window.reshape(b * h, n * d)
-            if (cls._plain(up, nn.Linear) and cls._plain(act, nn.ReLU) and cls._plain(down, nn.Linear) and not torch.is_autocast_enabled()
+            if (cls._plain(up, nn.Linear) and cls._plain(act, nn.ReLU) and cls._plain(down, nn.Linear) and ops.plain_call()
                     and ops.skinny_linear_supported(x, up.weight, up.bias) and ops.skinny_linear_supported(x, down.weight, down.bias, width=up.weight.shape[0])):
                 return ops.skinny_linear(ops.skinny_linear(x, up.weight, up.bias, act="relu"), down.weight, down.bias).view(b, h, 1, -1)
         return mlp(window[:, :, None])
@@ -332,8 +332,8 @@ class SparseAttention(nn.Module):
         if out is not None:
             return out
         # projections of a few rows by the same kernels (bit-equal to the whole-layer call and to decode_session.DecodeSession)
-        norm, gate, gates = self.norm, self.to_strategy_combine[0], None
-        if (inp.dtype == bf16 and self._plain(norm, nn.RMSNorm) and self._plain(self.to_qkv, nn.Linear) and not torch.is_autocast_enabled()
+        norm, gate, gates, kernels = self.norm, self.to_strategy_combine[0], None, ops.plain_call()
+        if (inp.dtype == bf16 and self._plain(norm, nn.RMSNorm) and self._plain(self.to_qkv, nn.Linear) and kernels
                 and tuple(norm.normalized_shape) == tuple(inp.shape[-1:]) and ops.rms_norm_supported(inp, norm.weight)
                 and ops.skinny_linear_supported(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight)):
             eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
@@ -398,7 +398,7 @@ class SparseAttention(nn.Module):
             merged = merged.reshape(b, 1, self.heads, D)[..., :d].reshape(b, 1, self.heads * d)
         merged = merged.to(qkv.dtype)
         heads = self.combine_heads
-        if self._plain(heads, nn.Linear) and not torch.is_autocast_enabled() and ops.skinny_linear_supported(merged, heads.weight, heads.bias):
+        if kernels and self._plain(heads, nn.Linear) and ops.skinny_linear_supported(merged, heads.weight, heads.bias):
             out = ops.skinny_linear(merged, heads.weight, heads.bias)
         else:
             out = heads(merged)

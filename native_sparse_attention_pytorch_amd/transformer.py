@@ -64,7 +64,7 @@ class Transformer(nn.Module):
         linear, residual), each step rounded as the layers would."""
         from . import ops
         plain = SparseAttention._plain
-        if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+        if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and ops.plain_call()
                 and plain(ff, nn.Sequential) and len(ff) == 4):
             norm, up, act, down = ff
             if (plain(norm, nn.RMSNorm) and plain(up, nn.Linear) and plain(act, nn.GELU) and plain(down, nn.Linear) and act.approximate == 'none'
@@ -80,7 +80,7 @@ class Transformer(nn.Module):
         """to_logits(norm(tokens)) for one token per sequence."""
         from . import ops
         plain, norm, out = SparseAttention._plain, self.norm, self.to_logits
-        if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+        if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and ops.plain_call()
                 and plain(norm, nn.RMSNorm) and plain(out, nn.Linear) and norm.normalized_shape == tuple(tokens.shape[-1:])
                 and ops.rms_norm_supported(tokens, norm.weight) and ops.skinny_linear_supported(tokens, out.weight, out.bias, norm.weight)):
             return ops.skinny_linear(tokens, out.weight, out.bias, norm.weight, torch.finfo(torch.float32).eps if norm.eps is None else norm.eps)

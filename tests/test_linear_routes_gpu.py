@@ -40,3 +40,26 @@ def test_what_only_the_operator_serves():
     with forward_ad.dual_level():
         y = ops.linear(forward_ad.make_dual(x, x + 1), w)
         close(forward_ad.unpack_dual(y).tangent, F.linear(x + 1, w))
+    # the weight batched: an address would be that of the whole stack
+    stack = _r(3, 16, 64)
+    close(torch.vmap(lambda u: ops.linear(x, u))(stack), F.linear(x, stack.reshape(48, 64)).view(8, 3, 16).transpose(0, 1))
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("trace", ["compile", "make_fx", "make_fx fake", "make_fx pre_dispatch", "jit.trace"])
+def test_traces_record_the_operator(trace):
+    """A traced projection computes on the inputs it is run on: a kernel launched while tracing would leave its result as a constant."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from native_sparse_attention_pytorch_amd import ops
+    x, w, b = _r(8, 64), _r(16, 64), _r(16)
+    args, other = (x, w, b), (x.flip(0) * 2, w + 1, b)
+    if trace == "compile":
+        torch._dynamo.reset()
+        run = torch.compile(ops.linear, backend="eager", fullgraph=True)
+        run(*args)
+    elif trace == "jit.trace":
+        run = torch.jit.trace(ops.linear, args, check_trace=False)
+    else:
+        run = make_fx(ops.linear, tracing_mode="fake" if "fake" in trace else "real", pre_dispatch="pre" in trace)(*args)
+    got, want = run(*other), F.linear(*other)
+    torch.testing.assert_close(got, want, rtol=0, atol=64 * 2 ** -24 * 1024)
