@@ -29,9 +29,10 @@ def rel_err(a, b):
 
 def assert_close(got, want, atol, rtol, what=""):
     got, want = got.float().cpu(), want.float().cpu()
+    assert got.shape == want.shape, f"{what}: shape {tuple(got.shape)}, want {tuple(want.shape)}"
     err = (got - want).abs()
     tol = atol + rtol * want.abs()
-    bad = err > tol
+    bad = ~((err <= tol) & err.isfinite() | (got == want))      # (out of any tolerance: a NaN, an infinity where another value is wanted)
     if bad.any():
         i = torch.nonzero(bad)[0].tolist()
         raise AssertionError(f"{what}: {int(bad.sum())}/{bad.numel()} elements out of tolerance; "
