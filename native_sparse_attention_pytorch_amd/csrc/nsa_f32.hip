@@ -112,11 +112,11 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // `total` keys; key(v) -> row of k / v (v < total), -1 for a padding key past the sequence end (logit 0, value 0), -2 - m for
-// row m of mk / mv.  Tiles first, first + step, ...
+// row m of mk / mv.  Tiles first, first + step, ...  `flat`: every key scores 0, whatever it holds.
 template <int DT, class Key>
 __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ piece, int* __restrict__ rows_s, const float (&q)[DT][64], const float* __restrict__ kb,
                                           const float* __restrict__ vb, const float* __restrict__ mk, const float* __restrict__ mv, int total,
-                                          int first, int step, Key key, RowsState<DT>& S, int lane) {
+                                          int first, int step, bool flat, Key key, RowsState<DT>& S, int lane) {
   const int tiles = (total + 63) >> 6;
   if (first >= tiles) return;
   const int chunk = lane & 15, r0 = lane >> 4;
@@ -176,15 +176,15 @@ __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ 
     float s[4], tmax = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      s[i] = v0 + i < total ? (s0[i] + s1[i]) * A.scale : -INFINITY;
+      s[i] = v0 + i < total ? (flat ? 0.f : (s0[i] + s1[i]) * A.scale) : -INFINITY;
       tmax = fmaxf(tmax, s[i]);
     }
-    const float mn = fmaxf(S.m, max_mod4(tmax));       // finite: every tile holds at least one key
-    const float alpha = expf(S.m - mn);
+    const float mn = fmaxf(S.m, max_mod4(tmax)), mref = mn == -INFINITY ? 0.f : mn;      // (keys whose scores overflow to -inf weigh nothing)
+    const float alpha = expf(S.m - mref);              // m = -inf: 0
     S.m = mn;
     float p[4], ps = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { p[i] = expf(s[i] - mn); ps += p[i]; }
+    for (int i = 0; i < 4; ++i) { p[i] = expf(s[i] - mref); ps += p[i]; }
     S.l = S.l * alpha + ps;
     floatx4 al;
 #pragma unroll
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
   const float* mk = A.memk != nullptr ? A.memk + (long)hk * A.mem * A.d : kb;
   const float* mv = A.memv != nullptr ? A.memv + (long)hk * A.mem * A.d : vb;
   // A query of a non-causal selection whose slots are all dead attends their blocks uniformly, zero padding included: the
-  // reference fills all its logits with the same value (NSA.py:809-815).  Zero queries over all slots give the same.
+  // reference fills all its logits with the same value (NSA.py:809-815).
   bool dead = false;
   if constexpr (SELECT) {
     if (A.uniform) {
@@ -271,12 +271,6 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
       for (int ft = 0; ft < DT; ++ft)
 #pragma unroll
         for (int e = 0; e < 64; ++e) qr[ft][e] = qp[min(64 * ft + e, last)];
-      if (SELECT && dead) {
-#pragma unroll
-        for (int ft = 0; ft < DT; ++ft)
-#pragma unroll
-          for (int e = 0; e < 64; ++e) qr[ft][e] = 0.f;
-      }
     }
     RowsState<DT> S;
     S.m = -INFINITY;
@@ -303,7 +297,7 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
         if (blk >= 0) blocks[__popcll(live & ((1ull << lane) - 1))] = blk;
         __builtin_amdgcn_wave_barrier();
         const bool last = s0 + 64 >= A.S;
-        rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, kb, vb, cnt * A.B + (last ? own_keys : 0), first, step, [&](int v) {
+        rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, kb, vb, cnt * A.B + (last ? own_keys : 0), first, step, dead, [&](int v) {
           const int slot = v / A.B, off = v - slot * A.B;
           const int row = (slot < cnt ? blocks[slot] : own) * A.B + off;
           return row < A.nk ? row : -1;
@@ -314,7 +308,7 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
       int lo, hi;
       f32_interval(A, pos, lo, hi);
       const int own_mem = A.memk != nullptr ? A.mem : 0;
-      rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, mk, mv, hi - lo + 1, first, step, [&](int v) {
+      rows_walk<DT>(A, piece, rows_s[wave], qr, kb, vb, mk, mv, hi - lo + 1, first, step, false, [&](int v) {
         const int u = lo + v;
         return u < own_mem ? -2 - u : u - own_mem;
       }, S, lane);

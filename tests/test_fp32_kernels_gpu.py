@@ -76,6 +76,59 @@ def test_selection(b, hq, hk, n, d, B, S, causal, qoff):
     assert_close(lse, want_lse, 1e-5, 1e-5, "lse")
 
 
+def _overflowing(shape, rows, seed):
+    """Keys whose first `rows` rows score -inf in fp32 against queries with 1e20 as their first feature."""
+    k = _rand(shape, seed)
+    k[..., 0] = 0
+    k[..., :rows, 0] = -1e30
+    return k
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n", [300, 2100])                       # a work-group per query; a wave per query
+def test_selected_blocks_that_score_minus_infinity(n, d):
+    """The first tile of every query holds such a block alone: it weighs nothing and the blocks after it are attended as ever."""
+    from native_sparse_attention_pytorch_amd.ops import native_sparse_attend_f32
+    q, k, v = _rand((1, 4, n, d), 1), _overflowing((1, 1, n, d), 64, 2), _rand((1, 1, n, d), 3)
+    q[..., 0] = 1e20
+    idx = torch.stack((torch.zeros(n, dtype=torch.long), 1 + torch.arange(n) % (n // 64)), -1)[None, None]
+    msk = torch.ones_like(idx, dtype=torch.bool)
+    want = O.select_attend(q.double(), k.double(), v.double(), idx, msk, 64, causal=True)
+    got = native_sparse_attend_f32(q.to(DEV), k.to(DEV), v.to(DEV), 64, idx.to(DEV), msk.to(DEV))
+    torch.cuda.synchronize()
+    assert_close(got, want, 1e-5, 1e-5, "out")
+
+
+@pytest.mark.parametrize("n,win", [(420, 130), (1400, 130), (4200, 40)])      # a work-group, a wave per query; 32-row tiles
+def test_interval_keys_that_score_minus_infinity(n, win):
+    from native_sparse_attention_pytorch_amd.ops import dense_attend_f32
+    q, k, v = _rand((1, 2, n, 64), 1), _overflowing((1, 1, n, 64), 300, 2), _rand((1, 1, n, 64), 3)
+    q[..., 0] = 1e20
+    got = dense_attend_f32(q.to(DEV), k.to(DEV), v.to(DEV), 0, True, win)[0][:, :, 300:340]      # (queries with at least one other key)
+    torch.cuda.synchronize()
+    i, j = torch.arange(300, 340)[:, None], torch.arange(n)[None, :]
+    sim = (q[:, :, 300:340].double() @ k.double().transpose(-1, -2) / 8).masked_fill((j > i) | (i - j > win), float("-inf"))
+    assert_close(got, sim.softmax(-1) @ v.double(), 1e-5, 1e-5, "out")
+
+
+def test_queries_without_a_live_slot_do_not_read_their_keys_scores():
+    """They attend their slots' blocks uniformly (NSA.py:809-815), also where the keys are infinite."""
+    from native_sparse_attention_pytorch_amd.ops import native_sparse_attend_f32
+    n = 130
+    q, k, v = (_rand((1, 2, n, 64), i) for i in range(3))
+    k, v = k[:, :1], v[:, :1]
+    idx = torch.tensor([0, 3]).expand(1, 1, n, 2).contiguous()
+    msk = torch.zeros_like(idx, dtype=torch.bool)
+    args = lambda key: (q.to(DEV), key.to(DEV), v.to(DEV), 32, idx.to(DEV), msk.to(DEV), False)
+    want = native_sparse_attend_f32(*args(k))
+    k[:, :, :5] = float("inf")
+    got = native_sparse_attend_f32(*args(k))
+    torch.cuda.synchronize()
+    mean = torch.cat((v[:, :, :32], v[:, :, 96:128]), 2).double().mean(2, keepdim=True).expand(1, 2, n, 64)
+    assert torch.equal(got, want)
+    assert_close(got, mean, 1e-5, 1e-5, "out")
+
+
 @pytest.mark.parametrize("rows,k,n,bias,act", [(1, 8, 1, True, None), (31, 264, 33, True, "relu"), (32, 512, 32, False, None), (33, 72, 100, True, None),
                                                (256, 512, 40, True, "relu")])
 def test_linear_f32(rows, k, n, bias, act):
