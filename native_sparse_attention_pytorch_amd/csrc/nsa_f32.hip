@@ -379,7 +379,8 @@ __global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const
   constexpr int VS = D + 8;                              // V row stride: the halves' rows (4 apart) lie 32 banks apart
   constexpr int LD = D / 32;                             // 16-byte loads per thread and tile of K (and of V)
   __shared__ float k_s[2][32 * D];                       // chunk c of row r at c ^ (r % 16)
-  __shared__ float v_s[2][32 * VS];
+  __shared__ float v_s[2][32 * VS];                      // (zeros for values that are not finite)
+  __shared__ int odd_s;                                  // there was such a value
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n_ = lane & 31, h = lane >> 5;
   const int bh = blockIdx.y, b = bh / A.hk, hk = bh % A.hk;
   const float* kb = k + b * A.sk[0] + hk * A.sk[1];
@@ -437,13 +438,23 @@ __global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const
   };
   const int t_first = g_lo & ~31;
   fetch(t_first);
+  if (tid == 0) odd_s = 0;
+  __syncthreads();
+  bool odd = false;
   int buf = 0;
   for (int t0 = t_first; t0 <= g_hi; t0 += 32, buf ^= 1) {
 #pragma unroll
     for (int u = 0; u < LD; ++u) {
       const int e = u * 256 + tid, r = e / (D / 4), c = e % (D / 4);
       *reinterpret_cast<floatx4*>(&k_s[buf][r * D + 4 * (c ^ (r & 15))]) = kx[u];
-      *reinterpret_cast<floatx4*>(&v_s[buf][r * VS + 4 * c]) = vx[u];
+      floatx4 x;
+#pragma unroll
+      for (int e2 = 0; e2 < 4; ++e2) {
+        const bool finite = fabsf(vx[u][e2]) < INFINITY;
+        odd |= !finite;
+        x[e2] = finite ? vx[u][e2] : 0.f;
+      }
+      *reinterpret_cast<floatx4*>(&v_s[buf][r * VS + 4 * c]) = x;
     }
     __syncthreads();          // (the other buffer was read before this barrier by every wave: it may be written in the next round)
     if (t0 + 32 <= g_hi) fetch(t0 + 32);
@@ -493,6 +504,28 @@ __global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const
       for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int ft = 0; ft < D / 32; ++ft) o[ft] = mfma32x2(vv[i][ft], sv[i8 + i], o[ft]);
+    }
+  }
+  // A value that is not finite is left out of the products, where a weight of zero times it would be NaN in every row of its tile,
+  // and added here to the rows that see its key.
+  if (odd) odd_s = 1;
+  __syncthreads();
+  if (odd_s) {
+#pragma unroll 1
+    for (int kr = g_lo; kr <= g_hi; ++kr) {
+      const float* vr = kr < own_mem ? A.memv + ((long)hk * A.mem + kr) * A.d : vb + (long)(kr - own_mem) * A.sv[2];
+      const bool visible = (unsigned)(kr - lo) <= seen;
+#pragma unroll
+      for (int ft = 0; ft < D / 32; ++ft)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int f0 = 32 * ft + 8 * u + 4 * h;
+          if (f0 >= A.d) continue;
+          const floatx4 x = *reinterpret_cast<const floatx4*>(vr + f0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (visible && !(fabsf(x[e]) < INFINITY)) o[ft][4 * u + e] += x[e];
+        }
     }
   }
   l = halves_sum(l);

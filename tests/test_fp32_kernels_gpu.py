@@ -111,6 +111,32 @@ def test_interval_keys_that_score_minus_infinity(n, win):
     assert_close(got, sim.softmax(-1) @ v.double(), 1e-5, 1e-5, "out")
 
 
+@pytest.mark.parametrize("d", [64, 100, 128])
+@pytest.mark.parametrize("mode,win,st", [(0, 70, 1), (1, 0, 8)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), "both"])
+def test_values_a_query_does_not_see_stay_out_of_its_result(value, mode, win, st, d):
+    """32-row tiles (4200 queries): a value row that is not finite reaches the queries that see its key and no others."""
+    from native_sparse_attention_pytorch_amd.ops import dense_attend_f32
+    n, mem = 4200, mode                                           # (the strided prefix stands behind a memory row)
+    keys = n // st
+    q, k, v = _rand((1, 2, n, d), 1), _rand((1, 1, mem + keys, d), 2), _rand((1, 1, mem + keys, d), 3)
+    rows = [mem + keys // 2, mem + keys - 40]
+    run = lambda: dense_attend_f32(q.to(DEV), k.to(DEV), v.to(DEV), mode, True, win, st, mem)[0].cpu()
+    clean = run()
+    v[:, :, rows[0], 3], v[:, :, rows[1], 3] = (float("inf"), float("-inf")) if value == "both" else (value, value)
+    v[:, :, rows[0], d - 1] = v[:, :, rows[0], 3]
+    got = run()
+    i, j = torch.arange(n), torch.tensor(rows) - mem
+    see = (j[:, None] <= i) & (i - j[:, None] <= win) if mode == 0 else (j[:, None] + 1) * st <= i           # [row, query]
+    want = clean.clone()
+    for r, first in enumerate(rows):
+        for f in (3, d - 1) if r == 0 else (3,):
+            want[:, :, see[r], f] += v[0, 0, first, f]
+    assert torch.equal(got.isnan(), want.isnan())
+    same = want.isnan() | (got == want)
+    assert same.all(), (~same).nonzero()[:5]
+
+
 def test_queries_without_a_live_slot_do_not_read_their_keys_scores():
     """They attend their slots' blocks uniformly (NSA.py:809-815), also where the keys are infinite."""
     from native_sparse_attention_pytorch_amd.ops import native_sparse_attend_f32
