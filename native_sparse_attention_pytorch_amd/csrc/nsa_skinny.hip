@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kSkinnyThreads, 4) void skinny_linear_kernel(const 
       const float u = (float)(__bf16)t;
       t = 0.5f * u * (1.0f + erff(u * 0.70710678118654752f));
     } else if (A.act == NSA_ACT_RELU) {
-      t = fmaxf(t, 0.f);
+      t = t < 0.f ? 0.f : t;                              // (NaN stays, as the layer leaves it)
     }
     if (o == 0 && A.res != nullptr) t = (float)(__bf16)t + (float)A.res[row * A.rs + n0 + f];
     A.y[o][row * A.ys[o] + n0 + f] = (__bf16)t;
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(int rows, int K, int N,
 #pragma unroll
     for (int v = 0; v < 8; ++v) t += part_s[v][row][f];
     if (bias != nullptr) t += bias[n0 + f];
-    if (act == NSA_ACT_RELU) t = fmaxf(t, 0.f);
+    if (act == NSA_ACT_RELU) t = t < 0.f ? 0.f : t;      // (NaN stays)
     y[(long)(m0 + row) * N + n0 + f] = t;
   }
 }

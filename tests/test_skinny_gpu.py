@@ -62,6 +62,18 @@ def test_skinny_epilogue(rows, k, n, act, res):
     assert got.shape == (rows, 1, n) and (err <= tol).all(), (err - tol).max().item()
 
 
+@pytest.mark.parametrize("dtype, act", [(torch.bfloat16, None), (torch.bfloat16, "relu"), (torch.bfloat16, "gelu"), (torch.float32, None), (torch.float32, "relu")])
+def test_what_is_not_finite_passes_the_epilogue(dtype, act):
+    """NaN and infinities through the activations as the layers hand them on (relu(NaN) is NaN)."""
+    from native_sparse_attention_pytorch_amd import ops
+    fn = ops.skinny_linear if dtype == torch.bfloat16 else ops.linear_f32
+    bias = torch.tensor([float("nan"), float("inf"), float("-inf"), 1., -1.])
+    want = {None: lambda t: t, "relu": torch.relu, "gelu": torch.nn.functional.gelu}[act](bias.to(DEV, dtype)).expand(3, 5)
+    got = fn(torch.zeros(3, 64, device=DEV, dtype=dtype), torch.zeros(5, 64, device=DEV, dtype=dtype), bias.to(DEV, dtype), act=act)
+    torch.cuda.synchronize()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 def test_decode_layer_fills_the_newest_rows_and_reports_the_selection():
     """The whole-layer call: rows of the caches and of the open window, the selection's views, against the general path."""
     from native_sparse_attention_pytorch_amd import SparseAttention, ops
