@@ -231,7 +231,7 @@ class SparseAttention(nn.Module):
         # the default network (flatten, linear, relu, linear) layer by layer, so that its projections go through ops.linear
         if not cls._plain(mlp, nn.Sequential):
             return mlp(windows)
-        if (len(mlp) == 4 and windows.dtype == torch.float32 and type(mlp[0]) is _FlattenWindow and cls._plain(mlp[1], nn.Linear)
+        if (len(mlp) == 4 and windows.dtype == torch.float32 and cls._plain(mlp[0], _FlattenWindow) and cls._plain(mlp[1], nn.Linear)
                 and cls._plain(mlp[2], nn.ReLU) and not torch.is_grad_enabled() and ops.plain_call()):
             x = windows.flatten(-2)
             if ops.linear_f32_supported(x, mlp[1].weight, mlp[1].bias):
@@ -307,7 +307,7 @@ class SparseAttention(nn.Module):
     def _compress_rows(cls, mlp, window):
         """The compression network on one complete window per sequence, 'b h cbs d' -> 'b h 1 d'."""
         b, h, n, d = window.shape
-        if cls._plain(mlp, nn.Sequential) and len(mlp) == 4 and type(mlp[0]) is _FlattenWindow and window.dtype == torch.bfloat16:
+        if cls._plain(mlp, nn.Sequential) and len(mlp) == 4 and cls._plain(mlp[0], _FlattenWindow) and window.dtype == torch.bfloat16:
             _, up, act, down = mlp
             x = window.reshape(b * h, n * d)
             if (cls._plain(up, nn.Linear) and cls._plain(act, nn.ReLU) and cls._plain(down, nn.Linear) and ops.plain_call()
