@@ -141,9 +141,9 @@ def test_inputs_off_a_boundary_are_copied(calls):
 @pytest.mark.parametrize("hook", ["register_forward_hook", "register_forward_pre_hook"])
 def test_hooks_on_the_flatten_layer_run(calls, dtype, hook):
     """The compression network's first layer is its own call whenever something hangs on it."""
-    m = SparseAttention(dim=128, dim_head=64, heads=4, kv_heads=2, causal=True, sliding_window_size=16, compress_block_size=16,
+    m = SparseAttention(dim=128, dim_head=64, heads=4, kv_heads=2, causal=True, sliding_window_size=16, compress_block_size=8,
                         compress_block_sliding_stride=8, selection_block_size=16, num_selected_blocks=2).to(dtype)
-    run = (lambda: m._compress_rows(m.k_compress, _dev(2, 2, 16, 64))) if dtype == BF16 else (lambda: m._compress(m.k_compress, _dev(2, 2, 3, 16, 64, dtype=F32)))
+    run = (lambda: m._compress_rows(m.k_compress, _dev(2, 2, 8, 64))) if dtype == BF16 else (lambda: m._compress(m.k_compress, _dev(2, 2, 3, 8, 64, dtype=F32)))
     with torch.no_grad():
         run()
         assert calls
