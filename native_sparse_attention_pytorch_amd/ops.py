@@ -1374,7 +1374,7 @@ def decode_step(q: Tensor, k: Tensor, v: Tensor, freqs: Tensor, pos: int, keys: 
     for t in (keys, vals) + ((ck, cv) if nc else ()):
         if t.dtype != _BF16 or not t.is_cuda or not _rows_ok(t):
             raise RuntimeError("decode_step: caches must be bf16 device tensors with unit feature stride and 16-byte aligned rows")
-        if t.dim() != 4 or t.shape[0] != b or t.shape[1] != hk or t.shape[3] != d:
+        if t.dim() != 4 or t.shape[0] < b or t.shape[1] < hk or t.shape[3] < d:
             raise RuntimeError("decode_step: caches must be 'b hk n d' of the new token's batch, heads and features")
     if nc and cv.shape[2] < nc:
         raise RuntimeError("decode_step: fewer compressed values than keys")

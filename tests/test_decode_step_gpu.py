@@ -115,3 +115,21 @@ def test_caches_of_another_shape_are_refused(wrong):
     with pytest.raises(RuntimeError, match="batch, heads"):
         ops.decode_step(q, k, k, freqs, 8, z(b, hk, 9, 64), z(b, hk, 9, 64), None, None, None, None, None, None, gl, per_block=2, block=16, num_sel=2,
                         share=True, window=16)
+
+
+def test_caches_of_more_sequences_or_heads_are_read_from_their_start():
+    """Buffers larger than the step (more sequences, more heads): the step takes their first ones."""
+    from native_sparse_attention_pytorch_amd import ops
+    g = torch.Generator().manual_seed(1)
+    r = lambda *s: torch.randn(*s, generator=g).to(BF16).to(DEV)
+    q, k, v, gl, freqs = r(2, 4, 1, 64), r(2, 2, 1, 64), r(2, 2, 1, 64), r(2, 1, 12), torch.ones(32, device=DEV)
+    big = [r(3, 3, n, 64) for n in (41, 41, 10, 10)]
+    first = [t[:2, :2].clone() for t in big]
+    run = lambda c: ops.decode_step(q, k, v, freqs, 40, *c, None, None, None, None, gl, per_block=2, block=16, num_sel=2, share=True, window=16)[0]
+    rest = [t.clone() for t in big]
+    got, want = run(big), run(first)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and all(torch.equal(a[:2, :2], b) for a, b in zip(big, first))
+    for a, b in zip(big, rest):
+        b[:2, :2] = a[:2, :2]
+        assert torch.equal(a, b)
