@@ -1690,11 +1690,21 @@ def _wgrad_splits(rows: int, n_in: int, n_out: int, replayed: bool = False) -> i
 
 
 def linear_f32_supported(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> bool:
-    """An fp32 projection small enough that the GEMM library's tiles leave most of the chip idle.  Measured, this kernel / the
-    library in us: 240 x 256 -> 256 4.8 / 64.7, 240 x 512 -> 24 6.2 / 19.9, 62 x 512 -> 1536 6.7 / 6.8, 256 x 512 -> 1536 11.6 / 8.5
-    (the library's call takes the host 14 us longer), 384 x 256 -> 256 4.8 / 6.1, 256 x 1024 -> 1024 12.3 / 9.1."""
+    """An fp32 projection that `linear_f32` serves and the GEMM library does not serve better.  Measured on the GPU alone, this kernel
+    / the library in us (its call takes the host another 12):
+      up to 256 outputs the library's tiles leave most of the chip idle: 240 x 256 -> 256 4.0 / 59, 240 x 512 -> 24 5.6 / 18, 1 x 512 -> 256 5.0 / 12.4;
+      more of them cost this kernel a second round once its 32 x 32 tiles exceed the CUs: 256 x 256 -> 1024 (256 tiles) 4.6 / 5.6, 192 x 256 ->
+      1536 (288) 6.4 / 5.5, 256 x 512 -> 1536 (384) 10.4 / 7.6; with K above 256 the two meet at half of that: 62 x 512 -> 1536 (96) 6.0 / 6.1,
+      128 x 512 -> 1024 (128) 6.1 / 6.0, 128 x 512 -> 1536 (192) 6.4 / 6.2;
+      for 2 to 31 rows and more than 256 outputs the library has a kernel that wins when K exceeds 256: 8 x 512 -> 512 5.2 / 4.3, 31 x 320 -> 300
+      4.4 / 3.9, but 8 x 256 -> 512 3.6 / 3.7, 1 x 512 -> 512 5.0 / 6.0, 32 x 512 -> 512 5.8 / 5.9."""
     rows, k = x.numel() // max(x.shape[-1], 1), x.shape[-1]
-    return x.is_cuda and x.dtype == torch.float32 and 0 < rows <= 256 and k <= 512 and k % 8 == 0 and _weight_ready(x, k, weight) and _vectors_ready(x, weight, bias, None)
+    if not (x.is_cuda and x.dtype == torch.float32 and 0 < rows <= 256 and k <= 512 and k % 8 == 0 and _weight_ready(x, k, weight)
+            and _vectors_ready(x, weight, bias, None)):
+        return False
+    n = weight.shape[0]
+    tiles = -(-rows // 32) * -(-n // 32)
+    return n <= 256 or (tiles <= 256 if k <= 256 else tiles <= 128 and not 1 < rows < 32)
 
 
 def _laid_out(t: Tensor) -> Tensor:

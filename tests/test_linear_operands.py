@@ -151,3 +151,14 @@ def test_hooks_on_the_flatten_layer_run(calls, dtype, hook):
         getattr(m.k_compress[0], hook)(lambda *args: seen.append(len(args)) or None)
         run()
     assert len(seen) == 1
+
+
+@pytest.mark.parametrize("rows, k, n, own", [
+    (62, 512, 1536, True), (240, 512, 24, True), (256, 512, 256, True),       # the smallest layer's projections; few outputs
+    (256, 512, 1536, False), (128, 512, 3072, False), (256, 256, 6144, False),    # more tiles than the chip takes at once
+    (256, 256, 1024, True), (160, 256, 2048, False),
+    (8, 512, 512, False), (31, 320, 300, False), (1, 512, 512, True), (32, 512, 512, True), (8, 256, 512, True),
+    (257, 64, 64, False), (8, 520, 64, False), (8, 60, 64, False),
+])
+def test_fp32_projections_that_the_library_serves_better_stay_with_it(rows, k, n, own):
+    assert ops.linear_f32_supported(_dev(rows, k, dtype=F32), _dev(n, k, dtype=F32)) is own
