@@ -143,16 +143,17 @@ class DecodeSession:
             torch.cuda.current_stream(dev).wait_stream(side)
             # [0]: ordinary step, [1]: step that completes a window.  A direct step reads the caller's token and writes a new
             # result itself (recorded, it would need a copy of the token into a fixed buffer and one of the result out of
-            # another, each a launch like the other five): of its second graph only the window is recorded
+            # another, each a launch like the other five): of its graphs only the window of the second is recorded
             self.graphs, self.outs = [], []
             for event in (False, True):
-                g = torch.cuda.CUDAGraph()
+                g = None if self.direct and not event else torch.cuda.CUDAGraph()
                 out = None
-                with torch.no_grad(), torch.cuda.graph(g):
-                    if not (self.direct and event):
-                        out = self.layer_step(self.x_buf, advance=1)
-                    if event:
-                        self.compress_window()
+                if g is not None:
+                    with torch.no_grad(), torch.cuda.graph(g):
+                        if not self.direct:
+                            out = self.layer_step(self.x_buf, advance=1)
+                        if event:
+                            self.compress_window()
                 self.graphs.append(g)
                 self.outs.append(out)
             if self.direct:

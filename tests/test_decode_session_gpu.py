@@ -104,3 +104,8 @@ def test_a_step_cannot_be_recorded():
             session.step(x)
     assert session.pos == 37
     assert torch.equal(session.step(x), type(session)(m, cache, max_len=64).step(x))
+
+
+def test_a_direct_session_records_nothing_but_its_windows():
+    _, _, session = _session()
+    assert session.direct and session.graphs[0] is None and session.graphs[1] is not None and session.outs == [None, None]
