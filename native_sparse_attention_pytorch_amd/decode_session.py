@@ -130,7 +130,7 @@ class DecodeSession:
         # launches, ~35 us), with the GEMM library's (~20 us of host time each) when the weights are what takes time
         self.direct = self.own_norm and self.fused_gate and m._plain(out, torch.nn.Linear) and m.to_qkv.bias is None and (
             (self.own_in and self.own_out) or self.w_cat.numel() * 2 >= 32 << 20)
-        self.graphs = None
+        self._graphs = None
         if capture:
             # the libraries initialise themselves on first use (outside the capture); the warm-up steps write row `pos` of
             # the caches and row `nc` of the compressed caches, which the first real steps overwrite, and leave both counters alone
@@ -143,23 +143,30 @@ class DecodeSession:
             torch.cuda.current_stream(dev).wait_stream(side)
             # [0]: ordinary step, [1]: step that completes a window.  A direct step reads the caller's token and writes a new
             # result itself (recorded, it would need a copy of the token into a fixed buffer and one of the result out of
-            # another, each a launch like the other five): of its graphs only the window of the second is recorded
-            self.graphs, self.outs = [], []
-            for event in (False, True):
-                g = None if self.direct and not event else torch.cuda.CUDAGraph()
-                out = None
-                if g is not None:
-                    with torch.no_grad(), torch.cuda.graph(g):
-                        if not self.direct:
-                            out = self.layer_step(self.x_buf, advance=1)
-                        if event:
-                            self.compress_window()
-                self.graphs.append(g)
-                self.outs.append(out)
+            # another, each a launch like the other five): only the window that completes is recorded for it
+            self._graphs, self.outs = [None, None], [None, None]
+            for event in ((True,) if self.direct else (False, True)):
+                self._record(event, step=not self.direct)
             if self.direct:
                 self._prepare_direct(merged)
 
     # ---------------------------------------------------------------------------------------
+
+    def _record(self, event: bool, step: bool):
+        self._graphs[event] = g = torch.cuda.CUDAGraph()
+        with torch.no_grad(), torch.cuda.graph(g):
+            if step:
+                self.outs[event] = self.layer_step(self.x_buf, advance=1)
+            if event:
+                self.compress_window()
+
+    @property
+    def graphs(self):
+        """[an ordinary step, one that completes a window] as recorded, for a caller that replays them itself (`x_buf` the token, `outs` the
+        results); None with capture=False.  Direct steps do not replay the first: it is recorded when it is asked for."""
+        if self._graphs is not None and self._graphs[0] is None:
+            self._record(False, step=True)
+        return self._graphs
 
     def _make_desc(self, dev):
         m = self.module
@@ -284,7 +291,7 @@ class DecodeSession:
     @torch.no_grad()
     def step(self, x: torch.Tensor) -> torch.Tensor:
         """x 'b 1 dim', or what is broadcast to it: the token at position `self.pos`.  Returns the layer output 'b 1 dim' (a new tensor)."""
-        if self.graphs is None:
+        if self._graphs is None:
             raise RuntimeError("DecodeSession was built with capture=False (its launches belong to an enclosing graph)")
         if self.pos >= self.max_len:
             raise RuntimeError(f"DecodeSession: capacity of {self.max_len} tokens reached")
@@ -297,11 +304,11 @@ class DecodeSession:
         if self.direct:
             out = self._step_direct(x)
             if event:
-                self.graphs[1].replay()
+                self._graphs[1].replay()
             self.advance_host(event)
             return out
         self.x_buf.copy_(x)
-        self.graphs[event].replay()
+        self._graphs[event].replay()
         self.advance_host(event)
         return self.outs[event].clone()
 

@@ -106,6 +106,13 @@ def test_a_step_cannot_be_recorded():
     assert torch.equal(session.step(x), type(session)(m, cache, max_len=64).step(x))
 
 
-def test_a_direct_session_records_nothing_but_its_windows():
-    _, _, session = _session()
-    assert session.direct and session.graphs[0] is None and session.graphs[1] is not None and session.outs == [None, None]
+def test_a_direct_session_records_a_step_only_for_a_caller_that_replays_it():
+    m, cache, session = _session()
+    x = torch.randn(4, 1, 128, device=DEV, dtype=BF16)
+    assert session.direct and session._graphs[0] is None and session._graphs[1] is not None
+    session.x_buf.copy_(x)
+    for replay in range(3):
+        session.state[0] = 37
+        session.graphs[0].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(session.outs[0], type(session)(m, cache, max_len=64).step(x)) and int(session.state[0]) == 38

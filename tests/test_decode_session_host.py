@@ -21,7 +21,7 @@ def test_a_step_runs_on_the_session_s_device(monkeypatch):
     monkeypatch.setattr(torch.cuda, "device", device)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     s = object.__new__(DecodeSession)
-    s.graphs, s.direct, s.pos, s.nc, s.max_len, s.st, s.max_nc = [], True, 0, 0, 8, 4, 2
+    s._graphs, s.direct, s.pos, s.nc, s.max_len, s.st, s.max_nc = [], True, 0, 0, 8, 4, 2
     s.K = SimpleNamespace(device=torch.device("cuda", 3))
     s._step_direct = lambda x: current[0]
     assert s.step(None) == 3 and current[0] == 0 and s.pos == 1
