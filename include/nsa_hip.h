@@ -390,8 +390,10 @@ int nsa_decode_combine(const nsa_decode_desc* compressed, const void* ws_compres
                        const void* gate_logits, void* out, void* stream);
 
 /* The attention part of one decode step (NSA.py:377-545 without the projections and the compression of
- * a completed window) as one host call: nsa_decode_prep, the compressed branch, nsa_decode_topk, the
- * selected-block branch, the sliding branch and nsa_decode_combine, with all intermediates in `ws`.
+ * a completed window) as one host call and three launches, with all intermediates in `ws`: what
+ * nsa_decode_prep does is part of the sliding branch, which shares a launch with the compressed branch;
+ * the selected-block branch makes its own selection; the merge is that of nsa_decode_combine.  (per_block
+ * other than a power of two up to 32: the selection is a fourth launch, nsa_decode_topk.)
  * pos = rows already in the key / value caches (the new token's position); the caches must have row
  * pos free.  num_sel is the configured number of blocks; min(num_sel, num_compressed / per_block) are
  * selected, their indices (int32) and mask (uint8), [batch, kv_heads or heads, k], are left in the

@@ -898,10 +898,10 @@ extern "C" int nsa_decode_combine(const nsa_decode_desc* compressed, const void*
 }
 
 // ---------------------------------------------------------------------------- whole step
-// The attention part of one decode step as a single host call: prep, compressed branch, block
-// selection, selected-block branch, sliding branch, merge + gate.  The launches are the same as
-// through the separate entry points; what goes away is the host-side work between them, which
-// at small batch is most of a step's time.
+// The attention part of one decode step as a single host call and three launches: the sliding branch, which rotates the queries
+// and brings the new token into the caches, together with the compressed branch, which leaves its logits pooled per block; the
+// selected-block branch, whose work-groups make the selection themselves; merge + gate.  (Blocks of other than 1, 2, 4 .. 32
+// compressed keys: one logit per key and head, and the top-k kernel as a launch of its own.)
 
 namespace nsa {
 
