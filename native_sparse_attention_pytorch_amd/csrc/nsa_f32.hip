@@ -251,11 +251,8 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
   if constexpr (SELECT) {
     if (A.uniform) {
       dead = true;
-      for (int s = lane; s < A.S; s += 64) {
-        const size_t at = ((size_t)bh * A.n + i) * A.S + s;
-        const long j = A.idx64 ? (long)reinterpret_cast<const long long*>(idx)[at] : (long)reinterpret_cast<const int*>(idx)[at];
-        if (fmask[at] && j >= 0 && j < A.W) dead = false;
-      }
+      for (int s = lane; s < A.S; s += 64)
+        if (fmask[((size_t)bh * A.n + i) * A.S + s]) dead = false;      // (a live slot that names no block: nothing attended, as before)
       dead = !__any(!dead);
     }
   }

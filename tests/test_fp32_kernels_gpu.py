@@ -155,6 +155,17 @@ def test_queries_without_a_live_slot_do_not_read_their_keys_scores():
     assert_close(got, mean, 1e-5, 1e-5, "out")
 
 
+def test_live_slots_that_name_no_block_attend_nothing():
+    """Not causal, an index out of range under a live slot: the query is not one without live slots, and has nothing to attend."""
+    from native_sparse_attention_pytorch_amd.ops import native_sparse_attend_f32
+    n = 128
+    q, k, v = (_rand((1, 2, n, 64), i)[:, :h].to(DEV) for i, h in ((1, 2), (2, 1), (3, 1)))
+    idx = torch.tensor([-1, 5]).expand(1, 1, n, 2).contiguous().to(DEV)
+    out, lse = native_sparse_attend_f32(q, k, v, 32, idx, torch.ones_like(idx, dtype=torch.bool), False, return_lse=True)
+    torch.cuda.synchronize()
+    assert not out.any() and (lse == float("-inf")).all()
+
+
 @pytest.mark.parametrize("rows,k,n,bias,act", [(1, 8, 1, True, None), (31, 264, 33, True, "relu"), (32, 512, 32, False, None), (33, 72, 100, True, None),
                                                (256, 512, 40, True, "relu")])
 def test_linear_f32(rows, k, n, bias, act):
