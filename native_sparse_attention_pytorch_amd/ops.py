@@ -453,7 +453,11 @@ def _importance_products_backward(q, ck, dpooled, num_mem, stride, sel_block, sh
     block's npf compressed keys and, if shared, the group's heads) with respect to q and ck.  The
     logits are linear in both, so this is two small dense GEMMs per (batch, kv head); entries that
     were -inf carry zero gradient by construction of the softmax that follows.  Returns (dq 'b hk n d' (shared) or 'b hq n d', dck
-    'b hk nb d' of every key of a block, c): both still to be multiplied by c."""
+    'b hk nb d' of every key of a block, c): both still to be multiplied by c, both fp32 (a backward inside an autocast region would
+    hand out 16-bit products)."""
+    if torch.is_autocast_enabled(q.device.type):
+        with torch.autocast(q.device.type, enabled=False):
+            return _importance_products_backward(q, ck, dpooled, num_mem, stride, sel_block, share, scale)
     b, hq, n, d = q.shape
     hk = ck.shape[1]
     g = hq // hk
@@ -483,6 +487,9 @@ def _importance_backward(q, ck, dpooled, num_mem, stride, sel_block, share, scal
 def _add_repeated(base: Tensor, small: Tensor, out: Tensor, head_repeat: int, row_offset: int, row_repeat: int, c: float) -> Tensor:
     """out (bf16, may be base) = base + c * small, small's heads and rows repeated (nsa_add_repeated)."""
     b, h, n, d = base.shape
+    if (small.dtype != torch.float32 or base.dtype not in (torch.float32, _BF16) or out.dtype != _BF16 or not base.is_contiguous()
+            or not out.is_contiguous() or out.shape != base.shape or small.shape[:2] != (b, h // head_repeat) or small.shape[3] != d):
+        raise RuntimeError("_add_repeated: fp32 'b h/head_repeat rows d' onto contiguous fp32 or bf16 'b h n d'")
     small = small.contiguous()
     _lib.check(_lib.lib().nsa_add_repeated(_ptr(base), int(base.dtype == torch.float32), b, h, n, d, _ptr(small), head_repeat, row_offset, row_repeat,
                                            small.shape[2], float(c), _ptr(out), _stream()), "nsa_add_repeated")
