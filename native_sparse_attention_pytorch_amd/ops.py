@@ -772,6 +772,9 @@ def _(scores, k, apply_softmax, seq, block):
 
 @torch.library.custom_op("nsa_amd::topk_bwd", mutates_args=())
 def topk_bwd(logits: Tensor, idx: Tensor, dvals: Tensor) -> Tensor:
+    if (logits.dtype != torch.float32 or not logits.is_cuda or idx.dtype != torch.int32 or idx.device != logits.device or dvals.device != logits.device
+            or dvals.shape != idx.shape or idx.shape[:-1] != logits.shape[:-1]):
+        raise RuntimeError("topk_bwd: fp32 logits '... nb' on the device, int32 indices and gradients '... k'")
     logits, idx, dvals = logits.contiguous(), idx.contiguous(), dvals.to(torch.float32).contiguous()
     out = torch.empty_like(logits)
     nb, k = logits.shape[-1], idx.shape[-1]
@@ -818,6 +821,8 @@ def importance_topk(importance_logits: Tensor, num_selected: int, prefix=None, r
     `raw` = (scale, seq, causal block or 0, own block or 0): the logits are fp32 products that the kernel scales and masks
     (`importance_topk_f32`; no gradient)."""
     if raw is not None:
+        if importance_logits.dtype != torch.float32 or not importance_logits.is_cuda:
+            raise RuntimeError("importance scores must be fp32 device tensors")
         rows = importance_logits.detach().contiguous()
         shp = (*rows.shape[:-1], int(num_selected))
         idx = torch.empty(shp, dtype=torch.int32, device=rows.device)

@@ -28,6 +28,22 @@ def test_a_summand_of_another_type_is_refused(monkeypatch):
             ops._add_repeated(b, small, torch.empty_like(base), 1, 0, 1, 1.0)
 
 
+def test_scores_of_another_type_are_refused(monkeypatch):
+    """The masked top-k and the gradient of its values read fp32 rows, as the top-k itself, which refuses others."""
+    class OnDevice(torch.Tensor):
+        is_cuda = True
+    monkeypatch.setattr(_lib, "lib", lambda: pytest.fail("reached the library"))
+    dev = lambda *s, dtype=torch.float32: torch.zeros(s, dtype=dtype).as_subclass(OnDevice)
+    half, raw = dev(1, 2, 8, 4, dtype=torch.bfloat16), (0.25, 8, 2, 2)
+    for call in (lambda: ops.importance_topk(half, 2, raw=raw), lambda: ops.importance_topk(torch.zeros(1, 2, 8, 4), 2, raw=raw),
+                 lambda: ops.topk_bwd._init_fn(half, dev(1, 2, 8, 2, dtype=torch.int32), dev(1, 2, 8, 2)),
+                 lambda: ops.topk_bwd._init_fn(dev(1, 2, 8, 4), dev(1, 2, 8, 2, dtype=torch.int64), dev(1, 2, 8, 2)),
+                 lambda: ops.topk_bwd._init_fn(dev(1, 2, 8, 4), dev(1, 2, 8, 2, dtype=torch.int32), dev(1, 2, 8, 3)),
+                 lambda: ops.topk_bwd._init_fn(dev(1, 2, 8, 4), dev(1, 2, 6, 2, dtype=torch.int32), dev(1, 2, 6, 2))):
+        with pytest.raises(RuntimeError):
+            call()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("share", [True, False])
 def test_backward_inside_autocast_equals_backward_outside(share):
