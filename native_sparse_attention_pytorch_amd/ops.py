@@ -2124,11 +2124,20 @@ class _QkvPrepF32(torch.autograd.Function):
         return dqkv, None, *pos, None, None, None, None, None, None
 
 
+def qkv_prep_f32_operands(qkv: Tensor, freqs: Tensor, k_positions: Tensor, v_positions: Tensor, kv_heads: int, dim_head: int, block: int) -> bool:
+    """Frequencies and intra-window positions as the kernel reads them (operators broadcast others)."""
+    return (all(t.device == qkv.device for t in (freqs, k_positions, v_positions)) and freqs.shape == (dim_head // 2,)
+            and k_positions.shape == v_positions.shape == (kv_heads, block, dim_head))
+
+
 def qkv_prep_f32(qkv: Tensor, freqs: Tensor, k_positions: Tensor, v_positions: Tensor, heads: int, kv_heads: int, dim_head: int,
                  compress_block_size: int, compress_stride: int, offset: int = 0):
     """`qkv_prep` for the fp32 forward: (q, rotated q, rotated k, v, k windows, v windows), all fp32; q and v are views of
     the projection.  dim_head 64 or 128.  Differentiable in the projection and the positions."""
     if qkv.dtype != torch.float32 or dim_head not in (64, 128) or not qkv.is_cuda:
         raise RuntimeError("qkv_prep_f32: needs an fp32 device projection with dim_head 64 or 128")
+    if qkv.dim() != 3 or qkv.shape[2] != (heads + 2 * kv_heads) * dim_head or not qkv_prep_f32_operands(
+            qkv, freqs, k_positions, v_positions, kv_heads, dim_head, compress_block_size or k_positions.shape[1]):
+        raise RuntimeError("qkv_prep_f32: projection 'b n ((h + 2 hk) d)', frequencies 'd/2' and positions 'hk block d' on its device")
     return _QkvPrepF32.apply(qkv, freqs, k_positions, v_positions, int(heads), int(kv_heads), int(dim_head), int(compress_block_size),
                              int(compress_stride), int(offset))

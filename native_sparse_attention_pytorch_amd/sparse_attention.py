@@ -214,11 +214,14 @@ class SparseAttention(nn.Module):
             return False
         return ops.rms_norm_supported(inp, norm.weight) and (inp.requires_grad or any(p.requires_grad for p in self.parameters()))
 
-    def _plain_rotary(self, batch):
-        """Rotation and window split may be the kernel's under autograd: frequencies that are not trained, no hooks, its own types."""
-        rot = self.rotary_emb
-        return (self._plain(rot, RotaryEmbedding) and not rot.freqs.requires_grad and batch <= 65535
-                and all(p.dtype == torch.float32 for p in (self.k_intrablock_positions, self.v_intrablock_positions)))
+    def _prep_by_kernel(self, qkv, recording):
+        """Rotation and window split of an fp32 projection may be the kernel's: frequencies and positions of the sizes and on the device it
+        reads them from; under autograd also frequencies that are not trained, no hooks, its own types."""
+        rot, pos = self.rotary_emb, (self.k_intrablock_positions, self.v_intrablock_positions)
+        if self.dim_head not in (64, 128) or not ops.qkv_prep_f32_operands(qkv, rot.freqs, *pos, self.kv_heads, self.dim_head, self.compress_block_size):
+            return False
+        return not recording or (self._plain(rot, RotaryEmbedding) and not rot.freqs.requires_grad and qkv.shape[0] <= 65535
+                                 and all(p.dtype == torch.float32 for p in pos))
 
     def _normed(self, x):
         norm = self.norm
@@ -468,7 +471,7 @@ class SparseAttention(nn.Module):
         L = (n // st) * st
         recording = torch.is_grad_enabled() and (qkv.requires_grad or any(p.requires_grad for p in self.parameters()))
         qa, va = q, v                                    # as the attention branches read them (the caches hand out q, k, v themselves)
-        if d in (64, 128) and (not recording or self._plain_rotary(b)):
+        if self._prep_by_kernel(qkv, recording):
             qa, rq, rk, va, kw, vw = ops.qkv_prep_f32(qkv, self.rotary_emb.freqs, self.k_intrablock_positions, self.v_intrablock_positions,
                                                       self.heads, self.kv_heads, d, cbs, st)
         else:
