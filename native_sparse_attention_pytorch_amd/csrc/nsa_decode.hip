@@ -610,7 +610,7 @@ struct CombineArgs {
 template <int D>
 __global__ __launch_bounds__(384) void decode_combine_kernel(const CombineArgs A, const __bf16* __restrict__ gate_logits, __bf16* __restrict__ out) {
   constexpr int LPP = D / 4, PPR = 128 / LPP;              // lanes per partial, partials per round of a branch
-  __shared__ float w_s[3][kMaxParts];
+  __shared__ float w_s[3][kMaxParts], sum_s[3];
   __shared__ __align__(16) float acc_s[3][PPR][D];
   const int hq = A.P[0].hk * A.P[0].g;
   const int bh = blockIdx.x, b = bh / hq, head = bh % hq;
@@ -636,6 +636,7 @@ __global__ __launch_bounds__(384) void decode_combine_kernel(const CombineArgs A
     L = wave_reduce_sum(L);
     const float inv = L > 0.f ? 1.0f / L : 0.f;
     if (t < 64) {
+      if (lane == 0) sum_s[s] = L;
 #pragma unroll
       for (int r = 0; r < PT; ++r) w_s[s][lane + 64 * r] = mp[r] * inv;
     }
@@ -660,6 +661,7 @@ __global__ __launch_bounds__(384) void decode_combine_kernel(const CombineArgs A
       float o = 0.f;
 #pragma unroll
       for (int r = 0; r < PPR; ++r) o += acc_s[br][r][f];
+      o = sum_s[br] > 0.f ? o : 0.f;                       // no key, or a sum that is no number: nothing, as merge_head_partials
       float gl = (float)gate_logits[(long)b * A.gate_row + head * 3 + br];
       if (A.gate_bias != nullptr) gl += (float)A.gate_bias[head * 3 + br];
       res += (float)(__bf16)o / (1.f + __expf(-gl));       // branch outputs are rounded to bf16 as when each is merged on its own

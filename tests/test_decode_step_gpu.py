@@ -133,3 +133,22 @@ def test_caches_of_more_sequences_or_heads_are_read_from_their_start():
     for a, b in zip(big, rest):
         b[:2, :2] = a[:2, :2]
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_a_branch_whose_sum_is_no_number_adds_nothing(value, d):
+    """Keys that are not finite in the window: the branch is left out whole, as when it is merged on its own; the others stand."""
+    from native_sparse_attention_pytorch_amd import ops
+    g = torch.Generator().manual_seed(d)
+    r = lambda *s: torch.randn(*s, generator=g).to(BF16).to(DEV)
+    b, hq, hk, n = 2, 4, 2, 130
+    rq, ks, vs, gl = r(b, hq, 1, d), r(b, hk, n, d), r(b, hk, n, d), r(b, 1, 3 * hq)
+    ks[:, :, 70] = value
+    idx = torch.zeros(b, hk, 1, 1, dtype=torch.int32, device=DEV)
+    f = ops.decode_select_attend(rq, ks, vs, 64, 32, idx, torch.ones_like(idx, dtype=torch.bool), merge=False)      # the first 64 keys: finite
+    s = ops.decode_range_attend(rq, ks, vs, n - 65, 65, merge=False)
+    alone = ops.decode_range_attend(rq, ks, vs, n - 65, 65)
+    got, want = ops.decode_combine(gl, None, f, s), ops.decode_combine(gl, None, f, ops.decode_range_attend(rq, ks, torch.zeros_like(vs), 0, 64, merge=False))
+    torch.cuda.synchronize()
+    assert not alone.any() and torch.isfinite(got).all() and torch.equal(got, want)
