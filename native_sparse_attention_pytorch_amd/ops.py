@@ -1627,13 +1627,17 @@ def rms_norm(x: Tensor, weight: Tensor, eps: float | None = None) -> Tensor:
 
 # ------------------------------------------------------------------ projections
 
+_is_compiling, _is_autocast, _forward_ad = torch.compiler.is_compiling, torch.is_autocast_enabled, torch.autograd.forward_ad
+_transforms, _dispatch_modes, _tracing_state = torch._C._functorch.peek_interpreter_stack, torch._C._len_torch_dispatch_stack, torch._C._get_tracing_state
+_dispatch_key, _PRE_DISPATCH = torch._C._dispatch_tls_is_dispatch_key_included, torch._C.DispatchKey.PreDispatch
+
+
 def plain_call() -> bool:
     """Nothing is at work that an operator carries and a kernel launched by address loses: autocast, a compiler or another tracer (which
     would record the result as a constant), vmap, jvp, a forward-mode level, a dispatch mode.  Asked before any address is read:
     a batched or traced tensor has none."""
-    return not (torch.compiler.is_compiling() or torch.is_autocast_enabled() or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0
-                or torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0 or torch._C._get_tracing_state() is not None)
+    return not (_is_compiling() or _is_autocast() or _forward_ad._current_level >= 0 or _transforms() is not None or _dispatch_modes() > 0
+                or _dispatch_key(_PRE_DISPATCH) or _tracing_state() is not None)
 
 
 def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
@@ -1665,8 +1669,14 @@ def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_we
     """act(linear(rms_norm(x), weight, bias)) + residual for at most 32 rows in one kernel (see nsa_skinny_linear): a bf16
     projection of a decode step with what stands around it, every part optional.  Inference only (no autograd)."""
     _check_linear("skinny_linear", _BF16, x, weight, bias, norm_weight)
-    weight = _laid_out(weight)
-    bias, norm_weight = (t if t is None else _laid_out(t) for t in (bias, norm_weight))
+    return _skinny(x, _laid_out(weight), bias, None if norm_weight is None else _laid_out(norm_weight), eps, act, residual)
+
+
+def _skinny(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_weight: Tensor | None = None, eps: float = 0.0, act: str | None = None,
+            residual: Tensor | None = None) -> Tensor:
+    """`skinny_linear` of operands that `skinny_linear_supported` has seen."""
+    if bias is not None and not bias.is_contiguous():
+        bias = bias.contiguous()
     k, n = x.shape[-1], weight.shape[0]
     x2 = x.reshape(-1, k)
     if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
@@ -1674,8 +1684,8 @@ def skinny_linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_we
     rows = x2.shape[0]
     if residual is not None:
         residual = residual.reshape(rows, n)
-        if residual.dtype != _BF16 or residual.stride(1) != 1:
-            raise RuntimeError("skinny_linear: the residual must be bf16 with unit stride")
+        if residual.dtype != _BF16 or residual.device != x.device or residual.stride(1) != 1:
+            raise RuntimeError("skinny_linear: the residual must be bf16 on the same device with unit stride")
     y = x.new_empty((*x.shape[:-1], n))
     _lib.check(_lib.lib().nsa_skinny_linear(rows, k, n, x2.data_ptr(), x2.stride(0), _ptr(norm_weight), eps, weight.data_ptr(), _ptr(bias), _ACTS[act],
                                             _ptr(residual), 0 if residual is None else residual.stride(0), y.data_ptr(), n, _stream()),
@@ -1738,8 +1748,13 @@ def _check_linear(name: str, dtype: torch.dtype, x: Tensor, weight: Tensor, *oth
 def linear_f32(x: Tensor, weight: Tensor, bias: Tensor | None = None, act: str | None = None) -> Tensor:
     """act(linear(x, weight, bias)) in fp32 by nsa_linear_f32 (few rows, no gradient)."""
     _check_linear("linear_f32", torch.float32, x, weight, bias)
-    weight = _laid_out(weight)
-    bias = bias if bias is None else bias.contiguous()
+    return _few_rows_f32(x, _laid_out(weight), bias, act)
+
+
+def _few_rows_f32(x: Tensor, weight: Tensor, bias: Tensor | None, act: str | None = None) -> Tensor:
+    """`linear_f32` of operands that `linear_f32_supported` has seen."""
+    if bias is not None and not bias.is_contiguous():
+        bias = bias.contiguous()
     k, n = x.shape[-1], weight.shape[0]
     x2 = x.reshape(-1, k)
     if x2.stride(1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
@@ -1780,7 +1795,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     if (not (torch.is_grad_enabled() and weight.requires_grad) or torch.compiler.is_compiling() or x.dtype != weight.dtype
             or torch.is_autocast_enabled()):               # under autocast the library casts the operands itself
         if not torch.is_grad_enabled() and plain_call() and linear_f32_supported(x, weight, bias):
-            return linear_f32(x, weight, bias)
+            return _few_rows_f32(x, weight, bias)
         return torch.nn.functional.linear(x, weight, bias)
     return _Linear.apply(x, weight, bias)
 

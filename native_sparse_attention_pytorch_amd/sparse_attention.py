@@ -238,7 +238,7 @@ class SparseAttention(nn.Module):
                 and cls._plain(mlp[2], nn.ReLU) and not torch.is_grad_enabled() and ops.plain_call()):
             x = windows.flatten(-2)
             if ops.linear_f32_supported(x, mlp[1].weight, mlp[1].bias):
-                return cls._linear(mlp[3], ops.linear_f32(x, mlp[1].weight, mlp[1].bias, act="relu"))
+                return cls._linear(mlp[3], ops._few_rows_f32(x, mlp[1].weight, mlp[1].bias, act="relu"))
         for layer in mlp:
             windows = cls._linear(layer, windows)
         return windows
@@ -315,7 +315,7 @@ class SparseAttention(nn.Module):
             x = window.reshape(b * h, n * d)
             if (cls._plain(up, nn.Linear) and cls._plain(act, nn.ReLU) and cls._plain(down, nn.Linear) and ops.plain_call()
                     and ops.skinny_linear_supported(x, up.weight, up.bias) and ops.skinny_linear_supported(x, down.weight, down.bias, width=up.weight.shape[0])):
-                return ops.skinny_linear(ops.skinny_linear(x, up.weight, up.bias, act="relu"), down.weight, down.bias).view(b, h, 1, -1)
+                return ops._skinny(ops._skinny(x, up.weight, up.bias, act="relu"), down.weight, down.bias).view(b, h, 1, -1)
         return mlp(window[:, :, None])
 
     @torch.no_grad()
@@ -341,9 +341,9 @@ class SparseAttention(nn.Module):
                 and ops.skinny_linear_supported(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight)):
             eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
             x = None
-            qkv = ops.skinny_linear(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight, eps)
+            qkv = ops._skinny(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight, eps)
             if self._plain(gate, nn.Linear) and ops.skinny_linear_supported(inp, gate.weight, gate.bias, norm.weight):
-                gates = ops.skinny_linear(inp, gate.weight, gate.bias, norm.weight, eps)
+                gates = ops._skinny(inp, gate.weight, gate.bias, norm.weight, eps)
             else:
                 x = norm(inp)
         else:
@@ -402,7 +402,7 @@ class SparseAttention(nn.Module):
         merged = merged.to(qkv.dtype)
         heads = self.combine_heads
         if kernels and self._plain(heads, nn.Linear) and ops.skinny_linear_supported(merged, heads.weight, heads.bias):
-            out = ops.skinny_linear(merged, heads.weight, heads.bias)
+            out = ops._skinny(merged, heads.weight, heads.bias)
         else:
             out = heads(merged)
         if not return_cache:

@@ -72,8 +72,8 @@ class Transformer(nn.Module):
                     and ops.skinny_linear_supported(tokens, up.weight, up.bias, norm.weight)
                     and ops.skinny_linear_supported(tokens, down.weight, down.bias, width=up.weight.shape[0])):
                 eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
-                hidden = ops.skinny_linear(tokens, up.weight, up.bias, norm.weight, eps, act="gelu")
-                return ops.skinny_linear(hidden, down.weight, down.bias, residual=tokens)
+                hidden = ops._skinny(tokens, up.weight, up.bias, norm.weight, eps, act="gelu")
+                return ops._skinny(hidden, down.weight, down.bias, residual=tokens)
         return ff(tokens) + tokens
 
     def _decode_logits(self, tokens):
@@ -83,7 +83,7 @@ class Transformer(nn.Module):
         if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and ops.plain_call()
                 and plain(norm, nn.RMSNorm) and plain(out, nn.Linear) and norm.normalized_shape == tuple(tokens.shape[-1:])
                 and ops.rms_norm_supported(tokens, norm.weight) and ops.skinny_linear_supported(tokens, out.weight, out.bias, norm.weight)):
-            return ops.skinny_linear(tokens, out.weight, out.bias, norm.weight, torch.finfo(torch.float32).eps if norm.eps is None else norm.eps)
+            return ops._skinny(tokens, out.weight, out.bias, norm.weight, torch.finfo(torch.float32).eps if norm.eps is None else norm.eps)
         return out(norm(tokens))
 
     def _decode(self, ids, caches):
