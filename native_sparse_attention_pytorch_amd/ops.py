@@ -2021,7 +2021,7 @@ class _GateF32(torch.autograd.Function):
 def gate_combine_f32(logits: Tensor, compressed: Tensor, selected: Tensor, sliding: Tensor) -> Tensor:
     """`gate_combine` in fp32: pre-sigmoid logits 'b n (h s)', branches 'b h n d' -> 'b n (h d)'."""
     b, h, n, _ = compressed.shape
-    if logits.dtype != torch.float32 or logits.shape != (b, n, 3 * h) or selected.shape != compressed.shape or sliding.shape != compressed.shape:
+    if logits.dtype != torch.float32 or logits.device != compressed.device or logits.shape != (b, n, 3 * h) or selected.shape != compressed.shape or sliding.shape != compressed.shape:
         raise RuntimeError("gate_combine_f32: fp32 logits 'b n (h 3)' and three branches 'b h n d'")
     return _GateF32.apply(logits, compressed, selected, sliding)
 

@@ -153,6 +153,14 @@ def test_hooks_on_the_flatten_layer_run(calls, dtype, hook):
     assert len(seen) == 1
 
 
+def test_gate_logits_in_host_memory_are_refused(calls):
+    branch = torch.zeros(1, 2, 3, 8).as_subclass(OnDevice)
+    for logits in (torch.zeros(1, 3, 6, device="meta"), torch.zeros(1, 3, 6, dtype=BF16), torch.zeros(1, 3, 5)):
+        with pytest.raises(RuntimeError):
+            ops.gate_combine_f32(logits, branch, branch, branch)
+    assert not calls
+
+
 @pytest.mark.parametrize("rows, k, n, own", [
     (62, 512, 1536, True), (240, 512, 24, True), (256, 512, 256, True),       # the smallest layer's projections; few outputs
     (256, 512, 1536, False), (128, 512, 3072, False), (256, 256, 6144, False),    # more tiles than the chip takes at once
