@@ -646,7 +646,7 @@ __global__ __launch_bounds__(384) void decode_combine_kernel(const CombineArgs A
   if (A.part[s] != nullptr) {
     const int u = (P.units == P.hk) ? head / P.g : head, gi = (P.units == P.hk) ? head % P.g : 0;
     const float* base = A.part[s] + (long)(b * P.units + u) * P.nparts * P.rec + gi * D + 4 * (t % LPP);
-    // every wave of the attend kernels wrote a finite record (zeros when it saw no key), so the loads need no guard and overlap
+    // every wave of the attend kernels wrote its record (zeros when it saw no key), so the loads need no guard and overlap
 #pragma unroll 8
     for (int p = t / LPP; p < P.nparts; p += PPR) acc += w_s[s][p] * *reinterpret_cast<const floatx4*>(base + (long)p * P.rec);
   }

@@ -369,6 +369,8 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
 //   O^T = V^T P^T: step i takes the keys that register i of S^T holds, 8 (i / 4) + 4 h + i % 4, so P goes in as it is.
 // 64 MFMAs of 64 cycles per tile at d = 64: bound by the fp32 matrix rate (154 TFLOP/s by a large library GEMM).  Window 512, 4
 // heads x 4 kv heads, d = 64, 4096 queries: 0.104 ms (2.28 ms one query per wave in scalar FMAs), 8.6 GFLOP in 32-key tiles.
+// (Looking every value over for infinities and NaN on its way into LDS costs 0 to 1.5 %: window 512, 4 heads x 8 kv heads, d = 128, 4096
+// queries 366 -> 371 us.)
 
 template <int D>
 __global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const float* __restrict__ q, const float* __restrict__ k,
