@@ -196,9 +196,9 @@ class SparseAttention(nn.Module):
 
     @staticmethod
     def _plain(layer, kind):
-        """A library layer of exactly this kind on which nothing is hooked, neither on the instance nor globally: only then may
-        its weights be used directly (any hook is skipped when the layer's own `__call__` is)."""
-        return (type(layer) is kind and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
+        """A library layer of exactly this kind on which nothing is hooked, neither on the instance nor globally, and whose forward is its
+        class's: only then may its weights be used directly (any hook is skipped when the layer's own `__call__` is)."""
+        return (type(layer) is kind and "forward" not in layer.__dict__ and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
                 and not any(_GLOBAL_HOOKS))
 
     def _front_is_one_node(self, inp):

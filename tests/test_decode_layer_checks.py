@@ -150,3 +150,25 @@ def test_a_missing_cache_does_not_reach_the_layer_call():
     model.layers[0][0] = m
     with torch.no_grad(), pytest.raises(RuntimeError, match="GPU only"):      # the layer's own forward, which has no CPU path
         model(torch.zeros(4, 1, dtype=torch.long), cache=[None])
+
+
+def test_layers_whose_forward_was_replaced_are_called(reached, monkeypatch):
+    """A forward put on the instance (as offloading and tracing tools do) runs, for the layer itself and for the layers inside it."""
+    m, _, cache = _layer_and_cache()
+    seen = []
+    for layer in (m.norm, m.to_qkv, m.to_strategy_combine[0], m.combine_heads):
+        with monkeypatch.context() as patch:
+            patch.setattr(layer, "forward", lambda x: seen.append(1) or x)
+            assert _run(m, cache) is None and not reached
+            if isinstance(layer, nn.Linear):
+                SparseAttention._linear(layer, torch.zeros(1, 128, dtype=BF16))
+    assert len(seen) == 3
+    model = Transformer(num_tokens=16, dim=128, depth=1, heads=4, kv_heads=2).to(BF16)
+    model.layers[0][0] = m
+    monkeypatch.setattr(m, "forward", lambda tokens, cache=None, return_cache=False: (seen.append("attn") or torch.zeros_like(tokens), cache))
+    monkeypatch.setattr(model.token_emb, "forward", lambda ids: torch.zeros(4, 1, 128, dtype=BF16).as_subclass(OnDevice))
+    monkeypatch.setattr(model, "_decode_feed_forward", lambda ff, tokens: tokens)
+    monkeypatch.setattr(model, "_decode_logits", lambda tokens: tokens)
+    with torch.no_grad():
+        model(torch.zeros(4, 1, dtype=torch.long), cache=[cache])
+    assert seen[-1] == "attn" and not reached

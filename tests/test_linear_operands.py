@@ -3,6 +3,7 @@ library replaced by a recorder: they read a weight as contiguous rows of the inp
 refused, copied or left to the layer, as F.linear would have it."""
 import pytest
 import torch
+import torch.nn.functional as F
 from torch import nn
 
 from native_sparse_attention_pytorch_amd import SparseAttention, _lib, ops
@@ -77,15 +78,17 @@ def test_second_projections_the_kernel_cannot_read_stay_with_the_layer(calls, mo
     ff = FeedForward(64).to(BF16)
     layers = []
     for down, run in ((m.k_compress[3], lambda: m._compress_rows(m.k_compress, _dev(2, 2, 16, 64))), (ff[3], lambda: Transformer._decode_feed_forward(ff, _dev(2, 1, 64)))):
-        monkeypatch.setattr(_odd(down, how), "forward", lambda x, n=down.out_features: layers.append(n) or torch.zeros(*x.shape[:-1], n, dtype=BF16))
-        with torch.no_grad():
-            out = run()
-        assert out.shape[-1] == down.out_features
         if how == "plain":
-            assert not layers and [name for name, _ in calls] == ["nsa_skinny_linear"] * 2
+            with torch.no_grad():
+                assert run().shape[-1] == down.out_features
+            assert [name for name, _ in calls] == ["nsa_skinny_linear"] * 2
             calls.clear()
             continue
-        assert len(layers) == 1 and not calls
+        w = _odd(down, how).weight
+        with monkeypatch.context() as patch, torch.no_grad():
+            patch.setattr(F, "linear", lambda x, w, b=None: layers.append(w) or torch.zeros(*x.shape[:-1], w.shape[0], dtype=BF16))
+            assert run().shape[-1] == down.out_features
+        assert not calls and any(u is w for u in layers)
         layers.clear()
 
 
