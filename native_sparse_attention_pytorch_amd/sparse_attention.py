@@ -250,7 +250,7 @@ class SparseAttention(nn.Module):
     def _decode_whole(self, inp, cache, return_cache=True, residual=None):
         """The decode step of a bf16 layer with its default parts over bf16 caches as one library call (nsa_decode_layer: five
         launches; `residual` is added to the output); None when something about the layer, the caches or the sizes asks for the
-        general path.  Called without gradients."""
+        general path.  Called without gradients and in a plain call (ops.plain_call)."""
         (cache_k, cache_v), ((cache_ck, cache_cv), (run_k, run_v)) = cache
         norm, qkv, gate, out, bf16 = self.norm, self.to_qkv, self.to_strategy_combine[0], self.combine_heads, torch.bfloat16
         plain, d = self._plain, self.dim_head
@@ -259,8 +259,7 @@ class SparseAttention(nn.Module):
             return None
         b, dim, hd = inp.shape[0], inp.shape[2], self.heads * d
         mem, freqs, device = self.compress_mem_kv, self.rotary_emb.freqs, inp.device
-        if (b > 32 or dim % 32 or b * (max(dim, hd) + 8) > 65536 or norm.normalized_shape != (dim,)
-                or not ops.plain_call()):
+        if b > 32 or dim % 32 or b * (max(dim, hd) + 8) > 65536 or norm.normalized_shape != (dim,):
             return None
         for w in (norm.weight, qkv.weight, gate.weight, gate.bias, out.weight, out.bias, mem):
             if w is not None and (w.dtype != bf16 or w.device != device or not w.is_contiguous() or w.data_ptr() % 16):
@@ -331,11 +330,12 @@ class SparseAttention(nn.Module):
         G, bf16 = self.num_grouped_queries, torch.bfloat16
         freqs = self.rotary_emb.freqs
 
-        out = self._decode_whole(inp, cache, return_cache)
+        kernels = ops.plain_call()
+        out = self._decode_whole(inp, cache, return_cache) if kernels else None
         if out is not None:
             return out
         # projections of a few rows by the same kernels (bit-equal to the whole-layer call and to decode_session.DecodeSession)
-        norm, gate, gates, kernels = self.norm, self.to_strategy_combine[0], None, ops.plain_call()
+        norm, gate, gates = self.norm, self.to_strategy_combine[0], None
         if (inp.dtype == bf16 and self._plain(norm, nn.RMSNorm) and self._plain(self.to_qkv, nn.Linear) and kernels
                 and tuple(norm.normalized_shape) == tuple(inp.shape[-1:]) and ops.rms_norm_supported(inp, norm.weight)
                 and ops.skinny_linear_supported(inp, self.to_qkv.weight, self.to_qkv.bias, norm.weight)):

@@ -88,9 +88,10 @@ class Transformer(nn.Module):
 
     def _decode(self, ids, caches):
         """One token per sequence through the caches: (logits 'b 1 vocab', advanced caches)."""
+        from . import ops
         tokens = self.token_emb(ids[:, -1:])
         new = []
-        whole = not torch.is_grad_enabled()
+        whole = not torch.is_grad_enabled() and ops.plain_call()
         for (attn, ff), cache in zip(self.layers, caches):
             # a layer nothing is hooked on takes the residual into its last kernel
             step = attn._decode_whole(tokens, cache, residual=tokens) if whole and SparseAttention._plain(attn, SparseAttention) else None

@@ -172,3 +172,38 @@ def test_layers_whose_forward_was_replaced_are_called(reached, monkeypatch):
     with torch.no_grad():
         model(torch.zeros(4, 1, dtype=torch.long), cache=[cache])
     assert seen[-1] == "attn" and not reached
+
+
+def test_calls_that_are_not_plain_do_not(reached, monkeypatch):
+    """Autocast, tracers and transforms around a step (ops.plain_call): the general path, from the layer and from the model."""
+    m, _, cache = _layer_and_cache()
+    model = Transformer(num_tokens=16, dim=128, depth=1, heads=4, kv_heads=2).to(BF16)
+    model.layers[0][0] = m
+    x = torch.zeros(4, 1, 128, dtype=BF16).as_subclass(OnDevice)
+    monkeypatch.setattr(model.token_emb, "forward", lambda ids: x)
+
+    class General(Exception):
+        pass
+
+    def split(self, t):
+        raise General
+    monkeypatch.setattr(SparseAttention, "_split_heads", split)
+    for run in (lambda: m(x, cache=cache), lambda: model(torch.zeros(4, 1, dtype=torch.long), cache=[cache])):
+        monkeypatch.setattr(ops, "plain_call", lambda: False)
+        with torch.no_grad(), pytest.raises(General):
+            run()
+    assert not reached
+
+
+def test_plain_calls():
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    assert ops.plain_call()
+    seen = []
+    look = lambda t: seen.append(ops.plain_call()) or t + 1
+    one = torch.ones(2)
+    torch.vmap(look)(one), torch.func.jvp(look, (one,), (one,)), make_fx(look)(one), make_fx(look, pre_dispatch=True)(one)
+    torch.jit.trace(look, (one,), check_trace=False)
+    with forward_ad.dual_level():
+        look(one)
+    assert seen and not any(seen) and ops.plain_call()
