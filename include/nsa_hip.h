@@ -308,7 +308,7 @@ int nsa_colsum(const void* x, int32_t groups, int64_t group_stride, int64_t oute
                int64_t inner_stride, int32_t cols, void* out, int32_t out_fp32, float* workspace, void* stream);
 
 /* fp32 forward of the attention branches, for fp32 modules run for inference: products, softmax and
- * accumulation in fp32 on the vector ALUs, so that the result agrees with the reference's fp32 torch path
+ * accumulation in fp32 (on the matrix instructions: fp32 ones, or bf16 ones with operands split in three), so that the result agrees with the reference's fp32 torch path
  * to its own test tolerance (1e-5, tests/test_sparse_attn.py:86), which the bf16 MFMA kernels cannot.
  * Same contracts and descriptors as nsa_dense_fwd (without the importance logits, which are linear in q and
  * the compressed keys and cost one small fp32 GEMM) and nsa_select_fwd (no workspaces, no inverse index);

@@ -5,14 +5,15 @@
 // (NSA.py:153-184, 632-639, 841-850): any head dimension <= 128 that is a multiple of 4, any group
 // size, any block size.
 //
-// Two kernels, both on the fp32 matrix instructions (256 FLOP per cycle and CU, twice what scalar FMAs reach):
-//  * f32_tile_kernel  - interval masks (band, strided prefix): 32 rows (query, head) per wave against
-//    32-key tiles shared by the work-group, v_mfma_f32_32x32x2;
+// Two kernels:
+//  * f32_tile_kernel  - interval masks (band, strided prefix) and selections of a fair share of the blocks: 32 rows (query, head)
+//    per wave against 32-key tiles shared by the work-group, on the bf16 matrix instructions with operands split in three;
 //  * f32_rows_kernel  - one query of one kv head per wave (or per work-group) against 64-key tiles gathered
 //    from anywhere, v_mfma_f32_4x4x1 with 16 blocks = 64 keys x 4 heads: block selection, and interval
 //    masks with few queries (decode steps).
 #include <type_traits>
-#include "nsa_common.hpp"
+#include <algorithm>
+#include "nsa_split.hpp"
 #include "../../include/nsa_hip.h"
 
 namespace nsa {
@@ -20,7 +21,7 @@ namespace nsa {
 constexpr int kF32MaxD = 128;
 
 struct F32Args {
-  int b, hk, g, n, nk, d;          // n: number of queries (rows of q / out); nk: key rows after the memory slots
+  int b, hk, bh, g, n, nk, d;          // n: number of queries (rows of q / out); nk: key rows after the memory slots
   int qoff;                       // query row i sits at sequence position i + qoff
   float scale;
   long sq[3], sk[3], sv[3];
@@ -28,7 +29,7 @@ struct F32Args {
   int mode, causal, wb, wf, st, mem;
   const float *memk, *memv;       // the memory rows [hk, mem, d] when they are not the first rows of k / v, else null
   // selection
-  int S, B, W, idx64, uniform;
+  int S, B, W, idx64, uniform, lb;      // lb: log2 of the block, where it is a power of two
 };
 
 __device__ __forceinline__ floatx16 mfma32x2(float a, float b, floatx16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
@@ -363,159 +364,352 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
 
 // ------------------------------------------------------------------------------------------ tile
 //
-// Interval masks with many queries: a wave holds 32 rows (row r of a kv head = query r / G, head r % G, so any group size
-// fits), a work-group 128; tiles of 32 keys of K and V are shared through LDS, double-buffered, one barrier per tile.
-//   S^T = K Q^T: A = K (lane = key, half h: features 8 t + 4 h + j in step j of group t), B = Q in the same order;
-//   O^T = V^T P^T: step i takes the keys that register i of S^T holds, 8 (i / 4) + 4 h + i % 4, so P goes in as it is.
-// 64 MFMAs of 64 cycles per tile at d = 64: bound by the fp32 matrix rate (154 TFLOP/s by a large library GEMM).  Window 512, 4
-// heads x 4 kv heads, d = 64, 4096 queries: 0.104 ms (2.28 ms one query per wave in scalar FMAs), 8.6 GFLOP in 32-key tiles.
-// (Looking every value over for infinities and NaN on its way into LDS costs 0 to 1.5 %: window 512, 4 heads x 8 kv heads, d = 128, 4096
-// queries 366 -> 371 us.)
+// Many queries: a wave holds 32 rows (row r of a kv head = query r / G, head r % G, so any group size fits), a work-group 128;
+// tiles of 32 keys of K and V are shared through LDS, double-buffered, one barrier per tile.  The products are made of bf16
+// thirds (nsa_split.hpp): K and V are split on their way into LDS, once for the 128 rows, Q once and P where it is made.
+//   S^T = K Q^T: A = K (lane = key), B = Q (lane = row);  O^T = V^T P^T: A = V^T by the LDS transpose load, whose order of rows is the
+//   order in which S^T's registers hold the keys, so P goes in as it is.
+// Interval masks, and (SEL) block selections of few enough blocks: every tile of a block that one of the 128 rows selected is
+// multiplied and a row's own choice is a mask on the scores, which beats gathering while a query attends a fair share of the
+// blocks there are (f32_masked_tiles).
+// Per tile and wave at d = 64 48 MFMAs (1536 cycles) and some 450 vector instructions (the split of K, V and P 230, softmax 160),
+// of which two waves to a SIMD hide part of each other; a wave alone takes 2.4 us.  Against v_mfma_f32_32x32x2 tiles (64 MFMAs of 64
+// cycles): 2 x 2053 queries, 16 heads x 4 kv heads, window 512 117 -> 68 us, strided prefix 38 -> 28; 32 x 8 heads, d = 128, 2000 queries
+// 204 -> 152.  Error of the outputs against float64 1.6e-7 instead of 3.8e-7 (window 512): each row's sums are rounded once per 16
+// products instead of once per 2.
+constexpr int kTileBlocks = 128;         // blocks of a masked selection
 
-template <int D>
-__global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const float* __restrict__ q, const float* __restrict__ k,
-                                                          const float* __restrict__ v, float* __restrict__ out, float* __restrict__ lse) {
-  constexpr int VS = D + 8;                              // V row stride: the halves' rows (4 apart) lie 32 banks apart
-  constexpr int LD = D / 32;                             // 16-byte loads per thread and tile of K (and of V)
-  __shared__ float k_s[2][32 * D];                       // chunk c of row r at c ^ (r % 16)
-  __shared__ float v_s[2][32 * VS];                      // (zeros for values that are not finite)
+__device__ __forceinline__ void split_probs(const float (&p)[16], bf16x8 (&part)[3][2]) {
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t s[3];
+      split2(p[8 * u + 2 * j], p[8 * u + 2 * j + 1], s);
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) w[pl][j] = s[pl];
+    }
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) part[pl][u] = __builtin_bit_cast(bf16x8, uintx4{w[pl][0], w[pl][1], w[pl][2], w[pl][3]});
+  }
+}
+
+template <int D, bool SEL>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F32Args A, const float* __restrict__ q, const float* __restrict__ k,
+                                                                        const float* __restrict__ v, const void* __restrict__ idx,
+                                                                        const uint8_t* __restrict__ fmask, float* __restrict__ out,
+                                                                        float* __restrict__ lse) {
+  constexpr int KP = D + 8, VP = D + 16;                 // row strides: conflict-free row reads of K, transpose loads of V
+  constexpr int LD = D / 32, KS = D / 16, FT = D / 32;
+  __shared__ __align__(16) __bf16 k_s[2][3 * 32 * KP];
+  __shared__ __align__(16) __bf16 v_s[2][3 * 32 * VP];   // (zeros for values that are not finite)
   __shared__ int odd_s;                                  // there was such a value
+  __shared__ uint32_t mask_s[SEL ? 129 : 1][kTileBlocks / 32], any_s[kTileBlocks / 32];
+  __shared__ int repeated_s, big_s;                      // big_s: some key was that large (it stays set)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n_ = lane & 31, h = lane >> 5;
-  const int bh = blockIdx.y, b = bh / A.hk, hk = bh % A.hk;
+  // Longest key lists first (causal prefixes).  Where the launch fits the chip at two work-groups to a CU, the second half goes the
+  // other way round: the longest then shares its CU with the shortest.
+  const int tiles = gridDim.x / A.bh, nth = blockIdx.x / A.bh;
+  const int turned = gridDim.x <= 512 && (int)blockIdx.x >= 256 ? 256 / A.bh + tiles - 1 - nth : nth;
+  const int bh = blockIdx.x % A.bh, b = bh / A.hk, hk = bh % A.hk;
   const float* kb = k + b * A.sk[0] + hk * A.sk[1];
   const float* vb = v + b * A.sv[0] + hk * A.sv[1];
   const long all_rows = (long)A.n * A.g;
-  const long row0 = (long)(gridDim.x - 1 - blockIdx.x) * 128;              // longest key lists first (causal prefixes)
+  const long row0 = (long)(tiles - 1 - turned) * 128;
   const long row = row0 + wave * 32 + n_;
   const long rowc = row < all_rows ? row : all_rows - 1;
   const int qi = (int)(rowc / A.g), g = (int)(rowc - (long)qi * A.g);
-  int lo, hi;
-  f32_interval(A, qi + A.qoff, lo, hi);
-  // ranges of the wave's and of the work-group's rows (both ends grow with the query)
-  const int wq0 = (int)(min(row0 + wave * 32, all_rows - 1) / A.g), wq1 = (int)(min(row0 + wave * 32 + 31, all_rows - 1) / A.g);
   const int gq0 = (int)(row0 / A.g), gq1 = (int)(min(row0 + 127, all_rows - 1) / A.g);
-  int w_lo0, w_hi1, g_lo, g_hi, dummy;
-  f32_interval(A, wq0 + A.qoff, w_lo0, dummy);
-  f32_interval(A, wq1 + A.qoff, dummy, w_hi1);
-  f32_interval(A, gq0 + A.qoff, g_lo, dummy);
-  f32_interval(A, gq1 + A.qoff, dummy, g_hi);
-  if (A.mode == 1) { w_hi1 = max(w_hi1, A.mem - 1); g_hi = max(g_hi, A.mem - 1); }
-  hi = A.mode == 1 ? max(hi, A.mem - 1) : hi;
+  // Keys [lo, lo + seen] are visible to the row, and (SEL) those of its selected blocks.
+  // g_lo .. g_hi: what the work-group walks; w_lo .. w_hi: what the wave's rows see of the interval.
+  int lo, hi, w_lo, w_hi, g_lo, g_hi, dummy;
+  const int wq0 = (int)(min(row0 + wave * 32, all_rows - 1) / A.g), wq1 = (int)(min(row0 + wave * 32 + 31, all_rows - 1) / A.g);
+  if (SEL) {
+    hi = qi + A.qoff;
+    lo = (hi >> A.lb) << A.lb;
+    w_lo = ((wq0 + A.qoff) >> A.lb) << A.lb;
+    w_hi = wq1 + A.qoff;
+    g_lo = 0;
+    g_hi = gq1 + A.qoff;
+  } else {
+    f32_interval(A, qi + A.qoff, lo, hi);
+    f32_interval(A, wq0 + A.qoff, w_lo, dummy);
+    f32_interval(A, wq1 + A.qoff, dummy, w_hi);
+    f32_interval(A, gq0 + A.qoff, g_lo, dummy);
+    f32_interval(A, gq1 + A.qoff, dummy, g_hi);
+    if (A.mode == 1) { w_hi = max(w_hi, A.mem - 1); g_hi = max(g_hi, A.mem - 1); hi = max(hi, A.mem - 1); }
+  }
   // a key is visible if key - lo, as an unsigned number, is at most `seen`: one comparison, and no branch per element
   const unsigned seen = hi < lo ? 0u : (unsigned)(hi - lo);
   if (hi < lo) lo = 0x7fffffff;
 
-  float qr[D / 8][4];
-  {
-    const float* qp = q + b * A.sq[0] + (long)(hk * A.g + g) * A.sq[1] + (long)qi * A.sq[2];
-#pragma unroll
-    for (int t = 0; t < D / 8; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) qr[t][j] = qp[min(8 * t + 4 * h + j, A.d - 1)];      // (features past the head dimension meet zero keys)
+  unsigned long long any0 = 0, any1 = 0;                 // blocks that some row of the work-group attends
+  bool repeated = false;
+  const size_t slot0 = SEL ? ((size_t)bh * A.n + gq0) * A.S : 0;
+  auto block_of = [&](size_t at) {
+    if (!fmask[at]) return -1;
+    const long j = A.idx64 ? (long)reinterpret_cast<const long long*>(idx)[at] : (long)reinterpret_cast<const int*>(idx)[at];
+    return j >= 0 && j < A.W ? (int)j : -1;
+  };
+  if (SEL) {
+    for (int e = tid; e < 129 * (kTileBlocks / 32); e += 256) (&mask_s[0][0])[e] = 0;
+    if (tid < kTileBlocks / 32) any_s[tid] = 0;
+    if (tid == 0) repeated_s = 0;
+    __syncthreads();
+    const int total = (gq1 - gq0 + 1) * A.S;
+    for (int e = tid; e < total; e += 256) {
+      const int j = block_of(slot0 + e);
+      if (j < 0) continue;
+      const int qr = e / A.S;
+      const uint32_t bit = 1u << (j & 31);
+      // a block named twice, or the own block or a later one: the masks cannot say that (the scores' weights can, below)
+      if ((atomicOr(&mask_s[qr][j >> 5], bit) & bit) || j >= (gq0 + qr + A.qoff) >> A.lb) repeated_s = 1;
+      atomicOr(&any_s[j >> 5], bit);
+    }
+    for (int qr = tid; qr <= gq1 - gq0; qr += 256) {
+      const int own = (gq0 + qr + A.qoff) >> A.lb;
+      atomicOr(&any_s[own >> 5], 1u << (own & 31));
+    }
+    __syncthreads();
+    auto word = [&](int w) { return (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)any_s[w]); };
+    any0 = word(0) | word(1) << 32;
+    any1 = word(2) | word(3) << 32;
+    repeated = __builtin_amdgcn_readfirstlane(repeated_s) != 0;
+    if (repeated) g_hi = (A.W << A.lb) - 1;              // (zero padding behind the last key counts, as a score of 0)
   }
-  floatx16 o[D / 32];
+  // the first tile from t0 on that somebody attends
+  const uint32_t tile_bits = SEL ? (1u << max(1, 32 >> A.lb)) - 1u : 0;
+  auto attended = [&](int t0) {
+    if (SEL) {
+      while (t0 <= g_hi) {
+        const int j = t0 >> A.lb;
+        if (((j < 64 ? any0 >> j : any1 >> (j - 64)) & tile_bits) != 0) break;
+        t0 += 32;
+      }
+    }
+    return t0;
+  };
+
+  // Products of numbers below kBig do not overflow; where larger ones (or infinities) meet, a sum of leading products may not be
+  // finite, and the small ones then mean nothing.
+  constexpr float kBig = 1.152921504606846976e18f;       // 2^60
+  bool q_big;
+  bf16x8 qf[3][KS];
+  {
+    // (a negative scale goes into the queries, so that the largest product is the largest score)
+    const float sign = A.scale < 0.f ? -1.f : 1.f;
+    const float* qp = q + b * A.sq[0] + (long)(hk * A.g + g) * A.sq[1] + (long)qi * A.sq[2];
+    float big = 0.f;
 #pragma unroll
-  for (int ft = 0; ft < D / 32; ++ft) o[ft] = zero_acc();
-  float m = -INFINITY, l = 0.f;
+    for (int ks = 0; ks < KS; ++ks) {
+      uint32_t w[3][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int f = 16 * ks + 8 * h + 2 * j;
+        const float x0 = qp[min(f, A.d - 1)], x1 = qp[min(f + 1, A.d - 1)];
+        big = fmaxf(big, fmaxf(fabsf(x0), fabsf(x1)));
+        uint32_t s[3];
+        split2(f < A.d ? sign * x0 : 0.f, f + 1 < A.d ? sign * x1 : 0.f, s);
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) w[pl][j] = s[pl];
+      }
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) qf[pl][ks] = __builtin_bit_cast(bf16x8, uintx4{w[pl][0], w[pl][1], w[pl][2], w[pl][3]});
+    }
+    q_big = __any(big >= kBig);
+  }
+  floatx16 o[FT], os[FT];                                // sums of leading and of small products
+#pragma unroll
+  for (int ft = 0; ft < FT; ++ft) { o[ft] = zero_acc(); os[ft] = zero_acc(); }
+  const float c = fmaxf(fabsf(A.scale) * kLog2e, 1e-37f);      // weights are powers of two of (score - maximum) c (a scale of 0: no 0 x inf)
+  float m = -INFINITY, l = 0.f;                          // m: of the unscaled scores
 
   const int own_mem = A.memk != nullptr ? A.mem : 0;
+  const int last_key = SEL ? min(g_hi, A.nk - 1) : g_hi;
   floatx4 kx[LD], vx[LD];
+  // this thread's rows of a tile that lies within the keys: offsets from its first row (row strides: below 2^24)
+  unsigned k_at[LD], v_at[LD];
+#pragma unroll
+  for (int u = 0; u < LD; ++u) {
+    const int e = u * 256 + tid, r = e / (D / 4), ch = e % (D / 4);
+    k_at[u] = (unsigned)r * (unsigned)A.sk[2] + 4 * ch;
+    v_at[u] = (unsigned)r * (unsigned)A.sv[2] + 4 * ch;
+  }
+  const bool plain_rows = A.d == D && A.sk[2] >= 0 && A.sv[2] >= 0 && (A.sk[2] | A.sv[2]) >> 24 == 0;
   auto fetch = [&](int t0) {
+    if (plain_rows && t0 >= own_mem && t0 + 31 <= last_key) {
+      const float *kt = kb + (long)(t0 - own_mem) * A.sk[2], *vt = vb + (long)(t0 - own_mem) * A.sv[2];
+#pragma unroll
+      for (int u = 0; u < LD; ++u) {
+        kx[u] = *reinterpret_cast<const floatx4*>(kt + k_at[u]);
+        vx[u] = *reinterpret_cast<const floatx4*>(vt + v_at[u]);
+      }
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < LD; ++u) {
-      const int e = u * 256 + tid, r = e / (D / 4), c = e % (D / 4);
+      const int e = u * 256 + tid, r = e / (D / 4), ch = e % (D / 4);
       const int kr = t0 + r;
       floatx4 z = {0.f, 0.f, 0.f, 0.f};
       kx[u] = z;
       vx[u] = z;
-      if (kr <= g_hi && 4 * c < A.d) {
+      if (kr <= last_key && 4 * ch < A.d) {
         const bool own = kr < own_mem;
-        kx[u] = *reinterpret_cast<const floatx4*>((own ? A.memk + ((long)hk * A.mem + kr) * A.d : kb + (long)(kr - own_mem) * A.sk[2]) + 4 * c);
-        vx[u] = *reinterpret_cast<const floatx4*>((own ? A.memv + ((long)hk * A.mem + kr) * A.d : vb + (long)(kr - own_mem) * A.sv[2]) + 4 * c);
+        kx[u] = *reinterpret_cast<const floatx4*>((own ? A.memk + ((long)hk * A.mem + kr) * A.d : kb + (long)(kr - own_mem) * A.sk[2]) + 4 * ch);
+        vx[u] = *reinterpret_cast<const floatx4*>((own ? A.memv + ((long)hk * A.mem + kr) * A.d : vb + (long)(kr - own_mem) * A.sv[2]) + 4 * ch);
       }
     }
   };
-  const int t_first = g_lo & ~31;
-  fetch(t_first);
-  if (tid == 0) odd_s = 0;
+  int t0 = attended(g_lo & ~31);
+  fetch(t0);
+  if (tid == 0) { odd_s = 0; big_s = 0; }
   __syncthreads();
   bool odd = false;
   int buf = 0;
-  for (int t0 = t_first; t0 <= g_hi; t0 += 32, buf ^= 1) {
+  for (; t0 <= g_hi; buf ^= 1) {
+    bool k_big = false;
+    float zero = 0.f;
 #pragma unroll
     for (int u = 0; u < LD; ++u) {
-      const int e = u * 256 + tid, r = e / (D / 4), c = e % (D / 4);
-      *reinterpret_cast<floatx4*>(&k_s[buf][r * D + 4 * (c ^ (r & 15))]) = kx[u];
-      floatx4 x;
+      k_big |= fmaxf(fmaxf(fabsf(kx[u][0]), fabsf(kx[u][1])), fmaxf(fabsf(kx[u][2]), fabsf(kx[u][3]))) >= kBig;
 #pragma unroll
-      for (int e2 = 0; e2 < 4; ++e2) {
-        const bool finite = fabsf(vx[u][e2]) < INFINITY;
-        odd |= !finite;
-        x[e2] = finite ? vx[u][e2] : 0.f;
-      }
-      *reinterpret_cast<floatx4*>(&v_s[buf][r * VS + 4 * c]) = x;
+      for (int e = 0; e < 4; ++e) zero = __builtin_fmaf(vx[u][e], 0.f, zero);      // (NaN if one of them is not finite)
     }
+    if (__any(zero != 0.f)) {
+      odd = true;
+#pragma unroll
+      for (int u = 0; u < LD; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vx[u][e] = fabsf(vx[u][e]) < INFINITY ? vx[u][e] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < LD; ++u) {
+      const int e = u * 256 + tid, r = e / (D / 4), ch = e % (D / 4);
+      const Split3 ks = split4(kx[u]), vs = split4(vx[u]);
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) {
+        *reinterpret_cast<bf16x4*>(&k_s[buf][(pl * 32 + r) * KP + 4 * ch]) = ks.part[pl];
+        *reinterpret_cast<bf16x4*>(&v_s[buf][(pl * 32 + r) * VP + 4 * ch]) = vs.part[pl];
+      }
+    }
+    if (k_big) big_s = 1;
     __syncthreads();          // (the other buffer was read before this barrier by every wave: it may be written in the next round)
-    if (t0 + 32 <= g_hi) fetch(t0 + 32);
-    if (t0 > w_hi1 || t0 + 31 < w_lo0) continue;         // wave-uniform: nothing of this tile is visible to the wave
-    floatx16 s = zero_acc();
-    // (the K operands of 8 feature groups are read ahead of the first product that needs them: at one or two waves per SIMD an
-    // LDS round trip in front of every fourth MFMA is not hidden by other waves)
+    const int here = t0;
+    t0 = attended(t0 + 32);
+    if (t0 <= g_hi) fetch(t0);
+    uint32_t chosen = 0;      // bit i: the row selected block i of the tile
+    if (SEL) {
+      const int j = here >> A.lb;
+      chosen = (mask_s[qi - gq0][j >> 5] >> (j & 31)) & tile_bits;
+      if (!__any(chosen != 0) && (here > w_hi || here + 31 < w_lo)) continue;
+    } else if (here > w_hi || here + 31 < w_lo) {
+      continue;               // wave-uniform: nothing of this tile is visible to the wave
+    }
+    const int overflows = big_s;
+    floatx16 lead = zero_acc(), small = zero_acc();
+    // (operands are read a product group ahead: at one or two waves per SIMD an LDS round trip in front of every group is not hidden)
+    bf16x8 kf[2][3], vf[2][3];
+    auto read_k = [&](int ks) {
 #pragma unroll
-    for (int t8 = 0; t8 < D / 8; t8 += 8) {
-      floatx4 kk[8];
+      for (int pl = 0; pl < 3; ++pl) kf[ks & 1][pl] = *reinterpret_cast<const bf16x8*>(&k_s[buf][(pl * 32 + n_) * KP + 16 * ks + 8 * h]);
+    };
+    auto read_v = [&](int g) {                            // group g: keys 16 (g / FT), features 32 (g % FT)
 #pragma unroll
-      for (int t = 0; t < 8; ++t) kk[t] = *reinterpret_cast<const floatx4*>(&k_s[buf][n_ * D + 4 * ((2 * (t8 + t) + h) ^ (n_ & 15))]);
+      for (int pl = 0; pl < 3; ++pl) vf[g & 1][pl] = lds_transposed_operand(&v_s[buf][pl * 32 * VP], VP, 16 * (g / FT), 32 * (g % FT), lane);
+    };
+    read_k(0);
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+    for (int ks = 0; ks < KS; ++ks) {
+      if (ks + 1 < KS) read_k(ks + 1);
+      const bf16x8 (&kk)[3] = kf[ks & 1];
+      lead = mfma32(kk[0], qf[0][ks], lead);
+      small = mfma32(kk[0], qf[1][ks], small);
+      small = mfma32(kk[0], qf[2][ks], small);
+      small = mfma32(kk[1], qf[0][ks], small);
+      small = mfma32(kk[1], qf[1][ks], small);
+      small = mfma32(kk[2], qf[0][ks], small);
+    }
+    read_v(0);
+    if (q_big || __builtin_amdgcn_readfirstlane(overflows)) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) s = mfma32x2(kk[t][j], qr[t8 + t][j], s);
+      for (int i = 0; i < 16; ++i) small[i] = fabsf(lead[i]) < INFINITY ? small[i] : 0.f;
     }
     float sv[16], tmax = -INFINITY;
-    const int from_lo = t0 + 4 * h - lo;
+    const int from_lo = here + 4 * h - lo;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      sv[i] = (unsigned)(from_lo + 8 * (i / 4) + (i % 4)) <= seen ? s[i] * A.scale : -INFINITY;
-      tmax = fmaxf(tmax, sv[i]);
+    for (int a = 0; a < 4; ++a) {
+      const unsigned limit = SEL && ((chosen >> ((8 * a + 4 * h) >> A.lb)) & 1u) ? 0xffffffffu : seen;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * a + e;
+        sv[i] = (unsigned)(from_lo + 8 * a + e) <= limit ? lead[i] + small[i] : -INFINITY;
+        tmax = fmaxf(tmax, sv[i]);
+      }
     }
     tmax = halves_max(tmax);
-    const float mn = fmaxf(m, tmax), mref = mn == -INFINITY ? 0.f : mn;
-    const float alpha = expf(m - mref);                  // m = -inf: 0
+    // (the reference of a row's weights follows its maximum only when that has grown by more than 2^8: weights up to 256 are as
+    // exact as those up to 1, and nearly every tile spares the multiplication of the sums)
+    const float mn = (tmax - m) * c > 8.f ? tmax : m, mref = mn == -INFINITY ? 0.f : mn;
+    const float alpha = fast_exp2((m - mref) * c);       // m = -inf: 0
     m = mn;
     float ps = 0.f;
+    if (SEL && repeated) {
+      // weights: how often the row's live slots name a key's block, and once more where the key is the own block's
 #pragma unroll
-    for (int i = 0; i < 16; ++i) { sv[i] = expf(sv[i] - mref); ps += sv[i]; }
+      for (int a = 0; a < 4; ++a) {
+        const int j = (here + 8 * a + 4 * h) >> A.lb;
+        int times = 0;
+        for (int s = 0; s < A.S; ++s) times += block_of(slot0 + (size_t)(qi - gq0) * A.S + s) == j;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float w = (float)(times + ((unsigned)(from_lo + 8 * a + e) <= seen ? 1 : 0));
+          sv[4 * a + e] = w > 0.f ? w * fast_exp2((sv[4 * a + e] - mref) * c) : 0.f;
+          ps += sv[4 * a + e];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) { sv[i] = fast_exp2((sv[i] - mref) * c); ps += sv[i]; }
+    }
     l = l * alpha + ps;                                  // this half's keys
     if (__any(alpha != 1.0f)) {
 #pragma unroll
-      for (int ft = 0; ft < D / 32; ++ft)
+      for (int ft = 0; ft < FT; ++ft)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[ft][i] *= alpha;
+        for (int i = 0; i < 16; ++i) { o[ft][i] *= alpha; os[ft][i] *= alpha; }
     }
+    bf16x8 pf[3][2];
+    split_probs(sv, pf);
 #pragma unroll
-    for (int i8 = 0; i8 < 16; i8 += 8) {
-      float vv[8][D / 32];
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int ft = 0; ft < D / 32; ++ft) vv[i][ft] = v_s[buf][(8 * ((i8 + i) / 4) + 4 * h + (i % 4)) * VS + 32 * ft + n_];
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int ft = 0; ft < D / 32; ++ft) o[ft] = mfma32x2(vv[i][ft], sv[i8 + i], o[ft]);
+    for (int gr = 0; gr < 2 * FT; ++gr) {
+      if (gr + 1 < 2 * FT) read_v(gr + 1);
+      const bf16x8 (&vv)[3] = vf[gr & 1];
+      const int u = gr / FT, ft = gr % FT;
+      o[ft] = mfma32(vv[0], pf[0][u], o[ft]);
+      os[ft] = mfma32(vv[0], pf[1][u], os[ft]);
+      os[ft] = mfma32(vv[0], pf[2][u], os[ft]);
+      os[ft] = mfma32(vv[1], pf[0][u], os[ft]);
+      os[ft] = mfma32(vv[1], pf[1][u], os[ft]);
+      os[ft] = mfma32(vv[2], pf[0][u], os[ft]);
     }
   }
   // A value that is not finite is left out of the products, where a weight of zero times it would be NaN in every row of its tile,
   // and added here to the rows that see its key.
   if (odd) odd_s = 1;
+#pragma unroll
+  for (int ft = 0; ft < FT; ++ft)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[ft][i] += os[ft][i];
   __syncthreads();
   if (odd_s) {
 #pragma unroll 1
-    for (int kr = g_lo; kr <= g_hi; ++kr) {
+    for (int kr = g_lo; kr <= last_key; ++kr) {
       const float* vr = kr < own_mem ? A.memv + ((long)hk * A.mem + kr) * A.d : vb + (long)(kr - own_mem) * A.sv[2];
-      const bool visible = (unsigned)(kr - lo) <= seen;
+      bool visible = (unsigned)(kr - lo) <= seen;
+      if (SEL) visible |= (mask_s[qi - gq0][(kr >> A.lb) >> 5] >> ((kr >> A.lb) & 31)) & 1u;
 #pragma unroll
-      for (int ft = 0; ft < D / 32; ++ft)
+      for (int ft = 0; ft < FT; ++ft)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int f0 = 32 * ft + 8 * u + 4 * h;
@@ -533,14 +727,14 @@ __global__ __launch_bounds__(256, 2) void f32_tile_kernel(const F32Args A, const
   const long orow = ((long)b * A.hk * A.g + (long)hk * A.g + g) * A.n + qi;
   float* op = out + orow * A.d;
 #pragma unroll
-  for (int ft = 0; ft < D / 32; ++ft)
+  for (int ft = 0; ft < FT; ++ft)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int f0 = 32 * ft + 8 * u + 4 * h;
       if (f0 < A.d)
         *reinterpret_cast<floatx4*>(op + f0) = floatx4{o[ft][4 * u] * inv, o[ft][4 * u + 1] * inv, o[ft][4 * u + 2] * inv, o[ft][4 * u + 3] * inv};
     }
-  if (lse != nullptr && h == 0) lse[orow] = l > 0.f ? m + logf(l) : -INFINITY;
+  if (lse != nullptr && h == 0) lse[orow] = l > 0.f ? __builtin_fmaf(m, fabsf(A.scale), logf(l)) : -INFINITY;
 }
 
 static int f32_common(int batch, int kv_heads, int group, int seq, int q_offset, int dim_head, float scale, const int64_t* qs, const int64_t* ks,
@@ -549,7 +743,7 @@ static int f32_common(int batch, int kv_heads, int group, int seq, int q_offset,
   A.qoff = q_offset;
   if (dim_head <= 0 || dim_head > kF32MaxD || (dim_head & 3)) return NSA_E_UNSUPPORTED;
   if ((long)batch * kv_heads > 65535) return NSA_E_UNSUPPORTED;
-  A.b = batch; A.hk = kv_heads; A.g = group; A.n = seq; A.d = dim_head; A.scale = scale;
+  A.b = batch; A.hk = kv_heads; A.bh = batch * kv_heads; A.g = group; A.n = seq; A.d = dim_head; A.scale = scale;
   for (int t = 0; t < 3; ++t) {
     A.sq[t] = qs[t]; A.sk[t] = ks[t]; A.sv[t] = vs[t];
     if ((A.sk[t] | A.sv[t]) & 3) return NSA_E_ARG;       // key / value rows are read 16 bytes at a time
@@ -570,6 +764,37 @@ static void f32_launch_rows(const F32Args& A, const float* q, const float* k, co
   if (A.d <= 64) { if (shared) NSA_ROWS(1, 4); else NSA_ROWS(1, 1); }
   else { if (shared) NSA_ROWS(2, 4); else NSA_ROWS(2, 1); }
 #undef NSA_ROWS
+}
+
+template <bool SEL>
+static void f32_launch_tiles(const F32Args& A, const float* q, const float* k, const float* v, const void* idx, const uint8_t* fmask, float* out,
+                             float* lse, hipStream_t stream) {
+  const dim3 grid((unsigned)((((long)A.n * A.g + 127) / 128) * A.bh));
+  if (A.d <= 64) hipLaunchKernelGGL((f32_tile_kernel<64, SEL>), grid, dim3(256), 0, stream, A, q, k, v, idx, fmask, out, lse);
+  else hipLaunchKernelGGL((f32_tile_kernel<128, SEL>), grid, dim3(256), 0, stream, A, q, k, v, idx, fmask, out, lse);
+}
+
+// A work-group of the tile kernel needs some 128 rows, and the launch enough of them.  Interval masks, us row by row / in tiles:
+//   d = 64   2048 queries 38.9 / 37.8 (window 512), 15.2 / 16.2 (64); 4096 81 / 42 and 22 / 16; 2048 queries ungrouped 21 / 23
+//   d = 128   496 queries 21.3 / 17.4, 1024 27.6 / 26.2 (window 512), 19.8 / 19.9 (2); 4096 168 / 67 and 54 / 21
+static bool f32_tiles_fit(const F32Args& A) {
+  return (long)A.n * A.g >= 128 && (long)A.n * A.b * A.hk >= (A.d <= 64 ? 4096 : 512);
+}
+
+// Masked tiles instead of gathered blocks, where the blocks fit the masks and the estimate of the time (us) is lower:
+//   tiles   a work-group's walk to the last key, 2.4 us per 32 keys (d = 128: 5), or the chip's rate over all rows and half the keys
+//   gather  per query (four heads at a time) 1.4 ns (4.6) for 64 keys of its blocks + 3 (12)
+// Measured, gather / tiles: 16 blocks of 64, d = 64, G 4: 2 x 2053 queries x 4 441 / 159, 1024 x 4 103 / 77, 8192 x 4 984 / 782; 4 blocks of 16, G 2:
+// 8 x 1024 x 4 155 / 84, 4 x 1024 x 4 83 / 79, 1024 x 4 29 / 78, 4 x 2048 x 4 156 / 151; d = 128, 16 of 64: 2048 x 8 1303 / 338; 4 of 16: 2048 x 8 297 / 321.
+static bool f32_masked_tiles(F32Args& A) {
+  A.lb = 0;
+  while (A.lb < 30 && (1 << A.lb) < A.B) ++A.lb;
+  if (!A.causal || A.B < 4 || A.B != 1 << A.lb || A.W > kTileBlocks || !f32_tiles_fit(A)) return false;
+  const bool wide = A.d > 64;
+  const double queries = (double)A.n * A.b * A.hk, keys = (double)(A.S + 1) * A.B;
+  const double tiles = std::max(A.nk * (wide ? 0.16 : 0.075), queries * A.g * A.nk * (wide ? 1.9e-6 : 0.73e-6));
+  const double gather = queries * ((A.g + 3) / 4) * (wide ? 0.0046 * keys / 64 + 0.012 : 0.0014 * keys / 64 + 0.003);
+  return tiles < gather;
 }
 
 }  // namespace nsa
@@ -596,14 +821,10 @@ static int dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k
   } else {
     return NSA_E_ARG;
   }
-  // A wave of the tile kernel takes 32 rows through all their keys: below ~4096 queries too few waves with too long a walk.
-  // Window 512, d = 64, 4 heads: 2048 queries 65 us in tiles, 41 us row by row; 4096 queries 65 against 82 us.
-  if ((long)A.n * A.b * A.hk < 4096) {
+  if (!f32_tiles_fit(A)) {
     f32_launch_rows<false>(A, q, k, v, nullptr, nullptr, out, lse, (hipStream_t)stream);
   } else {
-    const dim3 grid((unsigned)(((long)A.n * A.g + 127) / 128), A.b * A.hk);
-    if (A.d <= 64) hipLaunchKernelGGL(f32_tile_kernel<64>, grid, dim3(256), 0, (hipStream_t)stream, A, q, k, v, out, lse);
-    else hipLaunchKernelGGL(f32_tile_kernel<128>, grid, dim3(256), 0, (hipStream_t)stream, A, q, k, v, out, lse);
+    f32_launch_tiles<false>(A, q, k, v, nullptr, nullptr, out, lse, (hipStream_t)stream);
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
@@ -632,7 +853,8 @@ extern "C" int nsa_select_fwd_f32(const nsa_select_desc* d, const float* q, cons
   A.nk = num_keys; A.S = d->num_sel; A.B = d->block; A.W = (num_keys + d->block - 1) / d->block; A.causal = d->causal ? 1 : 0;
   A.idx64 = d->idx_is_int64 ? 1 : 0;
   A.uniform = !A.causal && A.S > 0 && q_offset == 0 && num_keys == d->seq;
-  f32_launch_rows<true>(A, q, k, v, idx, fmask, out, lse, (hipStream_t)stream);
+  if (f32_masked_tiles(A)) f32_launch_tiles<true>(A, q, k, v, idx, fmask, out, lse, (hipStream_t)stream);
+  else f32_launch_rows<true>(A, q, k, v, idx, fmask, out, lse, (hipStream_t)stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
