@@ -292,6 +292,13 @@ int nsa_skinny_linear(int32_t rows, int32_t k, int32_t n, const void* x, int64_t
 int nsa_linear_f32(int32_t rows, int32_t k, int32_t n, const float* x, int64_t x_row_stride, const float* weight, const float* bias, int32_t act,
                    float* y, void* stream);
 
+/* y = x weight^T + bias (relu: its positive part) in fp32 for many rows, on the bf16 matrix instructions with the operands split in
+ * three (see nsa_gemm.hip; the sums are at least as exact as fp32 fused multiply-adds): x [m, k] with row stride x_row_stride, weight
+ * [n, k] contiguous, bias (optional) [n], y [m, n] contiguous.  x2, weight2, bias2, y2: a second product of the same sizes in the
+ * same launch, or all NULL.  k and the row stride multiples of 4 below 2^24, x and weight 16-byte aligned (NSA_E_ARG otherwise). */
+int nsa_gemm_f32(int32_t m, int32_t k, int32_t n, const float* x, int64_t x_row_stride, const float* weight, const float* bias, int32_t relu,
+                 float* y, const float* x2, const float* weight2, const float* bias2, float* y2, void* stream);
+
 /* Column sums of a bf16 matrix in fp32: the bias gradient of a projection (the sum of d_out over tokens that
  * autograd takes for the nn.Linear layers of NSA.py:244-262, 853) and the gradient of the intra-window positions
  * (the sum of the window gradients over batch and windows, NSA.py:599-600).  Row (o, i) of group g starts at

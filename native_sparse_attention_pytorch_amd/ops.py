@@ -1765,6 +1765,32 @@ def _few_rows_f32(x: Tensor, weight: Tensor, bias: Tensor | None, act: str | Non
     return y
 
 
+def gemm_f32_supported(x: Tensor, weight: Tensor, bias: Tensor | None = None, products: int = 1) -> bool:
+    """An fp32 projection, or two of the same sizes in one launch, that `nsa_gemm_f32` serves better than the GEMM library: from one
+    tile of 128 x 128 to a CU on.  us, library / this kernel (the fp32 matrix instructions end at 154 TFLOP/s):
+      4106 x 1024 -> 1536 (396 tiles) 144 / 90, 16384 x 1024 -> 1536 396 / 281, 8192 x 512 -> 1024 70 / 56, 2053 x 4096 -> 4096 562 / 481,
+      8192 x 4096 -> 6144 2747 / 2100; at the line 8192 x 512 -> 512 (256) 38 / 36, 4106 x 1024 -> 1024 (264) 93 / 84;
+      below it 500 x 4096 -> 6144 (192) 200 / 175 but 1024 x 2048 -> 2048 (128) 69 / 94, 2048 x 1024 -> 1024 (128) 35 / 51;
+      two of 1024 x 2048 -> 2048 137 / 104, two of 2048 x 1024 -> 1024 70 / 57."""
+    rows, k = x.numel() // max(x.shape[-1], 1), x.shape[-1]
+    return bool(x.is_cuda and x.dtype == torch.float32 and k % 4 == 0 and 4 <= k < 1 << 24
+                and products * -(-rows // 128) * -(-weight.shape[0] // 128) >= 256
+                and _weight_ready(x, k, weight) and _vectors_ready(x, weight, bias, None) and (bias is None or bias.is_contiguous())
+                and x.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
+def _gemm_f32(x: Tensor, weight: Tensor, bias: Tensor | None, act: str | None = None, second=None):
+    """act(linear(x, weight, bias)) of operands that `gemm_f32_supported` has seen; `second`: another (x, weight, bias) of the same
+    sizes, whose result is returned beside it."""
+    k, n = x.shape[-1], weight.shape[0]
+    y = x.new_empty((*x.shape[:-1], n))
+    x2, w2, b2 = second if second is not None else (None, None, None)
+    y2 = None if second is None else torch.empty_like(y)
+    _lib.check(_lib.lib().nsa_gemm_f32(x.numel() // k, k, n, x.data_ptr(), k, weight.data_ptr(), _ptr(bias), int(act == "relu"), y.data_ptr(),
+                                       _ptr(x2), _ptr(w2), _ptr(b2), _ptr(y2), _stream()), "nsa_gemm_f32")
+    return y if second is None else (y, y2)
+
+
 class _Linear(torch.autograd.Function):
     """F.linear whose weight gradient is a batched GEMM over slices of the token axis, summed in fp32 (see _wgrad_splits):
     the same products as the one GEMM autograd would launch (NSA.py:583 to_qkv, 853 to_strategy_combine, 858 combine_heads)."""
@@ -1773,6 +1799,8 @@ class _Linear(torch.autograd.Function):
     def forward(ctx, x, w, b):
         ctx.save_for_backward(x, w)
         ctx.has_bias = b is not None
+        if x.dtype == torch.float32 and plain_call() and gemm_f32_supported(x, w, b):
+            return _gemm_f32(x, w, b)
         return torch.nn.functional.linear(x, w, b)
 
     @staticmethod
@@ -1794,8 +1822,11 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     """torch.nn.functional.linear with the split weight-gradient GEMM (see _Linear)."""
     if (not (torch.is_grad_enabled() and weight.requires_grad) or torch.compiler.is_compiling() or x.dtype != weight.dtype
             or torch.is_autocast_enabled()):               # under autocast the library casts the operands itself
-        if not torch.is_grad_enabled() and plain_call() and linear_f32_supported(x, weight, bias):
-            return _few_rows_f32(x, weight, bias)
+        if x.dtype == torch.float32 and not torch.is_grad_enabled() and plain_call():
+            if linear_f32_supported(x, weight, bias):
+                return _few_rows_f32(x, weight, bias)
+            if gemm_f32_supported(x, weight, bias):
+                return _gemm_f32(x, weight, bias)
         return torch.nn.functional.linear(x, weight, bias)
     return _Linear.apply(x, weight, bias)
 

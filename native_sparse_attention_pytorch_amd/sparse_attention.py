@@ -243,6 +243,20 @@ class SparseAttention(nn.Module):
             windows = cls._linear(layer, windows)
         return windows
 
+    def _compress_both(self, kw, vw):
+        """The two compression networks.  Without gradients the first projections of two default networks of an fp32 module are one launch:
+        either alone has a tile for half of the chip at 1000 windows."""
+        nets = self.k_compress, self.v_compress
+        if (kw.shape[:3].numel() > 256 and kw.dtype == torch.float32 and not torch.is_grad_enabled() and ops.plain_call() and kw.shape == vw.shape
+                and all(self._plain(m, nn.Sequential) and len(m) == 4 and self._plain(m[0], _FlattenWindow) and self._plain(m[1], nn.Linear)
+                        and self._plain(m[2], nn.ReLU) for m in nets)):
+            x, (up_k, up_v) = (kw.flatten(-2), vw.flatten(-2)), (m[1] for m in nets)
+            if (up_k.weight.shape == up_v.weight.shape
+                    and all(ops.gemm_f32_supported(t, up.weight, up.bias, products=2) for t, up in zip(x, (up_k, up_v)))):
+                hidden = ops._gemm_f32(x[0], up_k.weight, up_k.bias, "relu", (x[1], up_v.weight, up_v.bias))
+                return tuple(self._linear(m[3], t) for m, t in zip(nets, hidden))
+        return self._compress(self.k_compress, kw), self._compress(self.v_compress, vw)
+
     def _split_heads(self, t):
         b, n, hd = t.shape
         return t.view(b, n, hd // self.dim_head, self.dim_head).permute(0, 2, 1, 3)
@@ -477,7 +491,7 @@ class SparseAttention(nn.Module):
         else:
             rq, rk = self.rotary_emb.rotate(q), self.rotary_emb.rotate(k)
             kw, vw = ops.windows_of(k, self.k_intrablock_positions, cbs, st), ops.windows_of(v, self.v_intrablock_positions, cbs, st)
-        ck0, cv0 = self._compress(self.k_compress, kw), self._compress(self.v_compress, vw)
+        ck0, cv0 = self._compress_both(kw, vw)
         if not torch.is_grad_enabled():
             return self._forward_fp32_values(x, q, k, v, rq, rk, ck0, cv0, return_cache)
         ck = torch.cat((self.compress_mem_kv[0][None].expand(b, -1, -1, -1), ck0), dim=-2)
