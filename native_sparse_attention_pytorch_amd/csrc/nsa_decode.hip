@@ -671,7 +671,8 @@ __global__ __launch_bounds__(384) void decode_combine_kernel(const CombineArgs A
   if (A.advance != nullptr && blockIdx.x == 0 && threadIdx.x == 0) A.advance[0] += 1;
 }
 
-static int make_decode_plan(const nsa_decode_desc* dsc, DecodePlan& P, bool step = false) {
+// `step`: the branch is one of a whole step's; `beside`: tiles of the other key range in its launch
+static int make_decode_plan(const nsa_decode_desc* dsc, DecodePlan& P, bool step = false, int beside = 0) {
   if (!dsc) return NSA_E_ARG;
   P = DecodePlan{};
   P.b = dsc->batch; P.hk = dsc->kv_heads; P.g = dsc->group; P.d = dsc->dim_head;
@@ -714,6 +715,14 @@ static int make_decode_plan(const nsa_decode_desc* dsc, DecodePlan& P, bool step
   int ns = (P.tiles + tpw * kDecodeWaves - 1) / (tpw * kDecodeWaves);
   const long cap = units >= most ? 1 : most / units;
   if (ns > cap) ns = (int)cap;
+  // The two key ranges of a step in wide heads: no more work-groups than the chip holds at once (four to a CU).  A second and
+  // third round, begun where the first drains, cost more than the longer walks: 16 steps at 32k context, 32 heads x 128, batch 32
+  // (2816 work-groups -> 1024) 2290 -> 2165 us, batch 16 (1792 -> 1024) 1640 -> 1555; 4000 tokens of context, batch 32 1580 -> 1542.
+  // (At 64 features a work-group takes half as much, and the limit above is the better one.)
+  if (step && P.mode == 0 && P.d == 128) {
+    auto groups = [&](int tiles, int t) { return (tiles + t * kDecodeWaves - 1) / (t * kDecodeWaves); };
+    for (int t = tpw; ns > 1 && (groups(P.tiles, t) + groups(beside, t)) * units > 1024; ++t) ns = groups(P.tiles, t + 1);
+  }
   if (ns > 64) ns = 64;
   if (ns < 1) ns = 1;
   P.nsplit = ns; P.nparts = ns * kDecodeWaves;
@@ -817,9 +826,9 @@ static int launch_combine(const DecodePlan* plans[3], const void* const ws[3], c
 }  // namespace nsa
 
 namespace nsa {
-static int decode_partials_bytes(const nsa_decode_desc* dsc, size_t* bytes, bool step) {
+static int decode_partials_bytes(const nsa_decode_desc* dsc, size_t* bytes, bool step, int beside = 0) {
   DecodePlan P;
-  if (int e = make_decode_plan(dsc, P, step)) return e;
+  if (int e = make_decode_plan(dsc, P, step, beside)) return e;
   if (!bytes) return NSA_E_ARG;
   *bytes = (size_t)P.b * P.units * P.nparts * P.rec * sizeof(float);
   return 0;
@@ -911,6 +920,7 @@ struct StepLayout {
   nsa_decode_desc c, f, s;
   int nb, k;                       // selection blocks available / selected this step
   int sel_units;                   // rows of idx per batch element
+  int tiles_c, tiles_s;            // 32-key tiles of the two key ranges
   int pooled;                      // the compressed branch leaves pooled logits and the selected-block branch selects
   size_t off_rq, off_wsc, off_wsf, off_wss, off_logits, off_idx, off_vals, off_fm, total;
   size_t wsc, wsf, wss;
@@ -947,11 +957,14 @@ static int make_step_layout(const nsa_decode_step_desc* d, StepLayout& L) {
     x->q_stride[0] = (int64_t)d->heads * d->dim_head; x->q_stride[1] = d->dim_head;
     for (int i = 0; i < 3; ++i) { x->k_stride[i] = d->kc_stride[i]; x->v_stride[i] = d->vc_stride[i]; }
   }
+  auto tiles = [](const nsa_decode_desc& x) { return (x.num_mem + 31) / 32 + (x.count + 31) / 32; };
+  L.tiles_c = d->num_compressed > 0 ? tiles(L.c) : 0;
+  L.tiles_s = tiles(L.s);
   if (d->num_compressed > 0)
-    if (int e = decode_partials_bytes(&L.c, &L.wsc, true)) return e;
+    if (int e = decode_partials_bytes(&L.c, &L.wsc, true, L.tiles_s)) return e;
   if (d->num_compressed <= 0) L.wsc = 0;
   if (int e = decode_partials_bytes(&L.f, &L.wsf, true)) return e;
-  if (int e = decode_partials_bytes(&L.s, &L.wss, true)) return e;
+  if (int e = decode_partials_bytes(&L.s, &L.wss, true, L.tiles_c)) return e;
   size_t o = 0;
   L.off_rq = o;     o = up256(o + (size_t)d->batch * d->heads * d->dim_head * 2);
   L.off_wsc = o;    o = up256(o + L.wsc);
@@ -1009,9 +1022,9 @@ int run_decode_step(const nsa_decode_step_desc* d, int32_t* state, const void* q
   if (L.k > 0 && (L.nb > 64 * 32 || L.k > 64)) return NSA_E_UNSUPPORTED;
   DecodePlan Pc{}, Pf, Ps;
   if (has_c)
-    if (int e = make_decode_plan(&L.c, Pc, true)) return e;
+    if (int e = make_decode_plan(&L.c, Pc, true, L.tiles_s)) return e;
   if (int e = make_decode_plan(&L.f, Pf, true)) return e;
-  if (int e = make_decode_plan(&L.s, Ps, true)) return e;
+  if (int e = make_decode_plan(&L.s, Ps, true, L.tiles_c)) return e;
   if (state != nullptr) {
     int kind = 1;
     for (DecodePlan* P : {&Pc, &Pf, &Ps}) {
