@@ -181,6 +181,14 @@ int nsa_topk(const float* scores, int64_t rows, int32_t nb, int32_t k, int32_t a
  * floor(query / own_block) cannot (NSA.py:676-691).  rows must be a multiple of seq. */
 int nsa_importance_topk(const float* scores, int64_t rows, int32_t nb, int32_t k, float scale, int32_t seq, int32_t causal_block,
                         int32_t own_block, int32_t* idx, float* vals, uint8_t* fmask, void* stream);
+/* The scores themselves as well, for up to 64 blocks: row (b, u, i) of idx / vals / fmask [batch, units, seq, k] (units: kv heads if
+ * share, else query heads) holds the k best of mean over the unit's heads of q . mean over a block's per_block compressed keys of ck,
+ * times scale.  q fp32 [batch, heads, seq, dim_head], ck [batch, kv_heads, >= blocks * per_block, dim_head] by element strides {batch, head,
+ * token} (multiples of 4, 16-byte aligned); dim_head a multiple of 4 up to 128; causal_block, own_block as above. */
+int nsa_importance_select_f32(int32_t batch, int32_t heads, int32_t kv_heads, int32_t seq, int32_t dim_head, const float* q,
+                              const int64_t* q_stride, const float* ck, const int64_t* ck_stride, int32_t blocks, int32_t per_block, int32_t share,
+                              int32_t k, float scale, int32_t causal_block, int32_t own_block, int32_t* idx, float* vals, uint8_t* fmask,
+                              void* stream);
 /* The same for the logits of a causal compressed forward (nsa_dense_fwd with pool = 2): row r belongs to query
  * r % seq, and only its columns below floor(query / block) - the selection blocks that lie completely before the
  * query, NSA.py:676-689 - are defined; the rest counts as -inf and is never read (about half the matrix).  Same
@@ -291,6 +299,17 @@ int nsa_skinny_linear(int32_t rows, int32_t k, int32_t n, const void* x, int64_t
  * (NSA_E_UNSUPPORTED otherwise), rows 16-byte aligned. */
 int nsa_linear_f32(int32_t rows, int32_t k, int32_t n, const float* x, int64_t x_row_stride, const float* weight, const float* bias, int32_t act,
                    float* y, void* stream);
+/* Two of them in one launch: x, x2 [rows, k] of the same row stride (or the same matrix), n and n2 outputs.  norm != 0: of the RMS norm of
+ * the rows, rms_norm(x) * norm_weight (NULL: ones) with `eps` added to the mean square. */
+int nsa_linear_pair_f32(int32_t rows, int32_t k, int64_t x_row_stride, int32_t norm, const float* norm_weight, float eps, int32_t act,
+                        const float* x, const float* weight, const float* bias, int32_t n, float* y, const float* x2, const float* weight2,
+                        const float* bias2, int32_t n2, float* y2, void* stream);
+/* y = merged weight^T + bias with merged [batch seq, heads dim_head] = sum over the three branches of sigmoid(logit) * branch, as
+ * nsa_gate_fwd_f32 gives it: logits [batch, seq, 3 heads], branches [batch, heads, seq, dim_head] by element strides {batch, head, token}
+ * (multiples of 4, 16-byte aligned), y [batch seq, n].  heads * dim_head a multiple of 8. */
+int nsa_gate_linear_f32(int32_t batch, int32_t heads, int32_t seq, int32_t dim_head, const float* logits, const float* c, const int64_t* c_stride,
+                        const float* f, const int64_t* f_stride, const float* s, const int64_t* s_stride, const float* weight, const float* bias,
+                        int32_t n, float* y, void* stream);
 
 /* y = x weight^T + bias (relu: its positive part) in fp32 for many rows, on the bf16 matrix instructions with the operands split in
  * three (see nsa_gemm.hip; the sums are at least as exact as fp32 fused multiply-adds): x [m, k] with row stride x_row_stride, weight
@@ -331,6 +350,9 @@ int nsa_dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, c
  * k / v hold the num_keys compressed rows alone. */
 int nsa_compress_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, const float* mem_k, const float* mem_v,
                          float* out, float* lse, int32_t q_offset, void* stream);
+/* nsa_compress_fwd_f32 and the sliding window (mode 0) of the same queries' rotated form, in one launch where they are few; no lse. */
+int nsa_compress_window_fwd_f32(const nsa_dense_desc* dc, const float* q, const float* ck, const float* cv, const float* mem_k, const float* mem_v,
+                                float* out_c, const nsa_dense_desc* dw, const float* rq, const float* k, const float* v, float* out_w, void* stream);
 /* (non-causal, no offset, num_keys = seq: a query whose slots are all dead attends their blocks uniformly, NSA.py:809-815; its lse is -inf) */
 int nsa_select_fwd_f32(const nsa_select_desc* d, const float* q, const float* k, const float* v, const void* idx,
                        const uint8_t* fmask, float* out, float* lse, int32_t num_keys, int32_t q_offset, void* stream);

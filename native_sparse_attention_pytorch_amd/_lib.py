@@ -82,6 +82,14 @@ def lib():
         L.nsa_selftest_mfma.restype = C.c_int
         L.nsa_gemm_f32.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, vp, C.c_int32, vp, vp, vp, vp, vp, vp]
         L.nsa_gemm_f32.restype = C.c_int
+        i32, i64, f32 = C.c_int32, C.c_int64, C.c_float
+        s3 = C.POINTER(C.c_int64)
+        L.nsa_linear_pair_f32.argtypes = [i32, i32, i64, i32, vp, f32, i32, vp, vp, vp, i32, vp, vp, vp, vp, i32, vp, vp]
+        L.nsa_gate_linear_f32.argtypes = [i32, i32, i32, i32, vp, vp, s3, vp, s3, vp, s3, vp, vp, i32, vp, vp]
+        L.nsa_compress_window_fwd_f32.argtypes = [C.POINTER(DenseDesc), vp, vp, vp, vp, vp, vp, C.POINTER(DenseDesc), vp, vp, vp, vp, vp]
+        L.nsa_importance_select_f32.argtypes = [i32, i32, i32, i32, i32, vp, s3, vp, s3, i32, i32, i32, i32, f32, i32, i32, vp, vp, vp, vp]
+        for name in ("nsa_linear_pair_f32", "nsa_gate_linear_f32", "nsa_compress_window_fwd_f32", "nsa_importance_select_f32"):
+            getattr(L, name).restype = C.c_int
         L.nsa_probe_row_traffic.argtypes = [vp, sz, vp, sz, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_uint32, vp]
         L.nsa_probe_row_traffic.restype = C.c_int
         L.nsa_select_fwd_timed.argtypes = L.nsa_select_fwd.argtypes + [vp, C.c_int]

@@ -228,12 +228,18 @@ __device__ __forceinline__ void rows_walk(const F32Args& A, float* __restrict__ 
 
 // SELECT: block selection, else interval masks.  WPQ: waves of a work-group that share a query (1 or 4; with 4 each takes
 // every fourth tile and the partial results are merged: few queries, long key lists).
+struct RowsShared {
+  float pieces[4 * kRowsPiece];
+  int blocks[4][64], rows[4][64];
+};
+
 template <int DT, bool SELECT, int WPQ>
-__global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const float* __restrict__ q, const float* __restrict__ k,
-                                                          const float* __restrict__ v, const void* __restrict__ idx,
-                                                          const uint8_t* __restrict__ fmask, float* __restrict__ out, float* __restrict__ lse) {
-  __shared__ float pieces[4 * kRowsPiece];
-  __shared__ int blocks_s[4][64], rows_s[4][64];
+__device__ __forceinline__ void f32_rows_body(const F32Args& A, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+                                              const void* __restrict__ idx, const uint8_t* __restrict__ fmask, float* __restrict__ out,
+                                              float* __restrict__ lse, RowsShared& sh) {
+  float* pieces = sh.pieces;
+  int (&blocks_s)[4][64] = sh.blocks;
+  int (&rows_s)[4][64] = sh.rows;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = WPQ == 1 ? blockIdx.x * 4 + wave : blockIdx.x;
   if (i >= A.n) return;                                   // (WPQ == 1: no work-group barrier follows)
@@ -360,6 +366,25 @@ __global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const
       __syncthreads();                                     // before the next heads' pieces overwrite the partials
     }
   }
+}
+
+template <int DT, bool SELECT, int WPQ>
+__global__ __launch_bounds__(256, 2) void f32_rows_kernel(const F32Args A, const float* __restrict__ q, const float* __restrict__ k,
+                                                          const float* __restrict__ v, const void* __restrict__ idx,
+                                                          const uint8_t* __restrict__ fmask, float* __restrict__ out, float* __restrict__ lse) {
+  __shared__ RowsShared sh;
+  f32_rows_body<DT, SELECT, WPQ>(A, q, k, v, idx, fmask, out, lse, sh);
+}
+
+// Two interval masks of as many queries in one launch (the compressed branch and the window of a few tokens: a launch each is
+// most of their time)
+struct RowsCall { F32Args A; const float *q, *k, *v; float* out; };
+
+template <int DT, int WPQ>
+__global__ __launch_bounds__(256, 2) void f32_rows_pair_kernel(const RowsCall X, const RowsCall Y) {
+  __shared__ RowsShared sh;
+  if (blockIdx.z == 0) f32_rows_body<DT, false, WPQ>(X.A, X.q, X.k, X.v, nullptr, nullptr, X.out, nullptr, sh);
+  else f32_rows_body<DT, false, WPQ>(Y.A, Y.q, Y.k, Y.v, nullptr, nullptr, Y.out, nullptr, sh);
 }
 
 // ------------------------------------------------------------------------------------------ tile
@@ -801,10 +826,7 @@ static bool f32_masked_tiles(F32Args& A) {
 
 using namespace nsa;
 
-static int dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, const float* mem_k, const float* mem_v, float* out,
-                         float* lse, int32_t q_offset, void* stream) {
-  if (!d || !q || !k || !v || !out) return NSA_E_ARG;
-  F32Args A{};
+static int dense_args_f32(const nsa_dense_desc* d, const float* mem_k, const float* mem_v, int32_t q_offset, F32Args& A) {
   const int rc = f32_common(d->batch, d->kv_heads, d->group, d->seq, q_offset, d->dim_head, d->scale, d->q_stride, d->k_stride, d->v_stride, A);
   if (rc) return rc;
   if (d->num_keys < 0 || d->num_mem < 0 || d->num_mem > 64) return NSA_E_ARG;
@@ -821,6 +843,14 @@ static int dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k
   } else {
     return NSA_E_ARG;
   }
+  return 0;
+}
+
+static int dense_fwd_f32(const nsa_dense_desc* d, const float* q, const float* k, const float* v, const float* mem_k, const float* mem_v, float* out,
+                         float* lse, int32_t q_offset, void* stream) {
+  if (!d || !q || !k || !v || !out) return NSA_E_ARG;
+  F32Args A{};
+  if (const int rc = dense_args_f32(d, mem_k, mem_v, q_offset, A)) return rc;
   if (!f32_tiles_fit(A)) {
     f32_launch_rows<false>(A, q, k, v, nullptr, nullptr, out, lse, (hipStream_t)stream);
   } else {
@@ -840,6 +870,35 @@ extern "C" int nsa_compress_fwd_f32(const nsa_dense_desc* d, const float* q, con
   if (!d || d->mode != 1 || d->num_mem <= 0 || !mem_k || !mem_v || ((reinterpret_cast<uintptr_t>(mem_k) | reinterpret_cast<uintptr_t>(mem_v)) & 15))
     return NSA_E_ARG;
   return dense_fwd_f32(d, q, k, v, mem_k, mem_v, out, lse, q_offset, stream);
+}
+
+extern "C" int nsa_compress_window_fwd_f32(const nsa_dense_desc* dc, const float* q, const float* ck, const float* cv, const float* mem_k, const float* mem_v,
+                                           float* out_c, const nsa_dense_desc* dw, const float* rq, const float* k, const float* v, float* out_w,
+                                           void* stream) {
+  if (!dc || !dw || !q || !ck || !cv || !mem_k || !mem_v || !out_c || !rq || !k || !v || !out_w) return NSA_E_ARG;
+  if (dc->mode != 1 || dc->num_mem <= 0 || dw->mode != 0 || ((reinterpret_cast<uintptr_t>(mem_k) | reinterpret_cast<uintptr_t>(mem_v)) & 15)) return NSA_E_ARG;
+  RowsCall X{}, Y{};
+  if (const int rc = dense_args_f32(dc, mem_k, mem_v, 0, X.A)) return rc;
+  if (const int rc = dense_args_f32(dw, nullptr, nullptr, 0, Y.A)) return rc;
+  if (X.A.n != Y.A.n || X.A.b != Y.A.b || X.A.hk != Y.A.hk || X.A.g != Y.A.g || X.A.d != Y.A.d) return NSA_E_ARG;
+  if (f32_tiles_fit(X.A)) {
+    if (const int rc = dense_fwd_f32(dc, q, ck, cv, mem_k, mem_v, out_c, nullptr, 0, stream)) return rc;
+    return dense_fwd_f32(dw, rq, k, v, nullptr, nullptr, out_w, nullptr, 0, stream);
+  }
+  X.q = q; X.k = ck; X.v = cv; X.out = out_c;
+  Y.q = rq; Y.k = k; Y.v = v; Y.out = out_w;
+  const bool shared = (long)X.A.n * X.A.b * X.A.hk < 1024;            // (as f32_launch_rows)
+  const dim3 grid(shared ? X.A.n : (X.A.n + 3) / 4, X.A.b * X.A.hk, 2);
+  hipStream_t st = (hipStream_t)stream;
+  if (X.A.d <= 64) {
+    if (shared) hipLaunchKernelGGL((f32_rows_pair_kernel<1, 4>), grid, dim3(256), 0, st, X, Y);
+    else hipLaunchKernelGGL((f32_rows_pair_kernel<1, 1>), grid, dim3(256), 0, st, X, Y);
+  } else {
+    if (shared) hipLaunchKernelGGL((f32_rows_pair_kernel<2, 4>), grid, dim3(256), 0, st, X, Y);
+    else hipLaunchKernelGGL((f32_rows_pair_kernel<2, 1>), grid, dim3(256), 0, st, X, Y);
+  }
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : (int)e;
 }
 
 extern "C" int nsa_select_fwd_f32(const nsa_select_desc* d, const float* q, const float* k, const float* v, const void* idx,

@@ -813,13 +813,24 @@ class _ImportanceTopk(torch.autograd.Function):
         return dl, None
 
 
-def importance_topk(importance_logits: Tensor, num_selected: int, prefix=None, raw=None):
+def importance_topk(importance_logits: Tensor, num_selected: int, prefix=None, raw=None, keys=None):
     """softmax with the -1e3 pad column (NSA.py:693-695) + topk (NSA.py:713) + `> 1e-10` mask
     (NSA.py:721).  Returns (values fp32, indices int32, fmask bool), each [..., num_selected];
     `values` is differentiable with respect to the logits.  `prefix` = (n, sel_block) as returned by
     `compress_attend(..., prefix_only=True)`: row i is read only below column i // sel_block (no gradient).
     `raw` = (scale, seq, causal block or 0, own block or 0): the logits are fp32 products that the kernel scales and masks
-    (`importance_topk_f32`; no gradient)."""
+    (`importance_topk_f32`; no gradient).  `keys` = (compressed keys, blocks, keys a block, heads share, causal block or 0, own block or 0):
+    instead of logits the queries 'b h n d' they are made from (`importance_select_f32`; no gradient)."""
+    if keys is not None:
+        q, (ck, nb, npf, share, causal_block, own_block) = importance_logits.detach(), keys
+        b, hq, n, d = q.shape
+        shp = (b, ck.shape[1] if share else hq, n, num_selected)
+        idx = torch.empty(shp, dtype=torch.int32, device=q.device)
+        vals = torch.empty(shp, dtype=torch.float32, device=q.device)
+        fm = torch.empty(shp, dtype=torch.bool, device=q.device)
+        _lib.check(_lib.lib().nsa_importance_select_f32(b, hq, ck.shape[1], n, d, _ptr(q), _s3(q), _ptr(ck), _s3(ck), nb, npf, share, num_selected, d ** -0.5,
+                                                        causal_block, own_block, _ptr(idx), _ptr(vals), _ptr(fm), _stream()), "nsa_importance_select_f32")
+        return vals, idx, fm
     if raw is not None:
         if importance_logits.dtype != torch.float32 or not importance_logits.is_cuda:
             raise RuntimeError("importance scores must be fp32 device tensors")
@@ -1724,9 +1735,52 @@ def linear_f32_supported(x: Tensor, weight: Tensor, bias: Tensor | None = None) 
     if not (x.is_cuda and x.dtype == torch.float32 and 0 < rows <= 256 and k <= 512 and k % 8 == 0 and _weight_ready(x, k, weight)
             and _vectors_ready(x, weight, bias, None)):
         return False
-    n = weight.shape[0]
+    return _few_rows_sizes(rows, k, weight.shape[0])
+
+
+def _few_rows_sizes(rows: int, k: int, n: int) -> bool:
     tiles = -(-rows // 32) * -(-n // 32)
     return n <= 256 or (tiles <= 256 if k <= 256 else tiles <= 128 and not 1 < rows < 32)
+
+
+def _rows_f32(x: Tensor) -> Tensor | None:
+    """x as a matrix of rows the fp32 projection kernel reads where they lie, or None."""
+    x2 = x.reshape(-1, x.shape[-1])
+    return x2 if x2.stride(1) == 1 and x2.stride(0) % 4 == 0 and x2.data_ptr() % 16 == 0 else None
+
+
+def linear_pair_f32(x: Tensor, first, second, norm_weight: Tensor | None = None, eps: float | None = None, x2: Tensor | None = None,
+                    act: str | None = None):
+    """act(linear(x, *first)) and act(linear(x2, *second)) of a few rows in one launch, `first` / `second` = (weight, bias); x2 None: both
+    of x.  eps not None: of rms_norm(x) * norm_weight.  None where one of them is not `linear_f32`'s to serve."""
+    if not all(linear_f32_supported(t, w, b) and (b is None or b.is_contiguous()) for t, (w, b) in ((x, first), (x if x2 is None else x2, second))):
+        return None
+    a = _rows_f32(x)
+    c = a if x2 is None else _rows_f32(x2)
+    if a is None or c is None or a.shape != c.shape or a.stride() != c.stride() or not _vectors_ready(x, first[0], None, norm_weight):
+        return None
+    rows, k = a.shape
+    y, y2 = (x.new_empty((*x.shape[:-1], w.shape[0])) for w in (first[0], second[0]))
+    _lib.check(_lib.lib().nsa_linear_pair_f32(rows, k, a.stride(0), int(eps is not None), _ptr(norm_weight), eps or 0.0, _ACTS[act], a.data_ptr(),
+                                              first[0].data_ptr(), _ptr(first[1]), first[0].shape[0], y.data_ptr(), c.data_ptr(), second[0].data_ptr(),
+                                              _ptr(second[1]), second[0].shape[0], y2.data_ptr(), _stream()), "nsa_linear_pair_f32")
+    return y, y2
+
+
+def gate_linear_f32(logits: Tensor, c: Tensor, f: Tensor, s: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
+    """linear(gate_combine_f32(logits, c, f, s), weight, bias) of a few tokens in one launch; None where that is not `linear_f32`'s to serve."""
+    b, h, n, d = c.shape
+    rows, k = b * n, h * d
+    if not (0 < rows <= 256 and k <= 512 and k % 8 == 0 and logits.dtype == torch.float32 and logits.is_cuda and logits.shape == (b, n, 3 * h)
+            and logits.is_contiguous() and _weight_ready(logits, k, weight) and _vectors_ready(logits, weight, bias, None)
+            and (bias is None or bias.is_contiguous()) and _few_rows_sizes(rows, k, weight.shape[0])
+            and all(t.shape == c.shape and t.dtype == torch.float32 and t.device == logits.device for t in (c, f, s))):
+        return None
+    c, f, s = _f32(c), _f32(f), _f32(s)
+    y = logits.new_empty((b, n, weight.shape[0]))
+    _lib.check(_lib.lib().nsa_gate_linear_f32(b, h, n, d, logits.data_ptr(), c.data_ptr(), _s3(c), f.data_ptr(), _s3(f), s.data_ptr(), _s3(s),
+                                              weight.data_ptr(), _ptr(bias), weight.shape[0], y.data_ptr(), _stream()), "nsa_gate_linear_f32")
+    return y
 
 
 def _laid_out(t: Tensor) -> Tensor:
@@ -2009,6 +2063,30 @@ def compress_attend_f32(q: Tensor, ck: Tensor, cv: Tensor, mem: Tensor, stride: 
 
 
 @torch.no_grad()
+def compress_window_f32(q: Tensor, ck: Tensor, cv: Tensor, mem: Tensor, stride: int, rq: Tensor, k: Tensor, v: Tensor, window: int, causal: bool):
+    """(`compress_attend_f32(q, ck, cv, mem, stride, causal)`, `dense_attend_f32(rq, k, v, 0, causal, window)[0]`): one launch for a few tokens."""
+    q, ck, cv, rq, k, v = (_f32(t) for t in (q, ck, cv, rq, k, v))
+    b, hq, n, d = q.shape
+    _check_f32_dim(d)
+    mem = mem.to(torch.float32).contiguous()
+    mem = mem.clone() if mem.data_ptr() % 16 else mem
+    hk, m = ck.shape[1], mem.shape[2]
+    if mem.shape != (2, hk, m, d) or cv.shape != ck.shape or ck.shape[0] != b or ck.shape[3] != d or mem.device != q.device:
+        raise RuntimeError("compress_window_f32: memory rows '2 hk m d' and compressed keys / values 'b hk nc d' of the queries' batch and features")
+    if rq.shape != q.shape or k.shape != (b, hk, n, d) or v.shape != k.shape:
+        raise RuntimeError("compress_window_f32: rotated queries as the queries, keys and values 'b hk n d'")
+    c_out, s_out = (torch.empty((b, hq, n, d), dtype=torch.float32, device=q.device) for _ in range(2))
+    scale = float(d ** -0.5)
+    dc = _dense_desc(q, ck, cv, c_out, c_out, 1, bool(causal), 0, int(stride), 0, False, 1, True, scale)
+    dc.num_mem, dc.num_keys = m, ck.shape[2]
+    dw = _dense_desc(rq, k, v, s_out, s_out, 0, bool(causal), int(window), 1, 0, False, 1, True, scale)
+    p = mem.data_ptr()
+    _lib.check(_lib.lib().nsa_compress_window_fwd_f32(C.byref(dc), _ptr(q), _ptr(ck) or p, _ptr(cv) or p, p, p + 4 * hk * m * d, _ptr(c_out), C.byref(dw),
+                                                      _ptr(rq), _ptr(k), _ptr(v), _ptr(s_out), _stream()), "nsa_compress_window_fwd_f32")
+    return c_out, s_out
+
+
+@torch.no_grad()
 def importance_topk_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool, causal: bool, num_selected: int, mask_own: bool = True):
     """`importance_topk(importance_logits_f32(...))` without gradients: the products from the same fp32 GEMM, scale and masks
     inside the top-k kernel.  Returns (values, idx, fmask)."""
@@ -2018,6 +2096,20 @@ def importance_topk_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, shar
     if nb > _TOPK_MAX_ROW or num_selected > _TOPK_MAX_K:
         return importance_topk(_importance_mask_f32(raw * (q.shape[-1] ** -0.5), stride, sel_block, causal, mask_own).contiguous(), num_selected)
     return importance_topk(raw, num_selected, raw=(q.shape[-1] ** -0.5, n, int(sel_block) if causal else 0, int(sel_block) if own else 0))
+
+
+@torch.no_grad()
+def importance_select_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool, causal: bool, num_selected: int, mask_own: bool = True):
+    """`importance_topk_f32` whose products are made by the top-k kernel as well for up to 64 blocks: four launches less, and a query's scores
+    the same whatever the number of queries beside it."""
+    b, hq, n, d = q.shape
+    hk, npf = ck.shape[1], sel_block // stride
+    nb, num_selected = ck.shape[2] // npf, int(num_selected)
+    if (0 < num_selected <= nb <= 64 and d <= 128 and d % 4 == 0 and n > 0 and q.dtype == ck.dtype == torch.float32 and q.is_cuda
+            and ck.device == q.device and ck.shape[0] == b and ck.shape[3] == d and b * hq <= 65535):
+        return importance_topk(_f32(q), num_selected, keys=(_f32(ck), nb, npf, int(share), int(sel_block) if causal else 0,
+                                                            int(sel_block) if mask_own and stride != sel_block else 0))
+    return importance_topk_f32(q, ck, stride, sel_block, share, causal, num_selected, mask_own)
 
 
 class _GateF32(torch.autograd.Function):
@@ -2116,33 +2208,39 @@ def windows_of(t: Tensor, pos: Tensor, block: int, stride: int) -> Tensor:
     return torch.nn.functional.pad(t[..., :L, :], (0, 0, block - stride, 0)).unfold(2, block, stride).permute(0, 1, 2, 4, 3) + pos[None, :, None]
 
 
+def _qkv_prep_f32(qkv: Tensor, freqs: Tensor, kpos: Tensor, vpos: Tensor, heads: int, kv_heads: int, d: int, block: int, stride: int, offset: int):
+    """The results of `qkv_prep_f32` and the frequencies in fp32."""
+    b, n, width = qkv.shape
+    if qkv.stride(2) != 1 or qkv.stride(1) % 8 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
+        qkv = qkv.clone(memory_format=torch.contiguous_format)
+    w = n // stride if block > 0 else 0
+    rq = torch.empty((b, heads, n, d), dtype=torch.float32, device=qkv.device)
+    rk = torch.empty((b, kv_heads, n, d), dtype=torch.float32, device=qkv.device)
+    kw = torch.empty((b, kv_heads, w, block, d), dtype=torch.float32, device=qkv.device)
+    vw = torch.empty_like(kw)
+    freqs32 = freqs.detach().to(torch.float32).contiguous()
+    kp = kpos.detach().to(torch.float32).contiguous() if w > 0 else None
+    vp = vpos.detach().to(torch.float32).contiguous() if w > 0 else None
+    dsc = _qkv_desc(qkv, heads, kv_heads, d, block, stride, offset)
+    dsc.fp32 = 2
+    _lib.check(_lib.lib().nsa_qkv_prep_fwd(C.byref(dsc), _ptr(qkv), _ptr(freqs32), _ptr(kp), _ptr(vp), None, _ptr(rq), _ptr(rk), None,
+                                           _ptr(kw) if w > 0 else None, _ptr(vw) if w > 0 else None, _stream()), "nsa_qkv_prep_fwd")
+    q = qkv[..., :heads * d].view(b, n, heads, d).permute(0, 2, 1, 3)
+    v = qkv[..., (heads + kv_heads) * d:].view(b, n, kv_heads, d).permute(0, 2, 1, 3)
+    return (q, rq, rk, v, kw, vw), freqs32
+
+
 class _QkvPrepF32(torch.autograd.Function):
     """`_QkvPrep` with every tensor in fp32: one kernel over the projection in each direction, instead of about fifty launches of
     rotation, window split, their gradients and the padded sums of the gradients of q, k and v."""
 
     @staticmethod
     def forward(ctx, qkv, freqs, kpos, vpos, heads, kv_heads, d, block, stride, offset):
-        b, n, width = qkv.shape
-        if qkv.stride(2) != 1 or qkv.stride(1) % 8 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
-            qkv = qkv.clone(memory_format=torch.contiguous_format)
-        w = n // stride if block > 0 else 0
-        rq = torch.empty((b, heads, n, d), dtype=torch.float32, device=qkv.device)
-        rk = torch.empty((b, kv_heads, n, d), dtype=torch.float32, device=qkv.device)
-        kw = torch.empty((b, kv_heads, w, block, d), dtype=torch.float32, device=qkv.device)
-        vw = torch.empty_like(kw)
-        freqs32 = freqs.detach().to(torch.float32).contiguous()
-        kp = kpos.detach().to(torch.float32).contiguous() if w > 0 else None
-        vp = vpos.detach().to(torch.float32).contiguous() if w > 0 else None
-        dsc = _qkv_desc(qkv, heads, kv_heads, d, block, stride, offset)
-        dsc.fp32 = 2
-        _lib.check(_lib.lib().nsa_qkv_prep_fwd(C.byref(dsc), _ptr(qkv), _ptr(freqs32), _ptr(kp), _ptr(vp), None, _ptr(rq), _ptr(rk), None,
-                                               _ptr(kw) if w > 0 else None, _ptr(vw) if w > 0 else None, _stream()), "nsa_qkv_prep_fwd")
-        q = qkv[..., :heads * d].view(b, n, heads, d).permute(0, 2, 1, 3)
-        v = qkv[..., (heads + kv_heads) * d:].view(b, n, kv_heads, d).permute(0, 2, 1, 3)
+        results, freqs32 = _qkv_prep_f32(qkv, freqs, kpos, vpos, heads, kv_heads, d, block, stride, offset)
         ctx.save_for_backward(freqs32)
-        ctx.meta = ((b, n, width), heads, kv_heads, d, block, stride, offset, tuple(kpos.shape), kpos.dtype, vpos.dtype)
+        ctx.meta = (tuple(qkv.shape), heads, kv_heads, d, block, stride, offset, tuple(kpos.shape), kpos.dtype, vpos.dtype)
         ctx.set_materialize_grads(False)
-        return q, rq, rk, v, kw, vw
+        return results
 
     @staticmethod
     def backward(ctx, dq, drq, drk, dv, dkw, dvw):
@@ -2185,5 +2283,7 @@ def qkv_prep_f32(qkv: Tensor, freqs: Tensor, k_positions: Tensor, v_positions: T
     if qkv.dim() != 3 or qkv.shape[2] != (heads + 2 * kv_heads) * dim_head or not qkv_prep_f32_operands(
             qkv, freqs, k_positions, v_positions, kv_heads, dim_head, compress_block_size or k_positions.shape[1]):
         raise RuntimeError("qkv_prep_f32: projection 'b n ((h + 2 hk) d)', frequencies 'd/2' and positions 'hk block d' on its device")
-    return _QkvPrepF32.apply(qkv, freqs, k_positions, v_positions, int(heads), int(kv_heads), int(dim_head), int(compress_block_size),
-                             int(compress_stride), int(offset))
+    args = (qkv, freqs, k_positions, v_positions, int(heads), int(kv_heads), int(dim_head), int(compress_block_size), int(compress_stride), int(offset))
+    if not torch.is_grad_enabled() and plain_call():
+        return _qkv_prep_f32(*args)[0]                                      # (nothing to record: the node around it is 10 us of host time)
+    return _QkvPrepF32.apply(*args)

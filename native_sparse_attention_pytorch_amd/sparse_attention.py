@@ -247,15 +247,39 @@ class SparseAttention(nn.Module):
         """The two compression networks.  Without gradients the first projections of two default networks of an fp32 module are one launch:
         either alone has a tile for half of the chip at 1000 windows."""
         nets = self.k_compress, self.v_compress
-        if (kw.shape[:3].numel() > 256 and kw.dtype == torch.float32 and not torch.is_grad_enabled() and ops.plain_call() and kw.shape == vw.shape
+        if (kw.dtype == torch.float32 and not torch.is_grad_enabled() and ops.plain_call() and kw.shape == vw.shape
                 and all(self._plain(m, nn.Sequential) and len(m) == 4 and self._plain(m[0], _FlattenWindow) and self._plain(m[1], nn.Linear)
                         and self._plain(m[2], nn.ReLU) for m in nets)):
-            x, (up_k, up_v) = (kw.flatten(-2), vw.flatten(-2)), (m[1] for m in nets)
-            if (up_k.weight.shape == up_v.weight.shape
+            (_, up_k, _, down_k), (_, up_v, _, down_v) = nets
+            x = kw.flatten(-2), vw.flatten(-2)
+            hidden = ops.linear_pair_f32(x[0], (up_k.weight, up_k.bias), (up_v.weight, up_v.bias), x2=x[1], act="relu")
+            if (hidden is None and up_k.weight.shape == up_v.weight.shape
                     and all(ops.gemm_f32_supported(t, up.weight, up.bias, products=2) for t, up in zip(x, (up_k, up_v)))):
                 hidden = ops._gemm_f32(x[0], up_k.weight, up_k.bias, "relu", (x[1], up_v.weight, up_v.bias))
-                return tuple(self._linear(m[3], t) for m, t in zip(nets, hidden))
+            if hidden is not None:
+                if self._plain(down_k, nn.Linear) and self._plain(down_v, nn.Linear):
+                    pair = ops.linear_pair_f32(hidden[0], (down_k.weight, down_k.bias), (down_v.weight, down_v.bias), x2=hidden[1])
+                    if pair is not None:
+                        return pair
+                return self._linear(down_k, hidden[0]), self._linear(down_v, hidden[1])
         return self._compress(self.k_compress, kw), self._compress(self.v_compress, vw)
+
+    def _front_fp32(self, inp):
+        """(qkv projection, gate logits) of the normed input of an fp32 module with its default layers, without gradients, as one launch for a
+        few tokens; None otherwise."""
+        norm, qkv, gate = self.norm, self.to_qkv, self.to_strategy_combine
+        if (torch.is_grad_enabled() or inp.dtype != torch.float32 or not self.fp32_kernels or self.dim_head > 128 or self.dim_head % 4
+                or inp.shape[0] * inp.shape[1] > 256 or not ops.plain_call()):
+            return None
+        if not (self._plain(norm, nn.RMSNorm) and self._plain(qkv, nn.Linear) and qkv.bias is None and norm.normalized_shape == tuple(inp.shape[-1:])
+                and self._gate_plain() and self._plain(gate[0], nn.Linear) and gate[0].weight.shape[0] == 3 * self.heads):
+            return None
+        eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
+        return ops.linear_pair_f32(inp, (qkv.weight, None), (gate[0].weight, gate[0].bias), norm.weight, eps)
+
+    def _gate_plain(self):
+        gate = self.to_strategy_combine
+        return (self._plain(gate, nn.Sequential) and len(gate) == 3 and self._plain(gate[1], nn.Sigmoid) and self._plain(gate[2], _GateLayout))
 
     def _split_heads(self, t):
         b, n, hd = t.shape
@@ -448,7 +472,7 @@ class SparseAttention(nn.Module):
         # selected blocks + own block up to the token (NSA.py:446-515)
         num_sel = min(self.num_selected_blocks, nc // (B // st))
         if num_sel > 0:
-            _, idx, fmask = ops.importance_topk_f32(q, cache_ck, st, B, self.query_heads_share_selected_kv, False, num_sel, mask_own=False)
+            _, idx, fmask = ops.importance_select_f32(q, cache_ck, st, B, self.query_heads_share_selected_kv, False, num_sel, mask_own=False)
         else:
             idx = torch.zeros((b, self.kv_heads, 1, 0), dtype=torch.int32, device=x.device)
             fmask = idx.bool()
@@ -472,11 +496,12 @@ class SparseAttention(nn.Module):
             return out
         return out, ((keys, vals), ((ck, cv), (run_k, run_v)))
 
-    def _forward_fp32(self, x, qkv, return_cache):
+    def _forward_fp32(self, x, qkv, return_cache, logits=None):
         """The parallel forward of an fp32 module: every attention branch through the fp32 kernels (ops.*_f32), the gate and
         the merge in fp32 - the same steps as `forward` (NSA.py:579-862).  Under autograd the values are still those of
-        the fp32 kernels and each branch's gradient comes from the bf16 kernels (ops.fp32_value_bf16_grad)."""
-        b, n, _ = x.shape
+        the fp32 kernels and each branch's gradient comes from the bf16 kernels (ops.fp32_value_bf16_grad).  `logits`: the gate's, where
+        they came with the projection (x is None then)."""
+        b, n, _ = qkv.shape
         st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
         M, d = self.num_mem_compress_kv, self.dim_head
         causal, win, share = self.causal, self.sliding_window_size, self.query_heads_share_selected_kv
@@ -493,7 +518,7 @@ class SparseAttention(nn.Module):
             kw, vw = ops.windows_of(k, self.k_intrablock_positions, cbs, st), ops.windows_of(v, self.v_intrablock_positions, cbs, st)
         ck0, cv0 = self._compress_both(kw, vw)
         if not torch.is_grad_enabled():
-            return self._forward_fp32_values(x, q, k, v, rq, rk, ck0, cv0, return_cache)
+            return self._forward_fp32_values(x, q, k, v, rq, rk, ck0, cv0, return_cache, logits)
         ck = torch.cat((self.compress_mem_kv[0][None].expand(b, -1, -1, -1), ck0), dim=-2)
         cv = torch.cat((self.compress_mem_kv[1][None].expand(b, -1, -1, -1), cv0), dim=-2)
         nc = ck0.shape[-2]
@@ -506,13 +531,13 @@ class SparseAttention(nn.Module):
                 vals, idx, fmask = ops.importance_topk(ops.importance_logits_f32(qa, ck0, st, B, share, causal).contiguous(), num_sel)
                 gates = vals + (1. - vals).detach()                              # straight-through gates (NSA.py:715)
             else:
-                _, idx, fmask = ops.importance_topk_f32(qa, ck0, st, B, share, causal, num_sel)
+                _, idx, fmask = ops.importance_select_f32(qa, ck0, st, B, share, causal, num_sel)
             block_causal = causal
         elif causal:
-            idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=x.device)
+            idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=qkv.device)
             fmask, block_causal = idx.bool(), True
         else:
-            idx = (torch.arange(n, device=x.device, dtype=torch.int32) // B)[None, None, :, None].expand(b, self.kv_heads, n, 1).contiguous()
+            idx = (torch.arange(n, device=qkv.device, dtype=torch.int32) // B)[None, None, :, None].expand(b, self.kv_heads, n, 1).contiguous()
             fmask, block_causal = torch.ones_like(idx, dtype=torch.bool), False
         sel32 = lambda q_, k_, v_, *g_: ops.native_sparse_attend_f32(q_, k_, v_, B, idx, fmask, include_block_causal=block_causal)
         sel16 = lambda q_, k_, v_, *g_: ops.native_sparse_attend(q_, k_, v_, B, idx, fmask, sel_scale=g_[0] if g_ else None,
@@ -525,26 +550,29 @@ class SparseAttention(nn.Module):
             return out
         return out, ((rk, v), ((ck0, cv0), (_open_window(k, L, cbs - st), _open_window(v, L, cbs - st))))
 
-    def _forward_fp32_values(self, x, q, k, v, rq, rk, ck0, cv0, return_cache):
+    def _forward_fp32_values(self, x, q, k, v, rq, rk, ck0, cv0, return_cache, logits=None):
         """The attention of `_forward_fp32` without gradients: a kernel per branch, the memory rows read from the parameter, scale
         and masks of the importance scores inside the top-k kernel, gate and head merge one kernel."""
-        b, n, _ = x.shape
+        b, _, n, _ = q.shape
         st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
         causal, nc = self.causal, ck0.shape[-2]
-        c_out = ops.compress_attend_f32(q, ck0, cv0, self.compress_mem_kv, st, causal)
+        c_out, s_out = ops.compress_window_f32(q, ck0, cv0, self.compress_mem_kv, st, rq, rk, v, self.sliding_window_size, causal)
         num_sel = min(self.num_selected_blocks, nc // (B // st))
         block_causal = causal
         if num_sel > 0:
-            _, idx, fmask = ops.importance_topk_f32(q, ck0, st, B, self.query_heads_share_selected_kv, causal, num_sel)
+            _, idx, fmask = ops.importance_select_f32(q, ck0, st, B, self.query_heads_share_selected_kv, causal, num_sel)
         elif causal:
-            idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=x.device)
+            idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=q.device)
             fmask = idx.bool()
         else:
-            idx = (torch.arange(n, device=x.device, dtype=torch.int32) // B)[None, None, :, None].expand(b, self.kv_heads, n, 1).contiguous()
+            idx = (torch.arange(n, device=q.device, dtype=torch.int32) // B)[None, None, :, None].expand(b, self.kv_heads, n, 1).contiguous()
             fmask = torch.ones_like(idx, dtype=torch.bool)
         f_out = ops.native_sparse_attend_f32(rq, rk, v, B, idx, fmask, include_block_causal=block_causal)
-        s_out, _ = ops.dense_attend_f32(rq, rk, v, 0, causal, self.sliding_window_size)
-        out = self._linear(self.combine_heads, self._gate_fp32(x, c_out, f_out, s_out))
+        out, heads = None, self.combine_heads
+        if logits is not None and self._plain(heads, nn.Linear):
+            out = ops.gate_linear_f32(logits, c_out, f_out, s_out, heads.weight, heads.bias)
+        if out is None:
+            out = self._linear(heads, self._gate_fp32(x, c_out, f_out, s_out) if logits is None else ops.gate_combine_f32(logits, c_out, f_out, s_out))
         if not return_cache:
             return out
         L = (n // st) * st
@@ -553,7 +581,7 @@ class SparseAttention(nn.Module):
     def _gate_fp32(self, x, c_out, f_out, s_out):
         """Strategy gate and head merge in fp32: 'b n (h d)'."""
         gate = self.to_strategy_combine
-        if (self._plain(gate, nn.Sequential) and len(gate) == 3 and self._plain(gate[1], nn.Sigmoid) and self._plain(gate[2], _GateLayout)):
+        if self._gate_plain():
             logits = self._linear(gate[0], x)
             if logits.dtype == torch.float32:
                 return ops.gate_combine_f32(logits, c_out, f_out, s_out)
@@ -585,6 +613,9 @@ class SparseAttention(nn.Module):
             qkv, logits = ops.normed_projections(inp, self.norm.weight, self.norm.eps, self.to_qkv.weight,
                                                  self.to_strategy_combine[0].weight, self.to_strategy_combine[0].bias)
         else:
+            front = self._front_fp32(inp)
+            if front is not None:
+                return self._forward_fp32(None, front[0], return_cache, front[1])
             x = self._normed(inp)
             qkv = self._linear(self.to_qkv, x)
         if (x is not None and self.fp32_kernels and qkv.dtype == torch.float32
