@@ -318,6 +318,26 @@ int nsa_gate_linear_f32(int32_t batch, int32_t heads, int32_t seq, int32_t dim_h
 int nsa_gemm_f32(int32_t m, int32_t k, int32_t n, const float* x, int64_t x_row_stride, const float* weight, const float* bias, int32_t relu,
                  float* y, const float* x2, const float* weight2, const float* bias2, float* y2, void* stream);
 
+/* bf16 projections under training, fp32 sums.  nsa_gemm_bf16: y [m, n] = epilogue(x w^T + bias) (+ residual), x [m, k], w [n, k]
+ * (transposed: w [k, n], x w); all contiguous, act, residual and pre as y.  Epilogues: RELU; GELU (exact; the value before it goes to
+ * `pre` where that is not null); RELU_BWD / GELU_BWD multiply by the activation's slope at act (the output of the ReLU, the value
+ * before the GELU).  x2 .. pre2: a second product of the same sizes, or null (residual: the first only, without a second).
+ * k % 64 == 0, n % 8 == 0 (transposed: % 128), NSA_E_UNSUPPORTED otherwise.  Values are rounded where separate layers would round
+ * them: after the product and bias, after the activation, after the residual.
+ * nsa_wgrad_bf16: dw [n_out, n_in] = dy^T x and db [n_out] = the column sums of dy (or null) over `rows` rows, dy2 .. db2 a second one of
+ * the same sizes and strides, or null; n_out % 64 == 0 and n_in % 128 == 0; workspace of nsa_wgrad_bf16_workspace bytes each (0:
+ * unsupported sizes). */
+#define NSA_GEMM_RELU 1
+#define NSA_GEMM_GELU 2
+#define NSA_GEMM_RELU_BWD 3
+#define NSA_GEMM_GELU_BWD 4
+int nsa_gemm_bf16(int32_t transposed, int32_t m, int32_t n, int32_t k, int32_t epilogue, const void* x, const void* w, const void* bias,
+                  const void* act, const void* residual, void* y, void* pre, const void* x2, const void* w2, const void* bias2, const void* act2,
+                  void* y2, void* pre2, void* stream);
+int64_t nsa_wgrad_bf16_workspace(int64_t rows, int32_t n_out, int32_t n_in);
+int nsa_wgrad_bf16(int64_t rows, int32_t n_out, int32_t n_in, const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride,
+                   void* dw, void* db, const void* dy2, const void* x2, void* dw2, void* db2, float* workspace, void* stream);
+
 /* Column sums of a bf16 matrix in fp32: the bias gradient of a projection (the sum of d_out over tokens that
  * autograd takes for the nn.Linear layers of NSA.py:244-262, 853) and the gradient of the intra-window positions
  * (the sum of the window gradients over batch and windows, NSA.py:599-600).  Row (o, i) of group g starts at

@@ -82,6 +82,12 @@ def lib():
         L.nsa_selftest_mfma.restype = C.c_int
         L.nsa_gemm_f32.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, vp, C.c_int32, vp, vp, vp, vp, vp, vp]
         L.nsa_gemm_f32.restype = C.c_int
+        L.nsa_gemm_bf16.argtypes = [C.c_int32] * 5 + [vp] * 14
+        L.nsa_gemm_bf16.restype = C.c_int
+        L.nsa_wgrad_bf16_workspace.argtypes = [C.c_int64, C.c_int32, C.c_int32]
+        L.nsa_wgrad_bf16_workspace.restype = C.c_int64
+        L.nsa_wgrad_bf16.argtypes = [C.c_int64, C.c_int32, C.c_int32, vp, C.c_int64, vp, C.c_int64] + [vp] * 8
+        L.nsa_wgrad_bf16.restype = C.c_int
         i32, i64, f32 = C.c_int32, C.c_int64, C.c_float
         s3 = C.POINTER(C.c_int64)
         L.nsa_linear_pair_f32.argtypes = [i32, i32, i64, i32, vp, f32, i32, vp, vp, vp, i32, vp, vp, vp, vp, i32, vp, vp]

@@ -1865,9 +1865,13 @@ class _Linear(torch.autograd.Function):
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
             dx = (dy2 @ w).view(x.shape)
+        need_db = ctx.has_bias and ctx.needs_input_grad[2]
         if ctx.needs_input_grad[1]:
+            if _wgrad_supported(dy2, x2, w.dtype):
+                dw, db = _wgrad_bf16([(dy2, x2)], need_db)[0]
+                return dx, dw, db
             dw = _wgrad(dy2, x2, w.dtype)
-        if ctx.has_bias and ctx.needs_input_grad[2]:
+        if need_db:
             db = colsum(dy2) if colsum_supported(dy2) else dy2.sum(0)
         return dx, dw, db
 
@@ -1885,8 +1889,168 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     return _Linear.apply(x, weight, bias)
 
 
+_GEMM_MACS = 9 << 30
+
+
+def _wgrad_supported(dy2: Tensor, x2: Tensor, dtype) -> bool:
+    """A weight gradient that `nsa_wgrad_bf16` serves.  RULE"""
+    rows, n_out, n_in = x2.shape[0], dy2.shape[1], x2.shape[1]
+    return bool(x2.dtype == dy2.dtype == dtype == _BF16 and x2.is_cuda and rows > 0 and n_out % 64 == 0 and n_in % 128 == 0
+                and n_out < 1 << 15 and n_in < 1 << 15 and (n_out == 64 or rows * n_out * n_in <= _GEMM_MACS)
+                and not torch.is_grad_enabled() and plain_call() and not _in_batch(dy2) and _row_aligned(dy2) and _row_aligned(x2))
+
+
+_in_batch = torch._C._functorch.is_legacy_batchedtensor      # autograd.grad(..., is_grads_batched=True), which plain_call does not see
+
+
+def _row_aligned(t: Tensor) -> bool:
+    return t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.shape[1] <= t.stride(0) < 1 << 24 and t.data_ptr() % 16 == 0
+
+
+def _wgrad_bf16(pairs, bias: bool):
+    """[(dw, db)] of one or two (dy2, x2) of the same sizes and strides that `_wgrad_supported` has seen; db None without `bias`."""
+    L = _lib.lib()
+    (dy, x), (rows, n_out), n_in = pairs[0], pairs[0][0].shape, pairs[0][1].shape[1]
+    ws = torch.empty((len(pairs) * L.nsa_wgrad_bf16_workspace(rows, n_out, n_in) // 4,), dtype=torch.float32, device=x.device)
+    out = [(x.new_empty((n_out, n_in)), x.new_empty((n_out,)) if bias else None) for _ in pairs]
+    second = (None,) * 4 if len(pairs) == 1 else (_ptr(pairs[1][0]), _ptr(pairs[1][1]), _ptr(out[1][0]), _ptr(out[1][1]))
+    _lib.check(L.nsa_wgrad_bf16(rows, n_out, n_in, dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), _ptr(out[0][0]), _ptr(out[0][1]), *second,
+                                ws.data_ptr(), _stream()), "nsa_wgrad_bf16")
+    return out
+
+
+_EPILOGUES = {None: 0, "relu": 1, "gelu": 2, "relu_bwd": 3, "gelu_bwd": 4}
+
+
+def _gemm_bf16(xs, ws, biases=None, epilogue=None, acts=None, residual=None, transposed=False, keep=False):
+    """[epilogue(x w^T + bias) (+ residual)] (transposed: x w) of one or two contiguous operands of the same sizes, and with `keep` the
+    values before the epilogue."""
+    m, k = xs[0].shape
+    n = ws[0].shape[1 if transposed else 0]
+    two = len(xs) == 2
+    ys = [x.new_empty((m, n)) for x in xs]
+    pre = [torch.empty_like(y) for y in ys] if keep else None
+    pick = lambda ts, i: None if ts is None or i >= len(ts) or ts[i] is None else ts[i].data_ptr()
+    _lib.check(_lib.lib().nsa_gemm_bf16(int(transposed), m, n, k, _EPILOGUES[epilogue], xs[0].data_ptr(), ws[0].data_ptr(), pick(biases, 0),
+                                        pick(acts, 0), _ptr(residual), ys[0].data_ptr(), pick(pre, 0), pick(xs, 1), pick(ws, 1), pick(biases, 1),
+                                        pick(acts, 1), ys[1].data_ptr() if two else None, pick(pre, 1), _stream()), "nsa_gemm_bf16")
+    return (ys, pre) if keep else ys
+
+
+def _plain_mlp(act, eps, residual, norm_w, x, w1, b1, w2, b2):
+    F = torch.nn.functional
+    y = x if norm_w is None else F.rms_norm(x, norm_w.shape, norm_w, eps)
+    y = F.linear(F.gelu(F.linear(y, w1, b1)) if act == "gelu" else F.relu(F.linear(y, w1, b1)), w2, b2)
+    return y + x if residual else y
+
+
+class _Mlp(torch.autograd.Function):
+    """One or two networks linear - activation - linear of the same sizes in a bf16 module under autograd, each optionally behind an RMS
+    norm and with its input added (the feed-forward block, transformer.py:142-152; the compression networks, NSA.py:306-322): every
+    product is this library's kernel with what follows it in the product's epilogue, and a weight gradient comes with its bias's.
+    8 x 1024 tokens, 512 features, us in the layer: feed-forward with norm and residual NN, both compression networks NN."""
+
+    @staticmethod
+    def forward(ctx, act, eps, residual, norm_w, *nets):
+        nets = [nets[i:i + 5] for i in range(0, len(nets), 5)]
+        k = nets[0][0].shape[-1]
+        x2 = [net[0].reshape(-1, k).contiguous() for net in nets]
+        nw = rstd = None
+        xn = x2
+        if norm_w is not None:
+            nw = norm_w.detach().contiguous()
+            y, rstd = _rms_fwd(x2[0], nw, eps)
+            xn = [y]
+        w1, b1, w2, b2 = ([net[i] for net in nets] for i in (1, 2, 3, 4))
+        need = any(ctx.needs_input_grad)
+        if act == "gelu" and need:
+            hidden, slope_at = _gemm_bf16(xn, w1, b1, act, keep=True)
+        else:
+            hidden = slope_at = _gemm_bf16(xn, w1, b1, act)
+        out = _gemm_bf16(hidden, w2, b2, residual=x2[0] if residual else None)
+        if need:
+            ctx.save_for_backward(*(net[0] for net in nets), *w1, *b1, *w2, *b2, *hidden, *slope_at, *(() if nw is None else (norm_w, xn[0], rstd)))
+            ctx.args = (act, eps, residual, norm_w is not None, len(nets))
+        out = tuple(y.view(*net[0].shape[:-1], -1) for y, net in zip(out, nets))
+        return out if len(out) > 1 else out[0]
+
+    @staticmethod
+    def backward(ctx, *douts):
+        act, eps, residual, normed, n = ctx.args
+        xs, w1, b1, w2, b2, hidden, slope_at = (list(ctx.saved_tensors[i * n:(i + 1) * n]) for i in range(7))
+        norm_w, xn, rstd = ctx.saved_tensors[7 * n:] if normed else (None, None, None)
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled() or not plain_call() or any(map(_in_batch, douts)):
+            # gradients of the gradients, or a batch of them: through the separate layers
+            grads = [None, None, None, None]
+            for i, d in enumerate(douts):
+                args = [t if t is None or t.requires_grad else t.detach().requires_grad_() for t in (xs[i], w1[i], b1[i], w2[i], b2[i], norm_w)]
+                with torch.enable_grad():
+                    y = _plain_mlp(act, eps, residual, args[5], *args[:5])
+                got = torch.autograd.grad(y, [t for t in args if t is not None], d, create_graph=torch.is_grad_enabled())
+                grads += got[:5]
+                grads[3] = got[5] if normed else None
+            return tuple(g if w else None for g, w in zip(grads, need))
+        rows = [x.reshape(-1, x.shape[-1]).contiguous() for x in xs]
+        xn = rows if xn is None else [xn]
+        d2 = [d.reshape(-1, w.shape[0]).contiguous() for d, w in zip(douts, w2)]
+        wants = lambda i: any(need[4 + 5 * j + i] for j in range(n))
+        grads = [None] * len(need)
+
+        def put(i, values):
+            for j, v in enumerate(values):
+                grads[4 + 5 * j + i] = v
+
+        if wants(3) or wants(4):
+            got = _wgrad_bf16(list(zip(d2, hidden)), wants(4))
+            put(3, [g[0] for g in got])
+            put(4, [g[1] for g in got])
+        if need[3] or wants(0) or wants(1) or wants(2):
+            dh = _gemm_bf16(d2, w2, epilogue=act + "_bwd", acts=slope_at, transposed=True)
+            if wants(1) or wants(2):
+                got = _wgrad_bf16(list(zip(dh, xn)), wants(2))
+                put(1, [g[0] for g in got])
+                put(2, [g[1] for g in got])
+            if need[3] or wants(0):
+                dx = _gemm_bf16(dh, w1, residual=d2[0] if residual and not normed else None, transposed=True)
+                if normed:
+                    dx0, grads[3] = _rms_bwd(rows[0], norm_w.contiguous(), rstd, dx[0], need[3])
+                    dx = [dx0.add_(d2[0]) if residual else dx0]
+                put(0, [d.view(x.shape) for d, x in zip(dx, xs)])
+        return tuple(g if w else None for g, w in zip(grads, need))
+
+
+def mlp_supported(act: str, xs, nets, norm_w: Tensor | None = None) -> bool:
+    """Networks that `mlp` serves; `nets`: (w1, b1, w2, b2) each.  RULE"""
+    x, (w1, _, w2, _) = xs[0], nets[0]
+    if not (torch.is_grad_enabled() and x.is_cuda and x.dtype == _BF16 and w1.dim() == 2 and w2.dim() == 2 and plain_call()):
+        return False
+    k, hidden, out, rows = x.shape[-1], w1.shape[0], w2.shape[0], x.numel() // max(x.shape[-1], 1)
+    if not (rows > 0 and k % 128 == 0 and hidden % 128 == 0 and out % 64 == 0 and max(k, hidden, out) < 1 << 15
+            and len(xs) * rows * hidden * max(k, out) <= _GEMM_MACS):
+        return False
+    for y, (a, b, c, d) in zip(xs, nets):
+        if y.shape != x.shape or y.dtype != _BF16 or y.device != x.device or a.shape != (hidden, k) or c.shape != (out, hidden):
+            return False
+        if b is None or d is None or b.shape != (hidden,) or d.shape != (out,):
+            return False
+        if any(t.dtype != _BF16 or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in (a, b, c, d)):
+            return False
+    if norm_w is not None and (norm_w.shape != (k,) or not rms_norm_supported(x, norm_w)):
+        return False
+    return any(t.requires_grad for t in (*xs, *(t for net in nets for t in net)))
+
+
+def mlp(act: str, xs, nets, norm_w: Tensor | None = None, eps: float | None = None, residual: bool = False):
+    """w2 act(w1 norm(x) + b1) + b2 (+ x) for each of one or two inputs that `mlp_supported` has seen."""
+    eps = float(torch.finfo(torch.float32).eps if eps is None else eps)
+    return _Mlp.apply(act, eps, residual, norm_w, *(t for x, net in zip(xs, nets) for t in (x, *net)))
+
+
 def _wgrad(dy2: Tensor, x2: Tensor, dtype) -> Tensor:
     """Weight gradient 'o i' = dy2^T x2 of a projection, over slices of the token axis where that fills the chip."""
+    if _wgrad_supported(dy2, x2, dtype):
+        return _wgrad_bf16([(dy2, x2)], False)[0][0]
     rows, n_in, n_out = x2.shape[0], x2.shape[1], dy2.shape[1]
     s = _wgrad_splits(rows, n_in, n_out, capturing()) if x2.is_cuda and x2.dtype in (_BF16, torch.float16) and dy2.dtype == x2.dtype else 1
     if s > 1 and dy2.is_contiguous() and x2.is_contiguous():

@@ -247,6 +247,13 @@ class SparseAttention(nn.Module):
         """The two compression networks.  Without gradients the first projections of two default networks of an fp32 module are one launch:
         either alone has a tile for half of the chip at 1000 windows."""
         nets = self.k_compress, self.v_compress
+        if (kw.dtype == torch.bfloat16 and torch.is_grad_enabled()
+                and all(self._plain(m, nn.Sequential) and len(m) == 4 and self._plain(m[0], _FlattenWindow) and self._plain(m[1], nn.Linear)
+                        and self._plain(m[2], nn.ReLU) and self._plain(m[3], nn.Linear) for m in nets)):
+            x = kw.flatten(-2), vw.flatten(-2)
+            weights = [(up.weight, up.bias, down.weight, down.bias) for _, up, _, down in nets]
+            if ops.mlp_supported("relu", x, weights):
+                return ops.mlp("relu", x, weights)
         if (kw.dtype == torch.float32 and not torch.is_grad_enabled() and ops.plain_call() and kw.shape == vw.shape
                 and all(self._plain(m, nn.Sequential) and len(m) == 4 and self._plain(m[0], _FlattenWindow) and self._plain(m[1], nn.Linear)
                         and self._plain(m[2], nn.ReLU) for m in nets)):

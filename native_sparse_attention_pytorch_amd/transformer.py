@@ -46,17 +46,24 @@ class Transformer(nn.Module):
 
     @staticmethod
     def _feed_forward(ff, tokens):
-        """The feed-forward block (transformer.py:142-152 of the reference: norm, linear, GELU, linear).  While a HIP graph is
-        being recorded (training.GraphedStep) the two projections go through ops.linear, whose bias gradients are column sums
-        by this library's kernel: the library's own sum records a memset node that replays wrongly on this platform."""
+        """ff(tokens) + tokens (transformer.py:142-152 of the reference: norm, linear, GELU, linear).  A bf16 block of the default layers under
+        autograd is one node (ops.mlp) where its sizes allow.  While a HIP graph is being recorded (training.GraphedStep) the two
+        projections of any other go through ops.linear, whose bias gradients are column sums by this library's kernel: the library's own
+        sum records a memset node that replays wrongly on this platform."""
         from . import ops
-        if not (ops.capturing() and torch.is_grad_enabled() and tokens.dtype == torch.bfloat16 and isinstance(ff, nn.Sequential) and len(ff) == 4):
-            return ff(tokens)
-        norm, up, act, down = ff
         plain = SparseAttention._plain
+        if not (torch.is_grad_enabled() and tokens.dtype == torch.bfloat16 and isinstance(ff, nn.Sequential) and len(ff) == 4):
+            return ff(tokens) + tokens
+        norm, up, act, down = ff
         if not (plain(ff, nn.Sequential) and plain(norm, nn.RMSNorm) and plain(up, nn.Linear) and plain(act, nn.GELU) and plain(down, nn.Linear)):
-            return ff(tokens)
-        return ops.linear(act(ops.linear(norm(tokens), up.weight, up.bias)), down.weight, down.bias)
+            return ff(tokens) + tokens
+        net = up.weight, up.bias, down.weight, down.bias
+        if (act.approximate == 'none' and norm.weight is not None and norm.normalized_shape == tuple(tokens.shape[-1:])
+                and down.weight.shape[0] == tokens.shape[-1] and ops.mlp_supported("gelu", [tokens], [net], norm.weight)):
+            return ops.mlp("gelu", [tokens], [net], norm.weight, norm.eps, residual=True)
+        if not ops.capturing():
+            return ff(tokens) + tokens
+        return ops.linear(act(ops.linear(norm(tokens), up.weight, up.bias)), down.weight, down.bias) + tokens
 
     @staticmethod
     def _decode_feed_forward(ff, tokens):
@@ -127,7 +134,7 @@ class Transformer(nn.Module):
                 attn_out, layer_cache = attn(tokens), None
             caches.append(layer_cache)
             tokens = attn_out + tokens
-            tokens = self._feed_forward(ff, tokens) + tokens
+            tokens = self._feed_forward(ff, tokens)
         logits = self.to_logits(self.norm(tokens))
         if not return_loss:
             return (logits, caches) if return_cache else logits
