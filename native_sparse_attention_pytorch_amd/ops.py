@@ -78,17 +78,16 @@ def _unpad_groups(t: Tensor, hk: int, g: int, gp: int) -> Tensor:
     return t.reshape(b, hk, gp, *t.shape[2:])[:, :, :g].reshape(b, hk * g, *t.shape[2:])
 
 
+# packed: a field of a ctypes structure takes the host 0.3 us, an array in one 1.2 us
+_SELECT_DESC, _DENSE_DESC = struct.Struct("@9if12q"), struct.Struct("@14ifi15q")
+assert _SELECT_DESC.size == C.sizeof(_lib.SelectDesc) and _DENSE_DESC.size == C.sizeof(_lib.DenseDesc)
+
+
 def _select_desc(q, k, v, o, num_sel, block, causal, scale, idx_is_int64) -> _lib.SelectDesc:
     b, hq, n, d = q.shape
     hk = k.shape[1]
-    dsc = _lib.SelectDesc()
-    dsc.batch, dsc.kv_heads, dsc.group, dsc.seq = b, hk, hq // hk, n
-    dsc.num_sel, dsc.block, dsc.dim_head, dsc.causal = num_sel, block, d, int(causal)
-    dsc.idx_is_int64 = int(idx_is_int64)
-    dsc.scale = scale
-    for name, t in (("q_stride", q), ("k_stride", k), ("v_stride", v), ("o_stride", o)):
-        getattr(dsc, name)[:] = list(t.stride()[:3])
-    return dsc
+    return _lib.SelectDesc.from_buffer_copy(_SELECT_DESC.pack(b, hk, hq // hk, n, num_sel, block, d, bool(causal), bool(idx_is_int64), scale,
+                                                              *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *o.stride()[:3]))
 
 
 def _ws_sizes(dsc) -> tuple[int, int, int]:
@@ -370,14 +369,9 @@ def native_sparse_attend(fq: Tensor, fk: Tensor, fv: Tensor, block_size: int, se
 def _dense_desc(q, k, v, o, do, mode, causal, window, stride, num_mem, pool, sel_block, share, scale) -> _lib.DenseDesc:
     b, hq, n, d = q.shape
     hk = k.shape[1]
-    dsc = _lib.DenseDesc()
-    dsc.batch, dsc.kv_heads, dsc.group, dsc.seq = b, hk, hq // hk, n
-    dsc.num_keys, dsc.num_mem, dsc.dim_head = k.shape[2] - num_mem, num_mem, d
-    dsc.mode, dsc.causal, dsc.window, dsc.stride = mode, int(causal), window, stride
-    dsc.pool, dsc.sel_block, dsc.share, dsc.scale = int(pool), sel_block, int(share), scale
-    for name, t in (("q_stride", q), ("k_stride", k), ("v_stride", v), ("o_stride", o), ("do_stride", do)):
-        getattr(dsc, name)[:] = list(t.stride()[:3])
-    return dsc
+    return _lib.DenseDesc.from_buffer_copy(_DENSE_DESC.pack(b, hk, hq // hk, n, k.shape[2] - num_mem, num_mem, d, mode, bool(causal), window, stride,
+                                                            int(pool), sel_block, bool(share), scale, 0, *q.stride()[:3], *k.stride()[:3],
+                                                            *v.stride()[:3], *o.stride()[:3], *do.stride()[:3]))
 
 
 @torch.library.custom_op("nsa_amd::dense_fwd", mutates_args=())
@@ -1376,7 +1370,6 @@ def _decode_layer(layer: DecodeLayer, freqs, pos, keys, vals, ck, cv, mem, run_k
     return _StepResult(out, ws, desc, hk if share else layer.heads)
 
 
-@torch.no_grad()
 def decode_step(q: Tensor, k: Tensor, v: Tensor, freqs: Tensor, pos: int, keys: Tensor, vals: Tensor, ck: Tensor | None, cv: Tensor | None,
                 mem_k: Tensor | None, mem_v: Tensor | None, k_run_row: Tensor | None, v_run_row: Tensor | None, gate_logits: Tensor,
                 *, per_block: int, block: int, num_sel: int, share: bool, window: int, scale: float | None = None, layer=None):
@@ -1390,6 +1383,13 @@ def decode_step(q: Tensor, k: Tensor, v: Tensor, freqs: Tensor, pos: int, keys: 
     the first result is the layer's output 'b 1 dim'."""
     if layer is not None:
         return _decode_layer(layer, freqs, pos, keys, vals, ck, cv, mem_k, k_run_row, v_run_row, per_block, block, num_sel, share, window, scale)
+    return _decode_attention(q, k, v, freqs, pos, keys, vals, ck, cv, mem_k, mem_v, k_run_row, v_run_row, gate_logits, per_block, block, num_sel, share,
+                             window, scale)
+
+
+@torch.no_grad()
+def _decode_attention(q, k, v, freqs, pos, keys, vals, ck, cv, mem_k, mem_v, k_run_row, v_run_row, gate_logits, per_block, block, num_sel, share, window,
+                      scale):
     q, k, v = _prep(q), _prep(k), _prep(v)
     b, hq, _, d = q.shape
     hk = k.shape[1]
@@ -1653,8 +1653,10 @@ def plain_call() -> bool:
 
 def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
     """A weight the projection kernels read where it lies: rows of `width`, x's type and device, contiguous from a 16-byte boundary on."""
-    return bool(weight.dtype == x.dtype and weight.device == x.device and weight.dim() == 2 and weight.shape[1] == width
-                and weight.shape[0] > 0 and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+    if weight.dim() != 2:
+        return False
+    n, k = weight.shape
+    return bool(k == width and n > 0 and weight.dtype == x.dtype and weight.device == x.device and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
 
 
 def _vectors_ready(x: Tensor, weight: Tensor, bias: Tensor | None, norm_weight: Tensor | None) -> bool:
@@ -1667,7 +1669,8 @@ def _vectors_ready(x: Tensor, weight: Tensor, bias: Tensor | None, norm_weight: 
 def skinny_linear_supported(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_weight: Tensor | None = None, width: int | None = None) -> bool:
     """A projection of a few rows (a decode step) that `skinny_linear` serves.  `width`: the input is not x itself but as many rows
     of this many features, x's own projection."""
-    rows, k = x.numel() // x.shape[-1], x.shape[-1] if width is None else width
+    own = x.shape[-1]
+    rows, k = x.numel() // own, own if width is None else width
     return (x.is_cuda and x.dtype == _BF16 and 1 <= rows <= 32 and k % 32 == 0 and rows * (k + 8) <= 65536 and _weight_ready(x, k, weight)
             and _vectors_ready(x, weight, bias, norm_weight))
 
@@ -1688,19 +1691,29 @@ def _skinny(x: Tensor, weight: Tensor, bias: Tensor | None = None, norm_weight: 
     """`skinny_linear` of operands that `skinny_linear_supported` has seen."""
     if bias is not None and not bias.is_contiguous():
         bias = bias.contiguous()
-    k, n = x.shape[-1], weight.shape[0]
-    x2 = x.reshape(-1, k)
-    if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
-        x2 = x2.clone(memory_format=torch.contiguous_format)
-    rows = x2.shape[0]
+    *lead, k = x.shape
+    n = weight.shape[0]
+    ldx = k
+    if not x.is_contiguous() or x.data_ptr() % 16 or k % 8:
+        x = x.reshape(-1, k)
+        if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
+            x = x.clone(memory_format=torch.contiguous_format)
+        ldx = x.stride(0)
+    rows = x.numel() // k
+    ldr = 0
     if residual is not None:
-        residual = residual.reshape(rows, n)
-        if residual.dtype != _BF16 or residual.device != x.device or residual.stride(1) != 1:
+        if residual.dtype != _BF16 or residual.device != x.device:
             raise RuntimeError("skinny_linear: the residual must be bf16 on the same device with unit stride")
-    y = x.new_empty((*x.shape[:-1], n))
-    _lib.check(_lib.lib().nsa_skinny_linear(rows, k, n, x2.data_ptr(), x2.stride(0), _ptr(norm_weight), eps, weight.data_ptr(), _ptr(bias), _ACTS[act],
-                                            _ptr(residual), 0 if residual is None else residual.stride(0), y.data_ptr(), n, _stream()),
-               "nsa_skinny_linear")
+        ldr = n
+        if not residual.is_contiguous() or residual.numel() != rows * n:
+            residual = residual.reshape(rows, n)
+            ldr = residual.stride(0)
+            if residual.stride(1) != 1:
+                raise RuntimeError("skinny_linear: the residual must be bf16 on the same device with unit stride")
+    y = x.new_empty((*lead, n))
+    _lib.check(_lib.lib().nsa_skinny_linear(rows, k, n, x.data_ptr(), ldx, 0 if norm_weight is None else norm_weight.data_ptr(), eps, weight.data_ptr(),
+                                            0 if bias is None else bias.data_ptr(), _ACTS[act], 0 if residual is None else residual.data_ptr(), ldr,
+                                            y.data_ptr(), n, _stream()), "nsa_skinny_linear")
     return y
 
 

@@ -64,11 +64,13 @@ def _append_rows(t: torch.Tensor, extra: int = 1, dtype=torch.bfloat16, min_capa
 
 def _grown(t: torch.Tensor, min_capacity: int = 128) -> torch.Tensor:
     """`_append_rows` of one row to a bf16 cache of its own width, without the view of the new row."""
-    base, n = t._base, t.shape[2]
-    if (base is not None and getattr(base, "_nsa_filled", -1) == n and base.dim() == 4 and base.shape[2] > n and base.shape[:2] == t.shape[:2]
-            and base.shape[3] == t.shape[3] and base.dtype == torch.bfloat16 and t.data_ptr() == base.data_ptr() and t.stride() == base.stride()):
-        base._nsa_filled = n + 1
-        return base.narrow(2, 0, n + 1)
+    base, (b, h, n, d) = t._base, t.shape
+    if base is not None and getattr(base, "_nsa_filled", -1) == n and base.dim() == 4:
+        b0, h0, rows, d0 = base.shape
+        if (rows > n and b0 == b and h0 == h and d0 == d and base.dtype == torch.bfloat16 and t.data_ptr() == base.data_ptr()
+                and t.stride() == base.stride()):
+            base._nsa_filled = n + 1
+            return base.narrow(2, 0, n + 1)
     return _append_rows(t, min_capacity=min_capacity)[0]
 
 
@@ -96,6 +98,21 @@ class _GateLayout(nn.Module):
     def forward(self, x):                                   # 'b n (h s) -> b h n s'
         b, n, _ = x.shape
         return x.reshape(b, n, self.heads, 3).permute(0, 2, 1, 3)
+
+
+class _Attributes:
+    """An object's attributes as a table."""
+    def __init__(self, obj):
+        self.obj = obj
+
+    def __getitem__(self, name):
+        return getattr(self.obj, name)
+
+
+def _weights(layer):
+    """(weight, bias) of a library layer that `SparseAttention._plain` has seen (KeyError: they were taken out of its table)."""
+    p = layer._parameters
+    return p["weight"], p["bias"]
 
 
 def _global_hooks():
@@ -297,50 +314,67 @@ class SparseAttention(nn.Module):
         launches; `residual` is added to the output); None when something about the layer, the caches or the sizes asks for the
         general path.  Called without gradients and in a plain call (ops.plain_call)."""
         (cache_k, cache_v), ((cache_ck, cache_cv), (run_k, run_v)) = cache
-        norm, qkv, gate, out, bf16 = self.norm, self.to_qkv, self.to_strategy_combine[0], self.combine_heads, torch.bfloat16
-        plain, d = self._plain, self.dim_head
-        if not (self.causal and d in (64, 128) and inp.is_cuda and inp.dtype == bf16 and plain(norm, nn.RMSNorm) and plain(qkv, nn.Linear)
-                and plain(gate, nn.Linear) and plain(out, nn.Linear) and qkv.bias is None and norm.weight is not None and inp.dim() == 3 and inp.shape[1] == 1):
+        # A step of a small model is bound by this function: layers and weights come from nn.Module's own tables (its attribute lookup
+        # takes 0.5 us a name, and there were 45; a weight that is not there leaves the general path to say so) and each shape is read
+        # once (0.3 us).  8 sequences, a model of 6 layers: NN to NN us a layer and token.
+        try:
+            mods, own = (self._modules, self._parameters) if type(self) is SparseAttention else (_Attributes(self), _Attributes(self))
+            norm, qkv, gate, out, bf16 = mods["norm"], mods["to_qkv"], mods["to_strategy_combine"], mods["combine_heads"], torch.bfloat16
+            gate = gate._modules["0"] if type(gate) is nn.Sequential else gate[0]
+            mem, rot = own["compress_mem_kv"], mods["rotary_emb"]
+            plain, d = self._plain, self.dim_head
+            if not (self.causal and (d == 64 or d == 128) and inp.is_cuda and inp.dtype == bf16 and plain(norm, nn.RMSNorm) and plain(qkv, nn.Linear)
+                    and plain(gate, nn.Linear) and plain(out, nn.Linear) and inp.dim() == 3):
+                return None
+            weights = norm._parameters["weight"], qkv._parameters["weight"], *_weights(gate), *_weights(out)
+            if qkv._parameters["bias"] is not None or weights[0] is None:
+                return None
+            freqs = rot._parameters["freqs"] if type(rot) is RotaryEmbedding else rot.freqs
+        except KeyError:
             return None
-        b, dim, hd = inp.shape[0], inp.shape[2], self.heads * d
-        mem, freqs, device = self.compress_mem_kv, self.rotary_emb.freqs, inp.device
-        if b > 32 or dim % 32 or b * (max(dim, hd) + 8) > 65536 or norm.normalized_shape != (dim,):
+        w_norm, w_qkv, w_gate, b_gate, w_out, b_out = weights
+        (b, one, dim), heads, hk = inp.shape, self.heads, self.kv_heads
+        hd, device = heads * d, inp.device
+        if one != 1 or b > 32 or dim % 32 or b * (max(dim, hd) + 8) > 65536 or norm.normalized_shape != (dim,):
             return None
-        for w in (norm.weight, qkv.weight, gate.weight, gate.bias, out.weight, out.bias, mem):
+        for w in (*weights, mem):
             if w is not None and (w.dtype != bf16 or w.device != device or not w.is_contiguous() or w.data_ptr() % 16):
                 return None
         if not inp.is_contiguous() or inp.data_ptr() % 16:
             inp = inp.clone(memory_format=torch.contiguous_format)
         if residual is not None and not residual.is_contiguous():
             residual = residual.contiguous()
-        if (gate.weight.shape != (3 * self.heads, dim) or freqs.dtype not in (bf16, torch.float32) or not freqs.is_contiguous()
-                or freqs.device != device):
+        if (w_gate.shape != (3 * heads, dim) or freqs.dtype not in (bf16, torch.float32) or not freqs.is_contiguous() or freqs.device != device
+                or w_qkv.shape != (hd + 2 * hk * d, dim) or w_out.shape != (dim, hd) or freqs.shape != (d // 2,) or w_norm.shape != (dim,)
+                or (b_gate is not None and b_gate.shape != (3 * heads,)) or (b_out is not None and b_out.shape != (dim,)) or mem.dim() != 4):
             return None
-        hk = self.kv_heads
-        if (qkv.weight.shape != (hd + 2 * hk * d, dim) or out.weight.shape != (dim, hd) or freqs.shape != (d // 2,)
-                or norm.weight.shape != (dim,) or mem.dim() != 4 or mem.shape[:2] != (2, hk) or mem.shape[3] != d
-                or (gate.bias is not None and gate.bias.shape != (3 * self.heads,)) or (out.bias is not None and out.bias.shape != (dim,))):
+        two, mem_heads, _, mem_d = mem.shape
+        if two != 2 or mem_heads != hk or mem_d != d:
             return None
         # the kernels take batch, heads and lengths from one tensor of each pair
+        lengths = []
         for c, v in ((cache_k, cache_v), (cache_ck, cache_cv), (run_k, run_v)):
-            if c.shape != v.shape or c.dim() != 4 or c.shape[:2] != (b, hk) or c.shape[3] != d:
+            shape = c.shape
+            if shape != v.shape or len(shape) != 4 or c.dtype != bf16 or v.dtype != bf16 or c.device != device or v.device != device:
                 return None
-            if c.dtype != bf16 or v.dtype != bf16 or c.device != device or v.device != device:
+            cb, ch, rows, cd = shape
+            if cb != b or ch != hk or cd != d:
                 return None
+            lengths.append(rows)
+        pos, nc, opened = lengths
         st, cbs, B = self.compress_block_sliding_stride, self.compress_block_size, self.selection_block_size
-        nc, npf = cache_ck.shape[2], B // st
+        npf = B // st
         if min(self.num_selected_blocks, nc // npf) > 64 or nc // npf > 2048 or (nc and not (ops._rows_ok(cache_ck) and ops._rows_ok(cache_cv))):
             return None
         run_k, run_v = _grown(run_k, cbs), _grown(run_v, cbs)
         keys, vals = _grown(cache_k), _grown(cache_v)
         eps = norm.eps
-        layer = ops.DecodeLayer(inp, self.heads, norm.weight, torch.finfo(torch.float32).eps if eps is None else eps, qkv.weight, gate.weight, gate.bias,
-                                out.weight, out.bias, residual)
-        y = ops.decode_step(None, None, None, freqs, cache_k.shape[2], keys, vals, cache_ck if nc else None, cache_cv if nc else None, mem, None,
+        layer = ops.DecodeLayer(inp, heads, w_norm, torch.finfo(torch.float32).eps if eps is None else eps, w_qkv, w_gate, b_gate, w_out, b_out, residual)
+        y = ops.decode_step(None, None, None, freqs, pos, keys, vals, cache_ck if nc else None, cache_cv if nc else None, mem, None,
                             run_k, run_v, None, per_block=npf, block=B, num_sel=self.num_selected_blocks, share=self.query_heads_share_selected_kv,
                             window=self.sliding_window_size, scale=self.scale, layer=layer)[0]
         ck, cv = cache_ck, cache_cv
-        if run_k.shape[2] % cbs == 0:
+        if (opened + 1) % cbs == 0:
             next_ck = self._compress_rows(self.k_compress, run_k + self.k_intrablock_positions)
             next_cv = self._compress_rows(self.v_compress, run_v + self.v_intrablock_positions)
             run_k, run_v = run_k[..., st:, :], run_v[..., st:, :]

@@ -73,14 +73,15 @@ class Transformer(nn.Module):
         plain = SparseAttention._plain
         if (tokens.dtype == torch.bfloat16 and tokens.is_cuda and not torch.is_grad_enabled() and ops.plain_call()
                 and plain(ff, nn.Sequential) and len(ff) == 4):
-            norm, up, act, down = ff
-            if (plain(norm, nn.RMSNorm) and plain(up, nn.Linear) and plain(act, nn.GELU) and plain(down, nn.Linear) and act.approximate == 'none'
-                    and norm.normalized_shape == tuple(tokens.shape[-1:]) and ops.rms_norm_supported(tokens, norm.weight)
-                    and ops.skinny_linear_supported(tokens, up.weight, up.bias, norm.weight)
-                    and ops.skinny_linear_supported(tokens, down.weight, down.bias, width=up.weight.shape[0])):
-                eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
-                hidden = ops._skinny(tokens, up.weight, up.bias, norm.weight, eps, act="gelu")
-                return ops._skinny(hidden, down.weight, down.bias, residual=tokens)
+            norm, up, act, down = ff._modules.values()
+            if plain(norm, nn.RMSNorm) and plain(up, nn.Linear) and plain(act, nn.GELU) and plain(down, nn.Linear) and act.approximate == 'none':
+                # (each parameter is looked up once: see SparseAttention._decode_whole)
+                w_norm, w1, b1, w2, b2 = norm.weight, up.weight, up.bias, down.weight, down.bias
+                if (norm.normalized_shape == tuple(tokens.shape[-1:]) and ops.rms_norm_supported(tokens, w_norm)
+                        and ops.skinny_linear_supported(tokens, w1, b1, w_norm) and ops.skinny_linear_supported(tokens, w2, b2, width=w1.shape[0])):
+                    eps = torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
+                    hidden = ops._skinny(tokens, w1, b1, w_norm, eps, act="gelu")
+                    return ops._skinny(hidden, w2, b2, residual=tokens)
         return ff(tokens) + tokens
 
     def _decode_logits(self, tokens):
