@@ -1902,14 +1902,15 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     return _Linear.apply(x, weight, bias)
 
 
-_GEMM_MACS = 9 << 30
-
-
 def _wgrad_supported(dy2: Tensor, x2: Tensor, dtype) -> bool:
-    """A weight gradient that `nsa_wgrad_bf16` serves.  RULE"""
+    """A weight gradient that `nsa_wgrad_bf16` serves at least as well as the GEMM library (and its bias gradient, a pass of its own, for
+    1 to 2 us).  us on the GPU alone, library sliced by `_wgrad_splits` / this kernel (the library's call takes the host another 15):
+      4080 x 1024 -> 64 30.9 / 10.5, 4080 x 2048 -> 64 31.0 / 12.4, 4080 x 1024 -> 1024 35.0 / 27.1, 8192 x 512 -> 1024 26.2 / 25.6,
+      8192 x 2048 -> 512 33.4 / 34.8, 8192 x 512 -> 2048 35.2 / 35.9, 1000 x 512 -> 512 13.4 / 11.7;
+      above the line 4080 x 2048 -> 2048 (17 G) 55.8 / 58.3, 16384 x 1024 -> 1024 45.6 / 56.4, 16384 x 1024 -> 1536 67.7 / 82.9."""
     rows, n_out, n_in = x2.shape[0], dy2.shape[1], x2.shape[1]
     return bool(x2.dtype == dy2.dtype == dtype == _BF16 and x2.is_cuda and rows > 0 and n_out % 64 == 0 and n_in % 128 == 0
-                and n_out < 1 << 15 and n_in < 1 << 15 and (n_out == 64 or rows * n_out * n_in <= _GEMM_MACS)
+                and n_out < 1 << 15 and n_in < 1 << 15 and (n_out == 64 or rows * n_out * n_in <= 9 << 30)
                 and not torch.is_grad_enabled() and plain_call() and not _in_batch(dy2) and _row_aligned(dy2) and _row_aligned(x2))
 
 
@@ -1960,8 +1961,7 @@ def _plain_mlp(act, eps, residual, norm_w, x, w1, b1, w2, b2):
 class _Mlp(torch.autograd.Function):
     """One or two networks linear - activation - linear of the same sizes in a bf16 module under autograd, each optionally behind an RMS
     norm and with its input added (the feed-forward block, transformer.py:142-152; the compression networks, NSA.py:306-322): every
-    product is this library's kernel with what follows it in the product's epilogue, and a weight gradient comes with its bias's.
-    8 x 1024 tokens, 512 features, us in the layer: feed-forward with norm and residual NN, both compression networks NN."""
+    product is this library's kernel with what follows it in the product's epilogue, and a weight gradient comes with its bias's."""
 
     @staticmethod
     def forward(ctx, act, eps, residual, norm_w, *nets):
@@ -2034,13 +2034,18 @@ class _Mlp(torch.autograd.Function):
 
 
 def mlp_supported(act: str, xs, nets, norm_w: Tensor | None = None) -> bool:
-    """Networks that `mlp` serves; `nets`: (w1, b1, w2, b2) each.  RULE"""
+    """Networks that `mlp` serves better than the separate layers; `nets`: (w1, b1, w2, b2) each.  Forward and backward, us on the GPU alone,
+    layers / node (the host takes 320 / 250 for a feed-forward block and 490 / 270 for two networks):
+      feed-forward with norm and residual, 512 x 512 -> 2048 -> 512 114 / 110, 2048 rows 169 / 136, 8192 351 / 247, 16384 650 / 420;
+      8192 x 1024 -> 4096 -> 1024 (34 G products of a pass) 662 / 660, 4096 rows 381 / 396;
+      two networks, 1016 x 1024 -> 1024 -> 64 131 / 84, 4064 rows 185 / 145, 1016 x 2048 -> 2048 -> 64 185 / 156, 4080 rows (34 G) 380 / 357;
+      above the line 1000 x 4096 -> 4096 -> 128 (34 G) 350 / 408, 2040 rows 528 / 669: the library's larger tiles read the operands less often."""
     x, (w1, _, w2, _) = xs[0], nets[0]
     if not (torch.is_grad_enabled() and x.is_cuda and x.dtype == _BF16 and w1.dim() == 2 and w2.dim() == 2 and plain_call()):
         return False
     k, hidden, out, rows = x.shape[-1], w1.shape[0], w2.shape[0], x.numel() // max(x.shape[-1], 1)
     if not (rows > 0 and k % 128 == 0 and hidden % 128 == 0 and out % 64 == 0 and max(k, hidden, out) < 1 << 15
-            and len(xs) * rows * hidden * max(k, out) <= _GEMM_MACS):
+            and hidden * max(k, out) <= 1 << 22 and len(xs) * rows * hidden * max(k, out) <= 36 << 30):
         return False
     for y, (a, b, c, d) in zip(xs, nets):
         if y.shape != x.shape or y.dtype != _BF16 or y.device != x.device or a.shape != (hidden, k) or c.shape != (out, hidden):
