@@ -76,8 +76,15 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
   const long row_bytes = (long)P.g * P.D * 2;
   long ph = 256;
   while (ph * 2 * row_bytes <= (long)NSA_PHASE_BYTES && ph < (1L << 20)) ph *= 2;
-  P.chunk[0] = 256;  P.phase[0] = (int)ph;
-  P.chunk[1] = 256;  P.phase[1] = (int)(ph > 256 ? ph / 2 : ph);
+  // A unit is a serial chain of its pairs, 32 / group of them at a time, and a short sequence has few blocks: 289 tokens of 2 kv heads
+  // were 30 units of 256 pairs on 1024 SIMDs.  Shorter units where the launch would have under 2048 (a pair's results do not depend on
+  // its unit).  us with index build and merge, 256 pairs / this rule: 289 tokens, 16 / 2 heads, d 128, 15 blocks of 64 128 / 44; 1 x 512,
+  // 8 / 2 heads, 4 of 16 50 / 30; 2000, 16 / 2, d 128 160 / 99; 4 x 1024, 16 / 4 107 / 85; 4096, 16 / 4 116 / 98.  At 4096 units the last two
+  // take 85 and 103, 2 x 687 with 32 / 8 heads 99 instead of 92, 1 x 4000 of d 128 260 instead of 250.
+  long per = 256;
+  while (per > 32 && bh * pairs / per < 2048) per /= 2;
+  P.chunk[0] = (int)per;  P.phase[0] = (int)ph;
+  P.chunk[1] = (int)per;  P.phase[1] = (int)(ph > 256 ? ph / 2 : ph);
   // dK/dV walk: a unit keeps its accumulators for `chunk` pairs and leaves a 2 x 32KT x D fp32 partial behind, so long units
   // are cheaper per pair - but the chip holds 512 to 1024 work-groups of this kernel at a time, and a launch with fewer
   // units than a few rounds of that runs as long as its longest units whatever the rest does (seq 8k, 4 kv heads: 512 units
@@ -85,6 +92,9 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
   {
     const long want = bh * pairs / NSA_DKV_UNITS_WANTED;
     P.chunk[2] = NSA_DKV_CHUNK_FIXED ? NSA_DKV_CHUNK_FIXED : (want >= 1024 ? 1024 : want >= 512 ? 512 : 256);
+    // ... down to 64 pairs while there are under 512 of them: 289 tokens of 16 / 2 heads, d 128 138 / 62 us, 1 x 512 of 8 / 2 49 / 28 and of
+    // d 128 81 / 54, 1200 of 16 / 2, d 128 154 / 107 (units of 32 pairs: 59, 24, 66, 146; under 1024: 1899 of 16 / 4 83 instead of 71)
+    while (P.chunk[2] > 64 && bh * pairs / P.chunk[2] < 512) P.chunk[2] /= 2;
   }
   P.phase[2] = ((P.n + 255) / 256) * 256;
   for (int t = 0; t < 3; ++t) {
