@@ -139,6 +139,10 @@ int nsa_dense_fwd(const nsa_dense_desc* d, const void* q, const void* k, const v
 int nsa_dense_bwd(const nsa_dense_desc* d, const void* q, const void* k, const void* v,
                   const void* out, const void* d_out, const float* lse, void* bwd_ws, size_t bwd_bytes,
                   void* dq, void* dk, void* dv, void* stream);
+/* The same, added to what dq, dk and dv (bf16: not with dkv_fp32) hold, in fp32 with one rounding of the sum. */
+int nsa_dense_bwd_accumulate(const nsa_dense_desc* d, const void* q, const void* k, const void* v,
+                             const void* out, const void* d_out, const float* lse, void* bwd_ws, size_t bwd_bytes,
+                             void* dq, void* dk, void* dv, void* stream);
 
 /* Compressed attention with the block selection made inside the forward kernel.  Replaces, in one launch,
  * attend(q, ck, cv, cmask, return_sim=True) (NSA.py:153-184, 632-639), the importance scores (NSA.py:652-691), the

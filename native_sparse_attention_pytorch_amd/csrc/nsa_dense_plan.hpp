@@ -14,6 +14,7 @@ struct DensePlan {
   int pool, npf, nb, B, share, mask_own, nofill;
   int topk;                  // > 0: the forward selects this many blocks per query itself instead of writing the logits
   int dkv_fp32;              // dk / dv leave the reduce kernel as fp32 instead of bf16
+  int accumulate;            // the backward adds to what dq, dk and dv (bf16) hold
   float scale;
   int key_tiles, chunks, chunk_q;
   long sq[3], sk[3], sv[3], so[3], sdo[3];
@@ -31,6 +32,7 @@ static inline int make_dense_plan(const nsa_dense_desc* d, DensePlan& P) {
   P.b = d->batch; P.hkv = d->kv_heads; P.g = d->group; P.n = d->seq; P.nkeys = d->num_keys; P.mem = d->num_mem;
   P.krows = P.nkeys + P.mem; P.D = d->dim_head; P.mode = d->mode; P.causal = d->causal ? 1 : 0; P.scale = d->scale;
   P.dkv_fp32 = d->dkv_fp32 ? 1 : 0;
+  P.accumulate = 0;
   P.lg = 0;
   while ((1 << P.lg) < P.g) ++P.lg;
   const long bh = (long)P.b * P.hkv;

@@ -409,22 +409,31 @@ def _(q, k, v, mode, causal, window, stride, num_mem, pool, sel_block, share, sc
 @torch.library.custom_op("nsa_amd::dense_bwd", mutates_args=())
 def dense_bwd(q: Tensor, k: Tensor, v: Tensor, out: Tensor, dout: Tensor, lse: Tensor, mode: int, causal: bool, window: int,
               stride: int, num_mem: int, scale: float, dkv_fp32: bool = False) -> tuple[Tensor, Tensor, Tensor]:
+    return _dense_bwd(q, k, v, out, dout, lse, mode, causal, window, stride, num_mem, scale, dkv_fp32)
+
+
+def _dense_bwd(q, k, v, out, dout, lse, mode, causal, window, stride, num_mem, scale, dkv_fp32=False, into=None):
+    """Gradients (dq, dk, dv), in new tensors or added to `into` (contiguous, bf16, of q's, k's and v's shapes)."""
     q, k, v, out = _prep(q), _prep(k), _prep(v), _prep(out)
     dout = _prep(dout if dout.dtype == _BF16 else dout.to(_BF16))
     b, hq, n, d = q.shape
     hk, nk = k.shape[1], k.shape[2]
-    dq = torch.empty((b, hq, n, d), dtype=_BF16, device=q.device)
-    kv_dtype = torch.float32 if dkv_fp32 else _BF16
-    dk = torch.empty((b, hk, nk, d), dtype=kv_dtype, device=q.device)
-    dv = torch.empty((b, hk, nk, d), dtype=kv_dtype, device=q.device)
+    if into is None:
+        dq = torch.empty((b, hq, n, d), dtype=_BF16, device=q.device)
+        kv_dtype = torch.float32 if dkv_fp32 else _BF16
+        dk = torch.empty((b, hk, nk, d), dtype=kv_dtype, device=q.device)
+        dv = torch.empty((b, hk, nk, d), dtype=kv_dtype, device=q.device)
+    else:
+        dq, dk, dv = into
     dsc = _dense_desc(q, k, v, out, dout, mode, causal, window, stride, num_mem, False, 1, True, scale)
     dsc.dkv_fp32 = int(dkv_fp32)
     wb = C.c_size_t()
     L = _lib.lib()
     _lib.check(L.nsa_dense_workspace_bytes(C.byref(dsc), C.byref(wb)), "nsa_dense_workspace_bytes")
     ws = torch.empty(wb.value, dtype=torch.uint8, device=q.device)
-    _lib.check(L.nsa_dense_bwd(C.byref(dsc), _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(dout), _ptr(lse), _ptr(ws), wb.value,
-                               _ptr(dq), _ptr(dk), _ptr(dv), _stream()), "nsa_dense_bwd")
+    call = L.nsa_dense_bwd if into is None else L.nsa_dense_bwd_accumulate
+    _lib.check(call(C.byref(dsc), _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(dout), _ptr(lse), _ptr(ws), wb.value, _ptr(dq), _ptr(dk), _ptr(dv),
+                    _stream()), "nsa_dense_bwd")
     return dq, dk, dv
 
 
@@ -530,6 +539,43 @@ def sliding_attend(q: Tensor, k: Tensor, v: Tensor, window_size: int, causal: bo
     qp, g, gp = _pad_groups(_pad_dim(q, D), k.shape[1])
     out, _, _ = _dense_fwd(qp, _pad_dim(k, D), _pad_dim(v, D), 0, bool(causal), int(window_size), 1, 0, 0, 1, True, float(d ** -0.5))
     return _unpad_groups(out, k.shape[1], g, gp)[..., :d]
+
+
+class _SelectAndSlide(torch.autograd.Function):
+    """The selection and sliding branches of one q, k, v: the sliding backward adds its gradients to the selection's."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, idx, fmask, gates, block, window, scale):
+        out, lse, index_ws = select_fwd._init_fn(q, k, v, idx, fmask, gates, block, True, scale)
+        slid, slid_lse, _ = dense_fwd._init_fn(q, k, v, 0, True, window, 1, 0, 0, 1, True, scale)
+        ctx.save_for_backward(q, k, v, idx, fmask, index_ws, out, lse, slid, slid_lse)
+        ctx.args = (block, window, scale, None if gates is None or not gates.requires_grad else gates.dtype)
+        ctx.set_materialize_grads(False)
+        return out, slid
+
+    @staticmethod
+    def backward(ctx, dout, dslid):
+        q, k, v, idx, fmask, index_ws, out, lse, slid, slid_lse = ctx.saved_tensors
+        block, window, scale, gates = ctx.args
+        into = dgates = None
+        if dout is not None:
+            *into, dsel = select_bwd._init_fn(q, k, v, out, dout, lse, idx, fmask, index_ws, block, True, scale, gates is not None, None)
+            dgates = None if gates is None else dsel.to(gates)
+        if dslid is not None:
+            into = _dense_bwd(q, k, v, slid, dslid, slid_lse, 0, True, window, 1, 0, scale, into=into)
+        return (*((None,) * 3 if into is None else into), None, None, dgates, None, None, None)
+
+
+def select_and_slide(q: Tensor, k: Tensor, v: Tensor, block_size: int, idx: Tensor, fmask: Tensor, gates: Tensor | None, window: int):
+    """(native_sparse_attend(q, k, v, block_size, idx, fmask, gates), sliding_attend(q, k, v, window)) of a causal bf16 module under
+    autograd as one node; None where the two calls do more than one launch of the kernels each."""
+    (b, hq, n, d), hk = q.shape, k.shape[1]
+    g = hq // max(hk, 1)
+    if not (torch.is_grad_enabled() and plain_call() and (q.requires_grad or k.requires_grad or v.requires_grad) and q.dtype == k.dtype == v.dtype == _BF16
+            and d in (64, 128) and hq == g * hk and g & (g - 1) == 0 and idx.shape[1] == hk and block_size <= 64 and idx.shape[-1] <= _MAX_SLOTS
+            and _batch_pieces(b, hk) is None):
+        return None
+    return _SelectAndSlide.apply(q, k, v, idx, fmask, gates, int(block_size), int(window), float(d ** -0.5))
 
 
 def compress_attend(q: Tensor, ck: Tensor, cv: Tensor, num_mem: int, stride: int, causal: bool,

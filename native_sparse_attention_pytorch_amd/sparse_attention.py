@@ -711,10 +711,13 @@ class SparseAttention(nn.Module):
             rq16, rk16 = ops.rotary_pair(q.to(bf16), k.to(bf16), self.rotary_emb.freqs)
             v16 = v.to(bf16)
 
+        both = None
         if num_sel > 0:
             # straight-through gates (NSA.py:715): value 1, gradient flows into the importance scores
             gates = (vals + (1. - vals).detach()) if self.use_diff_topk else None
-            f_out = ops.native_sparse_attend(rq16, rk16, v16, B, idx, fmask, sel_scale=gates, include_block_causal=self.causal)
+            both = ops.select_and_slide(rq16, rk16, v16, B, idx, fmask, gates, self.sliding_window_size) if self.causal else None
+            if both is None:
+                f_out = ops.native_sparse_attend(rq16, rk16, v16, B, idx, fmask, sel_scale=gates, include_block_causal=self.causal)
         elif self.causal:
             # nothing selectable: block-diagonal causal attention (NSA.py:821-837)
             idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=inp.device)
@@ -725,7 +728,10 @@ class SparseAttention(nn.Module):
             f_out = ops.native_sparse_attend(rq16, rk16, v16, B, own.contiguous(), torch.ones_like(own, dtype=torch.bool),
                                              include_block_causal=False)
 
-        s_out = ops.sliding_attend(rq16, rk16, v16, self.sliding_window_size, causal=self.causal)
+        if both is None:
+            s_out = ops.sliding_attend(rq16, rk16, v16, self.sliding_window_size, causal=self.causal)
+        else:
+            f_out, s_out = both
 
         if logits is None:
             logits = self._linear(self.to_strategy_combine[0], x)

@@ -1,0 +1,53 @@
+"""The selection and sliding branches as one node whose backward sums their gradients in the kernels (nsa_dense_bwd_accumulate), against the
+two branches by themselves."""
+
+import pytest
+import torch
+
+from tests.util import causal_random_selection
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# ragged lengths, one tile, both head widths, groups of 1 and 8, a window longer than the sequence
+@pytest.mark.parametrize("b,hq,hk,n,d,B,S,window,gated", [(2, 4, 2, 200, 64, 16, 3, 7, False), (1, 8, 1, 333, 128, 64, 2, 64, True), (1, 2, 2, 64, 64, 32, 1, 500, True),
+                                                         (2, 8, 4, 1030, 64, 16, 4, 64, False), (1, 4, 2, 1, 128, 16, 1, 3, False)])
+def test_gradients_are_the_sum_of_the_branches(b, hq, hk, n, d, B, S, window, gated):
+    """The separate branches' gradients are each rounded to bf16 and added in bf16, the node's are one of them rounded plus the other in
+    fp32 with one rounding: they differ by at most the other's rounding and those of the two sums, 2^-9 of each value's magnitude."""
+    from native_sparse_attention_pytorch_amd import ops
+    print(b, hq, hk, n, d, B, S, window, flush=True)
+    g = torch.Generator().manual_seed(n)
+    r = lambda h: (torch.randn(b, h, n, d, generator=g) * d ** -0.25).to(DEV, torch.bfloat16)
+    q, k, v = (t.requires_grad_() for t in (r(hq), r(hk), r(hk)))
+    douts = [r(hq), r(hq)]
+    idx, live = (t.to(DEV) for t in causal_random_selection(b, hk, n, B, S, seed=5))
+    gates = torch.ones(idx.shape, device=DEV, requires_grad=True) if gated else None
+    leaves = [q, k, v] + ([gates] if gated else [])
+    both = ops.select_and_slide(q, k, v, B, idx, live, gates, window)
+    alone = ops.native_sparse_attend(q, k, v, B, idx, live, sel_scale=gates), ops.sliding_attend(q, k, v, window)
+    assert all(torch.equal(x, y) for x, y in zip(both, alone))
+    first = torch.autograd.grad(alone[0], leaves, douts[0], retain_graph=True)
+    second = torch.autograd.grad(alone[1], leaves[:3], douts[1], retain_graph=True)
+    got = torch.autograd.grad(both, leaves, douts, retain_graph=True)
+    for x, s, t in zip(got, first, second):
+        s, t = s.float(), t.float()
+        assert ((x.float() - (s + t)).abs() <= 2 ** -8 * ((s + t).abs() + t.abs()) + 1e-30).all()
+    if gated:
+        assert torch.equal(got[3], first[3])
+    # either branch by itself
+    assert all(torch.equal(x, y) for x, y in zip(torch.autograd.grad(both[0], leaves, douts[0], retain_graph=True), first))
+    assert all(torch.equal(x, y) for x, y in zip(torch.autograd.grad(both[1], leaves[:3], douts[1]), second))
+
+
+def test_what_the_node_does_not_take():
+    from native_sparse_attention_pytorch_amd import ops
+    z = lambda h, d=64: torch.zeros(1, h, 32, d, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    idx = torch.zeros(1, 2, 32, 1, device=DEV, dtype=torch.int64)
+    call = lambda q, k, B=16, i=idx: ops.select_and_slide(q, k, k, B, i, i.bool(), None, 8)
+    assert call(z(4), z(2)) is not None
+    assert call(z(6), z(2)) is None and call(z(4, 32), z(2, 32)) is None and call(z(4), z(2), B=128) is None
+    assert call(z(4), z(2), i=idx.repeat_interleave(2, 1)) is None and call(z(4).float(), z(2).float()) is None
+    with torch.no_grad():
+        assert call(z(4), z(2)) is None
