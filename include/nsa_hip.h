@@ -34,6 +34,9 @@ int nsa_abi_version(void);
  * A[32x16] * B[16x32] (row-major bf16) and T[32x32] = X[32x32] (bf16) passed through the
  * identity-operand register transpose.  No reference counterpart (Triton hides layouts). */
 int nsa_selftest_mfma(const void* A, const void* B, float* C, const void* X, float* T, void* stream);
+/* The order in which the fp32 tile kernel's work-groups take `tiles` tiles of `pairs` (batch, kv head) pairs, on the host:
+ * out[id] = pair * tiles + tile of work-group id, each of them once. */
+int nsa_selftest_f32_tiles(int32_t pairs, int32_t tiles, int32_t* out);
 
 /* Memory-system probe with the access pattern of the block-selection walks (no reference counterpart; used by
  * bench.py to state the ceiling next to the walks' achieved GB/s).  `waves` wavefronts each repeat `iters` times:

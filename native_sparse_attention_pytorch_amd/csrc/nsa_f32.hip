@@ -404,6 +404,15 @@ __global__ __launch_bounds__(256, 2) void f32_rows_pair_kernel(const RowsCall X,
 // products instead of once per 2.
 constexpr int kTileBlocks = 128;         // blocks of a masked selection
 
+// Which tile of 128 rows of which (batch, kv head) pair a work-group takes.  Longest key lists first (causal prefixes).  Where the
+// launch fits the chip at two work-groups to a CU, the second half goes the other way round: the longest then shares its CU with the
+// shortest.  (The ids are turned, not the tiles: a pair's tiles may lie on both sides of id 256.)
+struct TilePlace { int pair, tile; };
+__host__ __device__ inline TilePlace f32_tile_place(int id, int grid, int pairs) {
+  if (grid <= 512 && id >= 256) id = 255 + grid - id;
+  return TilePlace{id % pairs, grid / pairs - 1 - id / pairs};
+}
+
 __device__ __forceinline__ void split_probs(const float (&p)[16], bf16x8 (&part)[3][2]) {
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
@@ -433,15 +442,12 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
   __shared__ uint32_t mask_s[SEL ? 129 : 1][kTileBlocks / 32], any_s[kTileBlocks / 32];
   __shared__ int repeated_s, big_s;                      // big_s: some key was that large (it stays set)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n_ = lane & 31, h = lane >> 5;
-  // Longest key lists first (causal prefixes).  Where the launch fits the chip at two work-groups to a CU, the second half goes the
-  // other way round: the longest then shares its CU with the shortest.
-  const int tiles = gridDim.x / A.bh, nth = blockIdx.x / A.bh;
-  const int turned = gridDim.x <= 512 && (int)blockIdx.x >= 256 ? 256 / A.bh + tiles - 1 - nth : nth;
-  const int bh = blockIdx.x % A.bh, b = bh / A.hk, hk = bh % A.hk;
+  const TilePlace at = f32_tile_place(blockIdx.x, gridDim.x, A.bh);
+  const int b = at.pair / A.hk, hk = at.pair % A.hk;
   const float* kb = k + b * A.sk[0] + hk * A.sk[1];
   const float* vb = v + b * A.sv[0] + hk * A.sv[1];
   const long all_rows = (long)A.n * A.g;
-  const long row0 = (long)(tiles - 1 - turned) * 128;
+  const long row0 = (long)at.tile * 128;
   const long row = row0 + wave * 32 + n_;
   const long rowc = row < all_rows ? row : all_rows - 1;
   const int qi = (int)(rowc / A.g), g = (int)(rowc - (long)qi * A.g);
@@ -471,7 +477,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
 
   unsigned long long any0 = 0, any1 = 0;                 // blocks that some row of the work-group attends
   bool repeated = false;
-  const size_t slot0 = SEL ? ((size_t)bh * A.n + gq0) * A.S : 0;
+  const size_t slot0 = SEL ? ((size_t)at.pair * A.n + gq0) * A.S : 0;
   auto block_of = [&](size_t at) {
     if (!fmask[at]) return -1;
     const long j = A.idx64 ? (long)reinterpret_cast<const long long*>(idx)[at] : (long)reinterpret_cast<const int*>(idx)[at];
@@ -870,6 +876,15 @@ extern "C" int nsa_compress_fwd_f32(const nsa_dense_desc* d, const float* q, con
   if (!d || d->mode != 1 || d->num_mem <= 0 || !mem_k || !mem_v || ((reinterpret_cast<uintptr_t>(mem_k) | reinterpret_cast<uintptr_t>(mem_v)) & 15))
     return NSA_E_ARG;
   return dense_fwd_f32(d, q, k, v, mem_k, mem_v, out, lse, q_offset, stream);
+}
+
+extern "C" int nsa_selftest_f32_tiles(int32_t pairs, int32_t tiles, int32_t* out) {
+  if (!out || pairs <= 0 || tiles <= 0) return NSA_E_ARG;
+  for (int id = 0; id < pairs * tiles; ++id) {
+    const TilePlace at = f32_tile_place(id, pairs * tiles, pairs);
+    out[id] = at.pair * tiles + at.tile;
+  }
+  return 0;
 }
 
 extern "C" int nsa_compress_window_fwd_f32(const nsa_dense_desc* dc, const float* q, const float* ck, const float* cv, const float* mem_k, const float* mem_v,
