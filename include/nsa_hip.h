@@ -35,8 +35,8 @@ int nsa_abi_version(void);
  * identity-operand register transpose.  No reference counterpart (Triton hides layouts). */
 int nsa_selftest_mfma(const void* A, const void* B, float* C, const void* X, float* T, void* stream);
 /* The order in which the fp32 tile kernel's work-groups take `tiles` tiles of `pairs` (batch, kv head) pairs, on the host:
- * out[id] = pair * tiles + tile of work-group id, each of them once. */
-int nsa_selftest_f32_tiles(int32_t pairs, int32_t tiles, int32_t* out);
+ * out[id] = pair * tiles + tile of work-group id, each of them once.  two_to_a_cu: a CU holds two (dim_head up to 64). */
+int nsa_selftest_f32_tiles(int32_t pairs, int32_t tiles, int32_t two_to_a_cu, int32_t* out);
 
 /* Memory-system probe with the access pattern of the block-selection walks (no reference counterpart; used by
  * bench.py to state the ceiling next to the walks' achieved GB/s).  `waves` wavefronts each repeat `iters` times:

@@ -80,7 +80,7 @@ def lib():
         L.nsa_select_bwd.argtypes = [C.POINTER(SelectDesc)] + [vp] * 11 + [sz] + [vp] * 5
         L.nsa_selftest_mfma.argtypes = [vp] * 6
         L.nsa_selftest_mfma.restype = C.c_int
-        L.nsa_selftest_f32_tiles.argtypes = [C.c_int32, C.c_int32, vp]
+        L.nsa_selftest_f32_tiles.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp]
         L.nsa_selftest_f32_tiles.restype = C.c_int
         L.nsa_gemm_f32.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, C.c_int64, vp, vp, C.c_int32, vp, vp, vp, vp, vp, vp]
         L.nsa_gemm_f32.restype = C.c_int

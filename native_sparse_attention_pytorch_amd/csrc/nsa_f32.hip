@@ -406,10 +406,12 @@ constexpr int kTileBlocks = 128;         // blocks of a masked selection
 
 // Which tile of 128 rows of which (batch, kv head) pair a work-group takes.  Longest key lists first (causal prefixes).  Where the
 // launch fits the chip at two work-groups to a CU, the second half goes the other way round: the longest then shares its CU with the
-// shortest.  (The ids are turned, not the tiles: a pair's tiles may lie on both sides of id 256.)
+// shortest (1 x 4096 queries, 16 heads x 4 kv heads, d = 64: window of all 268 -> 258 us, strided prefix 27.9 -> 27.2, masked
+// selection 296 -> 291).  At d = 128 a CU holds one, and the second half starts where the first ends: longest first there, too (1 x
+// 2000 queries, 32 x 8 heads, turned 300 us, not 242).  The ids are turned, not the tiles: a pair's tiles may lie on both sides of id 256.
 struct TilePlace { int pair, tile; };
-__host__ __device__ inline TilePlace f32_tile_place(int id, int grid, int pairs) {
-  if (grid <= 512 && id >= 256) id = 255 + grid - id;
+__host__ __device__ inline TilePlace f32_tile_place(int id, int grid, int pairs, bool two_to_a_cu) {
+  if (two_to_a_cu && grid <= 512 && id >= 256) id = 255 + grid - id;
   return TilePlace{id % pairs, grid / pairs - 1 - id / pairs};
 }
 
@@ -442,7 +444,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
   __shared__ uint32_t mask_s[SEL ? 129 : 1][kTileBlocks / 32], any_s[kTileBlocks / 32];
   __shared__ int repeated_s, big_s;                      // big_s: some key was that large (it stays set)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n_ = lane & 31, h = lane >> 5;
-  const TilePlace at = f32_tile_place(blockIdx.x, gridDim.x, A.bh);
+  const TilePlace at = f32_tile_place(blockIdx.x, gridDim.x, A.bh, D == 64);
   const int b = at.pair / A.hk, hk = at.pair % A.hk;
   const float* kb = k + b * A.sk[0] + hk * A.sk[1];
   const float* vb = v + b * A.sv[0] + hk * A.sv[1];
@@ -878,10 +880,10 @@ extern "C" int nsa_compress_fwd_f32(const nsa_dense_desc* d, const float* q, con
   return dense_fwd_f32(d, q, k, v, mem_k, mem_v, out, lse, q_offset, stream);
 }
 
-extern "C" int nsa_selftest_f32_tiles(int32_t pairs, int32_t tiles, int32_t* out) {
+extern "C" int nsa_selftest_f32_tiles(int32_t pairs, int32_t tiles, int32_t two_to_a_cu, int32_t* out) {
   if (!out || pairs <= 0 || tiles <= 0) return NSA_E_ARG;
   for (int id = 0; id < pairs * tiles; ++id) {
-    const TilePlace at = f32_tile_place(id, pairs * tiles, pairs);
+    const TilePlace at = f32_tile_place(id, pairs * tiles, pairs, two_to_a_cu != 0);
     out[id] = at.pair * tiles + at.tile;
   }
   return 0;

@@ -13,24 +13,26 @@ from tests.util import assert_close
 DEV = "cuda"
 
 
-def _order(pairs, tiles):
+def _order(pairs, tiles, two=True):
     from native_sparse_attention_pytorch_amd import _lib
     out = (C.c_int32 * (pairs * tiles))()
-    assert _lib.lib().nsa_selftest_f32_tiles(pairs, tiles, out) == 0
+    assert _lib.lib().nsa_selftest_f32_tiles(pairs, tiles, two, out) == 0
     return list(out)
 
 
-def test_each_tile_once():
+@pytest.mark.parametrize("two", [True, False])
+def test_each_tile_once(two):
     for pairs in range(1, 521):
         for tiles in range(1, 520 // pairs + 1):
-            assert sorted(_order(pairs, tiles)) == list(range(pairs * tiles)), (pairs, tiles)
+            assert sorted(_order(pairs, tiles, two)) == list(range(pairs * tiles)), (pairs, tiles)
 
 
 def test_longest_first_and_in_pairs():
     """The last tiles, whose key lists are the longest, come first; work-groups 256 apart share a CU, and the two together have as long a
-    walk everywhere, to one tile."""
+    walk everywhere, to one tile.  Where a CU holds one, the order is not turned."""
     assert [t % 24 for t in _order(12, 24)[:24:12]] == [23, 22]
     assert {o % 32 + p % 32 for o, p in zip(_order(16, 32)[:256], _order(16, 32)[256:])} <= {30, 31, 32}
+    assert [t % 32 for t in _order(16, 32, False)] == [31 - i // 16 for i in range(512)]
     assert [t % 60 for t in _order(10, 60)] == [59 - i // 10 for i in range(600)]
 
 
