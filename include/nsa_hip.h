@@ -319,7 +319,7 @@ int nsa_gate_linear_f32(int32_t batch, int32_t heads, int32_t seq, int32_t dim_h
                         int32_t n, float* y, void* stream);
 
 /* y = x weight^T + bias (relu: its positive part) in fp32 for many rows, on the bf16 matrix instructions with the operands split in
- * three (see nsa_gemm.hip; the sums are at least as exact as fp32 fused multiply-adds): x [m, k] with row stride x_row_stride, weight
+ * three (see nsa_split.hpp; for operands above 2^-110 the sums are at least as exact as fp32 fused multiply-adds): x [m, k] with row stride x_row_stride, weight
  * [n, k] contiguous, bias (optional) [n], y [m, n] contiguous.  x2, weight2, bias2, y2: a second product of the same sizes in the
  * same launch, or all NULL.  k and the row stride multiples of 4 below 2^24, x and weight 16-byte aligned (NSA_E_ARG otherwise). */
 int nsa_gemm_f32(int32_t m, int32_t k, int32_t n, const float* x, int64_t x_row_stride, const float* weight, const float* bias, int32_t relu,

@@ -397,11 +397,10 @@ __global__ __launch_bounds__(256, 2) void f32_rows_pair_kernel(const RowsCall X,
 // Interval masks, and (SEL) block selections of few enough blocks: every tile of a block that one of the 128 rows selected is
 // multiplied and a row's own choice is a mask on the scores, which beats gathering while a query attends a fair share of the
 // blocks there are (f32_masked_tiles).
-// Per tile and wave at d = 64 48 MFMAs (1536 cycles) and some 450 vector instructions (the split of K, V and P 230, softmax 160),
-// of which two waves to a SIMD hide part of each other; a wave alone takes 2.4 us.  Against v_mfma_f32_32x32x2 tiles (64 MFMAs of 64
-// cycles): 2 x 2053 queries, 16 heads x 4 kv heads, window 512 117 -> 68 us, strided prefix 38 -> 28; 32 x 8 heads, d = 128, 2000 queries
-// 204 -> 152.  Error of the outputs against float64 1.6e-7 instead of 3.8e-7 (window 512): each row's sums are rounded once per 16
-// products instead of once per 2.
+// Per tile and wave at d = 64 64 MFMAs (2048 cycles) and some 450 vector instructions (the split of K, V and P 230, softmax 160),
+// of which two waves to a SIMD hide part of each other; a wave alone takes 2.6 us.  Against v_mfma_f32_32x32x2 tiles (64 MFMAs of 64
+// cycles): 2 x 2053 queries, 16 heads x 4 kv heads, window 512 110 -> 72 us, strided prefix 34 -> 28; 32 x 8 heads, d = 128, 2000 queries
+// 181 -> 155.  Error of the outputs against float64, rms: window 512 3.9e-8 -> 1.6e-8, two keys 6.6e-8 -> 4.6e-8.
 constexpr int kTileBlocks = 128;         // blocks of a masked selection
 
 // Which tile of 128 rows of which (batch, kv head) pair a work-group takes.  Longest key lists first (causal prefixes).  Where the
@@ -661,7 +660,9 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
       small = mfma32(kk[0], qf[2][ks], small);
       small = mfma32(kk[1], qf[0][ks], small);
       small = mfma32(kk[1], qf[1][ks], small);
+      small = mfma32(kk[1], qf[2][ks], small);
       small = mfma32(kk[2], qf[0][ks], small);
+      small = mfma32(kk[2], qf[1][ks], small);
     }
     read_v(0);
     if (q_big || __builtin_amdgcn_readfirstlane(overflows)) {
@@ -724,7 +725,9 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
       os[ft] = mfma32(vv[0], pf[2][u], os[ft]);
       os[ft] = mfma32(vv[1], pf[0][u], os[ft]);
       os[ft] = mfma32(vv[1], pf[1][u], os[ft]);
+      os[ft] = mfma32(vv[1], pf[2][u], os[ft]);
       os[ft] = mfma32(vv[2], pf[0][u], os[ft]);
+      os[ft] = mfma32(vv[2], pf[1][u], os[ft]);
     }
   }
   // A value that is not finite is left out of the products, where a weight of zero times it would be NaN in every row of its tile,
@@ -808,24 +811,26 @@ static void f32_launch_tiles(const F32Args& A, const float* q, const float* k, c
 }
 
 // A work-group of the tile kernel needs some 128 rows, and the launch enough of them.  Interval masks, us row by row / in tiles:
-//   d = 64   2048 queries 38.9 / 37.8 (window 512), 15.2 / 16.2 (64); 4096 81 / 42 and 22 / 16; 2048 queries ungrouped 21 / 23
-//   d = 128   496 queries 21.3 / 17.4, 1024 27.6 / 26.2 (window 512), 19.8 / 19.9 (2); 4096 168 / 67 and 54 / 21
+//   d = 64   2048 queries, 16 / 4 heads 38 / 42 (window 512), 12.8 / 14.6 (64); 4096 76 / 45 and 22 / 16; 3072 59 / 44 and 21 / 15, window 2 12 / 13;
+//            8 / 8 heads 2048 20.5 / 24.7 and 10.6 / 20.4, 4096 56 / 41 and 19 / 20.5
+//   d = 128  32 / 8 heads 512 queries 21 / 21, 768 40 / 25, 1024 27.6 / 27.7 (window 512), 20 / 21 (2); 2048 58 / 42 and 28 / 21
 static bool f32_tiles_fit(const F32Args& A) {
   return (long)A.n * A.g >= 128 && (long)A.n * A.b * A.hk >= (A.d <= 64 ? 4096 : 512);
 }
 
 // Masked tiles instead of gathered blocks, where the blocks fit the masks and the estimate of the time (us) is lower:
-//   tiles   a work-group's walk to the last key, 2.4 us per 32 keys (d = 128: 5), or the chip's rate over all rows and half the keys
+//   tiles   a work-group's walk to the last key, 2.5 us per 32 keys (d = 128: 5), or the chip's rate over all rows and half the keys
 //   gather  per query (four heads at a time) 1.4 ns (4.6) for 64 keys of its blocks + 3 (12)
-// Measured, gather / tiles: 16 blocks of 64, d = 64, G 4: 2 x 2053 queries x 4 441 / 159, 1024 x 4 103 / 77, 8192 x 4 984 / 782; 4 blocks of 16, G 2:
-// 8 x 1024 x 4 155 / 84, 4 x 1024 x 4 83 / 79, 1024 x 4 29 / 78, 4 x 2048 x 4 156 / 151; d = 128, 16 of 64: 2048 x 8 1303 / 338; 4 of 16: 2048 x 8 297 / 321.
+// Measured, gather / tiles: 16 blocks of 64, d = 64, G 4: 2 x 2053 queries x 4 451 / 183, 1024 x 4 99 / 85, 8192 x 4 979 / 882; 4 blocks of 64, G 1 4000 x 8
+// 328 / 306; 4 blocks of 16, G 2: 8 x 1024 x 4 154 / 90, 4 x 1024 x 4 82 / 86, 2 x 1024 x 4 45 / 85, 4 x 2048 x 4 157 / 165; d = 128, 16 of 64: 2048 x 8 1301 / 314;
+// 4 of 16: 2048 x 8 297 / 298; 4 of 64: 8192 x 8 2351 / 3381.
 static bool f32_masked_tiles(F32Args& A) {
   A.lb = 0;
   while (A.lb < 30 && (1 << A.lb) < A.B) ++A.lb;
   if (!A.causal || A.B < 4 || A.B != 1 << A.lb || A.W > kTileBlocks || !f32_tiles_fit(A)) return false;
   const bool wide = A.d > 64;
   const double queries = (double)A.n * A.b * A.hk, keys = (double)(A.S + 1) * A.B;
-  const double tiles = std::max(A.nk * (wide ? 0.16 : 0.075), queries * A.g * A.nk * (wide ? 1.9e-6 : 0.73e-6));
+  const double tiles = std::max(A.nk * (wide ? 0.16 : 0.079), queries * A.g * A.nk * (wide ? 1.9e-6 : 0.8e-6));
   const double gather = queries * ((A.g + 3) / 4) * (wide ? 0.0046 * keys / 64 + 0.012 : 0.0014 * keys / 64 + 0.003);
   return tiles < gather;
 }

@@ -1879,15 +1879,18 @@ def _few_rows_f32(x: Tensor, weight: Tensor, bias: Tensor | None, act: str | Non
 
 
 def gemm_f32_supported(x: Tensor, weight: Tensor, bias: Tensor | None = None, products: int = 1) -> bool:
-    """An fp32 projection, or two of the same sizes in one launch, that `nsa_gemm_f32` serves better than the GEMM library: from one
-    tile of 128 x 128 to a CU on.  us, library / this kernel (the fp32 matrix instructions end at 154 TFLOP/s):
-      4106 x 1024 -> 1536 (396 tiles) 144 / 90, 16384 x 1024 -> 1536 396 / 281, 8192 x 512 -> 1024 70 / 56, 2053 x 4096 -> 4096 562 / 481,
-      8192 x 4096 -> 6144 2747 / 2100; at the line 8192 x 512 -> 512 (256) 38 / 36, 4106 x 1024 -> 1024 (264) 93 / 84;
-      below it 500 x 4096 -> 6144 (192) 200 / 175 but 1024 x 2048 -> 2048 (128) 69 / 94, 2048 x 1024 -> 1024 (128) 35 / 51;
-      two of 1024 x 2048 -> 2048 137 / 104, two of 2048 x 1024 -> 1024 70 / 57."""
+    """An fp32 projection, or two of the same sizes in one launch, that `nsa_gemm_f32` serves better than the GEMM library, by the number of
+    its 128 x 128 tiles: two of them fit a CU, and a first or second round of few leaves most of the chip idle.  us, library / this kernel
+    (the fp32 matrix instructions end at 154 TFLOP/s):
+      4106 x 1024 -> 1536 (396 tiles) 126 / 99, 8192 x 512 -> 1024 (512) 65 / 63, 2053 x 4096 -> 4608 (612) 617 / 580, 16384 x 1024 -> 1536 362 / 319,
+      8192 x 4096 -> 6144 2736 / 2459; below 352 4106 x 1024 -> 1024 (264) 82 / 91, 2560 x 1024 -> 2048 (320) 87 / 94, 8192 x 512 -> 512 (256) 35 / 37.5
+      (but 8192 x 512 -> 576 62 / 53); between 512 and 608 2304 x 4096 -> 4096 (576) 542 / 573, 4352 x 1024 -> 2048 (544) 163 / 153;
+      two of 1024 x 2048 -> 2048 (256) 132 / 114, two of 2048 x 1024 -> 1024 (256) 76 / 63, two of 4064 x 1024 -> 1024 (512) 141 / 113;
+      up to 64 features, bound by the results, 33000 -> 128 (258) 18.9 / 17.8, 9000 -> 512 (284) 30 / 18."""
     rows, k = x.numel() // max(x.shape[-1], 1), x.shape[-1]
-    return bool(x.is_cuda and x.dtype == torch.float32 and k % 4 == 0 and 4 <= k < 1 << 24
-                and products * -(-rows // 128) * -(-weight.shape[0] // 128) >= 256
+    tiles = products * -(-rows // 128) * -(-weight.shape[0] // 128)
+    many = tiles >= 256 if products > 1 or k <= 64 else 352 <= tiles <= 512 or tiles >= 608
+    return bool(x.is_cuda and x.dtype == torch.float32 and k % 4 == 0 and 4 <= k < 1 << 24 and many
                 and _weight_ready(x, k, weight) and _vectors_ready(x, weight, bias, None) and (bias is None or bias.is_contiguous())
                 and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
