@@ -554,7 +554,11 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
   floatx16 o[FT], os[FT];                                // sums of leading and of small products
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) { o[ft] = zero_acc(); os[ft] = zero_acc(); }
-  const float c = fmaxf(fabsf(A.scale) * kLog2e, 1e-37f);      // weights are powers of two of (score - maximum) c (a scale of 0: no 0 x inf)
+  // Weights are powers of two of (score - maximum) (c + c_lo), scale x log2 e in two parts: the rounding of c alone would change every
+  // weight of a row the same way.  c is cut off, so that c_lo is positive and a score of minus infinity stays one (a scale of 0 as well).
+  const float scale = fabsf(A.scale), c = fmaxf(scale * kLog2e * (1.f - 0x1p-22f), 1e-37f);
+  const float c_lo = fmaxf(__builtin_fmaf(scale, kLog2e, -c) + scale * 1.925963e-8f, 2e-38f);
+  auto weight = [&](float below) { return fast_exp2(__builtin_fmaf(below, c_lo, below * c)); };
   float m = -INFINITY, l = 0.f;                          // m: of the unscaled scores
 
   const int own_mem = A.memk != nullptr ? A.mem : 0;
@@ -682,10 +686,10 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
       }
     }
     tmax = halves_max(tmax);
-    // (the reference of a row's weights follows its maximum only when that has grown by more than 2^8: weights up to 256 are as
-    // exact as those up to 1, and nearly every tile spares the multiplication of the sums)
-    const float mn = (tmax - m) * c > 8.f ? tmax : m, mref = mn == -INFINITY ? 0.f : mn;
-    const float alpha = fast_exp2((m - mref) * c);       // m = -inf: 0
+    // (a reference that lags behind the maximum would spare most tiles the multiplication of the sums, 1 to 4 % of the time, but weights
+    // above 1 carry large values over the end of fp32, and the lse of 512 keys was 3.4e-7 off in the mean, not 2.8e-7)
+    const float mn = fmaxf(m, tmax), mref = mn == -INFINITY ? 0.f : mn;
+    const float alpha = weight(m - mref);                // m = -inf: 0
     m = mn;
     float ps = 0.f;
     if (SEL && repeated) {
@@ -698,13 +702,13 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void f32_tile_kernel(const F3
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float w = (float)(times + ((unsigned)(from_lo + 8 * a + e) <= seen ? 1 : 0));
-          sv[4 * a + e] = w > 0.f ? w * fast_exp2((sv[4 * a + e] - mref) * c) : 0.f;
+          sv[4 * a + e] = w > 0.f ? w * weight(sv[4 * a + e] - mref) : 0.f;
           ps += sv[4 * a + e];
         }
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) { sv[i] = fast_exp2((sv[i] - mref) * c); ps += sv[i]; }
+      for (int i = 0; i < 16; ++i) { sv[i] = weight(sv[i] - mref); ps += sv[i]; }
     }
     l = l * alpha + ps;                                  // this half's keys
     if (__any(alpha != 1.0f)) {
