@@ -32,8 +32,6 @@ struct F32Args {
   int S, B, W, idx64, uniform, lb;      // lb: log2 of the block, where it is a power of two
 };
 
-__device__ __forceinline__ floatx16 mfma32x2(float a, float b, floatx16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-
 // First and last key row (memory slots included, they are always visible) that the query at `pos` sees
 __device__ __forceinline__ void f32_interval(const F32Args& A, int pos, int& lo, int& hi) {
   if (A.mode == 0) { lo = max(0, pos - A.wb); hi = min(A.nk - 1, pos + A.wf); }
