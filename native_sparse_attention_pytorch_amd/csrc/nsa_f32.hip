@@ -816,8 +816,13 @@ static void f32_launch_tiles(const F32Args& A, const float* q, const float* k, c
 //   d = 64   2048 queries, 16 / 4 heads 38 / 42 (window 512), 12.8 / 14.6 (64); 4096 76 / 45 and 22 / 16; 3072 59 / 44 and 21 / 15, window 2 12 / 13;
 //            8 / 8 heads 2048 20.5 / 24.7 and 10.6 / 20.4, 4096 56 / 41 and 19 / 20.5
 //   d = 128  32 / 8 heads 512 queries 21 / 21, 768 40 / 25, 1024 27.6 / 27.7 (window 512), 20 / 21 (2); 2048 58 / 42 and 28 / 21
+//            narrow windows of groups of 1 and 2, 1024 to 2048 queries: 8 / 8 heads, 1024 18 / 28 (2 to 32), 26 / 28 (64), 2048 22 / 32 (2), 26 / 32 (32), 34 / 36
+//            (64); 16 / 8 heads, 1024 20 / 25 (2 to 32); but 768 31 / 23 (2), 3200 40 / 32 (2)
 static bool f32_tiles_fit(const F32Args& A) {
-  return (long)A.n * A.g >= 128 && (long)A.n * A.b * A.hk >= (A.d <= 64 ? 4096 : 512);
+  const long queries = (long)A.n * A.b * A.hk;
+  if ((long)A.n * A.g < 128 || queries < (A.d <= 64 ? 4096 : 512)) return false;
+  const bool narrow = A.B == 0 && A.mode == 0 && A.g <= 2 && A.wb < 48 && A.wf < 48;      // (a window, not a selection)
+  return !(A.d > 64 && narrow && queries >= 1024 && queries <= 2048);
 }
 
 // Masked tiles instead of gathered blocks, where the blocks fit the masks and the estimate of the time (us) is lower:

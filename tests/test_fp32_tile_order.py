@@ -88,3 +88,15 @@ def test_every_row_is_written(b, hq, hk, n, d, monkeypatch):
     seen = seen + ((j // B == i // B) & (j <= i)).double()
     for name, got, ref in zip(("out", "lse"), (f_out, f_lse), _attention(rq, k, v, seen.repeat_interleave(hq // hk, 1))):
         assert_close(got, ref, 1e-5, 1e-5, "selected blocks, " + name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,hq,hk,n,window,causal", [(1, 8, 8, 127, 3, True), (1, 8, 8, 128, 2, True), (2, 16, 8, 128, 47, False), (1, 8, 8, 256, 48, True), (1, 8, 8, 257, 5, False)])
+def test_narrow_windows_of_ungrouped_heads(b, hq, hk, n, window, causal):
+    """Both sides of the lines between rows and tiles at 128 features."""
+    from native_sparse_attention_pytorch_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n)
+    q, k, v = (torch.randn(b, h, n, 128, generator=g, device=DEV) for h in (hq, hk, hk))
+    for name, got, ref in zip(("out", "lse"), ops.dense_attend_f32(q, k, v, 0, causal, window),
+                              _attention(q, k, v, _visible(0, n, n, 0, window, 1, causal).double())):
+        assert_close(got, ref, 1e-5, 1e-5, name)
