@@ -2016,11 +2016,11 @@ class _Mlp(torch.autograd.Function):
     def forward(ctx, act, eps, residual, norm_w, *nets):
         nets = [nets[i:i + 5] for i in range(0, len(nets), 5)]
         k = nets[0][0].shape[-1]
-        x2 = [net[0].reshape(-1, k).contiguous() for net in nets]
+        x2 = [_laid_out(net[0].reshape(-1, k)) for net in nets]
         nw = rstd = None
         xn = x2
         if norm_w is not None:
-            nw = norm_w.detach().contiguous()
+            nw = _laid_out(norm_w.detach())
             y, rstd = _rms_fwd(x2[0], nw, eps)
             xn = [y]
         w1, b1, w2, b2 = ([net[i] for net in nets] for i in (1, 2, 3, 4))
@@ -2053,9 +2053,9 @@ class _Mlp(torch.autograd.Function):
                 grads += got[:5]
                 grads[3] = got[5] if normed else None
             return tuple(g if w else None for g, w in zip(grads, need))
-        rows = [x.reshape(-1, x.shape[-1]).contiguous() for x in xs]
+        rows = [_laid_out(x.reshape(-1, x.shape[-1])) for x in xs]
         xn = rows if xn is None else [xn]
-        d2 = [d.reshape(-1, w.shape[0]).contiguous() for d, w in zip(douts, w2)]
+        d2 = [_laid_out(d.reshape(-1, w.shape[0])) for d, w in zip(douts, w2)]
         wants = lambda i: any(need[4 + 5 * j + i] for j in range(n))
         grads = [None] * len(need)
 
@@ -2076,7 +2076,7 @@ class _Mlp(torch.autograd.Function):
             if need[3] or wants(0):
                 dx = _gemm_bf16(dh, w1, residual=d2[0] if residual and not normed else None, transposed=True)
                 if normed:
-                    dx0, grads[3] = _rms_bwd(rows[0], norm_w.contiguous(), rstd, dx[0], need[3])
+                    dx0, grads[3] = _rms_bwd(rows[0], _laid_out(norm_w), rstd, dx[0], need[3])
                     dx = [dx0.add_(d2[0]) if residual else dx0]
                 put(0, [d.view(x.shape) for d, x in zip(dx, xs)])
         return tuple(g if w else None for g, w in zip(grads, need))

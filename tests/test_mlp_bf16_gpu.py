@@ -69,6 +69,26 @@ def test_gradients_of_gradients_and_batches_of_them():
         assert (a.float() - b.float()).norm() <= 2 ** -6 * b.float().norm()      # (both in bf16, second derivatives of sums of squares)
 
 
+@pytest.mark.parametrize("act,residual", [("gelu", True), ("relu", False)])
+def test_operands_off_a_16_byte_boundary(act, residual):
+    """Inputs, norm weight and incoming gradients that are contiguous views at an odd offset."""
+    from native_sparse_attention_pytorch_amd import ops
+    g = torch.Generator().manual_seed(5)
+    odd = lambda s: torch.randn(1 + s.numel(), generator=g).to(DEV, torch.bfloat16)[1:].view(s)
+    shape = torch.Size((3, 50, 128))
+    x, d, nw = odd(shape), odd(shape), odd(torch.Size((128,))) if residual else None
+    net = _net(128, 256, 128, g)
+    assert x.is_contiguous() and x.data_ptr() % 16 and d.data_ptr() % 16
+    res = []
+    for t, e, w in ((x, d, nw), (x.clone(), d.clone(), None if nw is None else nw.clone())):
+        leaves = [t.requires_grad_(), *net] + ([w.requires_grad_()] if residual else [])
+        assert ops.mlp_supported(act, [t], [tuple(net)], w)
+        y = ops.mlp(act, [t], [tuple(net)], w, residual=residual)
+        res.append([y, *torch.autograd.grad(y, leaves, e)])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
 def test_what_the_node_does_not_take():
     from native_sparse_attention_pytorch_amd import ops
     g = torch.Generator().manual_seed(1)
