@@ -105,8 +105,34 @@ def _direct(op):
     return op if torch.compiler.is_compiling() else op._init_fn
 
 
+class _NoFurther(torch.autograd.Function):
+    """The first `n` tensors, as functions of the others that cannot be differentiated."""
+
+    @staticmethod
+    def forward(ctx, n, *tensors):
+        return tuple(None if t is None else t.view_as(t) for t in tensors[:n])
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise RuntimeError("gradients of the attention kernels cannot be differentiated again")
+
+
+def _once(backward):
+    """A backward made by kernels.  Under create_graph its gradients depend on all that it read and refuse to be differentiated: as plain
+    tensors a second derivative would take them for constants."""
+    def call(ctx, *grads):
+        if not torch.is_grad_enabled():
+            return backward(ctx, *grads)
+        read = ctx.saved_tensors
+        with torch.no_grad():
+            got = backward(ctx, *grads)
+        return _NoFurther.apply(len(got), *got, *read, *grads)
+    return call
+
+
 def _eager_function(op, setup, backward):
     raw = op._init_fn
+    backward = _once(backward)
 
     class Fn(torch.autograd.Function):
         @staticmethod
@@ -554,6 +580,7 @@ class _SelectAndSlide(torch.autograd.Function):
         return out, slid
 
     @staticmethod
+    @_once
     def backward(ctx, dout, dslid):
         q, k, v, idx, fmask, index_ws, out, lse, slid, slid_lse = ctx.saved_tensors
         block, window, scale, gates = ctx.args

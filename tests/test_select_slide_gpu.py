@@ -51,3 +51,21 @@ def test_what_the_node_does_not_take():
     assert call(z(4), z(2), i=idx.repeat_interleave(2, 1)) is None and call(z(4).float(), z(2).float()) is None
     with torch.no_grad():
         assert call(z(4), z(2)) is None
+
+
+def test_gradients_of_gradients_are_refused():
+    """The backward kernels' results are no functions of their operands to autograd: differentiating them again raises, where it would leave
+    out what depends on them - also where only the inputs and not the incoming gradients ask for it."""
+    from native_sparse_attention_pytorch_amd import ops
+    b, hq, hk, n, B, S, window = 1, 4, 2, 100, 16, 2, 9
+    g = torch.Generator().manual_seed(0)
+    q, k, v = (torch.randn(b, h, n, 64, generator=g).to(DEV, torch.bfloat16).requires_grad_() for h in (hq, hk, hk))
+    idx, live = (t.to(DEV) for t in causal_random_selection(b, hk, n, B, S, seed=5))
+    for name, f in (("node", lambda: sum(ops.select_and_slide(q, k, v, B, idx, live, None, window))),
+                    ("selection", lambda: ops.native_sparse_attend(q, k, v, B, idx, live)),
+                    ("window", lambda: ops.sliding_attend(q, k, v, window))):
+        plain = torch.autograd.grad(f().sum(), (q, k, v))
+        first = torch.autograd.grad(f().sum(), (q, k, v), create_graph=True)
+        assert all(torch.equal(x, y) for x, y in zip(plain, first)), name
+        with pytest.raises(RuntimeError, match="cannot be differentiated again"):
+            torch.autograd.grad(sum(t.float().square().sum() for t in (*first, q)), q)
