@@ -49,6 +49,15 @@ def test_networks_as_one_node(rows, act, k, hidden, out, nets, whole):
         assert err < 2 ** -7, (name, err)
 
 
+# products of 512 tiles of 128 rows and more take those instead of tiles of 64: a last tile of 1, 34, 64, 65 and 128 rows
+@pytest.mark.parametrize("rows", (4097, 4130, 4160, 4161, 4224))
+@pytest.mark.parametrize("act,k,hidden,out,nets,whole", [("gelu", 128, 2048, 128, 1, True), ("relu", 128, 1024, 64, 2, False), ("gelu", 2048, 128, 2048, 1, True)])
+def test_tiles_of_128_rows(rows, act, k, hidden, out, nets, whole):
+    """The wide side of each network; the bounds are those of the test above."""
+    assert -(-rows // 128) * (max(k, hidden) // 128) * nets >= 512
+    test_networks_as_one_node(rows, act, k, hidden, out, nets, whole)
+
+
 def test_gradients_of_gradients_and_batches_of_them():
     """What the separate layers do beyond one backward pass, by the separate layers."""
     from native_sparse_attention_pytorch_amd import ops
