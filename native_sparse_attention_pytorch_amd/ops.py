@@ -1956,7 +1956,7 @@ class _Linear(torch.autograd.Function):
             dx = (dy2 @ w).view(x.shape)
         need_db = ctx.has_bias and ctx.needs_input_grad[2]
         if ctx.needs_input_grad[1]:
-            if _wgrad_supported(dy2, x2, w.dtype):
+            if _wgrad_supported(dy2, x2, w.dtype, need_db):
                 dw, db = _wgrad_bf16([(dy2, x2)], need_db)[0]
                 return dx, dw, db
             dw = _wgrad(dy2, x2, w.dtype)
@@ -1978,16 +1978,30 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     return _Linear.apply(x, weight, bias)
 
 
-def _wgrad_supported(dy2: Tensor, x2: Tensor, dtype) -> bool:
-    """A weight gradient that `nsa_wgrad_bf16` serves at least as well as the GEMM library (and its bias gradient, a pass of its own, for
-    1 to 2 us).  us on the GPU alone, library sliced by `_wgrad_splits` / this kernel (the library's call takes the host another 15):
-      4080 x 1024 -> 64 30.9 / 10.5, 4080 x 2048 -> 64 31.0 / 12.4, 4080 x 1024 -> 1024 35.0 / 27.1, 8192 x 512 -> 1024 26.2 / 25.6,
-      8192 x 2048 -> 512 33.4 / 34.8, 8192 x 512 -> 2048 35.2 / 35.9, 1000 x 512 -> 512 13.4 / 11.7;
-      above the line 4080 x 2048 -> 2048 (17 G) 55.8 / 58.3, 16384 x 1024 -> 1024 45.6 / 56.4, 16384 x 1024 -> 1536 67.7 / 82.9."""
+def _wgrad_supported(dy2: Tensor, x2: Tensor, dtype, sums: bool = True) -> bool:
+    """A weight gradient - with `sums` and the bias gradient, a pass of its own in the library - that `nsa_wgrad_bf16` serves at least as
+    well as the GEMM library, sliced by `_wgrad_splits` where that slices.  us on the GPU alone, library / this kernel (the library's call
+    takes the host another 15):
+      alone   the library gives a tile all rows, 7 us a thousand, so many rows are this kernel's: 3000 x 512 -> 1536 28.8 / 22.5, 3000 x 1024 -> 2048
+              36 / 31, 6000 x 1024 -> 1024 47 / 31, 12000 x 512 -> 1536 45 / 38; few are not: 2048 x 1024 -> 1024 17 / 25, 1000 x 512 -> 2048 13.5 / 19.4, 500 x
+              4096 -> 4096 30 / 48; few with few tiles: 1000 x 512 -> 512 (16 of 128 x 128) 12.9 / 10.7, 300 rows 7.3 / 10.2;
+              in slices it is as fast but for the smallest weights: 8192 x 512 -> 1536 28.7 / 30.5, 8192 x 1024 -> 1024 35.0 / 35.5, 8192 x 512 -> 512 22.0 / 21.9;
+      sums    fewer than 64 tiles 9.9 / 7.9 (64 x 512 -> 1536) to 57 / 41 (12000 rows), more of them 2048 x 1024 -> 1024 23.1 / 25.4, 1000 x 2048 -> 2048 29 / 27, 300 x
+              2048 -> 2048 17 / 22, but 3000 x 1024 -> 1536 40 / 29, 8192 x 512 -> 2048 45 / 38;
+      above 9 G products 4080 x 2048 -> 2048 (17) 60 / 57, 16384 x 1024 -> 1024 48.9 / 56.3."""
     rows, n_out, n_in = x2.shape[0], dy2.shape[1], x2.shape[1]
-    return bool(x2.dtype == dy2.dtype == dtype == _BF16 and x2.is_cuda and rows > 0 and n_out % 64 == 0 and n_in % 128 == 0
-                and n_out < 1 << 15 and n_in < 1 << 15 and (n_out == 64 or rows * n_out * n_in <= 9 << 30)
-                and not torch.is_grad_enabled() and plain_call() and not _in_batch(dy2) and _row_aligned(dy2) and _row_aligned(x2))
+    if not (x2.dtype == dy2.dtype == dtype == _BF16 and x2.is_cuda and rows > 0 and n_out % 64 == 0 and n_in % 128 == 0
+            and n_out < 1 << 15 and n_in < 1 << 15 and not torch.is_grad_enabled() and plain_call() and not _in_batch(dy2)
+            and _row_aligned(dy2) and _row_aligned(x2)):
+        return False
+    tiles = n_out * n_in >> 14
+    if n_out > 64 and rows * n_out * n_in > 9 << 30:
+        return False
+    if sums:
+        return tiles < 64 or rows > 2048
+    if tiles <= 16:
+        return rows >= 600
+    return rows > 2048 and _wgrad_splits(rows, n_in, n_out, capturing()) == 1
 
 
 _in_batch = torch._C._functorch.is_legacy_batchedtensor      # autograd.grad(..., is_grads_batched=True), which plain_call does not see
@@ -2143,7 +2157,7 @@ def mlp(act: str, xs, nets, norm_w: Tensor | None = None, eps: float | None = No
 
 def _wgrad(dy2: Tensor, x2: Tensor, dtype) -> Tensor:
     """Weight gradient 'o i' = dy2^T x2 of a projection, over slices of the token axis where that fills the chip."""
-    if _wgrad_supported(dy2, x2, dtype):
+    if _wgrad_supported(dy2, x2, dtype, False):
         return _wgrad_bf16([(dy2, x2)], False)[0][0]
     rows, n_in, n_out = x2.shape[0], x2.shape[1], dy2.shape[1]
     s = _wgrad_splits(rows, n_in, n_out, capturing()) if x2.is_cuda and x2.dtype in (_BF16, torch.float16) and dy2.dtype == x2.dtype else 1
