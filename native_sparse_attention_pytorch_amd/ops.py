@@ -2124,19 +2124,28 @@ class _Mlp(torch.autograd.Function):
 
 
 def mlp_supported(act: str, xs, nets, norm_w: Tensor | None = None) -> bool:
-    """Networks that `mlp` serves better than the separate layers; `nets`: (w1, b1, w2, b2) each.  Forward and backward, us on the GPU alone,
-    layers / node (the host takes 320 / 250 for a feed-forward block and 490 / 270 for two networks):
-      feed-forward with norm and residual, 512 x 512 -> 2048 -> 512 114 / 110, 2048 rows 169 / 136, 8192 351 / 247, 16384 650 / 420;
-      8192 x 1024 -> 4096 -> 1024 (34 G products of a pass) 662 / 660, 4096 rows 381 / 396;
-      two networks, 1016 x 1024 -> 1024 -> 64 131 / 84, 4064 rows 185 / 145, 1016 x 2048 -> 2048 -> 64 185 / 156, 4080 rows (34 G) 380 / 357;
-      above the line 1000 x 4096 -> 4096 -> 128 (34 G) 350 / 408, 2040 rows 528 / 669: the library's larger tiles read the operands less often."""
+    """Networks that `mlp` serves better than the separate layers; `nets`: (w1, b1, w2, b2) each.  Forward and backward, layers / node, us on the
+    GPU alone (the host takes 270 to 380 / 160 to 260 for a feed-forward block, 440 to 570 / 160 to 280 for two networks):
+      two networks, 64 x 1024 -> 1024 -> 64 95 / 58, 1016 rows 139 / 78, 4064 183 / 141, 15000 400 / 384; 500 x 2048 -> 2048 -> 64 154 / 125, 4080 rows (34 G products of a
+      pass) 383 / 374; above the line 1000 x 4096 -> 4096 -> 128 362 / 424, 500 rows 297 / 305: the library's larger tiles read the operands less often;
+      feed-forward with norm and residual, 512 x 512 -> 2048 -> 512 105 / 106, 2048 rows 162 / 129, 8192 344 / 248, 32768 1115 / 806; 15000 x 768 -> 3072 871 / 819;
+      8192 x 1024 -> 2048 438 / 374; wider ones up to where the GPU and not the host is the longer: 1024 x 1024 -> 4096 182 / 197 (with the host 372 / 264),
+      3000 rows 331 / 345 (369 / 313), above the line 4096 rows 380 / 390, 8192 667 / 677, 8000 x 1024 -> 3072 577 / 604;
+      recorded into a graph, without the host and with the layers' sums by kernels: 8192 x 512 -> 2048 274 / 247, 1000 rows 124 / 114, 2000 x 1024 -> 2048 191 / 164, but 512
+      x 512 -> 2048 98 / 105, 1024 x 768 -> 3072 146 / 158, 4096 x 768 -> 3072 283 / 285, 2048 x 1024 -> 4096 240 / 260, 16384 x 1024 -> 2048 661 / 706."""
     x, (w1, _, w2, _) = xs[0], nets[0]
     if not (torch.is_grad_enabled() and x.is_cuda and x.dtype == _BF16 and w1.dim() == 2 and w2.dim() == 2 and plain_call()):
         return False
     k, hidden, out, rows = x.shape[-1], w1.shape[0], w2.shape[0], x.numel() // max(x.shape[-1], 1)
+    size = hidden * max(k, out)
     if not (rows > 0 and k % 128 == 0 and hidden % 128 == 0 and out % 64 == 0 and max(k, hidden, out) < 1 << 15
-            and hidden * max(k, out) <= 1 << 22 and len(xs) * rows * hidden * max(k, out) <= 36 << 30):
+            and size <= 1 << 22 and len(xs) * rows * size <= 36 << 30):
         return False
+    if len(xs) == 1:
+        if size > 5 << 19 and rows * size > 12 << 30:
+            return False
+        if capturing() and not (size <= 2 << 20 and rows * size <= 16 << 30 and 1536 * rows >= size):
+            return False
     for y, (a, b, c, d) in zip(xs, nets):
         if y.shape != x.shape or y.dtype != _BF16 or y.device != x.device or a.shape != (hidden, k) or c.shape != (out, hidden):
             return False
