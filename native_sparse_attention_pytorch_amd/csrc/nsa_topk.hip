@@ -531,7 +531,8 @@ int decode_topk_launch(const float* logits, int32_t batch, int32_t kv_heads, int
 // means of the compressed keys into LDS once (npf keys to a block) and takes `per` queries per wave against them: the mean of the
 // group's heads (share) or one head, 64 dot products of d features, then softmax, rank and mask of the lane's own block as
 // topk_kernel has them.  Two means, a small GEMM and the top-k kernel otherwise: 2 x 2053 queries, 16 x 4 heads, d = 64, 32 blocks
-// 34 us in four launches -> 24 in one; 2 x 31 queries of 8 heads, 7 blocks 18 -> 4.8.
+// 30 us in four launches -> 23 in one; 2 x 31 queries of 8 heads, 7 blocks 14.5 -> 4.0.  Bound by its scalar products and their LDS reads,
+// half the GEMM's speed where there are many (8 x 4096 queries, 64 blocks 94 / 183): ops.importance_select_f32 has the line.
 namespace nsa {
 
 struct ImportanceArgs {

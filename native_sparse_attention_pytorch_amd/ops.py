@@ -2381,13 +2381,18 @@ def importance_topk_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, shar
 
 @torch.no_grad()
 def importance_select_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool, causal: bool, num_selected: int, mask_own: bool = True):
-    """`importance_topk_f32` whose products are made by the top-k kernel as well for up to 64 blocks: four launches less, and a query's scores
-    the same whatever the number of queries beside it."""
+    """`importance_topk_f32` whose products are made by the top-k kernel as well for up to 64 blocks, four launches less, while there are few
+    queries (of all batches and rows of a selection).  The kernel's products are scalar ones and each query's its own; us on the GPU alone, GEMM and
+    top-k / kernel:
+      62 queries x 7 blocks 14.5 / 4.0, 8212 x 32 22 / 14, 16424 x 32 30 / 23, 16384 x 32 20.8 / 19.8, 12000 x 46 23.2 / 20.1; d = 128 8000 x 15 21.5 / 12.9, 12000 x 23
+      28 / 20, 6000 x 46 23.5 / 20.4; above the lines 16384 x 64 24.4 / 30.1, 12288 x 64 20.9 / 23.1 and many queries of few blocks, 76800 x 4 48 / 54; far above
+      131072 x 64 94 / 183."""
     b, hq, n, d = q.shape
     hk, npf = ck.shape[1], sel_block // stride
     nb, num_selected = ck.shape[2] // npf, int(num_selected)
-    if (0 < num_selected <= nb <= 64 and d <= 128 and d % 4 == 0 and n > 0 and q.dtype == ck.dtype == torch.float32 and q.is_cuda
-            and ck.device == q.device and ck.shape[0] == b and ck.shape[3] == d and b * hq <= 65535):
+    queries = b * n * (hk if share else hq)
+    if (0 < num_selected <= nb <= 64 and d <= 128 and d % 4 == 0 and 0 < queries <= 20 << 10 and queries * nb * d <= 40 << 20
+            and q.dtype == ck.dtype == torch.float32 and q.is_cuda and ck.device == q.device and ck.shape[0] == b and ck.shape[3] == d and b * hq <= 65535):
         return importance_topk(_f32(q), num_selected, keys=(_f32(ck), nb, npf, int(share), int(sel_block) if causal else 0,
                                                             int(sel_block) if mask_own and stride != sel_block else 0))
     return importance_topk_f32(q, ck, stride, sel_block, share, causal, num_selected, mask_own)

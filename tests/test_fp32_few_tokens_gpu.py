@@ -121,6 +121,15 @@ def test_importance_and_selection(b, hq, hk, n, d, stride, B, k, causal, own, sh
     assert torch.equal(dead, vals == 0)
 
 
+@pytest.mark.parametrize("b,n,share", [(6, 1024, True), (3, 1024, False), (2, 2049, True)])
+def test_importance_of_many_queries(b, n, share):
+    """Above the lines the products are the library's."""
+    from native_sparse_attention_pytorch_amd import ops
+    q, ck = _r(b, 8, n, 64), _r(b, 4, n // 8, 64, seed=1)
+    for x, y in zip(ops.importance_select_f32(q, ck, 8, 32, share, True, 4), ops.importance_topk_f32(q, ck, 8, 32, share, True, 4)):
+        assert torch.equal(x, y)
+
+
 def test_scores_that_are_not_numbers():
     from native_sparse_attention_pytorch_amd import ops
     q, ck = _r(1, 4, 50, 64), _r(1, 2, 25, 64, seed=1)
