@@ -1729,7 +1729,13 @@ def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
     if weight.dim() != 2:
         return False
     n, k = weight.shape
-    return bool(k == width and n > 0 and weight.dtype == x.dtype and weight.device == x.device and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+    return bool(k == width and n > 0 and weight.dtype == x.dtype and weight.device == x.device and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+                and _on_current_device(x))
+
+
+def _on_current_device(x: Tensor) -> bool:
+    """A device tensor where `_stream` is; the library's products change to their operands' device, launches by address do not."""
+    return x.get_device() == torch.cuda.current_device()
 
 
 def _vectors_ready(x: Tensor, weight: Tensor, bias: Tensor | None, norm_weight: Tensor | None) -> bool:
@@ -1992,7 +1998,7 @@ def _wgrad_supported(dy2: Tensor, x2: Tensor, dtype, sums: bool = True) -> bool:
     rows, n_out, n_in = x2.shape[0], dy2.shape[1], x2.shape[1]
     if not (x2.dtype == dy2.dtype == dtype == _BF16 and x2.is_cuda and rows > 0 and n_out % 64 == 0 and n_in % 128 == 0
             and n_out < 1 << 15 and n_in < 1 << 15 and not torch.is_grad_enabled() and plain_call() and not _in_batch(dy2)
-            and _row_aligned(dy2) and _row_aligned(x2)):
+            and _row_aligned(dy2) and _row_aligned(x2) and _on_current_device(x2)):
         return False
     tiles = n_out * n_in >> 14
     if n_out > 64 and rows * n_out * n_in > 9 << 30:
@@ -2134,7 +2140,7 @@ def mlp_supported(act: str, xs, nets, norm_w: Tensor | None = None) -> bool:
       recorded into a graph, without the host and with the layers' sums by kernels: 8192 x 512 -> 2048 274 / 247, 1000 rows 124 / 114, 2000 x 1024 -> 2048 191 / 164, but 512
       x 512 -> 2048 98 / 105, 1024 x 768 -> 3072 146 / 158, 4096 x 768 -> 3072 283 / 285, 2048 x 1024 -> 4096 240 / 260, 16384 x 1024 -> 2048 661 / 706."""
     x, (w1, _, w2, _) = xs[0], nets[0]
-    if not (torch.is_grad_enabled() and x.is_cuda and x.dtype == _BF16 and w1.dim() == 2 and w2.dim() == 2 and plain_call()):
+    if not (torch.is_grad_enabled() and x.is_cuda and x.dtype == _BF16 and w1.dim() == 2 and w2.dim() == 2 and plain_call() and _on_current_device(x)):
         return False
     k, hidden, out, rows = x.shape[-1], w1.shape[0], w2.shape[0], x.numel() // max(x.shape[-1], 1)
     size = hidden * max(k, out)

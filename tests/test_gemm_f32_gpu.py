@@ -127,3 +127,24 @@ def test_both_compression_networks_in_one_launch(monkeypatch):
         layer._compress_both(kw, vw)
     handle.remove()
     assert seen
+
+
+def test_operands_of_another_device(monkeypatch):
+    """Where the current device is another one (told to the rules only), the library makes the products: a launch by address would go to a
+    stream of the wrong device."""
+    from native_sparse_attention_pytorch_amd import _lib, ops
+    x, w, few = _r(2049, 64), _r(2048, 64, seed=1), _r(4, 64)
+    h = lambda *s: _r(*s).bfloat16().requires_grad_()
+    net = h(256, 128), h(256), h(128, 256), h(128)
+    y, dy = h(700, 128), h(700, 64).detach()
+    with torch.no_grad():
+        assert ops.gemm_f32_supported(x, w) and ops.linear_f32_supported(few, w[:64]) and ops._wgrad_supported(dy, y, y.dtype)
+    assert ops.mlp_supported("relu", [y], [net])
+    other = torch.cuda.current_device() + 1
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: other)
+    monkeypatch.setattr(_lib, "lib", lambda: pytest.fail("launched"))
+    assert not ops.mlp_supported("relu", [y], [net])
+    with torch.no_grad():
+        assert not ops._wgrad_supported(dy, y, y.dtype)
+        for t, v in ((x, w), (few, w[:64])):
+            assert torch.equal(ops.linear(t, v), F.linear(t, v))
