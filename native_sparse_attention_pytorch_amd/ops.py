@@ -1844,7 +1844,8 @@ def _rows_f32(x: Tensor) -> Tensor | None:
 def linear_pair_f32(x: Tensor, first, second, norm_weight: Tensor | None = None, eps: float | None = None, x2: Tensor | None = None,
                     act: str | None = None):
     """act(linear(x, *first)) and act(linear(x2, *second)) of a few rows in one launch, `first` / `second` = (weight, bias); x2 None: both
-    of x.  eps not None: of rms_norm(x) * norm_weight.  None where one of them is not `linear_f32`'s to serve."""
+    of x.  eps not None: of rms_norm(x) * norm_weight.  None where one of them is not `linear_f32`'s to serve.  62 x 512 -> 1536 and 24 behind
+    the norm, us on the GPU alone: three launches 14.6, in one 9.0."""
     if not all(linear_f32_supported(t, w, b) and (b is None or b.is_contiguous()) for t, (w, b) in ((x, first), (x if x2 is None else x2, second))):
         return None
     a = _rows_f32(x)
@@ -1860,7 +1861,8 @@ def linear_pair_f32(x: Tensor, first, second, norm_weight: Tensor | None = None,
 
 
 def gate_linear_f32(logits: Tensor, c: Tensor, f: Tensor, s: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
-    """linear(gate_combine_f32(logits, c, f, s), weight, bias) of a few tokens in one launch; None where that is not `linear_f32`'s to serve."""
+    """linear(gate_combine_f32(logits, c, f, s), weight, bias) of a few tokens in one launch; None where that is not `linear_f32`'s to serve.
+    62 tokens of 512 features, apart / in one: with the host 25 / 13.5 us, on the GPU alone 8.7 / 12.6 (every tile makes the gated rows again)."""
     b, h, n, d = c.shape
     rows, k = b * n, h * d
     if not (0 < rows <= 256 and k <= 512 and k % 8 == 0 and logits.dtype == torch.float32 and logits.is_cuda and logits.shape == (b, n, 3 * h)
