@@ -1735,7 +1735,7 @@ def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
 
 def _on_current_device(x: Tensor) -> bool:
     """A device tensor where `_stream` is; the library's products change to their operands' device, launches by address do not."""
-    return x.get_device() == torch.cuda.current_device()
+    return x.get_device() == torch._C._cuda_getDevice()
 
 
 def _vectors_ready(x: Tensor, weight: Tensor, bias: Tensor | None, norm_weight: Tensor | None) -> bool:

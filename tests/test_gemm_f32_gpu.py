@@ -141,7 +141,7 @@ def test_operands_of_another_device(monkeypatch):
         assert ops.gemm_f32_supported(x, w) and ops.linear_f32_supported(few, w[:64]) and ops._wgrad_supported(dy, y, y.dtype)
     assert ops.mlp_supported("relu", [y], [net])
     other = torch.cuda.current_device() + 1
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: other)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: other)
     monkeypatch.setattr(_lib, "lib", lambda: pytest.fail("launched"))
     assert not ops.mlp_supported("relu", [y], [net])
     with torch.no_grad():
