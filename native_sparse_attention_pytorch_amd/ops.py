@@ -1734,8 +1734,10 @@ def _weight_ready(x: Tensor, width: int, weight: Tensor) -> bool:
 
 
 def _on_current_device(x: Tensor) -> bool:
-    """A device tensor where `_stream` is; the library's products change to their operands' device, launches by address do not."""
-    return x.get_device() == torch._C._cuda_getDevice()
+    """x lies where `_stream` is: the library's products change to their operands' device, launches by address do not.  (Of tensors on a
+    device; the others are told apart by is_cuda.)"""
+    index = x.get_device()
+    return index < 0 or index == torch._C._cuda_getDevice()
 
 
 def _vectors_ready(x: Tensor, weight: Tensor, bias: Tensor | None, norm_weight: Tensor | None) -> bool:
