@@ -117,22 +117,25 @@ class _NoFurther(torch.autograd.Function):
         raise RuntimeError("gradients of the attention kernels cannot be differentiated again")
 
 
-def _once(backward):
-    """A backward made by kernels.  Under create_graph its gradients depend on all that it read and refuse to be differentiated: as plain
-    tensors a second derivative would take them for constants."""
-    def call(ctx, *grads):
+def _once(kernels):
+    """`kernels(*args)` -> gradients.  Under create_graph these depend on all tensors among the arguments and refuse to be differentiated: as
+    plain tensors a second derivative would take them for constants."""
+    def call(*args):
         if not torch.is_grad_enabled():
-            return backward(ctx, *grads)
-        read = ctx.saved_tensors
+            return kernels(*args)
         with torch.no_grad():
-            got = backward(ctx, *grads)
-        return _NoFurther.apply(len(got), *got, *read, *grads)
+            got = kernels(*args)
+        return _NoFurther.apply(len(got), *got, *(a for a in args if isinstance(a, Tensor)))
     return call
+
+
+def _direct_bwd(op):
+    """`_direct` of an operator that makes gradients."""
+    return op if torch.compiler.is_compiling() else _once(op._init_fn)
 
 
 def _eager_function(op, setup, backward):
     raw = op._init_fn
-    backward = _once(backward)
 
     class Fn(torch.autograd.Function):
         @staticmethod
@@ -244,7 +247,7 @@ def _select_backward(ctx, dout, dlse, dws):
         return (None,) * 9
     if dout is None:
         dout = torch.zeros_like(out)
-    dq, dk, dv, dsel = _direct(select_bwd)(q, k, v, out, dout, lse, idx, fmask, index_ws, block, causal, scale, want, dlse)
+    dq, dk, dv, dsel = _direct_bwd(select_bwd)(q, k, v, out, dout, lse, idx, fmask, index_ws, block, causal, scale, want, dlse)
     return dq, dk, dv, None, None, (dsel.to(sdtype) if want else None), None, None, None
 
 
@@ -533,7 +536,7 @@ def _dense_backward(ctx, dout, dlse, dpooled):
         # the compressed keys are few and every one of their gradients is summed over all windows into the compression
         # network's parameters: they leave the kernel as fp32 and are rounded to the keys' dtype once, after the
         # importance term has been added
-        dq, dk, dv = _direct(dense_bwd)(q, k, v, out, dout, lse, mode, causal, window, stride, num_mem, scale,
+        dq, dk, dv = _direct_bwd(dense_bwd)(q, k, v, out, dout, lse, mode, causal, window, stride, num_mem, scale,
                                         mode == 1 and dpooled is not None and dpooled.numel() > 0)
     if dq is not None and dpooled is not None and dpooled.numel() > 0 and not torch.compiler.is_compiling() and not torch.is_grad_enabled():
         # both sums in one kernel each: scale, repetition over the group's heads / the block's keys, sum in fp32, one rounding
@@ -580,17 +583,21 @@ class _SelectAndSlide(torch.autograd.Function):
         return out, slid
 
     @staticmethod
-    @_once
     def backward(ctx, dout, dslid):
-        q, k, v, idx, fmask, index_ws, out, lse, slid, slid_lse = ctx.saved_tensors
         block, window, scale, gates = ctx.args
-        into = dgates = None
-        if dout is not None:
-            *into, dsel = select_bwd._init_fn(q, k, v, out, dout, lse, idx, fmask, index_ws, block, True, scale, gates is not None, None)
-            dgates = None if gates is None else dsel.to(gates)
-        if dslid is not None:
-            into = _dense_bwd(q, k, v, slid, dslid, slid_lse, 0, True, window, 1, 0, scale, into=into)
-        return (*((None,) * 3 if into is None else into), None, None, dgates, None, None, None)
+
+        def kernels(dout, dslid, q, k, v, idx, fmask, index_ws, out, lse, slid, slid_lse):
+            into = (None,) * 3
+            dgates = None
+            if dout is not None:
+                *into, dsel = select_bwd._init_fn(q, k, v, out, dout, lse, idx, fmask, index_ws, block, True, scale, gates is not None, None)
+                dgates = None if gates is None else dsel.to(gates)
+            if dslid is not None:
+                into = _dense_bwd(q, k, v, slid, dslid, slid_lse, 0, True, window, 1, 0, scale, into=None if dout is None else into)
+            return (*into, dgates)
+
+        dq, dk, dv, dgates = _once(kernels)(dout, dslid, *ctx.saved_tensors)
+        return dq, dk, dv, None, None, dgates, None, None, None
 
 
 def select_and_slide(q: Tensor, k: Tensor, v: Tensor, block_size: int, idx: Tensor, fmask: Tensor, gates: Tensor | None, window: int):
@@ -700,7 +707,7 @@ def _compress_topk_backward(ctx, dout, dlse, didx, dfm):
     causal, stride, num_mem, scale = ctx.args
     if dout is None:
         return (None,) * 9
-    dq, dk, dv = _direct(dense_bwd)(q, k, v, out, dout, lse, 1, causal, 0, stride, num_mem, scale, False)
+    dq, dk, dv = _direct_bwd(dense_bwd)(q, k, v, out, dout, lse, 1, causal, 0, stride, num_mem, scale, False)
     return (dq, dk, dv) + (None,) * 6
 
 
@@ -975,7 +982,7 @@ def _gate_setup(ctx, inputs, output):
 
 def _gate_backward(ctx, dout):
     logits, c, f, s = ctx.saved_tensors
-    return _direct(gate_bwd)(logits, c, f, s, dout)
+    return _direct_bwd(gate_bwd)(logits, c, f, s, dout)
 
 
 gate_fwd.register_autograd(_gate_backward, setup_context=_gate_setup)
@@ -2254,18 +2261,21 @@ class _Fp32ValueBf16Grad(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        tensors = ctx.saved_tensors
         need = ctx.needs_input_grad[2:]
-        with torch.enable_grad():
-            ins = [t.detach().to(_BF16).requires_grad_(bool(nd)) for t, nd in zip(tensors, need)]
-            out = ctx.fwd16(*ins)
-            wanted = [t for t in ins if t.requires_grad]
-            grads = iter(torch.autograd.grad(out, wanted, dout.to(out.dtype), allow_unused=True)) if wanted else iter(())
-        res = []
-        for t, nd in zip(tensors, need):
-            g = next(grads) if nd else None
-            res.append(None if g is None else g.to(t.dtype))
-        return (None, None, *res)
+
+        def kernels(dout, *tensors):
+            with torch.enable_grad():
+                ins = [t.detach().to(_BF16).requires_grad_(bool(nd)) for t, nd in zip(tensors, need)]
+                out = ctx.fwd16(*ins)
+                wanted = [t for t in ins if t.requires_grad]
+                grads = iter(torch.autograd.grad(out, wanted, dout.to(out.dtype), allow_unused=True)) if wanted else iter(())
+            res = []
+            for t, nd in zip(tensors, need):
+                g = next(grads) if nd else None
+                res.append(None if g is None else g.to(t.dtype))
+            return tuple(res)
+
+        return (None, None, *_once(kernels)(dout, *ctx.saved_tensors))
 
 
 def fp32_value_bf16_grad(fwd32, fwd16, *tensors: Tensor) -> Tensor:

@@ -63,9 +63,30 @@ def test_gradients_of_gradients_are_refused():
     idx, live = (t.to(DEV) for t in causal_random_selection(b, hk, n, B, S, seed=5))
     for name, f in (("node", lambda: sum(ops.select_and_slide(q, k, v, B, idx, live, None, window))),
                     ("selection", lambda: ops.native_sparse_attend(q, k, v, B, idx, live)),
-                    ("window", lambda: ops.sliding_attend(q, k, v, window))):
+                    ("window", lambda: ops.sliding_attend(q, k, v, window)),
+                    ("compressed", lambda: ops.compress_attend(q, k[:, :, :8], v[:, :, :8], 2, 16, True)[0]),
+                    ("in fp32", lambda: ops.fp32_value_bf16_grad(lambda *t: ops.dense_attend_f32(*(x.float() for x in t), 0, True, window)[0],
+                                                                 lambda *t: ops.sliding_attend(*t, window), q, k, v))):
         plain = torch.autograd.grad(f().sum(), (q, k, v))
         first = torch.autograd.grad(f().sum(), (q, k, v), create_graph=True)
         assert all(torch.equal(x, y) for x, y in zip(plain, first)), name
         with pytest.raises(RuntimeError, match="cannot be differentiated again"):
             torch.autograd.grad(sum(t.float().square().sum() for t in (*first, q)), q)
+
+
+def test_importance_scores_have_a_second_derivative():
+    """They are linear in queries and compressed keys, and their gradient is made of matrix products: against float64."""
+    from native_sparse_attention_pytorch_amd import ops
+    g = torch.Generator().manual_seed(1)
+    q, ck, cv = (torch.randn(1, h, m, 64, generator=g).to(DEV, torch.bfloat16).requires_grad_() for h, m in ((4, 100), (2, 7), (2, 7)))
+    res = []
+    for t, c in ((q, ck), (q.detach().double().requires_grad_(), ck.detach().double().requires_grad_())):
+        if t.dtype == torch.bfloat16:
+            logits = ops.compress_attend(t, c, cv, 1, 16, True, 16)[1]
+        else:
+            logits = ops.importance_logits_f32(t, c[:, :, 1:], 16, 16, True, True)
+        seen = logits.masked_fill(logits.isinf(), 0.)
+        dq, = torch.autograd.grad(seen.square().sum(), t, create_graph=True)
+        res.append(torch.autograd.grad(dq.square().sum(), (t, c)))
+    for x, y in zip(*res):
+        assert ((x.double() - y).norm() <= 2 ** -6 * y.norm()).item()      # (operands, scores and results in bf16)
