@@ -2002,7 +2002,8 @@ def _wgrad_supported(dy2: Tensor, x2: Tensor, dtype, sums: bool = True) -> bool:
       alone   the library gives a tile all rows, 7 us a thousand, so many rows are this kernel's: 3000 x 512 -> 1536 28.8 / 22.5, 3000 x 1024 -> 2048
               36 / 31, 6000 x 1024 -> 1024 47 / 31, 12000 x 512 -> 1536 45 / 38; few are not: 2048 x 1024 -> 1024 17 / 25, 1000 x 512 -> 2048 13.5 / 19.4, 500 x
               4096 -> 4096 30 / 48; few with few tiles: 1000 x 512 -> 512 (16 of 128 x 128) 12.9 / 10.7, 300 rows 7.3 / 10.2;
-              in slices it is as fast but for the smallest weights: 8192 x 512 -> 1536 28.7 / 30.5, 8192 x 1024 -> 1024 35.0 / 35.5, 8192 x 512 -> 512 22.0 / 21.9;
+              in slices it is as fast, 8192 x 512 -> 1536 28.7 / 30.5, 8192 x 1024 -> 1024 35.0 / 35.5, 8192 x 512 -> 512 22.0 / 21.9, and the host's time decides (a
+              model of 6 layers on 8192 tokens 11.51 / 11.39 ms a step; recorded into a graph the library has them);
       sums    fewer than 64 tiles 9.9 / 7.9 (64 x 512 -> 1536) to 57 / 41 (12000 rows), more of them 2048 x 1024 -> 1024 23.1 / 25.4, 1000 x 2048 -> 2048 29 / 27, 300 x
               2048 -> 2048 17 / 22, but 3000 x 1024 -> 1536 40 / 29, 8192 x 512 -> 2048 45 / 38;
       above 9 G products 4080 x 2048 -> 2048 (17) 60 / 57, 16384 x 1024 -> 1024 48.9 / 56.3."""
@@ -2018,7 +2019,7 @@ def _wgrad_supported(dy2: Tensor, x2: Tensor, dtype, sums: bool = True) -> bool:
         return tiles < 64 or rows > 2048
     if tiles <= 16:
         return rows >= 600
-    return rows > 2048 and _wgrad_splits(rows, n_in, n_out, capturing()) == 1
+    return rows > 2048 and not (capturing() and _wgrad_splits(rows, n_in, n_out, True) > 1)
 
 
 _in_batch = torch._C._functorch.is_legacy_batchedtensor      # autograd.grad(..., is_grads_batched=True), which plain_call does not see
@@ -2400,18 +2401,20 @@ def importance_topk_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, shar
 
 
 @torch.no_grad()
-def importance_select_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool, causal: bool, num_selected: int, mask_own: bool = True):
+def importance_select_f32(q: Tensor, ck: Tensor, stride: int, sel_block: int, share: bool, causal: bool, num_selected: int, mask_own: bool = True,
+                          host_bound: bool = False):
     """`importance_topk_f32` whose products are made by the top-k kernel as well for up to 64 blocks, four launches less, while there are few
     queries (of all batches and rows of a selection).  The kernel's products are scalar ones and each query's its own; us on the GPU alone, GEMM and
     top-k / kernel:
       62 queries x 7 blocks 14.5 / 4.0, 8212 x 32 22 / 14, 16424 x 32 30 / 23, 16384 x 32 20.8 / 19.8, 12000 x 46 23.2 / 20.1; d = 128 8000 x 15 21.5 / 12.9, 12000 x 23
       28 / 20, 6000 x 46 23.5 / 20.4; above the lines 16384 x 64 24.4 / 30.1, 12288 x 64 20.9 / 23.1 and many queries of few blocks, 76800 x 4 48 / 54; far above
-      131072 x 64 94 / 183."""
+      131072 x 64 94 / 183.  The launches take the host 48 / 13 us: where its time is the longer (`host_bound`: a training step of an fp32 layer, a hundred
+      launches), up to 32768 x 64 30 / 49, 8 x 1024 tokens a step 2.27 / 2.18 ms."""
     b, hq, n, d = q.shape
     hk, npf = ck.shape[1], sel_block // stride
     nb, num_selected = ck.shape[2] // npf, int(num_selected)
     queries = b * n * (hk if share else hq)
-    if (0 < num_selected <= nb <= 64 and d <= 128 and d % 4 == 0 and 0 < queries <= 20 << 10 and queries * nb * d <= 40 << 20
+    if (0 < num_selected <= nb <= 64 and d <= 128 and d % 4 == 0 and 0 < queries <= (32 if host_bound else 20) << 10 and queries * nb * d <= (128 if host_bound else 40) << 20
             and q.dtype == ck.dtype == torch.float32 and q.is_cuda and ck.device == q.device and ck.shape[0] == b and ck.shape[3] == d and b * hq <= 65535):
         return importance_topk(_f32(q), num_selected, keys=(_f32(ck), nb, npf, int(share), int(sel_block) if causal else 0,
                                                             int(sel_block) if mask_own and stride != sel_block else 0))

@@ -572,7 +572,7 @@ class SparseAttention(nn.Module):
                 vals, idx, fmask = ops.importance_topk(ops.importance_logits_f32(qa, ck0, st, B, share, causal).contiguous(), num_sel)
                 gates = vals + (1. - vals).detach()                              # straight-through gates (NSA.py:715)
             else:
-                _, idx, fmask = ops.importance_select_f32(qa, ck0, st, B, share, causal, num_sel)
+                _, idx, fmask = ops.importance_select_f32(qa, ck0, st, B, share, causal, num_sel, host_bound=True)
             block_causal = causal
         elif causal:
             idx = torch.zeros((b, self.kv_heads, n, 0), dtype=torch.int32, device=qkv.device)

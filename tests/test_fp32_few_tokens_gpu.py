@@ -130,6 +130,17 @@ def test_importance_of_many_queries(b, n, share):
         assert torch.equal(x, y)
 
 
+def test_importance_of_many_queries_of_a_waiting_host():
+    """The kernel's line where the host's time counts, against the GEMM's scores; and above it."""
+    from native_sparse_attention_pytorch_amd import ops
+    for b, same in ((8, False), (9, True)):
+        q, ck = _r(b, 8, 1024, 64), _r(b, 4, 128, 64, seed=1)
+        args = (q, ck, 8, 16, True, True, 4)
+        got, want = ops.importance_select_f32(*args, host_bound=True), ops.importance_topk_f32(*args)
+        assert_close(got[0], want[0], 1e-6, 1e-5, "values")
+        assert (not same) or all(torch.equal(x, y) for x, y in zip(got, want))
+
+
 def test_scores_that_are_not_numbers():
     from native_sparse_attention_pytorch_amd import ops
     q, ck = _r(1, 4, 50, 64), _r(1, 2, 25, 64, seed=1)
