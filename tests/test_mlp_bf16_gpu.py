@@ -125,3 +125,24 @@ def test_weight_gradients(rows, n_out, n_in, pad):
         (dw, db), = ops._wgrad_bf16([(dy, x)], True)
     for a, b in ((dw, dy.double().t() @ x.double()), (db, dy.double().sum(0))):
         assert ((a.double() - b).norm() <= 2 ** -8.5 * b.norm()).item()
+
+
+def test_lines_of_the_rules(monkeypatch):
+    """Either side of each line, by sizes alone (nothing is launched)."""
+    from native_sparse_attention_pytorch_amd import ops
+    z = lambda *s: torch.empty(s, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    net = lambda k, hidden, out: (z(hidden, k), z(hidden), z(out, hidden), z(out))
+    block = lambda rows, k, hidden: ops.mlp_supported("gelu", [z(rows, k)], [net(k, hidden, k)])
+    pair = lambda rows, k, out: ops.mlp_supported("relu", [z(rows, k)] * 2, [net(k, k, out)] * 2)
+    assert block(3072, 1024, 4096) and not block(3073, 1024, 4096) and block(16384, 512, 2048) and block(8192, 1024, 2048) and not block(8192, 1024, 3072)
+    assert pair(4080, 2048, 64) and not pair(1000, 4096, 128)
+
+    def wgrad(rows, n_in, n_out, sums):
+        with torch.no_grad():
+            return ops._wgrad_supported(z(rows, n_out).detach(), z(rows, n_in).detach(), torch.bfloat16, sums)
+    assert wgrad(2049, 2048, 1024, False) and not wgrad(2048, 2048, 1024, False) and not wgrad(2048, 2048, 1024, True)
+    assert wgrad(600, 512, 512, False) and not wgrad(599, 512, 512, False) and wgrad(8, 512, 512, True)
+    assert wgrad(8192, 512, 1024, False) and not wgrad(16384, 1024, 1024, True) and wgrad(16384, 1024, 64, False)
+    monkeypatch.setattr(ops, "capturing", lambda: True)
+    assert block(1000, 512, 2048) and not block(500, 512, 2048) and not block(2048, 1024, 4096) and not block(16384, 1024, 2048) and pair(64, 1024, 64)
+    assert not wgrad(8192, 512, 1024, False) and wgrad(8192, 512, 1024, True) and wgrad(8192, 512, 512, False)
