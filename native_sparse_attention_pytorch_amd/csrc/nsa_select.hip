@@ -17,6 +17,7 @@
 // streamed Q / dO rows are gathered with coalesced 16-byte loads, staged in row-major LDS tiles
 // and read back as row operands or through the LDS transpose load.
 #include "nsa_common.hpp"
+#include "nsa_select_bwd_block.hpp"
 #include "nsa_select_plan.hpp"
 
 namespace nsa {
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(1024) void sel_units_kernel(const SelPlan P, char* 
       const int L = ci.own + ci.count, nu = (L + P.chunk[t] - 1) >> csh;
       for (int k = 0; k < nu; ++k) {
         rec[2 * (acc + k)] = int4{j, ci.own, ci.first, k << csh};
-        rec[2 * (acc + k) + 1] = int4{min(L, (k + 1) << csh), 0, 0, 0};
+        rec[2 * (acc + k) + 1] = int4{min(L, (k + 1) << csh), nu, 0, 0};
       }
       acc += nu;
       if (++j == P.W) { j = 0; ++pp; }
@@ -760,9 +761,10 @@ __global__ __launch_bounds__(256) void sel_fwd_combine_kernel(const SelPlan P, c
 
 // delta[b,hq,i] = sum_d out * d_out   (TRI.py:696-756), less the gradient of the row's log-sum-exp when the caller has one:
 // d loss / d logit_j = p_j (dP_j - sum_k p_k dP_k) + d_lse p_j = p_j (dP_j - (delta - d_lse))
-template <int D>
-__global__ __launch_bounds__(256) void sel_delta_kernel(const SelPlan P, const __bf16* __restrict__ out, const __bf16* __restrict__ dout,
-                                                        const float* __restrict__ dlse, float* __restrict__ delta) {
+// With BLOCK it leaves what sel_bwd_block_kernel reads instead: -delta, behind it -lse log2 e, and a zero in the counter of its units.
+template <int D, bool BLOCK>
+__global__ __launch_bounds__(256) void sel_delta_kernel(const SelPlan P, const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
+                                                        const float* __restrict__ dlse, float* __restrict__ delta, unsigned* __restrict__ ticket) {
   constexpr int LPR = D / 8;                   // lanes per row
   constexpr int RPB = 256 / LPR;               // rows per block
   const int tid = threadIdx.x;
@@ -783,7 +785,12 @@ __global__ __launch_bounds__(256) void sel_delta_kernel(const SelPlan P, const _
   }
 #pragma unroll
   for (int m = LPR / 2; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
-  if (row < rows && (tid % LPR) == 0) delta[row] = dlse ? s - dlse[row] : s;
+  if (row < rows && (tid % LPR) == 0) {
+    const float dl = dlse ? s - dlse[row] : s;
+    delta[row] = BLOCK ? -dl : dl;
+    if (BLOCK) delta[rows + row] = -kLog2e * lse[row];
+  }
+  if (BLOCK && blockIdx.x == 0 && tid == 0) *ticket = 0u;
 }
 
 // dQ partial of every (query, slot) pair; same walk and register layout as the forward
@@ -923,9 +930,10 @@ __global__ __launch_bounds__(64) void sel_bwd_dq_kernel(const SelPlan P, const _
   }
 }
 
+// dq = mul * sum of a query's partials
 template <int D>
 __global__ __launch_bounds__(256) void sel_bwd_dq_combine_kernel(const SelPlan P, const void* idx, const uint8_t* fmask, const char* __restrict__ bws,
-                                                                __bf16* __restrict__ dq, float* __restrict__ sel_grads) {
+                                                                const float mul, __bf16* __restrict__ dq, float* __restrict__ sel_grads) {
   constexpr int CPR = D / 8;
   const bool two = merge_two_per_wave(P, CPR);
   const int lane = threadIdx.x & 63, half = two ? lane >> 5 : 0, sub = two ? lane & 31 : lane, width = two ? 32 : 64;
@@ -963,7 +971,7 @@ __global__ __launch_bounds__(256) void sel_bwd_dq_combine_kernel(const SelPlan P
     }
     bf16x8 r;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (__bf16)acc[e];
+    for (int e = 0; e < 8; ++e) r[e] = (__bf16)(mul * acc[e]);
     const long hq = hk * P.g + g;
     *reinterpret_cast<bf16x8*>(dq + (((long)b * P.hkv * P.g + hq) * P.n + i) * D + dd) = r;
   }
@@ -1410,19 +1418,26 @@ static int launch_bwd(const SelPlan& P, const void* q, const void* k, const void
   float* delta = reinterpret_cast<float*>((char*)bws + P.off_delta);
   const long rows = (long)P.bh * P.g * P.n;
   constexpr int RPB = 256 / (D / 8);
-  hipLaunchKernelGGL((sel_delta_kernel<D>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st, P, (const __bf16*)out, (const __bf16*)dout, dlse, delta);
+  unsigned* ticket = reinterpret_cast<unsigned*>((char*)bws + P.off_ticket);
+  const bool fused = sel_grads == nullptr, block = fused && P.block_walk;
+  if (block) hipLaunchKernelGGL((sel_delta_kernel<D, true>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st, P, (const __bf16*)out, (const __bf16*)dout, lse, dlse, delta, ticket);
+  else hipLaunchKernelGGL((sel_delta_kernel<D, false>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st, P, (const __bf16*)out, (const __bf16*)dout, lse, dlse, delta, ticket);
   NSA_LAUNCH_CHECK();
   mark(ev, nev, 1, st);
   // without gate gradients the dQ partials come out of the dK/dV walk (one gather of Q and dO
   // instead of two); with them the separate dQ walk, which also emits sel_grads, is used
-  const bool fused = sel_grads == nullptr;
   if (!fused) {
     hipLaunchKernelGGL((sel_bwd_dq_kernel<D, KT, true>), dim3(xcd_grid(P, 1)), dim3(64), 0, st, P, (const __bf16*)q, (const __bf16*)k, (const __bf16*)v,
                        (const __bf16*)dout, lse, delta, (const char*)iws, (char*)bws, sel_grads);
     NSA_LAUNCH_CHECK();
   }
   mark(ev, nev, 2, st);
-  if (fused) {
+  if (block) {
+    // one work-group a CU, whatever there is to do: those that find no unit end
+    const BlockArgs a = {P, small_div(P.SP), (const __bf16*)q, (const __bf16*)k, (const __bf16*)v, (const __bf16*)dout, delta + rows, delta,
+                         (const char*)iws, (char*)bws, ticket, (__bf16*)dk, (__bf16*)dv};
+    hipLaunchKernelGGL(sel_bwd_block_kernel, dim3(256), dim3(256), 0, st, a);
+  } else if (fused) {
     hipLaunchKernelGGL((sel_bwd_dkv_kernel<D, KT, true>), dim3(P.ub_kv, P.bh), dim3(64 * KT), 0, st, P, (const __bf16*)q, (const __bf16*)k, (const __bf16*)v,
                        (const __bf16*)dout, lse, delta, (const char*)iws, (char*)bws, (__bf16*)dk, (__bf16*)dv);
   } else {
@@ -1432,7 +1447,7 @@ static int launch_bwd(const SelPlan& P, const void* q, const void* k, const void
   NSA_LAUNCH_CHECK();
   mark(ev, nev, 3, st);
   const long nq = (long)P.bh * P.n, qpb = merge_two_per_wave(P, D / 8) ? 8 : 4;
-  hipLaunchKernelGGL((sel_bwd_dq_combine_kernel<D>), dim3((unsigned)((nq + qpb - 1) / qpb)), dim3(256), 0, st, P, idx, fmask, (const char*)bws, (__bf16*)dq, sel_grads);
+  hipLaunchKernelGGL((sel_bwd_dq_combine_kernel<D>), dim3((unsigned)((nq + qpb - 1) / qpb)), dim3(256), 0, st, P, idx, fmask, (const char*)bws, block ? P.scale : 1.0f, (__bf16*)dq, sel_grads);
   NSA_LAUNCH_CHECK();
   mark(ev, nev, 4, st);
   hipLaunchKernelGGL((sel_bwd_dkv_reduce_kernel<D, KT>), dim3(P.W, P.bh), dim3(256), 0, st, P, (const char*)iws, (const char*)bws, (__bf16*)dk, (__bf16*)dv);

@@ -32,14 +32,15 @@ struct SelPlan {
   size_t off_urec[3];        // per (batch*kv head, unit) a record of 8 ints: block, own, list start, v0, v1
   int ub_kv;                 // = ub[2]
   long list_cap;             // inverse-index entries reserved per (batch, kv head)
-  size_t prow;               // number of partial rows; row `prow` is a spare that padding rows write to
+  size_t prow;               // number of partial rows; `g` spare rows behind them are what padding rows write to
   long sq[3], sk[3], sv[3], so[3];
   // index workspace
   size_t off_cnt, off_blk, off_list, index_total;
   // forward workspace
   size_t off_opart, off_lsepart, fwd_total;
   // backward workspace
-  size_t off_delta, off_dqpart, off_dkvpart, bwd_total;
+  size_t off_delta, off_dqpart, off_dkvpart, off_ticket, bwd_total;
+  int block_walk;            // the backward walk without gate gradients is sel_bwd_block_kernel
 };
 
 static inline size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -89,12 +90,24 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
   // are cheaper per pair - but the chip holds 512 to 1024 work-groups of this kernel at a time, and a launch with fewer
   // units than a few rounds of that runs as long as its longest units whatever the rest does (seq 8k, 4 kv heads: 512 units
   // of 1024 pairs occupy half of the SIMDs for the whole launch).  Shorter units when the launch would have under ~4096.
+  // (shapes whose backward walk is sel_bwd_block_kernel where the strides allow it.  With fewer heads a group its row gathers have an
+  // offset per lane: 4096 tokens of 8 / 8 heads 150 us against the two-wave walk's 120, of 8 / 4 heads 109 against 98)
+  const bool long_units = P.D == 128 && P.B > 32 && P.g >= 4;
   {
     const long want = bh * pairs / NSA_DKV_UNITS_WANTED;
     P.chunk[2] = NSA_DKV_CHUNK_FIXED ? NSA_DKV_CHUNK_FIXED : (want >= 1024 ? 1024 : want >= 512 ? 512 : 256);
     // ... down to 64 pairs while there are under 512 of them: 289 tokens of 16 / 2 heads, d 128 138 / 62 us, 1 x 512 of 8 / 2 49 / 28 and of
     // d 128 81 / 54, 1200 of 16 / 2, d 128 154 / 107 (units of 32 pairs: 59, 24, 66, 146; under 1024: 1899 of 16 / 4 83 instead of 71)
     while (P.chunk[2] > 64 && bh * pairs / P.chunk[2] < 512) P.chunk[2] /= 2;
+    // sel_bwd_block_kernel takes a unit with four waves on one of 256 work-groups: few long units, about four for each of them while a
+    // unit is long, one for each below.  us of walk + reduction, 32 / 8 heads, 15 blocks, units of 256 / 512 / 1024 / 2048 pairs: 2048
+    // tokens 155 / 150 / 148, 4096 313 / 273 / 294 / 291, 8192 648 / 550 / 528 / 579, 32768 2630 / 2209 / 2010 / 1987; 16 / 2 heads, 64 / 128 /
+    // 256 / 512 pairs: 289 tokens 46 / 51 / 65 / 69, 1200 98 / 71 / 77 / 110, 2000 163 / 116 / 91 / 117
+    if (long_units && !NSA_DKV_CHUNK_FIXED) {
+      P.chunk[2] = 2048;
+      while (P.chunk[2] > 512 && bh * pairs / P.chunk[2] < 1000) P.chunk[2] /= 2;
+      while (P.chunk[2] > 64 && bh * pairs / P.chunk[2] < 250) P.chunk[2] /= 2;
+    }
   }
   P.phase[2] = ((P.n + 255) / 256) * 256;
   for (int t = 0; t < 3; ++t) {
@@ -122,11 +135,16 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
   P.off_lsepart = o; o = align_up(o + (prow + 1) * 4);
   P.fwd_total = o;
 
+  // sel_bwd_block_kernel addresses a kv head's Q and d_out rows, a block's K and V rows and the pairs of all heads with 32 bits
+  const long far_q = 2 * ((P.n - 1) * P.sq[2] + (P.g - 1) * P.sq[1] + P.D), far_o = 2 * ((P.n - 1) * P.so[2] + (P.g - 1) * P.so[1] + P.D);
+  P.block_walk = long_units && far_q <= 0xffffffffL && far_o <= 0xffffffffL && P.sk[2] >= 0 && P.sk[2] < (1L << 24) && P.sv[2] >= 0 && P.sv[2] < (1L << 24) &&
+                 bh * P.n * P.SP <= 0xffffffffL;
   const int KT = (P.B + 31) / 32;
   o = 0;
-  P.off_delta = o;   o = align_up(o + (size_t)bh * P.g * P.n * 4);
-  P.off_dqpart = o;  o = align_up(o + (prow + 1) * P.D * 2);
+  P.off_delta = o;   o = align_up(o + (size_t)bh * P.g * P.n * (long_units ? 8 : 4));
+  P.off_dqpart = o;  o = align_up(o + (prow + P.g) * P.D * 2);
   P.off_dkvpart = o; o = align_up(o + (size_t)bh * P.ub_kv * 2 * 32 * KT * P.D * 4);
+  P.off_ticket = o;  o = align_up(o + 4);
   P.bwd_total = o;
   return 0;
 }
