@@ -930,10 +930,9 @@ __global__ __launch_bounds__(64) void sel_bwd_dq_kernel(const SelPlan P, const _
   }
 }
 
-// dq = mul * sum of a query's partials
 template <int D>
 __global__ __launch_bounds__(256) void sel_bwd_dq_combine_kernel(const SelPlan P, const void* idx, const uint8_t* fmask, const char* __restrict__ bws,
-                                                                const float mul, __bf16* __restrict__ dq, float* __restrict__ sel_grads) {
+                                                                __bf16* __restrict__ dq, float* __restrict__ sel_grads) {
   constexpr int CPR = D / 8;
   const bool two = merge_two_per_wave(P, CPR);
   const int lane = threadIdx.x & 63, half = two ? lane >> 5 : 0, sub = two ? lane & 31 : lane, width = two ? 32 : 64;
@@ -971,7 +970,7 @@ __global__ __launch_bounds__(256) void sel_bwd_dq_combine_kernel(const SelPlan P
     }
     bf16x8 r;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (__bf16)(mul * acc[e]);
+    for (int e = 0; e < 8; ++e) r[e] = (__bf16)acc[e];
     const long hq = hk * P.g + g;
     *reinterpret_cast<bf16x8*>(dq + (((long)b * P.hkv * P.g + hq) * P.n + i) * D + dd) = r;
   }
@@ -1447,7 +1446,7 @@ static int launch_bwd(const SelPlan& P, const void* q, const void* k, const void
   NSA_LAUNCH_CHECK();
   mark(ev, nev, 3, st);
   const long nq = (long)P.bh * P.n, qpb = merge_two_per_wave(P, D / 8) ? 8 : 4;
-  hipLaunchKernelGGL((sel_bwd_dq_combine_kernel<D>), dim3((unsigned)((nq + qpb - 1) / qpb)), dim3(256), 0, st, P, idx, fmask, (const char*)bws, block ? P.scale : 1.0f, (__bf16*)dq, sel_grads);
+  hipLaunchKernelGGL((sel_bwd_dq_combine_kernel<D>), dim3((unsigned)((nq + qpb - 1) / qpb)), dim3(256), 0, st, P, idx, fmask, (const char*)bws, (__bf16*)dq, sel_grads);
   NSA_LAUNCH_CHECK();
   mark(ev, nev, 4, st);
   hipLaunchKernelGGL((sel_bwd_dkv_reduce_kernel<D, KT>), dim3(P.W, P.bh), dim3(256), 0, st, P, (const char*)iws, (const char*)bws, (__bf16*)dk, (__bf16*)dv);

@@ -40,6 +40,7 @@ __device__ __forceinline__ void mfma32_acc(floatx16& c, const bf16x8& a, const b
   if (FRESH) asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
+typedef __attribute__((address_space(1))) bf16x8* glb_x8;
 typedef __attribute__((address_space(3))) bf16x8* lds_x8;
 typedef __attribute__((address_space(3))) bf16x4* lds_x4;
 typedef __attribute__((address_space(3))) shortx4* lds_s4;
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void s
   const unsigned vq0 = chunk0 + (unsigned)lrow * sqh, vg0 = chunk0 + (unsigned)lrow * soh;
   const unsigned head_q = (unsigned)(n_ & (G - 1)) * sqh, head_g = (unsigned)(n_ & (G - 1)) * soh;
   const unsigned pair_bytes = (unsigned)G * (D * 2);
-  const float sc = A0->P.scale * kLog2e;
+  const float scale = A0->P.scale, sc = scale * kLog2e;
   const unsigned head_d = (unsigned)(n_ & (G - 1)) * (D * 2);
   char* const dqpart = A0->bws + A0->P.off_dqpart;
   char* const spare = dqpart + (unsigned long)((unsigned)A0->P.bh * per_head) * pair_bytes;
@@ -314,7 +315,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void s
     const int dt = c / 4, a = c % 4;
     bf16x4 r;
 #pragma unroll
-    for (int bb = 0; bb < 4; ++bb) r[bb] = (__bf16)Qa[dt][4 * a + bb];
+    for (int bb = 0; bb < 4; ++bb) r[bb] = (__bf16)(Qa[dt][4 * a + bb] * scale);
     *(lds_x4)(stw_a ^ (unsigned)(16 * c)) = r;
   };
   bf16x8 vv[NT];
@@ -323,7 +324,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void s
     vv[t] = lds_read8((str_a ^ (unsigned)(64 * (t & 3))) + t * 1024);
     pr[t] = pair_s[wave][slot][t * RPI + lrow_];
   };
-  auto store_dq = [&](int t) { __builtin_nontemporal_store(vv[t], reinterpret_cast<bf16x8*>(pr[t] + 16 * pos)); };
+  auto store_dq = [&](int t) { __builtin_nontemporal_store(vv[t], (glb_x8)(pr[t] + 16 * pos)); };
 
   constexpr int AH = 4, RING = AH + DT + 1;      // operands read ahead
   constexpr int mB = 2 * KS, mC = 4 * KS, mD = mC + 4 * DT, mE = mD + 4 * DT, mN = mE + 4 * DT;      // first MFMA of each phase
@@ -602,7 +603,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void s
       for (int i = 0; i < 64 * FPR / 256; ++i) {
         const int e = td + 256 * i, kl = e / FPR, c = e % FPR, col = half * (D / 2) + 4 * c;
         if (single_unit) {
-          const float mlt = which == 0 ? A->P.scale : 1.0f;
+          const float mlt = which == 0 ? scale : 1.0f;
           if (kl < keys) store4_bf16((which == 0 ? A->dk : A->dv) + ((size_t)done_bh * A->P.n + (size_t)done_blk * blockB + kl) * D + col, sum[i][0] * mlt, sum[i][1] * mlt, sum[i][2] * mlt, sum[i][3] * mlt);
         } else {
           *reinterpret_cast<floatx4*>(part + which * 64 * D + (size_t)kl * D + col) = sum[i];

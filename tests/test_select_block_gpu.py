@@ -28,8 +28,8 @@ def test_against_the_oracle(b, hq, hk, n, d, B, S):
 @pytest.mark.parametrize("layout", ["heads", "tokens", "sliced"])
 @pytest.mark.parametrize("b,hq,hk,n,B,S", [(2, 16, 2, 509, 64, 4), (1, 4, 1, 1300, 40, 15)])
 def test_against_the_other_walks(b, hq, hk, n, B, S, layout, causal):
-    """Same blocks, same sums: what differs is the order of fp32 additions and where the scale meets the rounding of a dQ partial
-    (bf16, half an ulp each: 2^-8 of a partial, less of the sum of several)."""
+    """Same blocks, same sums: what differs is the order of fp32 additions, which moves a bf16 result (or partial, or dS) by an ulp where it
+    lies near the middle of two: 2^-8 of the few it does that to."""
     from native_sparse_attention_pytorch_amd import native_sparse_attend
     print(f"case {b} {hq} {hk} {n} {B} {S} {layout} {causal}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(n + S)
@@ -55,7 +55,7 @@ def test_against_the_other_walks(b, hq, hk, n, B, S, layout, causal):
         ((out.float() * do.float()).sum() + (0.1 * lse.masked_fill(dead, 0.)).sum()).backward()
         grads.append([t.grad.float() for t in leaves])
     torch.cuda.synchronize()
-    for name, x, y, tol in zip("qkv", *grads, (2 ** -7, 2 ** -9, 2 ** -9)):
+    for name, x, y, tol in zip("qkv", *grads, (2 ** -8, 2 ** -9, 2 ** -9)):
         assert torch.isfinite(x).all(), name
         err = ((x - y).norm() / y.norm()).item()
         assert err < tol, (name, err)
