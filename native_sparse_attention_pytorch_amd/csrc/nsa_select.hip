@@ -361,6 +361,10 @@ static inline unsigned xcd_grid(const SelPlan& P, int t) {
   return 8u * (unsigned)((P.ub[t] + nsub_min - 1) / nsub_min);
 }
 
+}  // namespace nsa
+#include "nsa_select_fwd_rows.hpp"
+namespace nsa {
+
 struct RowInfo {
   int i, slot, lim, g;
   bool valid;
@@ -1377,8 +1381,16 @@ template <int D, int KT>
 static int launch_fwd(const SelPlan& P, const void* q, const void* k, const void* v, const void* idx, const uint8_t* fmask,
                       const void* iws, void* fws, void* out, float* lse, hipStream_t st, void* const* ev, int nev) {
   mark(ev, nev, 0, st);
-  hipLaunchKernelGGL((sel_fwd_kernel<D, KT>), dim3(xcd_grid(P, 0)), dim3(64), 0, st, P, (const __bf16*)q, (const __bf16*)k, (const __bf16*)v,
-                     (const char*)iws, (char*)fws);
+  // (blocks of 17 .. 32 keys stay with the register-staged walk: 8192 tokens, 32 / 8 heads, d 128, 32 keys 150 us against 164, 6000 tokens
+  // of 16 / 4 heads, d 64 57 against 58; of 16 keys, 4096 tokens, 8 / 8 heads, d 128 27 against 22, 8 x 1024 of 8 / 4 heads, d 64 21 against 18.6)
+  const bool by_dma = P.near_rows && (P.B > 32 || P.B <= 16);
+  if (by_dma && P.g * D >= 512)
+    hipLaunchKernelGGL((sel_fwd_rows_kernel<D, KT, true>), dim3(xcd_grid(P, 0)), dim3(64), 0, st, P, small_div(P.SP), (const __bf16*)q, (const __bf16*)k, (const __bf16*)v, (const char*)iws, (char*)fws);
+  else if (by_dma)
+    hipLaunchKernelGGL((sel_fwd_rows_kernel<D, KT, false>), dim3(xcd_grid(P, 0)), dim3(64), 0, st, P, small_div(P.SP), (const __bf16*)q, (const __bf16*)k, (const __bf16*)v, (const char*)iws, (char*)fws);
+  else
+    hipLaunchKernelGGL((sel_fwd_kernel<D, KT>), dim3(xcd_grid(P, 0)), dim3(64), 0, st, P, (const __bf16*)q, (const __bf16*)k, (const __bf16*)v,
+                       (const char*)iws, (char*)fws);
   NSA_LAUNCH_CHECK();
   mark(ev, nev, 1, st);
   const long nq = (long)P.bh * P.n, qpb = merge_two_per_wave(P, D / 8) ? 8 : 4;      // queries per work-group of the merge

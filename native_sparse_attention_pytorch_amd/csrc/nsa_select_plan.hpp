@@ -40,6 +40,7 @@ struct SelPlan {
   size_t off_opart, off_lsepart, fwd_total;
   // backward workspace
   size_t off_delta, off_dqpart, off_dkvpart, off_ticket, bwd_total;
+  int near_rows;             // byte offsets of a kv head's Q rows fit 32 bits
   int block_walk;            // the backward walk without gate gradients is sel_bwd_block_kernel
 };
 
@@ -137,7 +138,8 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
 
   // sel_bwd_block_kernel addresses a kv head's Q and d_out rows, a block's K and V rows and the pairs of all heads with 32 bits
   const long far_q = 2 * ((P.n - 1) * P.sq[2] + (P.g - 1) * P.sq[1] + P.D), far_o = 2 * ((P.n - 1) * P.so[2] + (P.g - 1) * P.so[1] + P.D);
-  P.block_walk = long_units && far_q <= 0xffffffffL && far_o <= 0xffffffffL && P.sk[2] >= 0 && P.sk[2] < (1L << 24) && P.sv[2] >= 0 && P.sv[2] < (1L << 24) &&
+  P.near_rows = far_q <= 0xffffffffL;
+  P.block_walk = long_units && P.near_rows && far_o <= 0xffffffffL && P.sk[2] >= 0 && P.sk[2] < (1L << 24) && P.sv[2] >= 0 && P.sv[2] < (1L << 24) &&
                  bh * P.n * P.SP <= 0xffffffffL;
   const int KT = (P.B + 31) / 32;
   o = 0;
