@@ -561,7 +561,11 @@ __global__ __launch_bounds__(256, 2) void dense_bwd_dq_kernel(const DensePlan P,
       for (int e = 0; e < 8; ++e) del_r = __builtin_fmaf((float)o8[e], (float)Gf[ks][e], del_r);
     }
     del_r = halves_sum(del_r);
-    if (valid && h == 0) delta[srow] = del_r;
+    // at 128 features negated, and behind all of them -lse log2e: as the dK / dV walk's products and exponents take them
+    if (valid && h == 0) {
+      delta[srow] = D == 128 ? -del_r : del_r;
+      if constexpr (D == 128) delta[(long)P.bh * P.g * P.n + srow] = -lse_r;
+    }
   }
   const Interval me = visible_range(P, i);
   const TileWalk walk = make_walk(P, q0, min(P.n - 1, q0 + 4 * ppt - 1));
@@ -708,14 +712,15 @@ __device__ __forceinline__ void chunk_range(const DensePlan& P, int T, int c, in
 // Work-group x of the dK/dV walk -> (key tile T, query chunk c); false for the padding ids of the grid.  Band mode:
 // tile-major, one contiguous range of key tiles per XCD (neighbouring tiles see almost the same queries).  Stride mode:
 // all key tiles of a query chunk on one XCD (they stream the same Q / dO rows), chunks dealt to the XCDs in a zig-zag
-// (rounds of 8 chunks, every other round reversed) because under the causal mask a later chunk sees more key tiles.
+// (rounds of 8 chunks, every other round reversed) because under the causal mask a later chunk sees more key tiles, and
+// from another XCD on for each kv head: fewer than 16 chunks fill no whole zig-zag.
 __device__ __forceinline__ bool chunk_of(const DensePlan& P, int x, int& T, int& c, int& qlo, int& qhi, int& c0, int& c1) {
   if (P.mode == 0) {
     const int v = xcd_contiguous(x, P.key_tiles * P.chunks);
     if (v >= P.key_tiles * P.chunks) return false;
     T = v / P.chunks; c = v % P.chunks;
   } else {
-    const int xc = x & 7, idx = x >> 3, round = idx / P.key_tiles;
+    const int xc = (x + (int)blockIdx.y * (P.chunks | 1)) & 7, idx = x >> 3, round = idx / P.key_tiles;
     T = idx % P.key_tiles;
     c = 8 * round + ((round & 1) ? 7 - xc : xc);
     if (c >= P.chunks) return false;
@@ -727,11 +732,12 @@ static inline unsigned dkv_grid(const DensePlan& P) {
   return P.mode == 0 ? xcd_grid_for(P.key_tiles * P.chunks) : 8u * (unsigned)(((P.chunks + 7) / 8) * P.key_tiles);
 }
 
+}  // namespace nsa
+#include "nsa_dense_bwd_keys.hpp"
+namespace nsa {
+
 #ifndef NSA_DKV_AHEAD
 #define NSA_DKV_AHEAD 3
-#endif
-#ifndef NSA_DKV_PIPE_MIN_D
-#define NSA_DKV_PIPE_MIN_D 128    // head dimensions from here on take dense_bwd_dkv_pipe_kernel (one wave per SIMD)
 #endif
 #ifndef NSA_DKV_STAGES
 #define NSA_DKV_STAGES 1      // measured on MI355X (compressed branch, seq 32k, d 128): 1, 2 or 3 tiles ahead all 4.7 ms
@@ -818,7 +824,7 @@ __global__ __launch_bounds__(128) void dense_bwd_dkv_kernel(const DensePlan P, c
     }
     if (kt == 0 && h == 0) {
       lse_s[n_] = valid ? cur.lse_r * kLog2e : INFINITY;   // +inf: a padding row gets p = 0
-      del_s[n_] = cur.del_r;
+      del_s[n_] = D == 128 ? -cur.del_r : cur.del_r;
       const Interval me = visible_range(P, i);
       lo_s[n_] = P.mode == 0 ? me.lo : 0;
       hi_s[n_] = P.mode == 0 ? me.hi : me.hi + P.mem;
@@ -909,7 +915,8 @@ __global__ __launch_bounds__(128) void dense_bwd_dkv_kernel(const DensePlan P, c
     }
 }
 
-// The same walk for head dimensions whose accumulators leave room for one wave per SIMD only (d = 128: 128 registers of dK / dV
+// The same walk for 128 features and bands whose tiles few rows see (more rows: dense_bwd_dkv_keys_kernel).  The accumulators leave room for
+// one wave per SIMD only (128 registers of dK / dV
 // accumulators, 64 of K / V operands).  With one wave per SIMD nothing overlaps a wave's MFMAs but its own instruction order,
 // so the step is laid out by hand and fenced (cycle stamps of the kernel above at d = 128: 23 % of a step in the tile's LDS
 // write, 11 % in two barriers, 6 % issuing loads, and the softmax entirely outside the MFMA runs):
@@ -1021,7 +1028,7 @@ __global__ __launch_bounds__(128) void dense_bwd_dkv_pipe_kernel(const DensePlan
     if (ktu == 0) {
       if (h == 0) {
         lse_s[buf][n_] = i0 + pq < c1 ? lse_r * kLog2e : INFINITY;   // +inf: a padding row gets p = 0
-        del_s[buf][n_] = del_r;
+        del_s[buf][n_] = D == 128 ? -del_r : del_r;
       }
     } else if (!whole_tile_visible(i0)) {
       if (h == 0) {
@@ -1290,9 +1297,14 @@ static int dense_bwd_launch(const DensePlan& P, const void* q, const void* k, co
                      (const __bf16*)v, (const __bf16*)out, (const __bf16*)dout, lse, delta, (__bf16*)dq);      // also writes delta
   NSA_LAUNCH_CHECK();
   const auto group_span = [&](const long* st) { return (long)(P.g - 1) * st[1] + (long)(P.n - 1) * st[2] + D; };
-  // the pipelined kernel's buffer loads take 32-bit byte offsets within one kv head's query heads (rows) and their lse / delta
-  if (D >= NSA_DKV_PIPE_MIN_D && group_span(P.sq) < (1l << 30) && group_span(P.sdo) < (1l << 30) && (long)P.g * P.n < (1l << 29))
-    hipLaunchKernelGGL((dense_bwd_dkv_pipe_kernel<D>), dim3(dkv_grid(P), P.bh), dim3(128), 0, st, P, (const __bf16*)q, (const __bf16*)k,
+  // buffer loads with 32-bit byte offsets within one kv head's query heads (rows) and their lse / delta
+  const bool near = D == 128 && group_span(P.sq) < (1l << 30) && group_span(P.sdo) < (1l << 30) && (long)P.g * P.n < (1l << 29);
+  // (the keys walk masks scores before they are scaled, and requests a tile's 64 rows of k / v from one base)
+  if (near && P.keys_walk && P.scale > 0.f && P.sk[2] < (1l << 24) && P.sv[2] < (1l << 24))
+    hipLaunchKernelGGL(dense_bwd_dkv_keys_kernel, dim3(dkv_grid(P), P.bh), dim3(256), 0, st, P, (const __bf16*)q, (const __bf16*)k,
+                       (const __bf16*)v, (const __bf16*)dout, delta, part);
+  else if (near)
+    hipLaunchKernelGGL((dense_bwd_dkv_pipe_kernel<128>), dim3(dkv_grid(P), P.bh), dim3(128), 0, st, P, (const __bf16*)q, (const __bf16*)k,
                        (const __bf16*)v, (const __bf16*)dout, lse, delta, part);
   else
     hipLaunchKernelGGL((dense_bwd_dkv_kernel<D>), dim3(dkv_grid(P), P.bh), dim3(128), 0, st, P, (const __bf16*)q, (const __bf16*)k,

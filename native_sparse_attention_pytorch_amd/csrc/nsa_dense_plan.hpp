@@ -17,6 +17,7 @@ struct DensePlan {
   int accumulate;            // the backward adds to what dq, dk and dv (bf16) hold
   float scale;
   int key_tiles, chunks, chunk_q;
+  int keys_walk;             // dK / dV by dense_bwd_dkv_keys_kernel (strides and scale allowing)
   long sq[3], sk[3], sv[3], so[3], sdo[3];
   size_t off_delta, off_part, bwd_total;
 };
@@ -71,22 +72,32 @@ static inline int make_dense_plan(const nsa_dense_desc* d, DensePlan& P) {
   // are cut into chunks of chunk_q; smaller chunks when there would be too few work-groups
   P.key_tiles = (P.krows + 63) / 64;
   const long span = P.mode == 0 ? ((long)64 + P.wb + P.wf < P.n ? (long)64 + P.wb + P.wf : P.n) : P.n;
-#ifndef NSA_DKV_MIN_WGS
-#define NSA_DKV_MIN_WGS 2048
-#endif
+  // At 128 features the keys walk, one work-group of it a CU, except for bands whose tiles few rows see: from 640 rows a tile on it is the
+  // faster one (dq + dK / dV, 2 x 8 heads, 8192 tokens, window 128: 192 rows, 169 us by the pipelined walk, 190 by the keys walk; window 512:
+  // 576 rows, 251 and 255; 32 / 8 heads, 8192 tokens, window 512: 2304 rows, 402 and 358).
+  P.keys_walk = P.D == 128 && (P.mode == 1 || span * P.g >= 640);
+  const auto groups = [&] { return bh * P.key_tiles * ((span + P.chunk_q - 1) / P.chunk_q); };
   if (P.mode == 0) {
-    // band: a tile's visible queries (64 + window of them) in equal chunks, as few as give the chip NSA_DKV_MIN_WGS work-groups
-    // (a chunk of 512 beside one of 64 is a work-group that runs eight times longer than its neighbour)
-    long want = (NSA_DKV_MIN_WGS + bh * P.key_tiles - 1) / (bh * P.key_tiles);
+    // band: a tile's visible queries (64 + window of them) in equal chunks, as few as give the chip so many work-groups
+    // (a chunk of 512 beside one of 64 is a work-group that runs eight times longer than its neighbour).  The keys walk's own 14 000 cycles
+    // before and behind its loop want few: 4096 tokens, 32 / 8 heads, window 512, from 512 on 186 us, from 768 on 216, from 2048 on 291.
+    const long from = P.keys_walk ? 512 : 2048;
+    long want = (from + bh * P.key_tiles - 1) / (bh * P.key_tiles);
     want = std::max<long>(1, std::min<long>(want, (span + 127) / 128));
     P.chunk_q = (int)(((span + want - 1) / want + 31) / 32 * 32);
+  } else if (P.keys_walk) {
+    // 8192 rows (4 MB of Q and dO: an XCD's cache), down to 2048 while there are fewer than four work-groups a CU (32 / 8 heads of compressed
+    // attention, dq + dK / dV: 8192 tokens 260 us, 318 with 4096 rows; 32768 tokens 2018 us, 2130 with 4096), on to 128 queries below two
+    P.chunk_q = 8192 >> P.lg;
+    while (P.chunk_q > 128 && P.chunk_q > (2048 >> P.lg) && groups() < 1024) P.chunk_q /= 2;
+    while (P.chunk_q > 128 && groups() < 512) P.chunk_q /= 2;
   } else {
     P.chunk_q = 1024;
-    while (P.chunk_q > 128 && bh * P.key_tiles * ((span + P.chunk_q - 1) / P.chunk_q) < 2048) P.chunk_q /= 2;
+    while (P.chunk_q > 128 && groups() < 2048) P.chunk_q /= 2;
   }
   P.chunks = (int)((span + P.chunk_q - 1) / P.chunk_q);
   size_t o = 0;
-  P.off_delta = o; o = dense_align_up(o + (size_t)bh * P.g * P.n * 4);
+  P.off_delta = o; o = dense_align_up(o + (size_t)bh * P.g * P.n * (P.D == 128 ? 8 : 4));      // delta, and at 128 features -lse log2e
   P.off_part = o;  o = dense_align_up(o + (size_t)bh * P.key_tiles * P.chunks * 2 * 64 * P.D * 4);
   P.bwd_total = o;
   return 0;
