@@ -140,7 +140,7 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
   const long far_q = 2 * ((P.n - 1) * P.sq[2] + (P.g - 1) * P.sq[1] + P.D), far_o = 2 * ((P.n - 1) * P.so[2] + (P.g - 1) * P.so[1] + P.D);
   P.near_rows = far_q <= 0xffffffffL;
   P.block_walk = long_units && P.near_rows && far_o <= 0xffffffffL && P.sk[2] >= 0 && P.sk[2] < (1L << 24) && P.sv[2] >= 0 && P.sv[2] < (1L << 24) &&
-                 bh * P.n * P.SP <= 0xffffffffL;
+                 bh * P.n * P.SP <= 0xffffffffL && P.scale > 0.f;      // (masked scores are -inf before they are scaled)
   const int KT = (P.B + 31) / 32;
   o = 0;
   P.off_delta = o;   o = align_up(o + (size_t)bh * P.g * P.n * (long_units ? 8 : 4));
