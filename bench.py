@@ -32,8 +32,8 @@ CFG = dict(batch=1, seq=32768, heads=32, kv_heads=8, dim_head=128, block=64, num
 # HBM bytes per launch on this workload come from the tracked rocprofv3 summary (FETCH_SIZE / WRITE_SIZE per dispatch,
 # scaled by streaming kernels of known size; the file states the commands), not from literals kept here
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "select_fwd_bwd_seq32k_hbm_traffic.txt")
-TRAFFIC_KERNELS = {"sel_fwd_kernel": "fwd_block_walk", "sel_fwd_combine_kernel": "fwd_merge", "sel_bwd_dq_combine_kernel": "bwd_dq_merge",
-                   "sel_bwd_dkv_kernel": "bwd_dkv_walk", "sel_bwd_dkv_reduce_kernel": "bwd_dkv_reduce", "sel_delta_kernel": "bwd_delta"}
+TRAFFIC_KERNELS = {"sel_fwd_rows_kernel": "fwd_block_walk", "sel_fwd_combine_kernel": "fwd_merge", "sel_bwd_dq_combine_kernel": "bwd_dq_merge",
+                   "sel_bwd_block_kernel": "bwd_dkv_walk", "sel_bwd_dkv_reduce_kernel": "bwd_dkv_reduce", "sel_delta_kernel": "bwd_delta"}
 
 
 def measured_traffic_bytes():

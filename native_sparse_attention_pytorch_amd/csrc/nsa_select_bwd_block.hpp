@@ -16,7 +16,7 @@
 //     c ^ 4 (r % 4): row reads and transpose loads both without bank conflicts.
 //   * work-groups stay and take units by number (an atomic counter; what a unit computes does not depend on who takes it), so that
 //     the next unit's lists, K and V rows and first tiles are under way while the sums of the last one are written.
-// Measured (MI355X): 2.54 -> 1.92 ms at seq 32k, 32 / 8 heads; 384 -> 269 us with its reduction at seq 4k.  In the loop the gathers
+// Measured (MI355X): 2.54 -> 1.86 ms at seq 32k, 32 / 8 heads; 384 -> 269 us with its reduction at seq 4k.  In the loop the gathers
 // and stores now run at what the memory gives their pattern (8.3 TB/s); 15 % of the time are the units' ends.  The same walk at 64
 // features, where a step has half the MFMAs and the same softmax, was slower than the two-wave walk (190 against 170 us at seq 8k).
 #pragma once
