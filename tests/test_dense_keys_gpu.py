@@ -35,6 +35,9 @@ def make(b, h, n, layout, g):
         return torch.randn(b, n, h, 128, generator=g, device="cuda").bfloat16().transpose(1, 2)
     if layout == "sliced":      # rows that start 16 bytes into wider ones
         return torch.randn(b, h, n, 144, generator=g, device="cuda").bfloat16()[..., 8:136]
+    if layout == "far":         # rows 2 MB apart: beyond the 32-bit offsets of all but the general walk
+        t = torch.empty(b, n, 2 ** 20, dtype=torch.bfloat16, device="cuda")[..., :128 * h].unflatten(2, (h, 128)).transpose(1, 2)
+        return t.copy_(torch.randn(b, h, n, 128, generator=g, device="cuda"))
     return torch.randn(b, h, n, 128, generator=g, device="cuda").bfloat16()
 
 
@@ -55,8 +58,10 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("layout", ["heads", "tokens", "sliced"])
-@pytest.mark.parametrize("mode,b,hq,hk,n,ws,mem,causal", CASES)
+@pytest.mark.parametrize("mode,b,hq,hk,n,ws,mem,causal,layout", [(*c, layout) for c in CASES for layout in ("heads", "tokens", "sliced")] + [
+    (0, 1, 4, 1, 1100, 300, 0, True, "far"),
+    (1, 1, 4, 2, 1100, 8, 1, True, "far"),
+])
 def test_against_float64(mode, b, hq, hk, n, ws, mem, causal, layout):
     """p and dS are rounded to bf16 and so are the results, 2^-9 each; out, which delta is taken from, adds as much to dS."""
     from native_sparse_attention_pytorch_amd import ops
@@ -65,7 +70,8 @@ def test_against_float64(mode, b, hq, hk, n, ws, mem, causal, layout):
     window, stride = (ws, 1) if mode == 0 else (0, ws)
     nkeys = n if mode == 0 else n // stride
     q, do = make(b, hq, n, layout, g), make(b, hq, n, layout, g)
-    k, v = make(b, hk, nkeys + mem, layout, g), make(b, hk, nkeys + mem, layout, g)
+    rows = "heads" if layout == "far" else layout
+    k, v = make(b, hk, nkeys + mem, rows, g), make(b, hk, nkeys + mem, rows, g)
     scale = 128 ** -0.5
     out, lse, _ = ops.dense_fwd(q, k, v, mode, causal, window, stride, mem, 0, 1, True, scale)
     grads = ops.dense_bwd(q, k, v, out, do, lse, mode, causal, window, stride, mem, scale)
