@@ -1367,7 +1367,7 @@ extern "C" int nsa_select_build_index(const nsa_select_desc* d, const void* idx,
   NSA_LAUNCH_CHECK();
   hipLaunchKernelGGL(sel_scan_kernel, dim3(P.bh), dim3(256), lds, st, P, iws);
   NSA_LAUNCH_CHECK();
-  hipLaunchKernelGGL(sel_units_kernel, dim3(P.bh, 3), dim3(1024), 0, st, P, iws);
+  hipLaunchKernelGGL(sel_units_kernel, dim3(P.bh, P.tables), dim3(1024), 0, st, P, iws);
   NSA_LAUNCH_CHECK();
   if (4 * lds <= 65536)
     hipLaunchKernelGGL(sel_fill_kernel<4>, dim3(P.nch, P.bh), dim3(256), 4 * lds, st, P, idx, fmask, iws);
@@ -1423,14 +1423,18 @@ extern "C" int nsa_select_fwd(const nsa_select_desc* d, const void* q, const voi
 }
 
 template <int D, int KT>
-static int launch_bwd(const SelPlan& P, const void* q, const void* k, const void* v, const void* out, const void* dout, const float* dlse, const float* lse,
+static int launch_bwd(const SelPlan& plan, const void* q, const void* k, const void* v, const void* out, const void* dout, const float* dlse, const float* lse,
                       const void* idx, const uint8_t* fmask, const void* iws, void* bws, void* dq, void* dk, void* dv, float* sel_grads, hipStream_t st, void* const* ev, int nev) {
   mark(ev, nev, 0, st);
+  const bool fused = sel_grads == nullptr, block = fused && plan.block_walk;
+  SelPlan P = plan;
+  if (!block && P.tables == 4) {      // the two-wave walk and the sum behind it find their own units as table 2
+    P.chunk[2] = P.chunk[3]; P.np[2] = P.np[3]; P.ub[2] = P.ub_kv = P.ub[3]; P.off_unit[2] = P.off_unit[3]; P.off_urec[2] = P.off_urec[3];
+  }
   float* delta = reinterpret_cast<float*>((char*)bws + P.off_delta);
   const long rows = (long)P.bh * P.g * P.n;
   constexpr int RPB = 256 / (D / 8);
   unsigned* ticket = reinterpret_cast<unsigned*>((char*)bws + P.off_ticket);
-  const bool fused = sel_grads == nullptr, block = fused && P.block_walk;
   if (block) hipLaunchKernelGGL((sel_delta_kernel<D, true>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st, P, (const __bf16*)out, (const __bf16*)dout, lse, dlse, delta, ticket);
   else hipLaunchKernelGGL((sel_delta_kernel<D, false>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st, P, (const __bf16*)out, (const __bf16*)dout, lse, dlse, delta, ticket);
   NSA_LAUNCH_CHECK();

@@ -26,13 +26,14 @@ struct SelPlan {
   // cell; cells are ordered phase-major so that units running at the same time gather Q rows of
   // the same query range (L2 reuse).  Table t: 0 = forward walk, 1 = dQ walk, 2 = dK/dV walk
   // (a single phase: the whole sequence, so a wave keeps its dK/dV accumulators as long as
-  // possible).
-  int chunk[3], phase[3], np[3], ub[3];
-  size_t off_unit[3];
-  size_t off_urec[3];        // per (batch*kv head, unit) a record of 8 ints: block, own, list start, v0, v1
-  int ub_kv;                 // = ub[2]
+  // possible), 3 = the same for sel_bwd_dkv_kernel where sel_bwd_block_kernel reads table 2.
+  int tables;                // 3, or 4 where both dK/dV walks may run: which of them does, each backward call decides
+  int chunk[4], phase[4], np[4], ub[4];
+  size_t off_unit[4];
+  size_t off_urec[4];        // per (batch*kv head, unit) a record of 8 ints: block, own, list start, v0, v1
+  int ub_kv;                 // dK/dV partials reserved per (batch, kv head): the longer of the tables
   long list_cap;             // inverse-index entries reserved per (batch, kv head)
-  size_t prow;               // number of partial rows; `g` spare rows behind them are what padding rows write to
+  size_t prow;               // number of partial rows; padding rows write to the spare rows behind them: one in the forward, g in the backward
   long sq[3], sk[3], sv[3], so[3];
   // index workspace
   size_t off_cnt, off_blk, off_list, index_total;
@@ -94,6 +95,8 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
   // (shapes whose backward walk is sel_bwd_block_kernel where the strides allow it.  With fewer heads a group its row gathers have an
   // offset per lane: 4096 tokens of 8 / 8 heads 150 us against the two-wave walk's 120, of 8 / 4 heads 109 against 98)
   const bool long_units = P.D == 128 && P.B > 32 && P.g >= 4;
+  P.tables = long_units ? 4 : 3;
+  P.chunk[3] = 0;
   {
     const long want = bh * pairs / NSA_DKV_UNITS_WANTED;
     P.chunk[2] = NSA_DKV_CHUNK_FIXED ? NSA_DKV_CHUNK_FIXED : (want >= 1024 ? 1024 : want >= 512 ? 512 : 256);
@@ -108,24 +111,37 @@ static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
       P.chunk[2] = 2048;
       while (P.chunk[2] > 512 && bh * pairs / P.chunk[2] < 1000) P.chunk[2] /= 2;
       while (P.chunk[2] > 64 && bh * pairs / P.chunk[2] < 250) P.chunk[2] /= 2;
+      // The two-wave walk at these shapes (gate gradients, far strides) has 512 work-groups on the chip and wants twice the units while they
+      // are short of 1024 pairs; slots beyond the number of blocks are dead.  us of a backward with gate gradients, units of 64 / 128 / 256 /
+      // 512 / 1024 / 2048 pairs: 16 / 2 heads, 15 blocks: 1000 tokens 129 / 125, 2000 218 / - / 203, 3000 300 / 267 / 245, 4096 383 / 324 /
+      // 331 / 360, 8192 822 / 649 / 667 / 706; 32 / 8 heads, 16 blocks: 400 tokens 70 / 72, 1024 180 / 157 / 141 / 177, 2048 - / 307 / 277 / 291,
+      // 4096 - / 681 / 620 / 588 / 625, 8192 - / - / 1286 / 1237 / 1234 / 1377, 16384 - / - / 2571 / 2455 / 2470 / 2545, 32768 - / - / 5150 /
+      // 4905 / 4937 / 4820
+      const long live = bh * P.n * ((P.S < P.W ? P.S : P.W) + P.causal);
+      P.chunk[3] = live / 2048 >= 2000 ? 2048 : 1024;
+      while (P.chunk[3] > 256 && live / P.chunk[3] < 1000) P.chunk[3] /= 2;
+      while (P.chunk[3] > 64 && live / P.chunk[3] < 250) P.chunk[3] /= 2;
+    } else if (long_units) {
+      P.chunk[3] = P.chunk[2];
     }
   }
-  P.phase[2] = ((P.n + 255) / 256) * 256;
-  for (int t = 0; t < 3; ++t) {
+  P.phase[2] = P.phase[3] = ((P.n + 255) / 256) * 256;
+  P.np[3] = P.ub[3] = 0;
+  for (int t = 0; t < P.tables; ++t) {
     P.np[t] = (P.n + P.phase[t] - 1) / P.phase[t];
     const long cells = (long)P.np[t] * P.W;
     const long ub = cells + (pairs + P.chunk[t] - 1) / P.chunk[t];
     if (ub > 0x3fffffffL) return NSA_E_UNSUPPORTED;
     P.ub[t] = (int)ub;
   }
-  P.ub_kv = P.ub[2];
+  P.ub_kv = P.ub[2] > P.ub[3] ? P.ub[2] : P.ub[3];
   P.list_cap = (long)P.n * (P.S > 0 ? P.S : 1);
 
   size_t o = 0;
   P.off_cnt = o;    o = align_up(o + (size_t)bh * P.nch * P.W * 4);
   P.off_blk = o;    o = align_up(o + (size_t)bh * (P.W + 1) * 4);
-  for (int t = 0; t < 3; ++t) { P.off_unit[t] = o; o = align_up(o + (size_t)bh * ((size_t)P.np[t] * P.W + 1) * 4); }
-  for (int t = 0; t < 3; ++t) { P.off_urec[t] = o; o = align_up(o + (size_t)bh * (size_t)P.ub[t] * 32); }
+  for (int t = 0; t < P.tables; ++t) { P.off_unit[t] = o; o = align_up(o + (size_t)bh * ((size_t)P.np[t] * P.W + 1) * 4); }
+  for (int t = 0; t < P.tables; ++t) { P.off_urec[t] = o; o = align_up(o + (size_t)bh * (size_t)P.ub[t] * 32); }
   P.off_list = o;   o = align_up(o + (size_t)bh * P.list_cap * 4);
   P.index_total = o;
 

@@ -59,3 +59,21 @@ def test_against_the_other_walks(b, hq, hk, n, B, S, layout, causal):
         assert torch.isfinite(x).all(), name
         err = ((x - y).norm() / y.norm()).item()
         assert err < tol, (name, err)
+
+
+@pytest.mark.parametrize("hq,hk,n,S", [(32, 8, 1024, 16), (16, 2, 4100, 15), (8, 2, 1500, 4)])
+def test_both_backwards_of_one_index(hq, hk, n, S):
+    """The walks with and without gate gradients have unit tables of their own in an index: either reads its own, whichever ran before.
+    (Tolerance: test_against_the_other_walks.)"""
+    from native_sparse_attention_pytorch_amd import ops
+    print(f"case {hq} {hk} {n} {S}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q, k, v, do = ((torch.randn(1, h, n, 128, generator=g, device="cuda") * 128 ** -0.25).bfloat16() for h in (hq, hk, hk, hq))
+    idx, live = (t.cuda() for t in causal_random_selection(1, hk, n, 64, S, seed=7))
+    out, lse, index = ops.select_fwd(q, k, v, idx, live, None, 64, True, 128 ** -0.5)
+    runs = [ops.select_bwd(q, k, v, out, do, lse, idx, live, index, 64, True, 128 ** -0.5, gated)[:3] for gated in (True, False, True)]
+    torch.cuda.synchronize()
+    for name, x, y, z, tol in zip("qkv", *runs, (2 ** -8, 2 ** -9, 2 ** -9)):
+        assert torch.equal(x, z), name
+        err = ((y.float() - x.float()).norm() / x.float().norm()).item()
+        assert err < tol, (name, err)
