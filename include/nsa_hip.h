@@ -136,6 +136,7 @@ typedef struct nsa_dense_desc {
   int64_t q_stride[3], k_stride[3], v_stride[3], o_stride[3], do_stride[3];
 } nsa_dense_desc;
 
+/* Scratch of the backward that `d` describes, strides and scale included: they decide which walk it takes. */
 int nsa_dense_workspace_bytes(const nsa_dense_desc* d, size_t* bwd_bytes);
 int nsa_dense_fwd(const nsa_dense_desc* d, const void* q, const void* k, const void* v,
                   void* out, float* lse, float* pooled, void* stream);

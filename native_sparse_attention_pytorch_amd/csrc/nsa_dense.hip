@@ -1296,14 +1296,10 @@ static int dense_bwd_launch(const DensePlan& P, const void* q, const void* k, co
   hipLaunchKernelGGL((dense_bwd_dq_kernel<D>), dim3(P.mode == 0 ? xcd_grid_for((P.n + qpw - 1) / qpw) : (unsigned)((P.n + qpw - 1) / qpw), P.bh), dim3(256), 0, st, P, (const __bf16*)q, (const __bf16*)k,
                      (const __bf16*)v, (const __bf16*)out, (const __bf16*)dout, lse, delta, (__bf16*)dq);      // also writes delta
   NSA_LAUNCH_CHECK();
-  const auto group_span = [&](const long* st) { return (long)(P.g - 1) * st[1] + (long)(P.n - 1) * st[2] + D; };
-  // buffer loads with 32-bit byte offsets within one kv head's query heads (rows) and their lse / delta
-  const bool near = D == 128 && group_span(P.sq) < (1l << 30) && group_span(P.sdo) < (1l << 30) && (long)P.g * P.n < (1l << 29);
-  // (the keys walk masks scores before they are scaled, and requests a tile's 64 rows of k / v from one base)
-  if (near && P.keys_walk && P.scale > 0.f && P.sk[2] < (1l << 24) && P.sv[2] < (1l << 24))
+  if (P.keys_walk)
     hipLaunchKernelGGL(dense_bwd_dkv_keys_kernel, dim3(dkv_grid(P), P.bh), dim3(256), 0, st, P, (const __bf16*)q, (const __bf16*)k,
                        (const __bf16*)v, (const __bf16*)dout, delta, part);
-  else if (near)
+  else if (P.near)
     hipLaunchKernelGGL((dense_bwd_dkv_pipe_kernel<128>), dim3(dkv_grid(P), P.bh), dim3(128), 0, st, P, (const __bf16*)q, (const __bf16*)k,
                        (const __bf16*)v, (const __bf16*)dout, lse, delta, part);
   else

@@ -17,7 +17,8 @@ struct DensePlan {
   int accumulate;            // the backward adds to what dq, dk and dv (bf16) hold
   float scale;
   int key_tiles, chunks, chunk_q;
-  int keys_walk;             // dK / dV by dense_bwd_dkv_keys_kernel (strides and scale allowing)
+  int near;                  // 32-bit byte offsets reach a kv head's Q and d_out rows (asked at 128 features)
+  int keys_walk;             // dK / dV by dense_bwd_dkv_keys_kernel
   long sq[3], sk[3], sv[3], so[3], sdo[3];
   size_t off_delta, off_part, bwd_total;
 };
@@ -72,10 +73,13 @@ static inline int make_dense_plan(const nsa_dense_desc* d, DensePlan& P) {
   // are cut into chunks of chunk_q; smaller chunks when there would be too few work-groups
   P.key_tiles = (P.krows + 63) / 64;
   const long span = P.mode == 0 ? ((long)64 + P.wb + P.wf < P.n ? (long)64 + P.wb + P.wf : P.n) : P.n;
+  const auto group_span = [&](const long* st) { return (long)(P.g - 1) * st[1] + (long)(P.n - 1) * st[2] + P.D; };
+  P.near = P.D == 128 && group_span(P.sq) < (1l << 30) && group_span(P.sdo) < (1l << 30) && (long)P.g * P.n < (1l << 29);
   // At 128 features the keys walk, one work-group of it a CU, except for bands whose tiles few rows see: from 640 rows a tile on it is the
   // faster one (dq + dK / dV, 2 x 8 heads, 8192 tokens, window 128: 192 rows, 169 us by the pipelined walk, 190 by the keys walk; window 512:
-  // 576 rows, 251 and 255; 32 / 8 heads, 8192 tokens, window 512: 2304 rows, 402 and 358).
-  P.keys_walk = P.D == 128 && (P.mode == 1 || span * P.g >= 640);
+  // 576 rows, 251 and 255; 32 / 8 heads, 8192 tokens, window 512: 2304 rows, 402 and 358).  It masks scores before they are scaled, and
+  // requests a tile's 64 rows of k / v from one base.
+  P.keys_walk = P.near && (P.mode == 1 || span * P.g >= 640) && P.scale > 0.f && P.sk[2] < (1l << 24) && P.sv[2] < (1l << 24);
   const auto groups = [&] { return bh * P.key_tiles * ((span + P.chunk_q - 1) / P.chunk_q); };
   if (P.mode == 0) {
     // band: a tile's visible queries (64 + window of them) in equal chunks, as few as give the chip so many work-groups
