@@ -917,9 +917,9 @@ __global__ __launch_bounds__(128) void dense_bwd_dkv_kernel(const DensePlan P, c
     }
 }
 
-// The same walk for 128 features and bands whose tiles few rows see (more rows: dense_bwd_dkv_keys_kernel).  The accumulators leave room for
-// one wave per SIMD only (128 registers of dK / dV
-// accumulators, 64 of K / V operands).  With one wave per SIMD nothing overlaps a wave's MFMAs but its own instruction order,
+// The same walk for 128 features where dense_bwd_dkv_keys_kernel does not take it: bands whose tiles few rows see, k / v rows far apart, a
+// scale that is not positive.  The accumulators leave room for one wave per SIMD only (128 registers of dK / dV accumulators, 64 of K / V
+// operands).  With one wave per SIMD nothing overlaps a wave's MFMAs but its own instruction order,
 // so the step is laid out by hand and fenced (cycle stamps of the kernel above at d = 128: 23 % of a step in the tile's LDS
 // write, 11 % in two barriers, 6 % issuing loads, and the softmax entirely outside the MFMA runs):
 //   * the tile's arithmetic is six runs of MFMAs in dependency order - S = Q K^T, dP = dO V^T, dV from rows 0-15, dV from rows
@@ -928,12 +928,11 @@ __global__ __launch_bounds__(128) void dense_bwd_dkv_kernel(const DensePlan P, c
 //   * the Q / dO tile is double-buffered in LDS: the next tile goes from its staging registers to the other buffer beside the
 //     S MFMAs, each row's staging register is reloaded with the tile after that right behind its store, and one barrier per
 //     step is left, which stands before the last run (see the loop).
-template <int D>
 __global__ __launch_bounds__(128) void dense_bwd_dkv_pipe_kernel(const DensePlan P, const __bf16* __restrict__ q, const __bf16* __restrict__ k,
                                                                  const __bf16* __restrict__ v, const __bf16* __restrict__ dout,
                                                                  const float* __restrict__ lse, const float* __restrict__ delta,
                                                                  float* __restrict__ part) {
-  constexpr int KS = D / 16, DT = D / 32, RS = D + 8;
+  constexpr int D = 128, KS = D / 16, DT = D / 32, RS = D + 8;
   __shared__ __align__(16) float lse_s[2][32];
   __shared__ __align__(16) float del_s[2][32];
   __shared__ __align__(16) int lo_s[2][32];
@@ -1030,7 +1029,7 @@ __global__ __launch_bounds__(128) void dense_bwd_dkv_pipe_kernel(const DensePlan
     if (ktu == 0) {
       if (h == 0) {
         lse_s[buf][n_] = i0 + pq < c1 ? lse_r * kLog2e : INFINITY;   // +inf: a padding row gets p = 0
-        del_s[buf][n_] = D == 128 ? -del_r : del_r;
+        del_s[buf][n_] = -del_r;
       }
     } else if (!whole_tile_visible(i0)) {
       if (h == 0) {
@@ -1302,7 +1301,7 @@ static int dense_bwd_launch(const DensePlan& P, const void* q, const void* k, co
     hipLaunchKernelGGL(dense_bwd_dkv_keys_kernel, dim3(dkv_grid(P), P.bh), dim3(256), 0, st, P, (const __bf16*)q, (const __bf16*)k,
                        (const __bf16*)v, (const __bf16*)dout, delta, part);
   else if (P.near)
-    hipLaunchKernelGGL((dense_bwd_dkv_pipe_kernel<128>), dim3(dkv_grid(P), P.bh), dim3(128), 0, st, P, (const __bf16*)q, (const __bf16*)k,
+    hipLaunchKernelGGL(dense_bwd_dkv_pipe_kernel, dim3(dkv_grid(P), P.bh), dim3(128), 0, st, P, (const __bf16*)q, (const __bf16*)k,
                        (const __bf16*)v, (const __bf16*)dout, lse, delta, part);
   else
     hipLaunchKernelGGL((dense_bwd_dkv_kernel<D>), dim3(dkv_grid(P), P.bh), dim3(128), 0, st, P, (const __bf16*)q, (const __bf16*)k,

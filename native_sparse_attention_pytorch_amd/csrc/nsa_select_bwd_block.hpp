@@ -25,17 +25,6 @@
 
 namespace nsa {
 
-// x / d for x < 2^31 (Granlund and Montgomery 1994): high word of 2 x * mul, shifted right by sh
-struct SmallDiv {
-  unsigned mul;
-  int sh;
-};
-static inline SmallDiv small_div(int d) {
-  int l = 0;
-  while ((1 << l) < d) ++l;
-  return {(unsigned)((((unsigned long)1 << (31 + l)) + d - 1) / d), l};
-}
-
 struct BlockArgs {
   SelPlan P;
   SmallDiv by_sp;

@@ -8,7 +8,8 @@
 // (4.3 GB of partial rows and their 4-byte lse's, 0.12 ms of it the latter) set the pace.  2048 tokens 77 -> 58 us; d 64, 16 / 4 heads:
 // 8192 tokens 86 -> 82 us, 4 x 4096 138 -> 130.
 #pragma once
-#include "nsa_select_bwd_block.hpp"
+#include "nsa_pipe.hpp"
+#include "nsa_select_plan.hpp"
 
 namespace nsa {
 

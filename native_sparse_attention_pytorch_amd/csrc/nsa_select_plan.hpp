@@ -45,6 +45,17 @@ struct SelPlan {
   int block_walk;            // the backward walk without gate gradients is sel_bwd_block_kernel
 };
 
+// x / d for x < 2^31 (Granlund and Montgomery 1994): high word of 2 x * mul, shifted right by sh
+struct SmallDiv {
+  unsigned mul;
+  int sh;
+};
+static inline SmallDiv small_div(int d) {
+  int l = 0;
+  while ((1 << l) < d) ++l;
+  return {(unsigned)((((unsigned long)1 << (31 + l)) + d - 1) / d), l};
+}
+
 static inline size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 static inline int make_plan(const nsa_select_desc* d, SelPlan& P) {
