@@ -25,19 +25,19 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 MFMA_PEAK_TFLOPS = 2500.0      # MI355X dense bf16
-HBM_PEAK_GBS = 8000.0
 
 CFG = dict(batch=1, seq=32768, heads=32, kv_heads=8, dim_head=128, block=64, num_sel=15)
 
-# HBM bytes per launch on this workload come from the tracked rocprofv3 summary (FETCH_SIZE / WRITE_SIZE per dispatch,
-# scaled by streaming kernels of known size; the file states the commands), not from literals kept here
+# Bytes per launch on this workload between L2 and the memory side (HBM and the 256 MB cache in front of it: rows which that serves are in
+# them) come from the tracked rocprofv3 summary (FETCH_SIZE / WRITE_SIZE per dispatch, scaled by streaming kernels of known size; the file
+# states the commands), not from literals kept here
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "select_fwd_bwd_seq32k_hbm_traffic.txt")
 TRAFFIC_KERNELS = {"sel_fwd_rows_kernel": "fwd_block_walk", "sel_fwd_combine_kernel": "fwd_merge", "sel_bwd_dq_combine_kernel": "bwd_dq_merge",
                    "sel_bwd_block_kernel": "bwd_dkv_walk", "sel_bwd_dkv_reduce_kernel": "bwd_dkv_reduce", "sel_delta_kernel": "bwd_delta"}
 
 
 def measured_traffic_bytes():
-    """{bench kernel name: HBM bytes per launch} from the summary's table (columns: kernel, raw counters, fetch_GB, write_GB,
+    """{bench kernel name: bytes per launch behind L2} from the summary's table (columns: kernel, raw counters, fetch_GB, write_GB,
     total_GB); empty when the file is missing."""
     out = {}
     try:
@@ -63,16 +63,16 @@ def selection(b, h, n, B, S, seed, device):
     return idx.masked_fill(~mask, 0).contiguous(), mask.contiguous()
 
 
-def ceiling_bytes(cfg, rows_per_pair=7):
-    """HBM bytes per step that the block-major walk cannot avoid: per live (query, kv head, slot) pair G*d bf16 of Q (forward)
-    and of Q and dO (backward), one G*d bf16 partial written and read again in each direction (7 rows); plus every tensor
-    once.  rows_per_pair=4 counts the partial exchange alone (as if every gather hit a cache)."""
+def exchange_bytes(cfg):
+    """Bytes per step that must cross HBM in a block-major walk: per live (query, kv head, slot) pair one G*d bf16 partial written and read
+    again in each direction - what is written between is far larger than any cache - and every tensor once.  (The three gathered rows a
+    pair, Q in the forward, Q and dO in the backward, come from a set that the memory-side cache holds.)"""
     b, n, hq, hk, d, B, S = cfg["batch"], cfg["seq"], cfg["heads"], cfg["kv_heads"], cfg["dim_head"], cfg["block"], cfg["num_sel"]
     W = math.ceil(n / B)
     pairs = b * hk * sum(B * (min(w, S) + 1) for w in range(W))
     row = (hq // hk) * d * 2
     once = (4 * b * hq * n * d + 6 * b * hk * n * d) * 2            # q, out, dO, dq; k, v, dk, dv (k, v read twice)
-    return pairs * row * rows_per_pair + once
+    return pairs * row * 4 + once
 
 
 def attended_pairs(b, hq, n, B, s_total):
@@ -272,16 +272,12 @@ def main():
     roofline = dict(bound="mfma", kernel=dom, achieved=round(achieved, 2), peak=MFMA_PEAK_TFLOPS, unit="TFLOP/s",
                     frac=round(achieved / MFMA_PEAK_TFLOPS, 4), traffic=traffic,
                     step_frac=round(value / MFMA_PEAK_TFLOPS, 4),
-                    # what this selection law allows at any kernel quality: a (query, block) pair's partial results must cross
-                    # HBM (2 KB written + 2 KB read per pair, forward and backward together) and its Q / dO rows be gathered
-                    # (3 KB); at the rate the memory system gives that access pattern (measured by the rowtraffic leg: ~5.3 TB/s
-                    # mixed gather / scatter, ~6 TB/s streams) the step cannot be shorter than those bytes take
-                    ceiling_frac=round(total_flop / (ceiling_bytes(cfg) / 5.5e12) / 1e12 / MFMA_PEAK_TFLOPS, 4),
-                    # the same with the exchange of partials alone (4 KB per pair at the 6 TB/s of plain streams)
-                    ceiling_exchange_only_frac=round(total_flop / (ceiling_bytes(cfg, 4) / 6.0e12) / 1e12 / MFMA_PEAK_TFLOPS, 4),
-                    # the kernels are HBM-bound in practice: measured bytes / measured time against 8 TB/s
-                    hbm_GBs={nm: round(traffic_all[nm] / (kern[nm] * 1e-3) / 1e9, 1) for nm in traffic_all},
-                    hbm_frac_step=round(sum(traffic_all.values()) / (ms_step * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if traffic_all else None,
+                    # what this selection law allows at any kernel quality: a pair's partial results cross HBM (4 KB, written and
+                    # read, forward and backward together) at the 6 TB/s that plain streams reach
+                    ceiling_exchange_only_frac=round(total_flop / (exchange_bytes(cfg) / 6.0e12) / 1e12 / MFMA_PEAK_TFLOPS, 4),
+                    # measured bytes behind L2 over measured time, to read beside the rowtraffic leg's rates
+                    behind_l2_GBs={nm: round(traffic_all[nm] / (kern[nm] * 1e-3) / 1e9, 1) for nm in traffic_all},
+                    behind_l2_GBs_step=round(sum(traffic_all.values()) / (ms_step * 1e-3) / 1e9, 1) if traffic_all else None,
                     traffic_source=os.path.relpath(TRAFFIC_SUMMARY, ROOT))
 
     res = dict(metric="NSA selection-attention fwd+bwd TFLOP/s at seq 32k (bf16)", value=round(value, 2), unit="TFLOP/s",
@@ -525,7 +521,7 @@ def main():
         res["generate_config5_bf16"] = dict(error=repr(ex))
 
     # what the memory system gives the walks' access pattern (random 1 KB rows, loads of a round in flight together): the
-    # ceiling to read the hbm_GBs figures against.  2 GB buffers = HBM; a 2 MB source = rows that stay in L2.
+    # rates to read the behind_l2_GBs figures against.  2 GB buffers = HBM; a 2 MB source = rows that stay in L2.
     try:
         leg("rowtraffic")
         big = 2 << 30
@@ -536,7 +532,9 @@ def main():
         for name, sr, rd, wr in (("gather_hbm", rows_big, 2, 0), ("scatter_hbm", rows_big, 0, 2), ("gather1_scatter1_hbm", rows_big, 1, 1),
                                  ("gather2_scatter1_hbm", rows_big, 2, 1), ("gather1_scatter2_hbm", rows_big, 1, 2),
                                  ("gather_l2_scatter_hbm", 2048, 1, 1),
-                                 # a gather set that fits the 256 MB memory-side cache (the Q and dO rows of one kv head at 32k: 134 MB)
+                                 # gather sets that fit the 256 MB memory-side cache: the Q rows of one kv head at 32k (forward walk), its Q and
+                                 # dO rows (backward walk), twice that
+                                 ("gather_32MB_scatter_hbm", (32 << 20) // 1024, 1, 1), ("gather2_64MB_scatter1_hbm", (64 << 20) // 1024, 2, 1),
                                  ("gather2_128MB_scatter1_hbm", (128 << 20) // 1024, 2, 1), ("gather_128MB", (128 << 20) // 1024, 2, 0)):
             best = None
             for rep in range(4):
